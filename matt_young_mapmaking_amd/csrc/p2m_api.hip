@@ -22,15 +22,17 @@
 #include "../../include/pks2map_gpu.h"
 #include "p2m_kernels.h"
 
-/* Scratch of p2m_products_noalloc: one array per GPU, kept for the life of
- * the process.  Layout: 8 doubles of partial sums, the 10000-bin dP/dy
- * histogram (u64), the cumulative dP/dy (float).  Its device address comes
- * from hipGetSymbolAddress once per device (the array's name is a host-side
- * stand-in in host code). */
+/* Scratch of the map products: the 10000-bin dP/dy histogram (u64), then the
+ * workgroups' partial sums of one map.  p2m_products keeps one per context;
+ * p2m_products_noalloc uses one array per GPU, kept for the life of the
+ * process, whose device address comes from hipGetSymbolAddress once per
+ * device (the array's name is a host-side stand-in in host code). */
+#define P2M_NDPDY 10000
 #define P2M_NOALLOC_BYTES (128 * 1024)
-#define P2M_NOALLOC_HIST_OFF 64
-#define P2M_NOALLOC_DPDY_OFF (64 + 8 * 10000)
-static_assert(P2M_NOALLOC_DPDY_OFF + 4 * 10000 <= P2M_NOALLOC_BYTES, "no-alloc scratch layout");
+#define P2M_PROD_PART_OFF (8 * P2M_NDPDY)
+#define P2M_PROD_PART_BYTES (8 * P2M_MOM_PART * P2M_MOM_BLOCKS)
+#define P2M_PROD_BYTES (P2M_PROD_PART_OFF + P2M_PROD_PART_BYTES)
+static_assert(P2M_PROD_BYTES <= P2M_NOALLOC_BYTES, "no-alloc scratch layout");
 static __device__ __align__(256) unsigned char scratch[P2M_NOALLOC_BYTES];
 static std::mutex g_scratch_mu;
 static void *g_scratch_ptr[64];
@@ -90,6 +92,8 @@ struct p2m_ctx {
     hipStream_t fs_stream = nullptr;            /* the flat-sky painter, beside the binning */
     hipEvent_t ev_dec = nullptr, ev_fs = nullptr;
     unsigned long long *h_pin = nullptr;   /* pinned host words for mid-call readbacks */
+    char *h_prod = nullptr;                /* pinned host copy of the products' scratch */
+    char *d_prod = nullptr;                /* the products' scratch */
     bool have_run = false;
     bool have_table[P2M_MAXMAPS] = {false};
     p2m_run run;
@@ -335,6 +339,10 @@ int p2m_create(p2m_ctx **out, const p2m_config *cfg)
         (void)hipGetLastError();
         c->h_pin = nullptr;
     }
+    if (hipHostMalloc((void **)&c->h_prod, P2M_PROD_BYTES + P2M_PROD_PART_BYTES, hipHostMallocDefault) != hipSuccess) {
+        (void)hipGetLastError();
+        c->h_prod = nullptr;
+    }
     c->hpnpix = cfg->nside > 0 ? 12LL * cfg->nside * cfg->nside : 0;
     c->fsnpix = (int64_t)cfg->npix_fs * cfg->npix_fs;
     int rc = 0;
@@ -356,6 +364,7 @@ int p2m_create(p2m_ctx **out, const p2m_config *cfg)
         }
     }
     if (!rc) rc |= dmalloc((void **)&c->d_ctr, sizeof(unsigned long long) * Ctr::ALL);
+    if (!rc) rc |= dmalloc((void **)&c->d_prod, P2M_PROD_BYTES);
     if (rc) { p2m_destroy(c); return P2M_E_NOMEM; }
     *out = c;
     int e = p2m_clear(c);
@@ -391,6 +400,8 @@ void p2m_destroy(p2m_ctx *c)
     dfree(c->d_halo_s); dfree(c->d_hot); dfree(c->d_bin); dfree(c->d_keys); dfree(c->d_vals); dfree(c->d_sort_tmp);
     for (int i = 0; i < 10; ++i) if (c->ev[i]) (void)hipEventDestroy(c->ev[i]);
     if (c->h_pin) (void)hipHostFree(c->h_pin);
+    if (c->h_prod) (void)hipHostFree(c->h_prod);
+    dfree(c->d_prod);
     if (c->ev_dec) (void)hipEventDestroy(c->ev_dec);
     if (c->ev_fs) (void)hipEventDestroy(c->ev_fs);
     if (c->fs_stream) (void)hipStreamDestroy(c->fs_stream);
@@ -1380,63 +1391,79 @@ static int autotune(p2m_ctx *c, int64_t n_halo, int64_t n_flat, unsigned long lo
 }
 
 /* ------------------------------------------------------------------ products + writers */
-extern "C" {
 
-int p2m_products(p2m_ctx *c, int slot, double moments[6], double rms[2], float dpdy[10000])
+/* Moments, RMS and dP/dy of one slot's maps, each map read once; the sums
+ * and the histogram go through `scratch` (P2M_PROD_BYTES of device memory)
+ * and one pinned copy, with one wait for the painter's stream. */
+static int products(p2m_ctx *c, int slot, char *scratch, double moments[6], double rms[2], float *dpdy)
 {
     if (!c) return P2M_E_INVALID;
     if (c->in_stream) return P2M_E_STATE;
     if (slot < 0 || slot >= c->cfg.n_maps) return P2M_E_INVALID;
     HIPCHK(hipSetDevice(c->cfg.device));
     { int rc = ensure_hp_valid(c); if (rc) return rc; }
-    double *d_out = nullptr;
-    unsigned long long *d_hist = nullptr;
-    if (dmalloc((void **)&d_out, sizeof(double) * 8)) return P2M_E_NOMEM;
-    if (dmalloc((void **)&d_hist, sizeof(unsigned long long) * 10000)) { dfree(d_out); return P2M_E_NOMEM; }
-    double res[2][4] = {{0}};
-    const int ndpdy = 10000;
-    const float dy = 1e-4f / (float)ndpdy;                 /* pks2map.f90:39-40 */
-    int rc = 0;
-    for (int which = 0; which < 2 && !rc; ++which) {
-        int64_t n = which == 0 ? c->fsnpix : c->hpnpix;
-        if (n <= 0) continue;
-        const float *m32 = which == 1 ? c->d_hp32[slot] : nullptr;
-        const double *m64 = which == 1 ? c->d_hp64[slot] : c->d_fs64[slot];
-        if (m32) m64 = nullptr;
-        p2m_launch_fill_f64(d_out, 8, c->stream);
-        if (which == 1) p2m_launch_fill_u64(d_hist, ndpdy, c->stream);
-        p2m_launch_moments(m32, m64, n, 0.0, d_out, which == 1 ? d_hist : nullptr, ndpdy, dy, c->stream);
-        double h1[8];
-        if (hipMemcpyAsync(h1, d_out, sizeof(h1), hipMemcpyDeviceToHost, c->stream) != hipSuccess ||
-            hipStreamSynchronize(c->stream) != hipSuccess) { rc = P2M_E_HIP; break; }
-        double mean = h1[0] / (double)n;
-        p2m_launch_fill_f64(d_out, 8, c->stream);
-        p2m_launch_moments(m32, m64, n, mean, d_out, nullptr, ndpdy, dy, c->stream);
-        double h2[8];
-        if (hipMemcpyAsync(h2, d_out, sizeof(h2), hipMemcpyDeviceToHost, c->stream) != hipSuccess ||
-            hipStreamSynchronize(c->stream) != hipSuccess) { rc = P2M_E_HIP; break; }
-        res[which][0] = h1[0] / (double)n; res[which][1] = h1[1] / (double)n; res[which][2] = h1[2] / (double)n;
-        res[which][3] = p2m_sqrt(h2[3] / (double)n);
-        if (which == 1 && dpdy) {
-            std::vector<unsigned long long> hist(ndpdy);
-            if (hipMemcpy(hist.data(), d_hist, sizeof(unsigned long long) * ndpdy, hipMemcpyDeviceToHost) != hipSuccess) {
-                rc = P2M_E_HIP; break;
-            }
-            /* dpdy = dpdy / real(hpnpix); cumulative (pks2map.f90:347, 355-357) */
-            for (int i = 0; i < ndpdy; ++i) dpdy[i] = (float)hist[i] / (float)n;
-            for (int i = 1; i < ndpdy; ++i) dpdy[i] = dpdy[i - 1] + dpdy[i];
-        }
+    char hbuf[P2M_PROD_BYTES + P2M_PROD_PART_BYTES];
+    char *h = c->h_prod ? c->h_prod : hbuf;
+    unsigned long long *d_hist = (unsigned long long *)scratch;
+    double *d_part = (double *)(scratch + P2M_PROD_PART_OFF);
+    const float dy = 1e-4f / (float)P2M_NDPDY;                 /* pks2map.f90:39-40 */
+    const int64_t n[2] = {c->fsnpix, c->hpnpix};
+    const char *hpart[2] = {h + P2M_PROD_BYTES, h + P2M_PROD_PART_OFF};
+    if (n[0] > 0) {
+        p2m_launch_moments(nullptr, c->d_fs64[slot], n[0], d_part, nullptr, P2M_NDPDY, dy, c->stream);
+        HIPCHK(hipGetLastError());
+        HIPCHK(hipMemcpyAsync(h + P2M_PROD_BYTES, d_part, P2M_PROD_PART_BYTES, hipMemcpyDeviceToHost, c->stream));
     }
-    dfree(d_out); dfree(d_hist);
-    if (rc) return rc;
+    if (n[1] > 0) {
+        /* the scratch keeps the last call's contents: cleared by a fill kernel */
+        if (dpdy) p2m_launch_fill_u64(d_hist, P2M_NDPDY, c->stream);
+        p2m_launch_moments(c->d_hp32[slot], c->d_hp64[slot], n[1], d_part, dpdy ? d_hist : nullptr, P2M_NDPDY, dy,
+                           c->stream);
+        HIPCHK(hipGetLastError());
+        HIPCHK(hipMemcpyAsync(h, scratch, P2M_PROD_BYTES, hipMemcpyDeviceToHost, c->stream));
+    }
+    HIPCHK(hipStreamSynchronize(c->stream));
+    double res[2][4] = {{0}};
+    for (int which = 0; which < 2; ++which) {
+        if (n[which] <= 0) continue;
+        const double *p = (const double *)hpart[which];
+        const int64_t chunk = p2m_moments_chunk(n[which]);
+        const int64_t nb = (n[which] + chunk - 1) / chunk;
+        const double dn = (double)n[which];
+        double s[3] = {0, 0, 0};
+        for (int64_t b = 0; b < nb; ++b)
+            for (int k = 0; k < 3; ++k) s[k] += p[b * P2M_MOM_PART + k];
+        const double mean = s[0] / dn;
+        double sq = 0.0;
+        for (int64_t b = 0; b < nb; ++b) {
+            const double cnt = (double)(b + 1 < nb ? chunk : n[which] - b * chunk);
+            const double d = p[b * P2M_MOM_PART + 3] - mean;
+            sq += p[b * P2M_MOM_PART + 4] + cnt * (d * d);
+        }
+        for (int k = 0; k < 3; ++k) res[which][k] = s[k] / dn;
+        res[which][3] = p2m_sqrt(sq / dn);
+    }
+    if (n[1] > 0 && dpdy) {
+        /* dpdy = dpdy / real(hpnpix); cumulative, in float and in order (pks2map.f90:347, 355-357) */
+        const unsigned long long *hist = (const unsigned long long *)h;
+        for (int i = 0; i < P2M_NDPDY; ++i) dpdy[i] = (float)hist[i] / (float)n[1];
+        for (int i = 1; i < P2M_NDPDY; ++i) dpdy[i] = dpdy[i - 1] + dpdy[i];
+    }
     if (moments) { for (int k = 0; k < 3; ++k) { moments[k] = res[0][k]; moments[3 + k] = res[1][k]; } }
     if (rms) { rms[0] = res[0][3]; rms[1] = res[1][3]; }
     return 0;
 }
 
-/* p2m_products without any allocation: the same kernels with the partial
- * sums, the histogram and the cumulative dP/dy in this device's scratch array.
- * Calls that overlap on one GPU share that array and race. */
+extern "C" {
+
+int p2m_products(p2m_ctx *c, int slot, double moments[6], double rms[2], float dpdy[10000])
+{
+    if (!c) return P2M_E_INVALID;
+    return products(c, slot, c->d_prod, moments, rms, dpdy);
+}
+
+/* The same in this device's process-wide scratch array; calls that overlap
+ * on one GPU share that array and race. */
 int p2m_products_noalloc(p2m_ctx *c, int slot, double moments[6], double rms[2], float dpdy[10000])
 {
     if (!c) return P2M_E_INVALID;
@@ -1445,44 +1472,7 @@ int p2m_products_noalloc(p2m_ctx *c, int slot, double moments[6], double rms[2],
     HIPCHK(hipSetDevice(c->cfg.device));
     void *base = nullptr;
     { int rc = scratch_for_device(c->cfg.device, &base); if (rc) return rc; }
-    double *d_out = (double *)base;
-    unsigned long long *d_hist = (unsigned long long *)((char *)base + P2M_NOALLOC_HIST_OFF);
-    float *d_dp = (float *)((char *)base + P2M_NOALLOC_DPDY_OFF);
-    { int rc = ensure_hp_valid(c); if (rc) return rc; }
-    double res[2][4] = {{0}};
-    const int ndpdy = 10000;
-    const float dy = 1e-4f / (float)ndpdy;                 /* pks2map.f90:39-40 */
-    for (int which = 0; which < 2; ++which) {
-        const int64_t n = which == 0 ? c->fsnpix : c->hpnpix;
-        if (n <= 0) continue;
-        const float *m32 = which == 1 ? c->d_hp32[slot] : nullptr;
-        const double *m64 = which == 1 ? c->d_hp64[slot] : c->d_fs64[slot];
-        if (m32) m64 = nullptr;
-        /* the scratch keeps the last call's contents: cleared by fill kernels */
-        p2m_launch_fill_f64(d_out, 8, c->stream);
-        if (which == 1) p2m_launch_fill_u64(d_hist, ndpdy, c->stream);
-        p2m_launch_moments(m32, m64, n, 0.0, d_out, which == 1 ? d_hist : nullptr, ndpdy, dy, c->stream);
-        double h1[8];
-        HIPCHK(hipMemcpyAsync(h1, d_out, sizeof(h1), hipMemcpyDeviceToHost, c->stream));
-        HIPCHK(hipStreamSynchronize(c->stream));
-        const double mean = h1[0] / (double)n;
-        p2m_launch_fill_f64(d_out, 8, c->stream);
-        p2m_launch_moments(m32, m64, n, mean, d_out, nullptr, ndpdy, dy, c->stream);
-        double h2[8];
-        HIPCHK(hipMemcpyAsync(h2, d_out, sizeof(h2), hipMemcpyDeviceToHost, c->stream));
-        HIPCHK(hipStreamSynchronize(c->stream));
-        res[which][0] = h1[0] / (double)n; res[which][1] = h1[1] / (double)n; res[which][2] = h1[2] / (double)n;
-        res[which][3] = p2m_sqrt(h2[3] / (double)n);
-        if (which == 1 && dpdy) {
-            p2m_launch_dpdy_cumulative(d_hist, ndpdy, (float)n, d_dp, c->stream);
-            HIPCHK(hipGetLastError());
-            HIPCHK(hipMemcpyAsync(dpdy, d_dp, sizeof(float) * ndpdy, hipMemcpyDeviceToHost, c->stream));
-            HIPCHK(hipStreamSynchronize(c->stream));
-        }
-    }
-    if (moments) { for (int k = 0; k < 3; ++k) { moments[k] = res[0][k]; moments[3 + k] = res[1][k]; } }
-    if (rms) { rms[0] = res[0][3]; rms[1] = res[1][3]; }
-    return 0;
+    return products(c, slot, (char *)base, moments, rms, dpdy);
 }
 
 }  /* extern "C" */

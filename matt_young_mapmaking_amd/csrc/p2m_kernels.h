@@ -184,9 +184,11 @@ size_t p2m_tile_lds_bytes(int mode, int n_maps, int log2w, int membership, int n
 int p2m_tile_occupancy(int mode, int n_maps, int wg, size_t lds);
 int p2m_launch_tile_paint(const TileArgs &a, int mode, int n_maps, int grid, int wg, hipStream_t s);
 int p2m_launch_fallback(const FallbackArgs &a, int64_t n_max, hipStream_t s);
-void p2m_launch_moments(const float *m32, const double *m64, int64_t n, double mean, double *out,
-                        unsigned long long *hist, int nb, float dy, hipStream_t s);
-void p2m_launch_dpdy_cumulative(const unsigned long long *hist, int nb, float npix, float *dpdy, hipStream_t s);
+#define P2M_MOM_BLOCKS 256       /* most workgroups of the moments kernel */
+#define P2M_MOM_PART 5           /* doubles each writes: sums of x, x^2, x^3, its mean, squares about it */
+int64_t p2m_moments_chunk(int64_t n);
+void p2m_launch_moments(const float *m32, const double *m64, int64_t n, double *part, unsigned long long *hist, int nb,
+                        float dy, hipStream_t s);
 void p2m_launch_f64_to_f32(const double *in, float *out, int64_t n, hipStream_t s);
 void p2m_launch_f32_to_f64(const float *in, double *out, int64_t n, hipStream_t s);
 
