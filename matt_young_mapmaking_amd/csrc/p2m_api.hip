@@ -75,11 +75,12 @@ namespace {
 
 const double CKMS = 2.99792458e10 / 1e5;   /* cosmology.f90:23 */
 
-struct Ctr {                 /* layout of one shard row of the device counter block; OVF is
-                                the paint counter (PAINT + OVF, shard 0 only) of binning
-                                overflow-list entries; ERR counts failed device-side range
+struct Ctr {                 /* layout of one shard row of the device counter block; PAIRS, GAPS and
+                                PIX are the decode's (halo, tile) pairs, halos that may have a ring
+                                gap and disc pixels (about);
+                                ERR counts failed device-side range
                                 checks, LOST the tiles marked for the repaint pass */
-    enum { ERR = 0, DEC = 1, LOST = 2, ITEMS = 4, N_FLAT = 5, N_CAND = 6, N_CAND0 = 7, PAINT = 8, OVF = 7,
+    enum { ERR = 0, DEC = 1, LOST = 2, PAIRS = 4, N_FLAT = 5, N_CAND = 6, N_CAND0 = 7, PAINT = 8, GAPS = 11, PIX = 15,
            TOTAL = P2M_CTR_STRIDE, ALL = P2M_CTR_STRIDE * P2M_SHARDS };
 };
 
@@ -125,37 +126,33 @@ struct p2m_ctx {
     bool hp_valid = true;       /* device HEALPix arrays hold the map (false after a lazy clear) */
     HaloRec *d_halo = nullptr;
     uint32_t *d_flat_idx = nullptr;
-    uint32_t *d_nr = nullptr;
-    unsigned long long *d_ring_off = nullptr;
-    uint32_t *d_runs = nullptr, *d_pos = nullptr;   /* per (halo, ring) item: run, first piece's slot */
-    int64_t runs_cap = 0;
-    uint4 *d_ovf = nullptr;                       /* pieces beyond an item's second */
-    int64_t ovf_cap = 0;
+    PairHalo *d_pair_halo = nullptr;              /* what the binning reads of a halo (tiled painters) */
+    TileHalo *d_hot = nullptr;                    /* what the FP32 painter stages of it */
+    uint32_t *d_n_pairs = nullptr;                /* tiles per halo, and their scan */
+    unsigned long long *d_pair_off = nullptr;
+    uint32_t *d_keys = nullptr, *d_vals = nullptr;  /* (halo, tile) pairs: as listed, then sorted by tile */
+    int64_t pair_cap = 0;
+    int counted_log2w = 0;                        /* the tile shape that n_pairs were counted at, and their sum */
+    unsigned long long counted_pairs = 0;
+    bool ask_gaps = false;                        /* the decode marked halos that may have a ring gap */
     int64_t halo_cap = 0;
     unsigned long long *d_ctr = nullptr;
     int log2w = 0, wg = 0;
     bool tuned = false;
-    std::vector<int32_t> tile_base;
-    int32_t *d_tile_base = nullptr;
-    int32_t *d_tile_ring = nullptr;
+    TileShape shape = {0, 0, 0};
+    int32_t *d_band_tile = nullptr; /* first tile of each band */
     int n_cu = 0;                   /* compute units of the device */
     TileDesc *d_tile_desc = nullptr;
-    double *d_ring_z = nullptr;     /* ring2z of every ring */
-    uint32_t *d_group = nullptr;    /* halo of every 64th (halo, ring) item */
-    int64_t group_cap = 0;
+    RingDesc *d_ring = nullptr;     /* geometry of every ring */
     uint32_t *d_fs_cnt = nullptr;   /* flat-sky box pixels per listed halo, and their scan */
     unsigned long long *d_fs_off = nullptr;
     int64_t fs_cap = 0;
     int64_t n_tiles = 0;
-    int n_rings = 0;
-    uint32_t *d_tile_cnt = nullptr;
     unsigned long long *d_tile_off = nullptr;
     void *d_scan_tmp = nullptr;
     size_t scan_tmp_bytes = 0;
     void *d_scan_tmp_fs = nullptr;              /* the flat-sky painter's own scan storage */
     size_t scan_tmp_fs_bytes = 0;
-    uint2 *d_segs = nullptr;
-    int64_t seg_cap = 0;
     /* host catalogues: two device slots that pieces of a block are copied
      * into on the copy stream, decoded from on the painter's stream */
     hipStream_t h2d_stream = nullptr;
@@ -171,21 +168,15 @@ struct p2m_ctx {
     /* per tile: 1 if the tile's deferred pixels did not all fit in the list
      * (the tile then wrote nothing and is painted again) */
     uint8_t *d_lost = nullptr;
-    unsigned int *d_tile_next = nullptr;   /* tile-queue counters of the FP32 painter */
+    unsigned int *d_tile_next = nullptr;   /* tile-queue counters */
     int n_redo = 0;
     /* the FP32 painter's last launch, kept for the repaint pass */
     TileArgs last_t;
     FallbackArgs last_f;
     int last_grid = 0;
-    int64_t last_nlisted = 0;
     bool last_fast = false;
     uint32_t *d_cand = nullptr;
     int64_t cand_cap = 0;
-    /* painted halos in spatial order (tiled painters) */
-    BinHalo *d_bin = nullptr;      /* fields the binning reads */
-    TileHalo *d_hot = nullptr;     /* fields the FP32 painter stages (FP32 mode) */
-    HaloRec *d_halo_s = nullptr;   /* full records (FP64 tiled mode) */
-    uint32_t *d_keys = nullptr, *d_vals = nullptr;
     void *d_sort_tmp = nullptr;
     size_t sort_tmp_bytes = 0;
     p2m_stats st;
@@ -221,48 +212,56 @@ static double host_lookup(const std::vector<double> &t, double tmin, double dt, 
 
 static bool is_pow2(int32_t x) { return x > 0 && (x & (x - 1)) == 0; }
 
+/* Rows and columns of a tile of up to 2^log2w pixels: at most 16 rings, 64
+ * pixels along each at the default 1024.  A map of few tiles (nside 128 and
+ * below at that size) takes fewer rings per tile, so that there are tiles for
+ * the CUs. */
+static TileShape tile_shape(int32_t nside, int log2w)
+{
+    TileShape g = {nside, log2w / 2 - 1 < 4 ? log2w / 2 - 1 : 4, 0};
+    g.log2c = log2w - g.log2r;
+    while (g.log2r > 0 && (12LL * nside * nside) >> (g.log2r + g.log2c) < 2048) --g.log2r;
+    return g;
+}
+
 static int build_tiles(p2m_ctx *c, int log2w)
 {
     int32_t ns = c->cfg.nside;
     if (ns <= 0) return 0;
-    if (c->log2w == log2w && c->d_tile_base) return 0;
-    c->n_rings = 4 * ns - 1;
-    c->tile_base.assign(c->n_rings, 0);
+    if (c->log2w == log2w && c->d_tile_desc) return 0;
+    const TileShape g = tile_shape(ns, log2w);
+    const int32_t nb = n_bands(g);
+    std::vector<int32_t> band_tile((size_t)nb + 1);
     int64_t acc = 0;
-    for (int r = 1; r <= c->n_rings; ++r) {
-        c->tile_base[r - 1] = (int32_t)acc;
-        acc += ring_tiles(ns, r, log2w);
+    for (int32_t b = 0; b < nb; ++b) {
+        int32_t r0, r1;
+        band_tile[(size_t)b] = (int32_t)acc;
+        acc += band_sectors(g, b, r0, r1);
     }
+    band_tile[(size_t)nb] = (int32_t)acc;
+    /* a pair's key holds the tile in 24 bits (at most 1.3e7 tiles: 64 pixels, nside 8192) */
+    if (acc >= (1 << 24)) return P2M_E_SIZE;
     c->n_tiles = acc;
-    std::vector<int32_t> tile_ring((size_t)acc);
-    for (int r = 1; r <= c->n_rings; ++r) {
-        const int64_t e = r < c->n_rings ? c->tile_base[r] : acc;
-        for (int64_t t = c->tile_base[r - 1]; t < e; ++t) tile_ring[(size_t)t] = r;
-    }
-    dfree(c->d_tile_base); dfree(c->d_tile_cnt); dfree(c->d_tile_off); dfree(c->d_tile_ring);
-    dfree(c->d_tile_desc); dfree(c->d_lost);
-    c->d_tile_base = nullptr; c->d_tile_cnt = nullptr; c->d_tile_off = nullptr;
-    c->d_tile_ring = nullptr; c->d_tile_desc = nullptr; c->d_lost = nullptr;
+    dfree(c->d_band_tile); dfree(c->d_tile_off); dfree(c->d_tile_desc); dfree(c->d_lost);
+    c->d_band_tile = nullptr; c->d_tile_off = nullptr; c->d_tile_desc = nullptr; c->d_lost = nullptr;
+    c->log2w = 0;
     int rc = 0;
     rc |= dmalloc((void **)&c->d_lost, (size_t)((acc + 3) / 4) * 4);
     if (!c->d_tile_next) rc |= dmalloc((void **)&c->d_tile_next, sizeof(unsigned int) * 8 * P2M_TQ_STRIDE);
-    rc |= dmalloc((void **)&c->d_tile_ring, sizeof(int32_t) * acc);
     rc |= dmalloc((void **)&c->d_tile_desc, sizeof(TileDesc) * acc);
-    rc |= dmalloc((void **)&c->d_tile_base, sizeof(int32_t) * c->n_rings);
-    rc |= dmalloc((void **)&c->d_tile_cnt, sizeof(uint32_t) * (c->n_tiles + 1));
+    rc |= dmalloc((void **)&c->d_band_tile, sizeof(int32_t) * (size_t)(nb + 1));
     rc |= dmalloc((void **)&c->d_tile_off, sizeof(unsigned long long) * (c->n_tiles + 1));
     if (rc) return P2M_E_NOMEM;
-    HIPCHK(hipMemcpy(c->d_tile_base, c->tile_base.data(), sizeof(int32_t) * c->n_rings, hipMemcpyHostToDevice));
-    HIPCHK(hipMemcpy(c->d_tile_ring, tile_ring.data(), sizeof(int32_t) * acc, hipMemcpyHostToDevice));
-    p2m_launch_tile_desc(ns, log2w, acc, c->d_tile_ring, c->d_tile_base, c->d_tile_desc, c->stream);
+    HIPCHK(hipMemcpy(c->d_band_tile, band_tile.data(), sizeof(int32_t) * (size_t)(nb + 1), hipMemcpyHostToDevice));
+    p2m_launch_tile_desc(g, c->d_band_tile, c->d_tile_desc, c->stream);
     p2m_launch_fill_u32((uint32_t *)c->d_lost, (acc + 3) / 4, 0u, c->stream);
     HIPCHK(hipGetLastError());
-    if (!c->d_ring_z) {
-        if (dmalloc((void **)&c->d_ring_z, sizeof(double) * c->n_rings)) return P2M_E_NOMEM;
-        p2m_launch_ring_z(ns, c->d_ring_z, c->stream);
+    if (!c->d_ring) {
+        if (dmalloc((void **)&c->d_ring, sizeof(RingDesc) * (size_t)(4 * ns - 1))) return P2M_E_NOMEM;
+        p2m_launch_ring_desc(ns, c->d_ring, c->stream);
         HIPCHK(hipGetLastError());
     }
-    c->scan_tmp_bytes = 0;
+    c->shape = g;
     c->log2w = log2w;
     return 0;
 }
@@ -393,11 +392,11 @@ void p2m_destroy(p2m_ctx *c)
     dfree(c->d_quad);
     dfree(c->d_count); dfree(c->d_hash); dfree(c->d_fs_count); dfree(c->d_fs_hash);
     dfree(c->d_rofz); dfree(c->d_zofr); dfree(c->d_inv_node2); dfree(c->d_inv_node2f); dfree(c->d_fb);
-    dfree(c->d_halo); dfree(c->d_flat_idx); dfree(c->d_nr); dfree(c->d_ring_off); dfree(c->d_runs); dfree(c->d_pos); dfree(c->d_ovf); dfree(c->d_ctr);
-    dfree(c->d_tile_base); dfree(c->d_tile_cnt); dfree(c->d_tile_off); dfree(c->d_scan_tmp); dfree(c->d_scan_tmp_fs);
-    dfree(c->d_tile_ring); dfree(c->d_tile_desc); dfree(c->d_group); dfree(c->d_ring_z); dfree(c->d_fs_cnt); dfree(c->d_fs_off);
-    dfree(c->d_segs); dfree(c->d_cand);
-    dfree(c->d_halo_s); dfree(c->d_hot); dfree(c->d_bin); dfree(c->d_keys); dfree(c->d_vals); dfree(c->d_sort_tmp);
+    dfree(c->d_halo); dfree(c->d_flat_idx); dfree(c->d_n_pairs); dfree(c->d_pair_off); dfree(c->d_ctr);
+    dfree(c->d_band_tile); dfree(c->d_tile_off); dfree(c->d_scan_tmp); dfree(c->d_scan_tmp_fs);
+    dfree(c->d_tile_desc); dfree(c->d_ring); dfree(c->d_fs_cnt); dfree(c->d_fs_off);
+    dfree(c->d_cand);
+    dfree(c->d_hot); dfree(c->d_pair_halo); dfree(c->d_keys); dfree(c->d_vals); dfree(c->d_sort_tmp);
     for (int i = 0; i < 10; ++i) if (c->ev[i]) (void)hipEventDestroy(c->ev[i]);
     if (c->h_pin) (void)hipHostFree(c->h_pin);
     if (c->h_prod) (void)hipHostFree(c->h_prod);
@@ -528,8 +527,8 @@ int p2m_load_table(p2m_ctx *c, int slot, const int32_t hdr_i[3], const float hdr
          * fits goes back to the library's choice */
         const int ml = c->cfg.precision == P2M_PREC_FP64 ? 1 : 2;
         const int mem = c->d_count != nullptr;
-        if (p2m_tile_lds_bytes(ml, c->cfg.n_maps, 10, mem, hdr_i[2]) > 160 * 1024) return P2M_E_SIZE;
-        if (c->tuned && c->log2w && p2m_tile_lds_bytes(ml, c->cfg.n_maps, c->log2w, mem, hdr_i[2]) > 160 * 1024)
+        if (p2m_tile_lds_bytes(ml, c->cfg.n_maps, 10, mem, hdr_i[2], 256) > 160 * 1024) return P2M_E_SIZE;
+        if (c->tuned && c->log2w && p2m_tile_lds_bytes(ml, c->cfg.n_maps, c->log2w, mem, hdr_i[2], c->wg) > 160 * 1024)
             c->tuned = false;
     }
     TabGeom &g = c->g;
@@ -606,7 +605,7 @@ int p2m_set_tile(p2m_ctx *c, int32_t tile_w, int32_t tile_wg)
     int l = 0;
     while ((1 << l) < tile_w) ++l;
     if (p2m_tile_lds_bytes(c->cfg.precision == P2M_PREC_FP64 ? 1 : 2, c->cfg.n_maps, l, c->d_count != nullptr,
-                           c->have_table[0] ? c->g.nrt : 200) > 160 * 1024)
+                           c->have_table[0] ? c->g.nrt : 200, tile_wg) > 160 * 1024)
         return P2M_E_INVALID;
     HIPCHK(hipSetDevice(c->cfg.device));
     int rc = build_tiles(c, l);
@@ -640,8 +639,6 @@ static int scan_counts(p2m_ctx *c, const uint32_t *cnt, unsigned long long *off,
     return scan_counts_on(cnt, off, n, &c->d_scan_tmp, &c->scan_tmp_bytes, c->stream);
 }
 
-/* The per-halo buffers exist after the first paint call even for an empty
- * catalogue: the binning writes the terminating ring count nr[n_halo]. */
 /* counter block summed over its shards (blocks until the stream is idle) */
 static int read_counters(p2m_ctx *c, unsigned long long out[Ctr::TOTAL], unsigned long long *raw = nullptr)
 {
@@ -661,27 +658,19 @@ static int ensure_halo_cap(p2m_ctx *c, int64_t n)
     if (n <= c->halo_cap && c->d_halo) return 0;
     dfree(c->d_halo); c->d_halo = nullptr; c->halo_cap = 0;
     dfree(c->d_flat_idx); c->d_flat_idx = nullptr;
-    dfree(c->d_nr); c->d_nr = nullptr;
-    dfree(c->d_ring_off); c->d_ring_off = nullptr;
-    dfree(c->d_halo_s); c->d_halo_s = nullptr;
+    dfree(c->d_n_pairs); c->d_n_pairs = nullptr;
+    dfree(c->d_pair_off); c->d_pair_off = nullptr;
     dfree(c->d_hot); c->d_hot = nullptr;
-    dfree(c->d_bin); c->d_bin = nullptr;
-    dfree(c->d_keys); c->d_keys = nullptr;
-    dfree(c->d_vals); c->d_vals = nullptr;
+    dfree(c->d_pair_halo); c->d_pair_halo = nullptr;
     int64_t cap = std::max<int64_t>(n, 1024);
     if (dmalloc((void **)&c->d_halo, sizeof(HaloRec) * cap)) return P2M_E_NOMEM;
     if (dmalloc((void **)&c->d_flat_idx, sizeof(uint32_t) * cap)) return P2M_E_NOMEM;
-    if (dmalloc((void **)&c->d_nr, sizeof(uint32_t) * (cap + 1))) return P2M_E_NOMEM;
-    if (dmalloc((void **)&c->d_ring_off, sizeof(unsigned long long) * (cap + 1))) return P2M_E_NOMEM;
     if (c->cfg.precision != P2M_PREC_PLAIN_FP64 && c->cfg.nside > 0) {
-        if (dmalloc((void **)&c->d_bin, sizeof(BinHalo) * cap)) return P2M_E_NOMEM;
-        if (c->cfg.precision == P2M_PREC_FP32_COMP) {
-            if (dmalloc((void **)&c->d_hot, sizeof(TileHalo) * cap)) return P2M_E_NOMEM;
-        } else {
-            if (dmalloc((void **)&c->d_halo_s, sizeof(HaloRec) * cap)) return P2M_E_NOMEM;
-        }
-        if (dmalloc((void **)&c->d_keys, sizeof(uint32_t) * 2 * cap)) return P2M_E_NOMEM;
-        if (dmalloc((void **)&c->d_vals, sizeof(uint32_t) * 2 * cap)) return P2M_E_NOMEM;
+        if (dmalloc((void **)&c->d_pair_halo, sizeof(PairHalo) * cap)) return P2M_E_NOMEM;
+        if (dmalloc((void **)&c->d_n_pairs, sizeof(uint32_t) * (cap + 1))) return P2M_E_NOMEM;
+        if (dmalloc((void **)&c->d_pair_off, sizeof(unsigned long long) * (cap + 1))) return P2M_E_NOMEM;
+        if (c->cfg.precision == P2M_PREC_FP32_COMP && dmalloc((void **)&c->d_hot, sizeof(TileHalo) * cap))
+            return P2M_E_NOMEM;
     }
     c->halo_cap = cap;
     return 0;
@@ -705,17 +694,12 @@ static int decode_chunk(p2m_ctx *c, const float *d_src, int64_t n, int64_t base)
     a.n_cand0 = c->d_ctr + Ctr::N_CAND0;
     a.n_flat_out = c->d_ctr + Ctr::N_FLAT;
     a.counters = c->d_ctr + Ctr::DEC;
-    a.keys = nullptr; a.vals = nullptr; a.nphi = 1; a.key_max = 0;
-    if (c->d_bin && c->cfg.nside > 0) {
-        a.keys = c->d_keys; a.vals = c->d_vals;
-        a.nphi = std::max(1, c->cfg.nside / 128);
-        a.key_max = p2m_key_max(c->cfg.nside, a.nphi);
-    }
+    a.hot = c->d_hot; a.pair_halo = c->d_pair_halo; a.n_pairs = c->d_n_pairs; a.shape = c->shape;
     p2m_launch_decode(a, c->stream);
     return hipGetLastError() == hipSuccess ? 0 : P2M_E_HIP;
 }
 
-static int autotune(p2m_ctx *c, int64_t n_halo, int64_t n_flat, unsigned long long n_items);
+static int autotune(p2m_ctx *c, int64_t n_halo, int64_t n_flat, unsigned long long n_pix);
 
 static int launch_flat(p2m_ctx *c, PaintArgs &pa, int64_t n_flat, hipStream_t s);
 
@@ -726,7 +710,8 @@ static void fs_join(p2m_ctx *c)
     (void)hipGetLastError();
 }
 
-static int paint_halos(p2m_ctx *c, int64_t n_halo, int64_t n_flat, unsigned long long n_items, bool allow_tune)
+/* n_pix: the pixels of the painted discs, about */
+static int paint_halos(p2m_ctx *c, int64_t n_halo, int64_t n_flat, unsigned long long n_pix, bool allow_tune)
 {
     const int mode = c->cfg.precision;
     unsigned long long *pc = c->d_ctr + Ctr::PAINT;
@@ -747,7 +732,7 @@ static int paint_halos(p2m_ctx *c, int64_t n_halo, int64_t n_flat, unsigned long
         /* tile shape first: the tuner's trials paint and clear both maps, so
          * this call's own painting (the flat-sky map included) starts after
          * the last trial */
-        if (allow_tune) { int rc = autotune(c, n_halo, n_flat, n_items); if (rc) return rc; }
+        if (allow_tune) { int rc = autotune(c, n_halo, n_flat, n_pix); if (rc) return rc; }
         else { int rc = build_tiles(c, 10); if (rc) return rc; c->wg = 256; c->tuned = true; }
     }
     HIPCHK(hipEventRecord(c->ev[2], c->stream));
@@ -776,99 +761,57 @@ static int paint_halos(p2m_ctx *c, int64_t n_halo, int64_t n_flat, unsigned long
             bool armed;
             ~FsJoin() { if (armed) (void)hipStreamWaitEvent(c->stream, c->ev_fs, 0); }
         } fs_guard{c, true};
-        /* painted halos in spatial order (keys written by decode):
-         * neighbouring halos share tiles */
-        {
-            const uint32_t key_max = p2m_key_max(c->cfg.nside, std::max(1, c->cfg.nside / 128));
+        /* (halo, tile) pairs: counted by the decode at the shape it knew,
+         * listed in halo order, sorted by tile */
+        BinArgs b;
+        memset(&b, 0, sizeof(b));
+        b.halos = c->d_pair_halo; b.n_halo = n_halo; b.shape = c->shape; b.band_tile = c->d_band_tile;
+        b.n_pairs = c->d_n_pairs; b.pair_off = c->d_pair_off; b.recs = c->d_halo; b.counters = pc;
+        const bool recount = c->counted_log2w != c->log2w;
+        if (recount) p2m_launch_pair_count(b, c->stream);
+        if (n_halo > 0) { int rc = scan_counts(c, c->d_n_pairs, c->d_pair_off, n_halo + 1); if (rc) return rc; }
+        if (recount && n_halo > 0) {
+            unsigned long long hv = 0, *hp = c->h_pin ? c->h_pin : &hv;
+            HIPCHK(hipMemcpyAsync(hp, c->d_pair_off + n_halo, sizeof(*hp), hipMemcpyDeviceToHost, c->stream));
+            HIPCHK(hipStreamSynchronize(c->stream));
+            c->counted_pairs = *hp;
+        }
+        c->counted_log2w = c->log2w;
+        const unsigned long long n_pairs = c->counted_pairs;
+        if ((int64_t)n_pairs > c->pair_cap || !c->d_keys || !c->d_vals) {
+            dfree(c->d_keys); dfree(c->d_vals); c->d_keys = nullptr; c->d_vals = nullptr; c->pair_cap = 0;
+            const int64_t cap = (int64_t)(n_pairs * 1.125) + 1024;
+            if (dmalloc((void **)&c->d_keys, sizeof(uint32_t) * 2 * cap)) return P2M_E_NOMEM;
+            if (dmalloc((void **)&c->d_vals, sizeof(uint32_t) * 2 * cap)) return P2M_E_NOMEM;
+            c->pair_cap = cap;
+        }
+        b.keys = c->d_keys; b.vals = c->d_vals; b.pair_cap = n_pairs;
+        if (n_pairs > 0) {
+            if (c->ask_gaps) {
+                /* in the place of the decode's count of such halos */
+                p2m_launch_clear_ctr(pc, 3, 1, c->stream);
+                p2m_launch_ring_gaps(b, c->stream);
+            }
+            p2m_launch_pair_emit(b, c->stream);
             size_t need = 0;
-            if (p2m_sort_halos(c->d_halo, n_halo, key_max, c->d_bin, c->d_hot, c->d_halo_s, c->g.nrt, c->g.nmht,
-                               c->d_keys, c->d_vals, nullptr, &need, c->d_nr, c->stream)) return P2M_E_HIP;
+            if (p2m_sort_pairs(c->d_keys, c->d_vals, n_pairs, c->n_tiles, nullptr, &need, c->stream)) return P2M_E_HIP;
             if (need > c->sort_tmp_bytes || !c->d_sort_tmp) {
                 dfree(c->d_sort_tmp); c->d_sort_tmp = nullptr; c->sort_tmp_bytes = 0;
                 if (dmalloc(&c->d_sort_tmp, need + 256)) return P2M_E_NOMEM;
                 c->sort_tmp_bytes = need + 256;
             }
             size_t bytes = c->sort_tmp_bytes;
-            if (p2m_sort_halos(c->d_halo, n_halo, key_max, c->d_bin, c->d_hot, c->d_halo_s, c->g.nrt, c->g.nmht,
-                               c->d_keys, c->d_vals, c->d_sort_tmp, &bytes, c->d_nr, c->stream)) return P2M_E_HIP;
+            if (p2m_sort_pairs(c->d_keys, c->d_vals, n_pairs, c->n_tiles, c->d_sort_tmp, &bytes, c->stream)) return P2M_E_HIP;
         }
-        const uint32_t *order = c->d_vals + n_halo;   /* spatial position -> slot */
-        BinArgs b;
-        memset(&b, 0, sizeof(b));
-        b.halos = c->d_bin; b.n_halo = n_halo; b.nside = c->cfg.nside; b.log2w = c->log2w;
-        b.nr = c->d_nr; b.ring_off = c->d_ring_off;
-        b.tile_base = c->d_tile_base; b.tile_cnt = c->d_tile_cnt;
-        b.tile_off = c->d_tile_off; b.segs = c->d_segs; b.counters = pc; b.ring_z = c->d_ring_z;
-        /* (halo, ring) item space: the gather wrote the item count of every
-         * halo (with no halo it did not run) */
-        if (n_halo <= 0) p2m_launch_ring_counts(b, c->stream);
-        { int rc = scan_counts(c, c->d_nr, c->d_ring_off, n_halo + 1); if (rc) return rc; }
-        /* n_items (= ring_off[n_halo]) was counted by the decode */
-        if ((int64_t)n_items > c->runs_cap || !c->d_runs || !c->d_pos) {
-            dfree(c->d_runs); dfree(c->d_pos); c->d_runs = nullptr; c->d_pos = nullptr; c->runs_cap = 0;
-            int64_t cap = (int64_t)(n_items * 1.25) + 1024;
-            if (dmalloc((void **)&c->d_runs, sizeof(uint32_t) * cap)) return P2M_E_NOMEM;
-            if (dmalloc((void **)&c->d_pos, sizeof(uint32_t) * cap)) return P2M_E_NOMEM;
-            c->runs_cap = cap;
-        }
-        if (!c->d_ovf || c->ovf_cap < (int64_t)(n_items / 8) + (1 << 16)) {
-            /* about 8% of the items cross a tile boundary at the default shape */
-            dfree(c->d_ovf); c->d_ovf = nullptr; c->ovf_cap = 0;
-            const int64_t cap = (int64_t)(n_items / 8) + (1 << 16);
-            if (dmalloc((void **)&c->d_ovf, sizeof(uint4) * cap)) return P2M_E_NOMEM;
-            c->ovf_cap = cap;
-        }
-        if ((int64_t)(n_items / 64 + 2) > c->group_cap || !c->d_group) {
-            dfree(c->d_group); c->d_group = nullptr; c->group_cap = 0;
-            const int64_t cap = (int64_t)((n_items / 64 + 2) * 1.25) + 1024;
-            if (dmalloc((void **)&c->d_group, sizeof(uint32_t) * cap)) return P2M_E_NOMEM;
-            c->group_cap = cap;
-        }
-        b.n_items = n_items; b.runs = c->d_runs; b.pos = c->d_pos; b.group_halo = c->d_group;
-        b.ovf = c->d_ovf; b.ovf_cap = c->ovf_cap; b.n_ovf = pc + Ctr::OVF;
-        b.n_tiles = c->n_tiles; b.err = c->d_ctr + Ctr::ERR;
-        p2m_launch_fill_u32(c->d_tile_cnt, c->n_tiles + 1, 0u, c->stream);
-        p2m_launch_seg_count(b, c->stream);
-        { int rc = scan_counts(c, c->d_tile_cnt, c->d_tile_off, c->n_tiles + 1); if (rc) return rc; }
-        /* segment and listed-pixel counts back to the host (pinned memory) */
-        unsigned long long nseg = 0, nlisted = 0;
-        {
-            unsigned long long hbuf[Ctr::ALL + 1];
-            unsigned long long *hb = c->h_pin ? c->h_pin : hbuf;
-            HIPCHK(hipMemcpyAsync(hb, c->d_ctr, sizeof(unsigned long long) * Ctr::ALL, hipMemcpyDeviceToHost, c->stream));
-            HIPCHK(hipMemcpyAsync(hb + Ctr::ALL, c->d_tile_off + c->n_tiles, sizeof(unsigned long long),
-                                  hipMemcpyDeviceToHost, c->stream));
-            HIPCHK(hipEventRecord(c->ev[6], c->stream));
-            HIPCHK(hipEventSynchronize(c->ev[6]));
-            const unsigned long long n_ovf = hb[Ctr::PAINT + Ctr::OVF];
-            if ((int64_t)n_ovf > c->ovf_cap) {
-                /* pieces beyond the overflow list (runs spanning three or
-                 * more tiles): grow it and count again */
-                dfree(c->d_ovf); c->d_ovf = nullptr; c->ovf_cap = 0;
-                const int64_t cap = (int64_t)(n_ovf * 1.25) + 1024;
-                if (dmalloc((void **)&c->d_ovf, sizeof(uint4) * cap)) return P2M_E_NOMEM;
-                c->ovf_cap = cap;
-                b.ovf = c->d_ovf; b.ovf_cap = cap;
-                p2m_launch_clear_ctr(pc, 0, 1, c->stream);
-                p2m_launch_clear_ctr(pc, 4, 1, c->stream);
-                p2m_launch_clear_ctr(pc, Ctr::OVF, 1, c->stream);
-                p2m_launch_fill_u32(c->d_tile_cnt, c->n_tiles + 1, 0u, c->stream);
-                p2m_launch_seg_count(b, c->stream);
-                { int rc = scan_counts(c, c->d_tile_cnt, c->d_tile_off, c->n_tiles + 1); if (rc) return rc; }
-                HIPCHK(hipMemcpyAsync(hb, c->d_ctr, sizeof(unsigned long long) * Ctr::ALL, hipMemcpyDeviceToHost, c->stream));
-                HIPCHK(hipMemcpyAsync(hb + Ctr::ALL, c->d_tile_off + c->n_tiles, sizeof(unsigned long long),
-                                      hipMemcpyDeviceToHost, c->stream));
-                HIPCHK(hipStreamSynchronize(c->stream));
-            }
-            nseg = hb[Ctr::ALL];
-            for (int sh = 0; sh < P2M_SHARDS; ++sh) nlisted += hb[sh * Ctr::TOTAL + Ctr::PAINT + 0];
-        }
+        const uint32_t *keys = c->d_keys + n_pairs, *vals = c->d_vals + n_pairs;     /* sorted */
+        p2m_launch_tile_bounds(keys, n_pairs, c->n_tiles, c->d_tile_off, c->stream);
+        HIPCHK(hipGetLastError());
         if (mode == P2M_PREC_FP32_COMP) {
             /* deferred FP64 pixels: ~5e-4 of the listed pixels in practice;
              * a list that fills up costs a repaint of the tiles that lost
              * pixels, after the list has grown (P2M_FB_CAP caps it, so that
              * the repaint can be exercised) */
-            int64_t need = (int64_t)(nlisted / 256) + (1 << 18);
+            int64_t need = (int64_t)(n_pix / 256) + (1 << 18);
             if (const char *e = getenv("P2M_FB_CAP")) {
                 const long long cap = atoll(e);
                 if (cap >= P2M_SHARDS && cap < need) need = cap;
@@ -879,24 +822,17 @@ static int paint_halos(p2m_ctx *c, int64_t n_halo, int64_t n_flat, unsigned long
                 c->fb_cap = need;
             }
         }
-        if ((int64_t)nseg > c->seg_cap || !c->d_segs) {
-            dfree(c->d_segs); c->d_segs = nullptr; c->seg_cap = 0;
-            int64_t cap = (int64_t)(nseg * 1.25) + 1024;
-            if (dmalloc((void **)&c->d_segs, sizeof(uint2) * cap)) return P2M_E_NOMEM;
-            c->seg_cap = cap;
-        }
-        b.segs = c->d_segs;
-        p2m_launch_seg_emit(b, c->stream);
-        HIPCHK(hipGetLastError());
         HIPCHK(hipEventRecord(c->ev[3], c->stream));
         TileArgs t;
         memset(&t, 0, sizeof(t));
-        t.halos = c->d_halo_s; t.hot = c->d_hot; t.nside = c->cfg.nside; t.log2w = c->log2w; t.n_rings = c->n_rings;
+        t.halos = c->d_halo; t.hot = c->d_hot; t.shape = c->shape; t.nside = c->cfg.nside;
+        t.log2w = c->log2w;
         t.n_maps = c->cfg.n_maps; t.profile = c->cfg.profile; t.accumulate = c->hp_zero ? 0 : 1;
-        t.n_tiles = c->n_tiles; t.tile_base = c->d_tile_base; t.desc = c->d_tile_desc; t.tile_off = c->d_tile_off; t.segs = c->d_segs;
+        t.n_tiles = c->n_tiles; t.desc = c->d_tile_desc; t.ring = c->d_ring; t.tile_off = c->d_tile_off;
+        t.keys = keys; t.vals = vals;
         t.g = c->g; t.n_flat = c->n_flat; t.inv_node2 = c->d_inv_node2;
         t.u_k1 = c->u_k1; t.u_k0 = c->u_k0; t.u_max = c->u_max; t.band = c->u_band; t.fr_clamp = c->fr_clamp; t.ir_clamp = c->ir_clamp;
-        t.band_c = 4e-6f;
+        t.band_c = (float)CHORD_BAND;
         t.inv_node2f = c->d_inv_node2f;
         t.n_quad = c->n_quad; t.tab_q = c->d_quad;
         t.fb = c->d_fb; t.fb_count = pc + 6; t.fb_cap = c->fb_cap;
@@ -909,7 +845,7 @@ static int paint_halos(p2m_ctx *c, int64_t n_halo, int64_t n_flat, unsigned long
          * of 8 for the XCD-aware tile order): no partial last round */
         int grid = (int)std::min<int64_t>(c->n_tiles, 8192);
         {
-            const size_t lds = p2m_tile_lds_bytes(mode, c->cfg.n_maps, c->log2w, c->d_count != nullptr, c->g.nrt);
+            const size_t lds = p2m_tile_lds_bytes(mode, c->cfg.n_maps, c->log2w, c->d_count != nullptr, c->g.nrt, c->wg);
             const int occ = p2m_tile_occupancy(mode, c->cfg.n_maps, c->wg, lds);
             if (occ > 0 && c->n_cu > 0) {
                 const int64_t res = ((int64_t)occ * c->n_cu) & ~(int64_t)7;
@@ -922,15 +858,15 @@ static int paint_halos(p2m_ctx *c, int64_t n_halo, int64_t n_flat, unsigned long
         if (mode == P2M_PREC_FP32_COMP) {
             FallbackArgs f;
             memset(&f, 0, sizeof(f));
-            f.halos = c->d_halo; f.order = order; f.fb = c->d_fb; f.fb_count = pc + 6; f.fb_cap = c->fb_cap;
+            f.halos = c->d_halo; f.fb = c->d_fb; f.fb_count = pc + 6; f.fb_cap = c->fb_cap;
             f.nside = c->cfg.nside; f.n_maps = c->cfg.n_maps; f.profile = c->cfg.profile;
             f.g = c->g; f.n_flat = c->n_flat;
             for (int m = 0; m < c->cfg.n_maps; ++m) { f.tab_flat[m] = c->d_flat[m]; f.map32[m] = c->d_hp32[m]; }
             f.count = c->d_count; f.hash = c->d_hash; f.counters = pc;
-            f.lost = c->d_lost; f.tile_base = c->d_tile_base; f.log2w = c->log2w; f.n_halo = n_halo;
+            f.lost = c->d_lost; f.desc = c->d_tile_desc; f.n_tiles = c->n_tiles; f.n_halo = n_halo;
             f.err = c->d_ctr + Ctr::ERR;
-            if (p2m_launch_fallback(f, (int64_t)(nlisted / 256) + 1024, c->stream)) return P2M_E_HIP;
-            c->last_t = t; c->last_f = f; c->last_grid = grid; c->last_nlisted = (int64_t)nlisted;
+            if (p2m_launch_fallback(f, (int64_t)(n_pix / 256) + 1024, c->stream)) return P2M_E_HIP;
+            c->last_t = t; c->last_f = f; c->last_grid = grid; 
         }
         c->last_fast = mode == P2M_PREC_FP32_COMP;
         HIPCHK(hipEventRecord(c->ev[4], c->stream));
@@ -1091,6 +1027,12 @@ static int pass_begin(p2m_ctx *c, int64_t n_total)
     HIPCHK(hipSetDevice(c->cfg.device));
     int rc = ensure_halo_cap(c, n_total);
     if (rc) return rc;
+    if (c->cfg.precision != P2M_PREC_PLAIN_FP64 && c->cfg.nside > 0) {
+        /* the decode counts tiles at the shape in force, or at the default
+         * one where the painter is still to choose */
+        if (!c->tuned) { rc = build_tiles(c, 10); if (rc) return rc; }
+        c->counted_log2w = c->log2w;
+    }
     if (n_total > 0 && n_total > c->cand_cap) {
         dfree(c->d_cand); c->d_cand = nullptr; c->cand_cap = 0;
         if (dmalloc((void **)&c->d_cand, sizeof(uint32_t) * n_total)) return P2M_E_NOMEM;
@@ -1194,7 +1136,9 @@ static int pass_finish(p2m_ctx *c, bool allow_tune)
     if (rc) return rc;
     int64_t n_halo = (int64_t)std::min<unsigned long long>(hc[Ctr::N_CAND], (unsigned long long)c->halo_cap);
     int64_t n_flat = (int64_t)std::min<unsigned long long>(hc[Ctr::N_FLAT], (unsigned long long)c->halo_cap);
-    rc = paint_halos(c, n_halo, n_flat, hc[Ctr::ITEMS], allow_tune);
+    c->counted_pairs = hc[Ctr::PAIRS];
+    c->ask_gaps = hc[Ctr::GAPS] != 0;
+    rc = paint_halos(c, n_halo, n_flat, hc[Ctr::PIX], allow_tune);
     if (rc) {
         /* nothing queued may outlive the call */
         (void)hipStreamSynchronize(c->fs_stream);
@@ -1334,7 +1278,7 @@ int p2m_fetch_membership(p2m_ctx *c, uint32_t *hc, uint64_t *hh, uint32_t *fc, u
 /* ------------------------------------------------------------------ autotuner */
 /* Times the binning + tile paint for each candidate tile shape on the
  * halos already decoded, keeps the fastest, and restores the maps. */
-static int autotune(p2m_ctx *c, int64_t n_halo, int64_t n_flat, unsigned long long n_items)
+static int autotune(p2m_ctx *c, int64_t n_halo, int64_t n_flat, unsigned long long n_pix)
 {
     static const int cand[][2] = {{9, 256}, {10, 256}, {11, 256}, {11, 128}, {12, 256}};
     int mode_ld = c->cfg.precision == P2M_PREC_FP64 ? 1 : 2;
@@ -1357,14 +1301,14 @@ static int autotune(p2m_ctx *c, int64_t n_halo, int64_t n_flat, unsigned long lo
     float best_ms = 1e30f;
     for (auto &cd : cand) {
         if (cd[0] > p2m_tile_max_log2w()) continue;
-        if (p2m_tile_lds_bytes(mode_ld, c->cfg.n_maps, cd[0], c->d_count != nullptr, c->g.nrt) > 160 * 1024) continue;
+        if (p2m_tile_lds_bytes(mode_ld, c->cfg.n_maps, cd[0], c->d_count != nullptr, c->g.nrt, cd[1]) > 160 * 1024) continue;
         int rc = build_tiles(c, cd[0]); if (rc) return rc;
         c->wg = cd[1]; c->tuned = true;
         c->hp_zero = true;
         /* each trial starts from zero paint counters, as a call does: the
          * deferred-pixel and overflow lists are appended at their counters */
         p2m_launch_clear_ctr(c->d_ctr, Ctr::PAINT, Ctr::TOTAL - Ctr::PAINT, c->stream);
-        rc = paint_halos(c, n_halo, n_flat, n_items, false);
+        rc = paint_halos(c, n_halo, n_flat, n_pix, false);
         if (rc == P2M_E_INVALID) {
             /* a shape the painter rejects at launch: the trial's flat-sky
              * paint is still on its stream, so the clear waits for it */

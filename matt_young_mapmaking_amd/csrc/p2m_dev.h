@@ -65,24 +65,31 @@ struct HaloRec {
     int32_t jmin, jmax, kmin, kmax;  /* flat-sky index box (haloproject.f90:124-128) */
 };
 
-/* The fields of a painted halo that the binning reads (query_disc per
- * ring), in spatial order. */
-struct BinHalo {
-    double cosang, zz0, a, phi0;
-    int32_t irmin, irmax;
-};
-
 /* The fields of a painted halo that the FP32 tile painter stages per
- * segment, packed into one 64-B line (written in spatial order). */
+ * (halo, ring) segment, packed into one 64-B line. */
 struct __attribute__((aligned(64))) TileHalo {
     double zz0, s0, phi0, thr;   /* as in HaloRec */
+    float thr_hi;                /* outer edge of the deferral band: thr (1 + CHORD_BAND) */
     float chi2;                  /* (float)(chi_r * chi_r) */
-    float vh;                    /* velocity factor; 0 when chi > chimaxt */
-    float fc, fm;                /* table fractions, rounded to float */
+    float w00, w10, w01, w11;    /* weights of the table cell's corners times the velocity factor, from
+                                    the table fractions rounded to float; 0 when chi > chimaxt */
     int32_t colbase;             /* nrt * ((imh - 1) + nmht * (ichi - 1)); 0 when chi > chimaxt */
     uint32_t pad;
-    unsigned long long hash;     /* membership hash of the catalogue index */
 };
+
+/* Half-width of the band around the disc edge, relative in chord^2, that the
+ * FP32 painter leaves to the FP64 decision. */
+#define CHORD_BAND 4e-6
+
+/* What the binning needs of a painted halo: its centre's azimuth and the
+ * disc's azimuth half-width, both in turns, and the rings the disc itself
+ * reaches (disc_rings), first | last << 16 (no ring: first > last), with
+ * the top bit set if it may have a ring gap. */
+struct PairHalo {
+    float turn, half;
+    uint32_t rings;
+};
+#define RINGS_ASK_GAPS 0x80000000u
 
 /* ------------------------------------------------------------ cosmology */
 P2M_DEV double tab_lookup(const double *t, int n, double tmin, double dt, double x)
@@ -116,7 +123,7 @@ P2M_DEV double deltacrit_z(const CosmoDev &c, double z)
 
 /* ------------------------------------------------------------ HEALPix */
 /* ring_num, pix_tools.F90:490-533 */
-P2M_DEV int32_t ring_num(int32_t nside, double z)
+P2M_HD int32_t ring_num(int32_t nside, double z)
 {
     int32_t iring = (int32_t)p2m_nint((double)nside * (2.0 - 1.5 * z));
     if (z > HPX_TWOTHIRD) {
@@ -132,7 +139,7 @@ P2M_DEV int32_t ring_num(int32_t nside, double z)
 }
 
 /* ring2z, pix_tools.F90:535-560 */
-P2M_DEV double ring2z(int32_t nside, int32_t ir)
+P2M_HD double ring2z(int32_t nside, int32_t ir)
 {
     double fn = (double)nside;
     if (ir < nside) {
@@ -169,9 +176,8 @@ P2M_HD void ring_info(int32_t nside, int32_t ring, int32_t &npr, int32_t &kshift
 /* Ring tiles: ring `ring` is cut into ceil(npr / W) tiles of W = 2^log2w
  * consecutive RING pixels, the last one narrower.  Tile `col` starts at
  * in-ring pixel ip0 = col W, holds `width` pixels, and its first map pixel is
- * first + ip0 (first: the ring's first pixel).  The host numbers the tiles
- * ring by ring with ring_tiles; k_tile_desc fills each descriptor with
- * tile_span. */
+ * first + ip0 (first: the ring's first pixel).  The painters' own tiles are
+ * bands of rings by sectors, below. */
 P2M_HD int32_t ring_tiles(int32_t nside, int32_t ring, int32_t log2w)
 {
     int32_t npr, kshift;
@@ -189,9 +195,108 @@ P2M_HD void tile_span(int32_t nside, int32_t ring, int32_t col, int32_t log2w, i
     width = npr - ip0 < (1 << log2w) ? npr - ip0 : (1 << log2w);
 }
 
+/* ------------------------------------------------------------ tiles */
+/* The map is painted in tiles of R = 2^log2r consecutive rings (a band; the
+ * last one may hold fewer) by one sector of azimuth.  A band's rings are
+ * each cut into the same number K of sectors, sector k of a ring of npr
+ * pixels being [floor(k npr / K), floor((k + 1) npr / K)): K is large
+ * enough that no sector is wider than C = 2^log2c pixels, nor (K >= 4, npr
+ * a multiple of 4) than a quarter of its ring.  Tiles are numbered sector
+ * by sector, band by band. */
+struct TileShape {
+    int32_t nside, log2r, log2c;
+};
+
+P2M_HD int32_t n_bands(const TileShape &g) { return ((4 * g.nside - 1) + (1 << g.log2r) - 1) >> g.log2r; }
+
+/* first and last ring of band `band` and its number of sectors */
+P2M_HD int32_t band_sectors(const TileShape &g, int32_t band, int32_t &r0, int32_t &r1)
+{
+    r0 = (band << g.log2r) + 1;
+    r1 = r0 + (1 << g.log2r) - 1;
+    if (r1 > 4 * g.nside - 1) r1 = 4 * g.nside - 1;
+    /* the longest ring of the band: 4 min(nside, the larger distance to a pole of its ends) */
+    int32_t m = r1 < 4 * g.nside - r0 ? r1 : 4 * g.nside - r0;
+    if (m > g.nside) m = g.nside;
+    const int32_t k = (4 * m + (1 << g.log2c) - 1) >> g.log2c;
+    return k < 4 ? 4 : k;
+}
+
+/* k npr < 2^31: K is at most 4 or npr / 2^log2c rounded up, npr at most 32768 */
+P2M_HD int32_t sector_start(int32_t npr, int32_t K, int32_t k) { return (int32_t)(((uint32_t)k * (uint32_t)npr) / (uint32_t)K); }
+
+/* Rings whose circle meets the disc, within the ring range [irmin, irmax] of
+ * query_disc (which adds a ring on either side): lat0 -+ dtheta as sines,
+ * 1 and -1 where a pole is inside.  The ring coordinate of a height is the
+ * one that ring_num rounds; it is taken 1e-4 of a ring wider, which is far
+ * above its rounding.  first > last if the disc lies between two rings. */
+P2M_HD double ring_coord(int32_t nside, double z)
+{
+    if (z > HPX_TWOTHIRD) return (double)nside * p2m_sqrt(3.0 * (1.0 - z));
+    if (z < -HPX_TWOTHIRD) return 4.0 * (double)nside - (double)nside * p2m_sqrt(3.0 * (1.0 + z));
+    return (double)nside * (2.0 - 1.5 * z);
+}
+
+P2M_HD uint32_t disc_rings(int32_t nside, double ztop, double zbot, int32_t irmin, int32_t irmax)
+{
+    int32_t a = (int32_t)p2m_ceil(ring_coord(nside, ztop) - 1e-4);
+    int32_t b = (int32_t)p2m_floor(ring_coord(nside, zbot) + 1e-4);
+    if (a < irmin) a = irmin;
+    if (b > irmax) b = irmax;
+    if (a > b) return 1u;        /* first 1, last 0 */
+    return (uint32_t)a | ((uint32_t)b << 16);
+}
+
+/* Azimuth half-width of a disc in turns, from its edge's chord^2 thr and the
+ * sine s0 of its centre's colatitude: sin(dphi) = sin(dtheta) / s0 where the
+ * disc holds no pole and is smaller than a hemisphere, else half a turn.
+ * FP32, widened by more than its error (asin's slope is below 8 for
+ * arguments up to 0.99). */
+P2M_HD float disc_half_turn(double thr, double s0)
+{
+    const float c2 = (float)thr, s = (float)s0;
+    const float sd = sqrtf(c2 * (1.0f - 0.25f * c2));          /* sin(dtheta) below a right angle */
+    if (!(c2 < 1.9f) || !(sd < 0.99f * s)) return 0.5f;
+    return asinf(sd / s) * (1.00001f / 6.2831853f) + 1e-6f;
+}
+
+/* The tiles a halo's disc may reach, in band order: f(band, sector, first
+ * row, rows), every tile once. */
+template <typename F>
+P2M_HD void halo_tiles(const TileShape &g, float turn, float half, uint32_t rings, F f)
+{
+    const int32_t ra = (int32_t)(rings & 0xffffu), rb = (int32_t)((rings >> 16) & 0x7fffu);
+    if (ra > rb) return;
+    const int32_t b0 = (ra - 1) >> g.log2r, b1 = (rb - 1) >> g.log2r;
+    for (int32_t band = b0; band <= b1; ++band) {
+        int32_t r0, r1;
+        const int32_t K = band_sectors(g, band, r0, r1);
+        const int32_t first = ra > r0 ? ra : r0, last = rb < r1 ? rb : r1;
+        int32_t n = K, k0 = 0;
+        if (half < 0.5f) {
+            /* a pixel ip of a ring lies at (ip + off) / npr turns, off 0 or
+             * 1/2, in the sector ceil((ip + 1) K / npr) - 1: not below the
+             * floor of its turn times K, at most a pixel's K / npr above */
+            const int32_t m0 = r0 < 4 * g.nside - r1 ? r0 : 4 * g.nside - r1;
+            const int32_t nmin = 4 * (m0 < g.nside ? m0 : g.nside);
+            const float fk = (float)K;
+            const double lo = ((double)turn - (double)half) * fk, hi = ((double)turn + (double)half) * fk + (double)(fk / (float)nmin);
+            k0 = (int32_t)p2m_floor(lo);
+            n = (int32_t)p2m_floor(hi + 1e-6) - k0 + 1;
+            if (n >= K) { n = K; k0 = 0; }
+            else if (k0 < 0) k0 += K;
+        }
+        for (int32_t j = 0; j < n; ++j) {
+            int32_t k = k0 + j;
+            if (k >= K) k -= K;
+            f(band, k, first - r0, last - first + 1);
+        }
+    }
+}
+
 /* Pixel-centre z and sin(theta) of ring `ring`, exactly as pix2vec_ring
  * computes them for any pixel of that ring (pixel_routines.F90:229-311). */
-P2M_DEV void ring_zsth(int32_t nside, int32_t ring, double &z, double &sth)
+P2M_HD void ring_zsth(int32_t nside, int32_t ring, double &z, double &sth)
 {
     if (ring < nside) {
         double fact2 = (3.0 * nside) * nside;
@@ -212,7 +317,7 @@ P2M_DEV void ring_zsth(int32_t nside, int32_t ring, double &z, double &sth)
 
 /* phi of pixel ip of ring `ring`: phi = (iphi + off) * HALFPI / den with the
  * association of pix2vec_ring. */
-P2M_DEV void ring_phi_param(int32_t nside, int32_t ring, double &off, double &den)
+P2M_HD void ring_phi_param(int32_t nside, int32_t ring, double &off, double &den)
 {
     if (ring < nside) { off = 0.5; den = (double)ring; }
     else if (ring <= 3 * nside) { off = 0.5 * (double)((ring + nside + 1) & 1); den = (double)nside; }
@@ -374,6 +479,133 @@ P2M_HD int32_t disc_ring_run_fast(const H &h, double z, int32_t npr, int32_t ksh
     if (np > npr) np = npr;
     lo = (int32_t)l;
     return (int32_t)np;
+}
+
+/* asin(sqrt(h)) for h in [0, 1] to 3e-7 relative: the angle is halved twice
+ * (sin^2(x/2) = h / (2 + 2 sqrt(1 - h))) and the series of asin(sqrt(y)) /
+ * sqrt(y) summed to y^6 for y <= 0.147; c is cos = sqrt(1 - h). */
+P2M_HD float asin_sqrt(float h, float c)
+{
+#if defined(__HIP_DEVICE_COMPILE__)
+#define P2M_RCPF(x) __builtin_amdgcn_rcpf(x)
+#define P2M_SQRTF(x) __builtin_amdgcn_sqrtf(x)
+#else
+#define P2M_RCPF(x) (1.0f / (x))
+#define P2M_SQRTF(x) sqrtf(x)
+#endif
+    const float y1 = h * P2M_RCPF(__builtin_fmaf(2.0f, c, 2.0f));
+    const float y = y1 * P2M_RCPF(__builtin_fmaf(2.0f, P2M_SQRTF(1.0f - y1), 2.0f));
+    float p = __builtin_fmaf(y, 0.01735276f, 0.02237216f);
+    p = __builtin_fmaf(y, p, 0.03038195f);
+    p = __builtin_fmaf(y, p, 0.04464286f);
+    p = __builtin_fmaf(y, p, 0.075f);
+    p = __builtin_fmaf(y, p, 0.16666667f);
+    p = __builtin_fmaf(y, p, 1.0f);
+    return 4.0f * P2M_SQRTF(y) * p;
+}
+
+/* The same run from the chord relation, for a ring whose pixels lie at
+ * azimuth (ip + off) kphi: the disc edge is where A + B sin^2(dphi / 2) = thr,
+ * A = (z - z0)^2 + (sth - s0)^2 and B = 4 sth s0 in FP64 as the painter forms
+ * them, the rest in FP32 relative to the ring pixel ipc nearest the centre,
+ * x_c = ((ipc + off) kphi - phi0) / 2 (|x_c| <= kphi / 4): the run is
+ * ceil((-dphi/2 - x_c) / (kphi/2)) .. floor((dphi/2 - x_c) / (kphi/2)) from
+ * ipc.  Returns the number of pixels and lo in [0, npr), or -1 where the
+ * exact evaluation has to decide: an end lies within the error of a pixel
+ * centre, the ring only touches the disc or the arc nearly closes the ring
+ * (sin^2(dphi/2) within 0.02 of 1).  Every pixel of the run is then among the
+ * np_max pixels from lo (the whole ring where that is not cheap to say).
+ *
+ * The error of sin^2(dphi/2) against the exact evaluation's is
+ * e = 4e-15 / B + 2e-15 / sth^2 (e_row: the second term), several times the
+ * FP64 rounding of either form (cosang, the product z z0 and 1 - z^2, over
+ * s0 sth); 2e-6 of dphi covers the FP32 quotient, roots and arc sine (the
+ * slope 1 / cos is at most 7), 3e-7 of a pixel x_c. */
+P2M_HD int32_t disc_ring_run_chord(double thr, double A, float B, float e_row, float xc, float ihphi, int32_t ipc,
+                                   int32_t npr, int32_t &lo, int32_t &np_max)
+{
+    const float rB = P2M_RCPF(B);
+    const float h2 = (float)(thr - A) * rB;
+    const float e = __builtin_fmaf(4e-15f, rB, e_row);
+    lo = 0;
+    np_max = npr;
+    if (h2 < -2.0f * e) return 0;
+    if (h2 > 1.00001f + 2.0f * e) return npr;
+    const float c = P2M_SQRTF(1.0f - h2);
+    const float X = asin_sqrt(h2, c);
+    const float t = X * ihphi, o = xc * ihphi;
+    const float fl = -t - o, fh = t - o;
+    const float eps = ihphi * e * 0.6f * P2M_RCPF(P2M_SQRTF(h2) * c) + __builtin_fmaf(t, 2e-6f, 3e-7f);
+    const bool range = h2 > 2.0f * e && h2 < 0.98f && eps < 0.25f;
+    const bool far = __builtin_fabsf(fl - __builtin_rintf(fl)) > eps && __builtin_fabsf(fh - __builtin_rintf(fh)) > eps;
+    if (!range) return -1;
+    /* undecided ends: the run with the pixels that may belong to it */
+    const int32_t nl = (int32_t)__builtin_ceilf(far ? fl : fl - eps), nh = (int32_t)__builtin_floorf(far ? fh : fh + eps);
+    int32_t l = ipc + nl;
+    if (l < 0) l += npr;
+    if (l >= npr) l -= npr;
+    lo = l;
+    const int32_t np = nh - nl + 1;
+    np_max = np < npr ? np : npr;
+    return far ? (np > 0 ? np_max : 0) : -1;
+}
+
+/* Rings of a disc without a pixel between rings with pixels (the row
+ * misalignment of discedge2fulldisc, quirk Q15), counted once per gap: an empty
+ * ring whose ring before holds a pixel and some ring after it too.
+ *
+ * A ring one ring spacing or more inside the disc's top or bottom is crossed
+ * over at least 2 sqrt(2 R - 1) ring spacings, R the disc's radius in them, and
+ * a pixel is at most 2.36 ring spacings wide (at the equator; 1.3 to 1.6 in
+ * the caps), so an interior ring can only be empty if R < 1.2: discs that meet
+ * three rings.  Asked exactly for the small ones of those, and, where the rings are short
+ * (within 16 of a pole) or the disc is wide (half a turn: a pole inside or
+ * near), of the two rings inside either end and of every short ring. */
+template <typename H>
+P2M_HD int32_t ring_run_of(const H &h, int32_t nside, int32_t ring)
+{
+    int32_t npr, kshift, lo = 0;
+    int64_t first;
+    ring_info(nside, ring, npr, kshift, first);
+    return disc_ring_run_fast(h, ring2z(nside, ring), npr, kshift, lo);
+}
+
+P2M_HD bool gaps_possible(int32_t nside, double ztop, double zbot, double a, float half, uint32_t rings)
+{
+    const int32_t ra = (int32_t)(rings & 0xffffu), rb = (int32_t)(rings >> 16);
+    if (rb - ra < 2) return false;
+    if (half >= 0.5f || ra < 16 || rb > 4 * nside - 16) return true;
+    if (rb - ra > 2) return false;
+    /* the middle of three rings: crossed over 2 sqrt(dt db) ring spacings, dt
+     * and db its distances from the top and bottom; a pixel there is 2.356
+     * sin^2(theta) of them wide at most (1.58 in the caps).  Empty only if
+     * that is shorter than 1.15 pixels. */
+    const double dt = (double)(ra + 1) - ring_coord(nside, ztop), db = ring_coord(nside, zbot) - (double)(ra + 1);
+    const double w2 = (2.356 * 1.15 * a) * (2.356 * 1.15 * a);
+    return 4.0 * dt * db < (w2 > 3.3 ? w2 : 3.3);
+}
+
+template <typename H>
+P2M_HD int32_t ring_gaps(const H &h, int32_t nside, uint32_t rings)
+{
+    const int32_t ra = (int32_t)(rings & 0xffffu), rb = (int32_t)(rings >> 16);
+    int32_t gaps = 0, asked = 0, before = 0;      /* `before`: the run of ring `asked` */
+    for (int32_t r = ra + 1; r < rb; ++r) {
+        if (r > ra + 2 && r < rb - 2 && r >= 16 && r <= 4 * nside - 16) {
+            r = rb - 3 < 4 * nside - 16 ? rb - 3 : 4 * nside - 16;      /* the next one is asked */
+            continue;
+        }
+        const int32_t run = ring_run_of(h, nside, r);
+        if (run <= 0) {
+            if (asked != r - 1) before = ring_run_of(h, nside, r - 1);
+            if (before > 0)
+                for (int32_t k = r + 1; k <= rb; ++k)
+                    if (ring_run_of(h, nside, k) > 0) { ++gaps; break; }
+        }
+        asked = r;
+        before = run;
+    }
+    return gaps;
 }
 
 /* ------------------------------------------------------------ profile */

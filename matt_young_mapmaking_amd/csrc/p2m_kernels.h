@@ -33,10 +33,12 @@ struct DecodeArgs {
     int64_t cap;
     uint32_t *flat_idx;          /* slots of halos the flat-sky painter covers */
     unsigned long long *n_flat_out;
-    uint32_t *keys, *vals;       /* spatial sort key and slot of each record (tiled painters) */
-    int32_t nphi;                /* azimuth bins of the key */
-    uint32_t key_max;            /* the largest key, also given to inert records */
-    unsigned long long *counters;/* sharded: [0] passed radial cut, [2] radius errors, [3] (halo, ring) items */
+    TileHalo *hot;               /* the FP32 painter's records (or NULL) */
+    PairHalo *pair_halo;         /* the binning's records (tiled painters, or NULL) */
+    uint32_t *n_pairs;           /* tiles each of them reaches, at shape */
+    TileShape shape;
+    unsigned long long *counters;/* sharded: [0] passed radial cut, [2] radius errors, [3] (halo, tile) pairs,
+                                    [10] halos that may have a ring gap, [14] pixels of the discs, about */
 };
 
 struct PaintArgs {
@@ -62,36 +64,32 @@ struct PaintArgs {
 };
 
 struct BinArgs {
-    const BinHalo *halos;         /* in spatial order */
+    const PairHalo *halos;
     int64_t n_halo;
-    int32_t nside, log2w;
-    uint32_t *nr;                 /* rings per halo (n_halo + 1 entries, last 0) */
-    const unsigned long long *ring_off;  /* exclusive scan of nr */
-    unsigned long long n_items;   /* total (halo, ring) items */
-    uint32_t *group_halo;         /* halo of item 64 g (n_items / 64 + 1 entries) */
-    const double *ring_z;         /* ring2z of every ring */
-    uint32_t *runs;               /* per item: first in-ring pixel | pixel count << 16 */
-    uint32_t *pos;                /* per item: slot of its first tile piece within its tile */
-    const int32_t *tile_base;     /* first tile of ring r+1 */
-    uint32_t *tile_cnt;           /* segments per tile */
-    const unsigned long long *tile_off;  /* exclusive scan of tile_cnt */
-    uint2 *segs;                  /* (halo, lo<<16 | len) */
-    uint4 *ovf;                   /* pieces after an item's first: (tile, slot, halo, lo<<16 | len) */
-    unsigned long long *n_ovf;    /* entries of ovf (one counter, not sharded) */
-    int64_t ovf_cap;
-    int64_t n_tiles;
-    unsigned long long *counters; /* [0] listed, [3] ring gaps, [4] segments */
-    unsigned long long *err;      /* sharded: pieces whose slot lies outside their tile's range */
+    TileShape shape;
+    const int32_t *band_tile;     /* first tile of each band */
+    uint32_t *n_pairs;            /* tiles per halo (n_halo + 1 entries, last 0) */
+    const unsigned long long *pair_off;  /* exclusive scan of n_pairs */
+    uint32_t *keys, *vals;        /* the pairs, see k_pair_count */
+    unsigned long long pair_cap;
+    const HaloRec *recs;          /* the full records */
+    unsigned long long *counters; /* [3] ring gaps */
 };
 
-/* Per-tile geometry, computed once per tile shape: the pixel-centre z and
- * sin(theta) of the tile's ring, its phi parameters (phi = (ip + off)
- * pi/2 / den, kphi = pi/2 / den), the ring's first map pixel, the ring,
- * the tile's first in-ring pixel and its width. */
-struct __attribute__((aligned(16))) TileDesc {
-    double zr, sth, off, den, kphi;
+/* Geometry of a ring: the pixel-centre z and sin(theta), its phi parameters
+ * (phi = (ip + off) pi/2 / den, den = npr / 4, kphi = pi/2 / den), its first
+ * map pixel and pixels; e_row: see disc_ring_run_chord. */
+struct __attribute__((aligned(16))) RingDesc {
+    double zr, sth, off, kphi;
     int64_t first;
-    int32_t ring, ip0, width, pad;
+    int32_t npr;
+    float e_row;
+    int64_t pad;
+};
+
+/* A tile: its first ring, its rings, its sector k of K. */
+struct __attribute__((aligned(16))) TileDesc {
+    int32_t ring0, rows, k, K;
 };
 
 #define P2M_TQ_STRIDE 32           /* tile-queue counters one 128-byte line apart */
@@ -99,12 +97,13 @@ struct __attribute__((aligned(16))) TileDesc {
 struct TileArgs {
     const HaloRec *halos;
     const TileHalo *hot;          /* the same halos, packed for the FP32 painter */
-    int32_t nside, log2w, n_rings, n_maps, profile, accumulate;
+    TileShape shape;
+    int32_t nside, log2w, n_maps, profile, accumulate;
     int64_t n_tiles;
-    const int32_t *tile_base;
-    const TileDesc *desc;         /* geometry of each tile */
+    const TileDesc *desc;
+    const RingDesc *ring;         /* of every ring */
     const unsigned long long *tile_off;
-    const uint2 *segs;
+    const uint32_t *keys, *vals;  /* the sorted pairs */
     TabGeom g;
     const float *tab_flat[P2M_MAXMAPS];
     const float *tab_q;           /* corner-quad table (k_build_quad): a pixel's nodes ir-1, ir of its
@@ -115,12 +114,12 @@ struct TileArgs {
     const float *inv_node2f;      /* the same in float */
     float u_k1, u_k0, u_max, band, fr_clamp;
     int32_t ir_clamp;             /* cell and fraction of r = rmint + 1e-5 (maptable.f90:190, 196, 200) */
-    float band_c;                 /* relative chord^2 band decided in FP64 */
+    float band_c;                 /* CHORD_BAND */
     double *map64[P2M_MAXMAPS];
     float *map32[P2M_MAXMAPS];
     uint32_t *count;
     unsigned long long *hash;
-    uint4 *fb;                    /* deferred FP64 pixels: (ring, ip, halo, 0), P2M_SHARDS sub-lists */
+    uint4 *fb;                    /* deferred FP64 pixels: (row, in-row pixel, halo, tile), P2M_SHARDS sub-lists */
     unsigned long long *fb_count; /* sharded: sub-list k's length at fb_count[k * P2M_CTR_STRIDE] */
     int64_t fb_cap;               /* total; each sub-list holds fb_cap / P2M_SHARDS */
     uint8_t *lost;                /* per tile: set when its deferred pixels did not all fit in fb;
@@ -128,16 +127,15 @@ struct TileArgs {
     int32_t redo;                 /* paint only the tiles marked lost, clearing the mark of each
                                      that now fits */
     int64_t n_halo;               /* records in hot / halos */
-    unsigned int *tile_next;      /* the FP32 painter's tile queues: one counter per XCD, P2M_TQ_STRIDE
+    unsigned int *tile_next;      /* the tile queues: one counter per XCD, P2M_TQ_STRIDE
                                      apart (zeroed by p2m_launch_tile_paint) */
-    unsigned long long *counters; /* [1] hp updates, [5] FP64 fallbacks */
-    unsigned long long *err;      /* sharded: segments whose halo or pixel range is out of bounds */
+    unsigned long long *counters; /* [0] listed, [1] hp updates, [4] segments, [5] FP64 fallbacks */
+    unsigned long long *err;      /* sharded: pairs whose halo or rows are out of bounds */
     unsigned long long *n_lost;   /* sharded: tiles marked lost */
 };
 
 struct FallbackArgs {
-    const HaloRec *halos;         /* records in slot order */
-    const uint32_t *order;        /* spatial position -> slot */
+    const HaloRec *halos;
     const uint4 *fb;
     const unsigned long long *fb_count;
     int64_t fb_cap;
@@ -149,10 +147,10 @@ struct FallbackArgs {
     uint32_t *count;
     unsigned long long *hash;
     const uint8_t *lost;          /* per tile: entries of a lost tile are skipped (it is painted again) */
-    const int32_t *tile_base;     /* first tile of ring r+1 */
-    int32_t log2w;
+    const TileDesc *desc;
+    int64_t n_tiles;
     int64_t n_halo;
-    unsigned long long *counters; /* [1] hp updates */
+    unsigned long long *counters; /* [0] listed, [1] hp updates */
     unsigned long long *err;      /* sharded: entries whose halo is out of range */
 };
 
@@ -166,21 +164,20 @@ void p2m_launch_paint_plain_hp(const PaintArgs &a, hipStream_t s);
 void p2m_launch_paint_fs(const PaintArgs &a, int plain, hipStream_t s);
 void p2m_launch_fs_counts(const PaintArgs &a, hipStream_t s);
 void p2m_launch_fs_paint(const PaintArgs &a, hipStream_t s);
-void p2m_launch_ring_counts(const BinArgs &b, hipStream_t s);
-void p2m_launch_ring_z(int32_t nside, double *z, hipStream_t s);
-void p2m_launch_tile_desc(int32_t nside, int32_t log2w, int64_t n_tiles, const int32_t *tile_ring,
-                          const int32_t *tile_base, TileDesc *desc, hipStream_t s);
-void p2m_launch_seg_count(const BinArgs &b, hipStream_t s);
-void p2m_launch_seg_emit(const BinArgs &b, hipStream_t s);
-uint32_t p2m_key_max(int32_t nside, int32_t nphi);
-int p2m_sort_halos(const HaloRec *in, int64_t n, uint32_t key_max, BinHalo *bin, TileHalo *hot, HaloRec *full,
-                   int32_t nrt, int32_t nmht, uint32_t *keys, uint32_t *vals, void *tmp, size_t *tmp_bytes,
-                   uint32_t *nr, hipStream_t s);
+void p2m_launch_pair_count(const BinArgs &b, hipStream_t s);
+void p2m_launch_ring_gaps(const BinArgs &b, hipStream_t s);
+void p2m_launch_pair_emit(const BinArgs &b, hipStream_t s);
+void p2m_launch_tile_bounds(const uint32_t *keys, unsigned long long n, int64_t n_tiles, unsigned long long *tile_off,
+                            hipStream_t s);
+int p2m_sort_pairs(uint32_t *keys, uint32_t *vals, unsigned long long n, int64_t n_tiles, void *tmp, size_t *tmp_bytes,
+                   hipStream_t s);
+void p2m_launch_ring_desc(int32_t nside, RingDesc *out, hipStream_t s);
+void p2m_launch_tile_desc(const TileShape &g, const int32_t *band_tile, TileDesc *desc, hipStream_t s);
 int p2m_scan_u32(const uint32_t *cnt, unsigned long long *off, int64_t n, void *tmp, size_t *tmp_bytes, hipStream_t s);
 int p2m_tile_max_log2w(void);
 void p2m_launch_build_quad(const float *slice, int64_t n_slice, int32_t nrt, int32_t nmht, int32_t nchit,
                            int32_t n_maps, int32_t slot, float *quad, hipStream_t s);
-size_t p2m_tile_lds_bytes(int mode, int n_maps, int log2w, int membership, int nrt);
+size_t p2m_tile_lds_bytes(int mode, int n_maps, int log2w, int membership, int nrt, int wg);
 int p2m_tile_occupancy(int mode, int n_maps, int wg, size_t lds);
 int p2m_launch_tile_paint(const TileArgs &a, int mode, int n_maps, int grid, int wg, hipStream_t s);
 int p2m_launch_fallback(const FallbackArgs &a, int64_t n_max, hipStream_t s);

@@ -5,16 +5,13 @@
  *                    then the FP64 per-halo setup of the survivors
  *                    (pks2map.f90:144-160, 264, 284-298; haloproject.f90:47-55,
  *                    93-128; maptable.f90:184-202; query_disc prologue)
- *  k_gather_halos    the survivors in spatial order (band of rings x azimuth),
- *                    packed for the binning and the FP32 painter, with each
- *                    halo's (halo, ring) item count
- *  k_ring_counts (a pass with no painted halo), k_group_heads, k_seg_count,
- *  k_seg_emit
- *                    bin the (halo, ring) pixel runs of query_disc into ring
- *                    tiles of W pixels (pix_tools.F90:712-800,
- *                    pixel_routines.F90:1823-1879)
- *  k_tile_fast       FP32 painter: workgroups take ring tiles from a queue per
- *                    XCD; per pixel the FP32 chord^2 test and profile value,
+ *  k_pair_count, k_pair_emit, k_tile_bounds
+ *                    (halo, tile) pairs of the painted halos, radix-sorted by
+ *                    tile: tiles are 16 rings by a sector of azimuth
+ *  k_tile_fast       FP32 painter: workgroups take tiles from a queue per
+ *                    XCD, their waves the halos' pixel runs on the tile's rings
+ *                    (pix_tools.F90:712-800, pixel_routines.F90:1823-1879);
+ *                    per pixel the FP32 chord^2 test and profile value,
  *                    summed in an FP64 LDS tile and written once as FP32;
  *                    pixels near a disc edge or a table-cell edge go to
  *  k_fallback        the exact FP64 decision and value (haloproject.f90:60-75,
@@ -31,7 +28,6 @@
  *  k_moments         map moments and the dP/dy histogram (pks2map.f90:321-357)
  */
 #include "p2m_kernels.h"
-#include "p2m_pieces.h"
 
 #include <hipcub/hipcub.hpp>
 #include <type_traits>
@@ -230,12 +226,14 @@ __global__ void __launch_bounds__(256) k_setup(DecodeArgs A)
     const CosmoDev &c = A.c;
     const TabGeom &g = A.g;
     __shared__ unsigned long long lds16[16];
-    unsigned long long tot_rad = 0, tot_rings = 0;
+    unsigned long long tot_rad = 0, tot_pairs = 0, tot_pix = 0, tot_gaps = 0;
     const unsigned long long kbeg = *A.n_cand0, kend = *A.n_cand;
     for (unsigned long long k0 = kbeg + blockIdx.x * (unsigned long long)blockDim.x; k0 < kend;
          k0 += (unsigned long long)gridDim.x * blockDim.x) {
         const unsigned long long k = k0 + threadIdx.x;
         bool painted = false;
+        uint32_t rings = 1u;               /* rings the disc meets: none (first 1, last 0) */
+        double ztop = 1.0, zbot = -1.0;
         HaloRec h;
         if (k < kend) {
             const int64_t i = A.cand[k];
@@ -273,6 +271,7 @@ __global__ void __launch_bounds__(256) k_setup(DecodeArgs A)
                 const double norm = p2m_sqrt((h.hx * h.hx + h.hy * h.hy) + h.hz * h.hz);
                 const double z0 = h.hz / norm;
                 h.irmin = 0; h.irmax = -1;
+                rings = 1u;
                 if (A.nside > 0) {
                     const double rlat0 = p2m_asin(z0);
                     const double rlat1 = rlat0 + dtheta, rlat2 = rlat0 - dtheta;
@@ -282,6 +281,8 @@ __global__ void __launch_bounds__(256) k_setup(DecodeArgs A)
                     const double zmin = (rlat2 <= -HPX_HALFPI) ? -1.0 : p2m_sin(rlat2);
                     const int32_t irmax = ring_num(A.nside, zmin);
                     h.irmax = irmax + 1 < 4 * A.nside - 1 ? irmax + 1 : 4 * A.nside - 1;
+                    rings = disc_rings(A.nside, zmax, zmin, h.irmin, h.irmax);
+                    ztop = zmax; zbot = zmin;
                 }
                 h.cosang = p2m_cos(dtheta);
                 const double x0 = h.hx / norm, y0 = h.hy / norm;
@@ -329,30 +330,46 @@ __global__ void __launch_bounds__(256) k_setup(DecodeArgs A)
             }
         }
         const bool flat = k < kend && painted && h.flat;
-        /* (halo, ring) items of this record, as the binning counts them */
-        if (k < kend && k < (unsigned long long)A.cap) tot_rings += h.irmax >= h.irmin ? (unsigned long long)(h.irmax - h.irmin + 1) : 1ULL;
         if (k < kend && k < (unsigned long long)A.cap) {
             A.out[k] = h;
-            if (A.keys) {
-                /* spatial key: band of 8 rings of the disc centre, then its azimuth bin */
-                uint32_t key = A.key_max;
-                if (painted && A.nside > 0) {
-                    const int32_t rc = ring_num(A.nside, h.zz0);
-                    double ph = h.phi0;
-                    if (ph < 0.0) ph += HPX_TWOPI;
-                    int32_t pb = (int32_t)(ph * (double)A.nphi / HPX_TWOPI);
-                    pb = pb < 0 ? 0 : (pb >= A.nphi ? A.nphi - 1 : pb);
-                    key = (uint32_t)((rc - 1) >> 3) * (uint32_t)A.nphi + (uint32_t)pb;
-                }
-                A.keys[k] = key;
-                A.vals[k] = (uint32_t)k;
+            if (A.hot) {
+                TileHalo t;
+                t.zz0 = h.zz0; t.s0 = h.s0; t.phi0 = h.phi0; t.thr = h.thr;
+                t.thr_hi = (float)(h.thr * (1.0 + CHORD_BAND));
+                t.chi2 = (float)(h.chi_r * h.chi_r);
+                const float v = h.chi_out ? 0.0f : (float)h.vh, fc = (float)h.fc, fm = (float)h.fm;
+                t.w00 = v * ((1.0f - fc) * (1.0f - fm));
+                t.w10 = v * (fc * (1.0f - fm));
+                t.w01 = v * ((1.0f - fc) * fm);
+                t.w11 = v * (fc * fm);
+                /* a halo beyond the table's chi range paints zeros (weights 0); its
+                 * cell indices may lie outside the table, so point it at column 0 */
+                t.colbase = h.chi_out ? 0 : g.nrt * ((h.imh - 1) + g.nmht * (h.ichi - 1));
+                t.pad = 0;
+                A.hot[k] = t;
+            }
+            if (A.pair_halo) {
+                PairHalo q;
+                q.turn = (float)(h.phi0 * (1.0 / HPX_TWOPI));
+                q.half = disc_half_turn(h.thr, h.s0);
+                q.rings = rings;
+                if (gaps_possible(A.nside, ztop, zbot, h.a, q.half, rings)) { q.rings |= RINGS_ASK_GAPS; tot_gaps++; }
+                A.pair_halo[k] = q;
+                uint32_t np = 0;
+                halo_tiles(A.shape, q.turn, q.half, rings, [&](int32_t, int32_t, int32_t, int32_t) { ++np; });
+                A.n_pairs[k] = np;
+                tot_pairs += np;
+                /* pixels of the disc, about: its share of the sphere is chord^2 / 4 */
+                if (painted) tot_pix += 1ULL + (unsigned long long)(3.0 * A.nside * A.nside * h.thr);
             }
         }
         const unsigned long long fs = wave_append(A.n_flat_out, flat);
         if (flat) A.flat_idx[fs] = (uint32_t)k;
     }
     block_count(&A.counters[2], tot_rad, lds16);
-    block_count(&A.counters[3], tot_rings, lds16);
+    block_count(&A.counters[3], tot_pairs, lds16);
+    block_count(&A.counters[14], tot_pix, lds16);
+    block_count(&A.counters[10], tot_gaps, lds16);
 }
 
 /* n_cand0 <- n_cand: the first candidate slot of the next chunk */
@@ -551,428 +568,112 @@ void p2m_launch_fs_paint(const PaintArgs &a, hipStream_t s)
 }
 
 /* ===================================================================== */
-/* binning of (halo, ring) runs into ring tiles                           */
+/* binning of halos into tiles                                            */
 /* ===================================================================== */
 
-__global__ void __launch_bounds__(256) k_ring_counts(BinArgs B)
+/* A painted halo reaches few tiles (about two at 1024 pixels, where its
+ * disc covers 13 rings on average), so the binning works on (halo, tile)
+ * pairs: they are counted per halo, listed in halo order with the tile as
+ * key, and radix-sorted by tile.  A pair's key holds the halo's rows in that
+ * tile below the tile's number, key = tile << 8 | first row << 4 | rows - 1,
+ * and only the tile's bits are sorted; its value is the halo's slot.  What a
+ * halo covers of a row is left to the painter, which has the row's geometry
+ * and the halo's constants at hand.
+ *
+ * Before, the (halo, ring) runs of every disc were cut at ring tiles,
+ * counted per tile through an LDS hash and scattered: 13 items a halo, two
+ * passes bound by load latency and LDS atomics.  Binning time, scans and sort
+ * included: 2e7 halos at nside 4096, 2.2e6 painted, 1.35 -> 0.39 ms; 2e7
+ * heavy halos at nside 2048, 1.7e7 painted, 6.0 -> 1.4 ms; 4e7 at nside 4096
+ * 17.9 -> 3.5 ms. */
+/* the fields of a record that the exact disc query reads */
+struct DiscRec { double cosang, zz0, a, phi0; };
+__device__ static inline DiscRec disc_rec(const HaloRec &h) { return {h.cosang, h.zz0, h.a, h.phi0}; }
+
+/* ring gaps of the halos marked RINGS_ASK_GAPS (launched only where the
+ * setup marked any) */
+__global__ void __launch_bounds__(256) k_ring_gaps(BinArgs B)
 {
-    for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i <= B.n_halo; i += (int64_t)gridDim.x * blockDim.x) {
-        uint32_t nr = 0;
-        if (i < B.n_halo) {
-            const BinHalo &h = B.halos[i];
-            nr = h.irmax >= h.irmin ? (uint32_t)(h.irmax - h.irmin + 1) : 1u;
-        }
-        B.nr[i] = nr;
-    }
-}
-
-/* Segment slots are assigned per workgroup through an LDS hash table keyed
- * by tile: a chunk of BIN_CH consecutive (halo, ring) items touches few
- * distinct tiles once the halos are in spatial order, so one global atomic
- * per (chunk, tile) reserves the slots of all its pieces.  A piece whose
- * tile finds no hash slot within BIN_PROBE probes takes one global atomic
- * of its own. */
-static_assert(offsetof(BinHalo, cosang) == 0 && offsetof(BinHalo, zz0) == 8 && offsetof(BinHalo, a) == 16 &&
-              offsetof(BinHalo, phi0) == 24 && offsetof(BinHalo, irmin) == 32 && offsetof(BinHalo, irmax) == 36 &&
-              sizeof(BinHalo) == 40, "BinHalo layout read by k_seg_count");
-
-#define BIN_CH 1024
-#define BIN_HASH 1024
-#define BIN_HASH_BITS 10
-#define BIN_PROBE 32
-#define BIN_EMPTY 0xffffffffu
-#define BIN_DIRECT 0x80000000u
-
-struct BinHash {
-    uint32_t key[BIN_HASH];
-    uint32_t cnt[BIN_HASH];
-};
-
-struct CountLDS : BinHash {
-    uint32_t prec[BIN_CH];       /* per item of the chunk: its first piece's slot code */
-};
-
-__device__ static inline int bin_slot(BinHash *L, uint32_t tile)
-{
-    uint32_t h = (tile * 2654435761u) >> (32 - BIN_HASH_BITS);
-    for (int k = 0; k < BIN_PROBE; ++k) {
-        const uint32_t prev = atomicCAS(&L->key[h], BIN_EMPTY, tile);
-        if (prev == BIN_EMPTY || prev == tile) return (int)h;
-        h = (h + 1) & (BIN_HASH - 1);
-    }
-    return -1;
-}
-
-__device__ static inline void bin_reset(BinHash *L)
-{
-    for (int k = threadIdx.x; k < BIN_HASH; k += blockDim.x) { L->key[k] = BIN_EMPTY; L->cnt[k] = 0; }
-}
-
-/* the items [start, end) of one wave (start a multiple of 64), with their
- * halo and ring offset: f(item, halo, k) for each item of this lane.  The
- * halo holding item 64g is group_halo[g]; the 64 items of a group span at
- * most 64 halos (every halo has at least one ring), so each lane finds its
- * halo by a 6-step shuffle search over off[h .. h+63]. */
-template <typename F>
-__device__ static inline void wave_range(const unsigned long long *off, const uint32_t *group_halo, int64_t n_halo,
-                                         unsigned long long start, unsigned long long end, F f)
-{
-    const int lane = __lane_id();
-    for (unsigned long long c = start; c < end; c += 64) {
-        const int64_t h = group_halo[c >> 6];
-        const unsigned long long item = c + lane;
-        const int64_t hl = h + lane;
-        const unsigned long long my_off = hl <= n_halo ? off[hl] : ~0ULL;
-        int j = 0;
-        for (int step = 32; step > 0; step >>= 1) {
-            unsigned long long o = __shfl(my_off, j + step);
-            if (o <= item) j += step;
-        }
-        const unsigned long long hoff = __shfl(my_off, j);
-        if (item < end) f(item, h + j, item - hoff);
-    }
-}
-
-/* z of every ring centre (ring2z) */
-__global__ void k_ring_z(int32_t nside, double *z)
-{
-    const int32_t r = blockIdx.x * blockDim.x + threadIdx.x + 1;
-    if (r <= 4 * nside - 1) z[r - 1] = ring2z(nside, r);
-}
-
-void p2m_launch_ring_z(int32_t nside, double *z, hipStream_t s)
-{
-    const int n = 4 * nside - 1;
-    hipLaunchKernelGGL(k_ring_z, dim3((n + 255) / 256), dim3(256), 0, s, nside, z);
-}
-
-/* group_halo[g] = the halo holding item 64 g */
-__global__ void __launch_bounds__(256) k_group_heads(BinArgs B)
-{
-    for (int64_t h = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; h < B.n_halo; h += (int64_t)gridDim.x * blockDim.x) {
-        const unsigned long long g0 = (B.ring_off[h] + 63) >> 6, g1 = (B.ring_off[h + 1] + 63) >> 6;
-        for (unsigned long long g = g0; g < g1; ++g) B.group_halo[g] = (uint32_t)h;
-    }
-}
-
-/* Per (halo, ring) item: the query_disc pixel run, its tile pieces and the
- * slot of each piece within its tile's segment list.  The first piece's slot
- * code is (hash slot << 16 | rank within the chunk's pieces of that tile)
- * until the chunk reserves its range in the tile, BIN_DIRECT | slot when
- * reserved on its own, BIN_EMPTY for none.  Later pieces (runs crossing a
- * tile boundary, about 8% of the items) take their slot on their own and are
- * listed in ovf with it. */
-__device__ static inline uint32_t slot_of(const BinHash &L, uint32_t code)
-{
-    if (code == BIN_EMPTY) return 0u;
-    if (code & BIN_DIRECT) return code & ~BIN_DIRECT;
-    return L.cnt[code >> 16] + (code & 0xffffu);
-}
-
-/* XCD-aware split of n work units over the grid: workgroup b runs on XCD
- * b % 8, and the workgroups of one XCD take one contiguous eighth of the
- * units, so the units in flight on an XCD are spatial neighbours whose tile
- * lists meet in its L2 (whole lines written before they leave it). */
-__device__ static inline void xcd_range(unsigned long long n, unsigned long long &beg, unsigned long long &end,
-                                        unsigned long long &step, unsigned long long lane_units, unsigned long long unit)
-{
-    const bool xcd = (gridDim.x % 8) == 0 && n >= 8;
-    const unsigned long long per_wg = lane_units;     /* units a workgroup takes per step */
-    if (xcd) {
-        const unsigned long long x = blockIdx.x % 8, l = blockIdx.x / 8;
-        beg = x * n / 8 + l * per_wg + unit;
-        end = (x + 1) * n / 8;
-        step = (unsigned long long)(gridDim.x / 8) * per_wg;
-    } else {
-        beg = (unsigned long long)blockIdx.x * per_wg + unit;
-        end = n;
-        step = (unsigned long long)gridDim.x * per_wg;
-    }
-}
-
-/* eight waves per SIMD (64 VGPRs, a few spilled): the pass waits on loads
- * and LDS atomics far more than it computes, so occupancy pays */
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8))) k_seg_count(BinArgs B)
-{
-    __shared__ CountLDS L;
     __shared__ unsigned long long lds16[16];
-    unsigned long long n_list = 0, n_seg = 0;
-    const unsigned long long nchunk = (B.n_items + BIN_CH - 1) / BIN_CH;
-    bin_reset(&L);
-    __syncthreads();
-    const int wv = threadIdx.x >> 6, nwv = blockDim.x >> 6;
-    const unsigned long long per = BIN_CH / nwv;
-    unsigned long long cbeg, cend, cstep;
-    xcd_range(nchunk, cbeg, cend, cstep, 1, 0);
-    for (unsigned long long ch = cbeg; ch < cend; ch += cstep) {
-        const unsigned long long c0 = ch * BIN_CH;
-        unsigned long long a = c0 + wv * per, e = a + per;
-        if (e > B.n_items) e = B.n_items;
-        wave_range(B.ring_off, B.group_halo, B.n_halo, a, e, [&](unsigned long long item, int64_t hi, unsigned long long k) {
-            const uint2 *hs = reinterpret_cast<const uint2 *>(B.halos + hi);
-            const uint2 q0 = hs[0], q1 = hs[1], q2 = hs[2], q3 = hs[3], q4 = hs[4];
-            pin2(q0); pin2(q1); pin2(q2); pin2(q3); pin2(q4);
-            BinHalo h;
-            h.cosang = dbl_of(q0.x, q0.y); h.zz0 = dbl_of(q1.x, q1.y);
-            h.a = dbl_of(q2.x, q2.y); h.phi0 = dbl_of(q3.x, q3.y);
-            h.irmin = (int32_t)q4.x; h.irmax = (int32_t)q4.y;
-            const int32_t ring = h.irmin + (int32_t)k;
-            int32_t lo = 0, np = 0;
-            int32_t npr, kshift; int64_t first;
-            if (ring <= h.irmax) {
-                ring_info(B.nside, ring, npr, kshift, first);
-                np = disc_ring_run_fast(h, B.ring_z[ring - 1], npr, kshift, lo);
+    unsigned long long gaps = 0;
+    for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < B.n_halo; i += (int64_t)gridDim.x * blockDim.x) {
+        const uint32_t rings = B.halos[i].rings;
+        if (rings & RINGS_ASK_GAPS) gaps += (unsigned long long)ring_gaps(disc_rec(B.recs[i]), B.shape.nside, rings & ~RINGS_ASK_GAPS);
+    }
+    block_count(&B.counters[3], gaps, lds16);
+}
+
+__global__ void __launch_bounds__(256) k_pair_count(BinArgs B)
+{
+    for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < B.n_halo; i += (int64_t)gridDim.x * blockDim.x) {
+        const PairHalo h = B.halos[i];
+        uint32_t n = 0;
+        halo_tiles(B.shape, h.turn, h.half, h.rings, [&](int32_t, int32_t, int32_t, int32_t) { ++n; });
+        B.n_pairs[i] = n;
+    }
+}
+
+__global__ void __launch_bounds__(256) k_pair_emit(BinArgs B)
+{
+    for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < B.n_halo; i += (int64_t)gridDim.x * blockDim.x) {
+        const PairHalo h = B.halos[i];
+        unsigned long long o = B.pair_off[i];
+        halo_tiles(B.shape, h.turn, h.half, h.rings, [&](int32_t band, int32_t k, int32_t row, int32_t rows) {
+            if (o < B.pair_cap) {
+                B.keys[o] = ((uint32_t)(B.band_tile[band] + k) << 8) | ((uint32_t)row << 4) | (uint32_t)(rows - 1);
+                B.vals[o] = (uint32_t)i;
             }
-            /* first pixel | count << 16: lo < npr and np <= npr <= 32768 for nside <= 8192 */
-            B.runs[item] = (uint32_t)lo | ((uint32_t)np << 16);
-            uint32_t code = BIN_EMPTY;
-            if (np > 0) {
-                n_list += (unsigned long long)np;
-                int j = 0;
-                run_pieces(lo, np, npr, B.tile_base[ring - 1], B.log2w, [&](int32_t tile, int32_t plo, int32_t len) {
-                    const int sl = j == 0 ? bin_slot(&L, (uint32_t)tile) : -1;
-                    if (sl >= 0) {
-                        code = ((uint32_t)sl << 16) | atomicAdd(&L.cnt[sl], 1u);
-                    } else {
-                        const uint32_t slot = atomicAdd(&B.tile_cnt[tile], 1u);
-                        if (j == 0) {
-                            code = BIN_DIRECT | slot;
-                        } else {
-                            const unsigned long long o = atomicAdd(B.n_ovf, 1ULL);
-                            if (o < (unsigned long long)B.ovf_cap)
-                                B.ovf[o] = make_uint4((uint32_t)tile, slot, (uint32_t)hi, ((uint32_t)plo << 16) | (uint32_t)len);
-                        }
-                    }
-                    ++j;
-                    n_seg++;
-                });
-            }
-            L.prec[item - c0] = code;
+            ++o;
         });
-        __syncthreads();
-        /* reserve each (chunk, tile) range; cnt[] then holds its first slot */
-        for (int k = threadIdx.x; k < BIN_HASH; k += blockDim.x)
-            if (L.key[k] != BIN_EMPTY) L.cnt[k] = atomicAdd(&B.tile_cnt[L.key[k]], L.cnt[k]);
-        __syncthreads();
-        const unsigned long long nin = B.n_items - c0 < BIN_CH ? B.n_items - c0 : BIN_CH;
-        for (unsigned long long k = threadIdx.x; k < nin; k += blockDim.x) B.pos[c0 + k] = slot_of(L, L.prec[k]);
-        __syncthreads();
-        bin_reset(&L);
-        __syncthreads();
-    }
-    block_count(&B.counters[0], n_list, lds16);
-    block_count(&B.counters[4], n_seg, lds16);
-}
-
-/* Scatter of every piece to its slot: segs[tile_off[tile] + slot].  A wave
- * takes 128 consecutive items, two per lane, with the loads of both issued
- * before either is used (the pass is bound by load latency); the pieces
- * after an item's first come from ovf. */
-#define EMIT_U 2
-__global__ void __launch_bounds__(256) k_seg_emit(BinArgs B)
-{
-    __shared__ unsigned long long lds16[16];
-    unsigned long long n_gaps = 0, n_err = 0;
-    const int lane = __lane_id();
-    const unsigned long long nunit = (B.n_items + 64 * EMIT_U - 1) / (64 * EMIT_U);
-    unsigned long long ubeg, uend, ustep;
-    xcd_range(nunit, ubeg, uend, ustep, blockDim.x >> 6, threadIdx.x >> 6);
-    for (unsigned long long un = ubeg; un < uend; un += ustep) {
-        const unsigned long long base = un * (64 * EMIT_U);
-        unsigned long long item[EMIT_U];
-        uint32_t run[EMIT_U], ps[EMIT_U];
-        int64_t hgrp[EMIT_U];
-        unsigned long long off[EMIT_U];
-#pragma unroll
-        for (int u = 0; u < EMIT_U; ++u) {
-            item[u] = base + 64 * u + lane;
-            const unsigned long long it = item[u] < B.n_items ? item[u] : B.n_items - 1;
-            run[u] = B.runs[it];
-            ps[u] = B.pos[it];
-            unsigned long long c = base + 64 * u;
-            if (c >= B.n_items) c = (B.n_items - 1) & ~63ULL;
-            hgrp[u] = B.group_halo[c >> 6];
-        }
-#pragma unroll
-        for (int u = 0; u < EMIT_U; ++u) {
-            const int64_t hl = hgrp[u] + lane;
-            off[u] = hl <= B.n_halo ? B.ring_off[hl] : ~0ULL;
-        }
-        int64_t hi[EMIT_U];
-        unsigned long long kk[EMIT_U];
-#pragma unroll
-        for (int u = 0; u < EMIT_U; ++u) {
-            int j = 0;
-            for (int step = 32; step > 0; step >>= 1) {
-                const unsigned long long o = __shfl(off[u], j + step);
-                if (o <= item[u]) j += step;
-            }
-            hi[u] = hgrp[u] + j;
-            kk[u] = item[u] - __shfl(off[u], j);
-        }
-        int32_t tb[EMIT_U], npr[EMIT_U];
-#pragma unroll
-        for (int u = 0; u < EMIT_U; ++u) {
-            const int64_t h = hi[u] < B.n_halo ? hi[u] : B.n_halo - 1;
-            int32_t ring = B.halos[h].irmin + (int32_t)kk[u];
-            ring = ring < 1 ? 1 : (ring > 4 * B.nside - 1 ? 4 * B.nside - 1 : ring);
-            int32_t kshift; int64_t first;
-            ring_info(B.nside, ring, npr[u], kshift, first);
-            tb[u] = B.tile_base[ring - 1];
-        }
-        int32_t tile[EMIT_U][2], plo[EMIT_U][2], len[EMIT_U][2];
-        bool live[EMIT_U];
-        unsigned long long to[EMIT_U], tn[EMIT_U];
-#pragma unroll
-        for (int u = 0; u < EMIT_U; ++u) {
-            const int32_t np = (int32_t)(run[u] >> 16);
-            live[u] = item[u] < B.n_items && np != 0;
-            if (live[u]) first_two_pieces((int32_t)(run[u] & 0xffffu), np, npr[u], tb[u], B.log2w, tile[u], plo[u], len[u]);
-            const int64_t tl = live[u] && tile[u][0] >= 0 && tile[u][0] < B.n_tiles ? tile[u][0] : 0;
-            to[u] = live[u] ? B.tile_off[tl] : 0;
-            tn[u] = live[u] ? B.tile_off[tl + 1] : 0;
-        }
-        /* a slot outside its tile's range is an error, never a store */
-#pragma unroll
-        for (int u = 0; u < EMIT_U; ++u) {
-            if (!live[u]) continue;
-            if (tile[u][0] < 0 || tile[u][0] >= B.n_tiles || to[u] + ps[u] >= tn[u]) { n_err++; continue; }
-            B.segs[to[u] + ps[u]] = make_uint2((uint32_t)hi[u], ((uint32_t)plo[u][0] << 16) | (uint32_t)len[u][0]);
-        }
-        /* an empty ring between non-empty rings of one disc, counted once per
-         * gap (the row misalignment of discedge2fulldisc, quirk Q15) */
-#pragma unroll
-        for (int u = 0; u < EMIT_U; ++u) {
-            if (item[u] < B.n_items && (run[u] >> 16) == 0 && kk[u] > 0 && (B.runs[item[u] - 1] >> 16) != 0) {
-                const unsigned long long endi = B.ring_off[hi[u] + 1];
-                for (unsigned long long j = item[u] + 1; j < endi; ++j)
-                    if ((B.runs[j] >> 16) != 0) { n_gaps++; break; }
-            }
-        }
-    }
-    const unsigned long long nov = *B.n_ovf < (unsigned long long)B.ovf_cap ? *B.n_ovf : (unsigned long long)B.ovf_cap;
-    for (unsigned long long o = (unsigned long long)blockIdx.x * blockDim.x + threadIdx.x; o < nov;
-         o += (unsigned long long)gridDim.x * blockDim.x) {
-        const uint4 v = B.ovf[o];
-        if (v.x >= (uint64_t)B.n_tiles || B.tile_off[v.x] + v.y >= B.tile_off[v.x + 1]) { n_err++; continue; }
-        B.segs[B.tile_off[v.x] + v.y] = make_uint2(v.z, v.w);
-    }
-    block_count(&B.counters[3], n_gaps, lds16);
-    block_count(B.err, n_err, lds16);
-}
-
-/* ------------------------------------------------------------------ */
-/* spatial order of the painted halos                                  */
-/* ------------------------------------------------------------------ */
-
-/* The fields read here lie in bytes [32, 112) and [128, 160) of the
- * 176-B record.  They are fetched with seven 16-B loads issued together and
- * one wait (field by field, the compiler put the loads of the FP32 fields
- * behind branches on chi_out, a memory round trip each). */
-static_assert(offsetof(HaloRec, hx) == 0 && offsetof(HaloRec, hy) == 8 && offsetof(HaloRec, hz) == 16 &&
-              offsetof(HaloRec, dtheta) == 24, "HaloRec layout read by k_fallback");
-static_assert(offsetof(HaloRec, zz0) == 32 && offsetof(HaloRec, phi0) == 40 && offsetof(HaloRec, a) == 48 &&
-              offsetof(HaloRec, cosang) == 56 && offsetof(HaloRec, s0) == 64 && offsetof(HaloRec, thr) == 72 &&
-              offsetof(HaloRec, chi_r) == 80 && offsetof(HaloRec, fc) == 88 && offsetof(HaloRec, fm) == 96 &&
-              offsetof(HaloRec, vh) == 104 && offsetof(HaloRec, cat) == 128 && offsetof(HaloRec, ichi) == 136 &&
-              offsetof(HaloRec, imh) == 140 && offsetof(HaloRec, irmin) == 144 && offsetof(HaloRec, irmax) == 148 &&
-              offsetof(HaloRec, chi_out) == 152 && sizeof(HaloRec) == 176, "HaloRec layout read by k_gather_halos");
-
-__global__ void __launch_bounds__(256) k_gather_halos(const HaloRec *in, const uint32_t *order, int64_t n,
-                                                      BinHalo *bin, TileHalo *hot, HaloRec *full, int32_t nrt, int32_t nmht,
-                                                      uint32_t *nr)
-{
-    /* nr: the (halo, ring) items of every halo in spatial order (its ring
-     * range, or one item for an inert record), and 0 after the last, as
-     * the scan into ring offsets needs */
-    if (blockIdx.x == 0 && threadIdx.x == 0) nr[n] = 0;
-    for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) {
-        const uint32_t o = order[i];
-        const uint4 *src = reinterpret_cast<const uint4 *>(in + o);
-        const uint4 c2 = src[2], c3 = src[3], c4 = src[4], c5 = src[5], c6 = src[6], c8 = src[8], c9 = src[9];
-        const double zz0 = dbl_of(c2.x, c2.y), phi0 = dbl_of(c2.z, c2.w);
-        const double a = dbl_of(c3.x, c3.y), cosang = dbl_of(c3.z, c3.w);
-        const double s0 = dbl_of(c4.x, c4.y), thr = dbl_of(c4.z, c4.w);
-        const double chi_r = dbl_of(c5.x, c5.y), fc = dbl_of(c5.z, c5.w);
-        const double fm = dbl_of(c6.x, c6.y), vh = dbl_of(c6.z, c6.w);
-        const int64_t cat = (int64_t)(((unsigned long long)c8.y << 32) | c8.x);
-        const int32_t ichi = (int32_t)c8.z, imh = (int32_t)c8.w;
-        const int32_t irmin = (int32_t)c9.x, irmax = (int32_t)c9.y, chi_out = (int32_t)c9.z;
-        BinHalo b;
-        b.cosang = cosang; b.zz0 = zz0; b.a = a; b.phi0 = phi0;
-        b.irmin = irmin; b.irmax = irmax;
-        bin[i] = b;
-        nr[i] = irmax >= irmin ? (uint32_t)(irmax - irmin + 1) : 1u;
-        if (hot) {
-            TileHalo t;
-            t.zz0 = zz0; t.s0 = s0; t.phi0 = phi0; t.thr = thr;
-            t.chi2 = (float)(chi_r * chi_r);
-            t.vh = chi_out ? 0.0f : (float)vh;
-            t.fc = (float)fc; t.fm = (float)fm;
-            /* a halo beyond the table's chi range paints zeros (vh = 0); its
-             * cell indices may lie outside the table, so point it at column 0 */
-            t.colbase = chi_out ? 0 : nrt * ((imh - 1) + nmht * (ichi - 1));
-            t.pad = 0;
-            t.hash = halo_hash(cat);
-            hot[i] = t;
-        }
-        if (full) full[i] = in[o];
     }
 }
 
-/* the largest key: the last azimuth bin of the last band, which the inert
- * records share (their place in the order does not matter), so that the
- * keys of nside 4096 fit 16 bits (two radix passes) */
-uint32_t p2m_key_max(int32_t nside, int32_t nphi)
+/* tile_off[t] = the first sorted pair of tile t or a later one, by binary
+ * search (empty stretches of the sky leave long runs of equal offsets) */
+__global__ void __launch_bounds__(256) k_tile_bounds(const uint32_t *__restrict__ keys, unsigned long long n, int64_t n_tiles,
+                                                     unsigned long long *tile_off)
 {
-    const uint32_t nband = (uint32_t)((4 * nside - 2) >> 3) + 1;
-    return nband * (uint32_t)nphi - 1;
-}
-
-/* Sorts the records by the key k_setup wrote (stable radix sort of
- * (key, slot)), then writes the binning, FP32 and (if asked) full records
- * in that order.  keys and vals hold 2n entries: input then output. */
-int p2m_sort_halos(const HaloRec *in, int64_t n, uint32_t key_max, BinHalo *bin, TileHalo *hot, HaloRec *full,
-                   int32_t nrt, int32_t nmht, uint32_t *keys, uint32_t *vals, void *tmp, size_t *tmp_bytes,
-                   uint32_t *nr, hipStream_t s)
-{
-    int bits = 1;
-    while ((1u << bits) <= key_max && bits < 32) ++bits;
-    if (!tmp) {
-        hipError_t e = hipcub::DeviceRadixSort::SortPairs(nullptr, *tmp_bytes, keys, keys + n, vals, vals + n,
-                                                          (int)n, 0, bits, s);
-        return e == hipSuccess ? 0 : -1;
+    for (int64_t t = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; t <= n_tiles; t += (int64_t)gridDim.x * blockDim.x) {
+        unsigned long long lo = 0, hi = n;
+        while (lo < hi) {
+            const unsigned long long mid = (lo + hi) >> 1;
+            if ((int64_t)(keys[mid] >> 8) < t) lo = mid + 1; else hi = mid;
+        }
+        tile_off[t] = lo;
     }
-    if (n <= 0) return 0;
-    hipError_t e = hipcub::DeviceRadixSort::SortPairs(tmp, *tmp_bytes, keys, keys + n, vals, vals + n,
-                                                      (int)n, 0, bits, s);
-    if (e != hipSuccess) return -1;
-    unsigned g = (unsigned)std::min<int64_t>((n + 255) / 256, 8192);
-    hipLaunchKernelGGL(k_gather_halos, dim3(g), dim3(256), 0, s, in, vals + n, n, bin, hot, full, nrt, nmht, nr);
-    return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 
 static unsigned bin_grid(int64_t n) { int64_t g = (n + 255) / 256; return (unsigned)(g > 8192 ? 8192 : (g < 1 ? 1 : g)); }
-void p2m_launch_ring_counts(const BinArgs &b, hipStream_t s)
+void p2m_launch_pair_count(const BinArgs &b, hipStream_t s)
 {
-    hipLaunchKernelGGL(k_ring_counts, dim3(bin_grid(b.n_halo + 1)), dim3(256), 0, s, b);
+    if (b.n_halo > 0) hipLaunchKernelGGL(k_pair_count, dim3(bin_grid(b.n_halo)), dim3(256), 0, s, b);
 }
-static unsigned chunk_grid(unsigned long long n_items)
+void p2m_launch_ring_gaps(const BinArgs &b, hipStream_t s)
 {
-    unsigned long long g = (n_items + BIN_CH - 1) / BIN_CH;
-    if (g >= 8) g &= ~7ULL;      /* a multiple of 8 for the XCD-aware split */
-    return (unsigned)(g > 2048 ? 2048 : (g < 1 ? 1 : g));
+    if (b.n_halo > 0) hipLaunchKernelGGL(k_ring_gaps, dim3(bin_grid(b.n_halo)), dim3(256), 0, s, b);
 }
-void p2m_launch_seg_count(const BinArgs &b, hipStream_t s)
+void p2m_launch_pair_emit(const BinArgs &b, hipStream_t s)
 {
-    if (b.n_items == 0) return;
-    hipLaunchKernelGGL(k_group_heads, dim3(bin_grid(b.n_halo)), dim3(256), 0, s, b);
-    hipLaunchKernelGGL(k_seg_count, dim3(chunk_grid(b.n_items)), dim3(256), 0, s, b);
+    if (b.n_halo > 0) hipLaunchKernelGGL(k_pair_emit, dim3(bin_grid(b.n_halo)), dim3(256), 0, s, b);
 }
-void p2m_launch_seg_emit(const BinArgs &b, hipStream_t s)
+void p2m_launch_tile_bounds(const uint32_t *keys, unsigned long long n, int64_t n_tiles, unsigned long long *tile_off, hipStream_t s)
 {
-    if (b.n_items == 0) return;
-    hipLaunchKernelGGL(k_seg_emit, dim3(chunk_grid(b.n_items)), dim3(256), 0, s, b);
+    hipLaunchKernelGGL(k_tile_bounds, dim3(bin_grid(n_tiles + 1)), dim3(256), 0, s, keys, n, n_tiles, tile_off);
+}
+
+/* stable radix sort of the pairs by their tile: keys and vals hold 2n
+ * entries, input then output */
+int p2m_sort_pairs(uint32_t *keys, uint32_t *vals, unsigned long long n, int64_t n_tiles, void *tmp, size_t *tmp_bytes,
+                   hipStream_t s)
+{
+    int bits = 1;
+    while ((1LL << bits) < n_tiles && bits < 24) ++bits;
+    hipError_t e;
+    if (n <= (unsigned long long)INT32_MAX)
+        e = hipcub::DeviceRadixSort::SortPairs(tmp, *tmp_bytes, keys, keys + n, vals, vals + n, (int)n, 8, 8 + bits, s);
+    else
+        e = hipcub::DeviceRadixSort::SortPairs(tmp, *tmp_bytes, keys, keys + n, vals, vals + n, (size_t)n, 8, 8 + bits, s);
+    return e == hipSuccess ? 0 : -1;
 }
 
 /* exclusive scan of uint32 counts into uint64 offsets with a 64-bit accumulator */
@@ -982,13 +683,55 @@ int p2m_scan_u32(const uint32_t *cnt, unsigned long long *off, int64_t n, void *
     return e == hipSuccess ? 0 : -1;
 }
 
+/* geometry of every ring */
+__global__ void k_ring_desc(int32_t nside, RingDesc *out)
+{
+    const int32_t r = blockIdx.x * blockDim.x + threadIdx.x + 1;
+    if (r > 4 * nside - 1) return;
+    RingDesc d;
+    int32_t kshift;
+    double den;
+    ring_info(nside, r, d.npr, kshift, d.first);
+    ring_zsth(nside, r, d.zr, d.sth);
+    ring_phi_param(nside, r, d.off, den);
+    d.kphi = HPX_HALFPI / den;
+    d.e_row = (float)(2e-15 / (d.sth * d.sth));
+    d.pad = 0;
+    out[r - 1] = d;
+}
+
+void p2m_launch_ring_desc(int32_t nside, RingDesc *out, hipStream_t s)
+{
+    const int n = 4 * nside - 1;
+    hipLaunchKernelGGL(k_ring_desc, dim3((n + 255) / 256), dim3(256), 0, s, nside, out);
+}
+
+__global__ void __launch_bounds__(256) k_tile_desc(TileShape g, int32_t nb, const int32_t *band_tile, TileDesc *desc)
+{
+    const int32_t b = blockIdx.x;
+    if (b >= nb) return;
+    TileDesc d;
+    int32_t r1;
+    d.K = band_sectors(g, b, d.ring0, r1);
+    d.rows = r1 - d.ring0 + 1;
+    for (int32_t k = threadIdx.x; k < d.K; k += blockDim.x) {
+        d.k = k;
+        desc[band_tile[b] + k] = d;
+    }
+}
+
+void p2m_launch_tile_desc(const TileShape &g, const int32_t *band_tile, TileDesc *desc, hipStream_t s)
+{
+    const int32_t nb = n_bands(g);
+    if (nb > 0) hipLaunchKernelGGL(k_tile_desc, dim3((unsigned)nb), dim3(256), 0, s, g, nb, band_tile, desc);
+}
 
 /* ===================================================================== */
-/* tiled painter                                                          */
+/* tiled painters                                                         */
 /* ===================================================================== */
 
 /* ------------------------------------------------------------------ */
-/* tile painters: common parts                                          */
+/* common parts                                                         */
 /* ------------------------------------------------------------------ */
 
 /* Workgroup barrier for LDS traffic only: waits for this wave's LDS
@@ -1006,105 +749,180 @@ __device__ static inline void lds_barrier()
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
 }
 
-#define FSEG 256                   /* segments staged per batch */
-#define FB_LDS 32                  /* deferred pixels of a tile buffered in LDS (flushed per tile) */
-#define PMAX 3072                  /* pixels per batch (>= the widest tile, 2048) */
+/* The lanes of a wave that pass data through LDS without a barrier: LDS
+ * serves a wave's operations in order, but the compiler must not move a
+ * lane's loads over other lanes' stores. */
+__device__ static inline void wave_lds_fence()
+{
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
 
-/* the part of a batch both painters share: segment starts and the pixel
- * -> segment map */
-struct BatchLDS {
-    uint32_t pre[FSEG + 1];        /* exclusive scan of the staged lengths */
-    uint32_t seg_of[PMAX / 4];     /* batch pixel -> segment (bytes) */
-    uint32_t wsum[16];
-    uint32_t nb;
+#define ASK_RUN 0x80000000u        /* a deferred pixel's halo word: it must lie in the halo's exact run */
+#define COUNT_LISTED 0x80000000u   /* its row word: it is counted as listed if it does */
+#define WSEG 64                    /* segments a wave stages at a time */
+#define WPIX 4096                  /* pixels of a wave's bitmap of segment starts */
+#define FB_LDS 24                  /* deferred pixels of a tile buffered in LDS (flushed per tile) */
+#define MAXROWS 16
+
+/* a row of the tile: its ring's geometry and its pixels */
+struct __attribute__((aligned(16))) TileRow {
+    double zr, sth, kphi;
+    int64_t pix0;                  /* first map pixel */
+    uint16_t ip0, width;           /* first in-ring pixel, pixels */
+    int32_t npr;                   /* pixels of the ring (4 den: phi = (ip + off) pi/2 / den) */
+    float off, e_row;
+    __device__ double den() const { return (double)(npr >> 2); }
+    __device__ double ik() const { return den() * (2.0 / HPX_PI); }      /* 1 / kphi */
+    __device__ int32_t kshift() const { return off > 0.25f ? 1 : 0; }
 };
 
-__global__ void __launch_bounds__(256) k_tile_desc(int32_t nside, int32_t log2w, int64_t n_tiles, const int32_t *tile_ring,
-                                                   const int32_t *tile_base, TileDesc *desc)
+struct TileCtl {
+    TileRow rows[2][MAXROWS];
+    /* the per-tile control words and rows come in two slots, used by
+     * alternate tiles, so that a tile's end needs no barrier before the next
+     * begins */
+    uint32_t nfb[2];               /* deferred pixels of the tile */
+    uint32_t lost[2];              /* a deferred pixel of the tile found the list full */
+    int32_t next_tile[2];          /* the tile this workgroup paints next */
+    unsigned long long fb_base;    /* list slot of the tile's deferred pixels */
+    uint4 fb[FB_LDS];
+};
+
+__device__ static inline void stage_row(TileRow &R, const RingDesc &d, int32_t K, int32_t k)
 {
-    for (int64_t t = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; t < n_tiles; t += (int64_t)gridDim.x * blockDim.x) {
-        TileDesc d;
-        d.ring = tile_ring[t];
-        tile_span(nside, d.ring, (int32_t)(t - tile_base[d.ring - 1]), log2w, d.first, d.ip0, d.width);
-        ring_zsth(nside, d.ring, d.zr, d.sth);
-        ring_phi_param(nside, d.ring, d.off, d.den);
-        d.kphi = HPX_HALFPI / d.den;
-        d.pad = 0;
-        desc[t] = d;
-    }
+    const int32_t i0 = sector_start(d.npr, K, k);
+    R.zr = d.zr; R.sth = d.sth; R.kphi = d.kphi;
+    R.off = (float)d.off;
+    R.ip0 = (uint16_t)i0;
+    R.width = (uint16_t)(sector_start(d.npr, K, k + 1) - i0);
+    R.npr = d.npr;
+    R.pix0 = d.first + i0;
+    R.e_row = d.e_row;
 }
 
-void p2m_launch_tile_desc(int32_t nside, int32_t log2w, int64_t n_tiles, const int32_t *tile_ring,
-                          const int32_t *tile_base, TileDesc *desc, hipStream_t s)
+/* bitwise or over the wave, in every lane; all lanes active */
+__device__ static inline uint32_t wave_or(uint32_t v)
 {
-    if (n_tiles <= 0) return;
-    int64_t g = (n_tiles + 255) / 256;
-    if (g > 8192) g = 8192;
-    hipLaunchKernelGGL(k_tile_desc, dim3((unsigned)g), dim3(256), 0, s, nside, log2w, n_tiles, tile_ring, tile_base, desc);
+    v |= (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x111, 0xf, 0xf, false);   /* row_shr:1 */
+    v |= (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x112, 0xf, 0xf, false);   /* row_shr:2 */
+    v |= (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x114, 0xf, 0xf, false);   /* row_shr:4 */
+    v |= (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x118, 0xf, 0xf, false);   /* row_shr:8 */
+    v |= (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x142, 0xa, 0xf, false);   /* row_bcast:15 */
+    v |= (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x143, 0xc, 0xf, false);   /* row_bcast:31 */
+    return (uint32_t)__builtin_amdgcn_readlane((int)v, 63);
 }
 
-/* XCD-aware tile order: workgroup b runs on XCD b % 8; the workgroups of
- * one XCD sweep one contiguous eighth of the tiles (ring-major), so tiles in
- * flight on an XCD are neighbours that share halos in its L2. */
-__device__ static inline void tile_range(const TileArgs &A, int64_t &tbeg, int64_t &tend, int64_t &tstep)
+/* The (halo, row) segments of a wave's next pairs, one per lane: the leading
+ * pairs (key, val hold pair `lane`, has whether there is one) whose rows add
+ * up to at most WSEG.  Returns how many pairs were taken; every pair has 1 to
+ * 16 rows, so at least one is.  A lane's pair is found from the bits that the
+ * pairs set at their first lanes: the number of bits at or below the lane. */
+struct Seg {
+    uint32_t val;                  /* the pair's value */
+    int32_t row;                   /* row of the tile */
+    int32_t lane0, rows;           /* first lane and rows of the pair */
+    bool act;                      /* this lane holds a segment */
+};
+
+__device__ static inline int wave_segments(uint32_t key, uint32_t val, bool has, Seg &g)
 {
-    const bool xcd = (gridDim.x % 8) == 0 && A.n_tiles >= 8;
-    tstep = xcd ? gridDim.x / 8 : gridDim.x;
-    tbeg = xcd ? (int64_t)(blockIdx.x % 8) * A.n_tiles / 8 + blockIdx.x / 8 : blockIdx.x;
-    tend = xcd ? (int64_t)(blockIdx.x % 8 + 1) * A.n_tiles / 8 : A.n_tiles;
+    const int lane = __lane_id();
+    const uint32_t nr = has ? (key & 15u) + 1u : 0u;
+    const uint32_t incl = wave_incl_scan(nr), excl = incl - nr;
+    const bool take = has && incl <= WSEG;
+    const unsigned long long tm = __ballot(take);
+    const int n = __popcll(tm);
+    const int S = __builtin_amdgcn_readlane((int)incl, n - 1);
+    const uint32_t bit = take ? 1u << (excl & 31u) : 0u;
+    const uint32_t mlo = wave_or(excl < 32u ? bit : 0u), mhi = wave_or(excl < 32u ? 0u : bit);
+    const unsigned long long m = ((unsigned long long)mhi << 32) | mlo;
+    g.act = lane < S;
+    const int below = (int)__builtin_amdgcn_mbcnt_hi(mhi, __builtin_amdgcn_mbcnt_lo(mlo, 0u));
+    int j = below + (int)((m >> lane) & 1ULL) - 1;
+    j = j < 0 ? 0 : j;
+    g.val = __shfl(val, j);
+    const uint32_t pk = __shfl(excl | (((key >> 4) & 15u) << 8) | (nr << 16), j);
+    g.lane0 = (int32_t)(pk & 255u);
+    g.rows = (int32_t)(pk >> 16);
+    g.row = (int32_t)((pk >> 8) & 15u) + lane - g.lane0;
+    return n;
 }
 
-/* Given this thread's staged length (0 if none; nstage segments staged),
- * forms pre[], takes the leading segments whose pixels fit in PMAX (a
- * segment is at most W <= PMAX pixels, so at least one) and builds the
- * pixel -> segment map.  Returns the number of segments in the batch; P
- * receives its pixel count.  Every thread calls; ends with a barrier. */
-__device__ static inline int batch_prepare(BatchLDS *bl, uint32_t len, int nstage, uint32_t &P)
+/* The part of a run (lo, np > 0 of a ring of npr pixels) in a row of `width`
+ * pixels from ip0: in-row pixels [a, a + len), and how many of them the run
+ * holds.  A run that leaves the row and comes round into it again leaves a
+ * gap [c, d) in it (a sector is at most a quarter of its ring, so the run
+ * then covers three quarters): the segment is the whole row and hole is
+ * set. */
+__device__ static inline int32_t clip_run(int32_t lo, int32_t np, const TileRow &R, int32_t &a, int32_t &len, int32_t &c,
+                                          int32_t &d)
 {
-    const int tid = threadIdx.x, lane = __lane_id(), wv = tid >> 6;
-    uint32_t v = wave_incl_scan(len);
-    if (lane == 63) bl->wsum[wv] = v;
-    lds_barrier();
-    uint32_t add = 0;
-    for (int k = 0; k < wv; ++k) add += bl->wsum[k];
-    v += add;
-    if (tid < nstage) bl->pre[tid + 1] = v;
-    if (tid == 0) bl->pre[0] = 0;
-    lds_barrier();
-    if (tid < nstage) {
-        const uint32_t e = bl->pre[tid + 1];
-        if (e <= PMAX && (tid + 1 == nstage || bl->pre[tid + 2] > PMAX)) bl->nb = (uint32_t)(tid + 1);
-    }
-    lds_barrier();
-    const int nb = (int)bl->nb;
-    P = bl->pre[nb];
-    /* each thread takes a run of whole words, finds the segment of its first
-     * pixel by binary search and walks forward */
-    const uint32_t nw = (P + 3) >> 2;
-    const uint32_t wpt = (nw + blockDim.x - 1) / blockDim.x;
-    const uint32_t w0 = tid * wpt;
-    const uint32_t w1 = w0 + wpt < nw ? w0 + wpt : nw;
-    if (w0 < w1) {
-        const uint32_t p0 = w0 * 4;
-        int lo_s = 0, hi_s = nb - 1;
-        while (lo_s < hi_s) {
-            const int mid = (lo_s + hi_s + 1) >> 1;
-            if (bl->pre[mid] <= p0) lo_s = mid; else hi_s = mid - 1;
-        }
-        uint32_t sg = (uint32_t)lo_s, nxt = bl->pre[sg + 1];
-        for (uint32_t w = w0; w < w1; ++w) {
-            uint32_t o = 0;
-            for (int bb = 0; bb < 4; ++bb) {
-                const uint32_t p = w * 4 + bb;
-                while (p >= nxt && (int)sg + 1 < nb) { ++sg; nxt = bl->pre[sg + 1]; }
-                o |= sg << (8 * bb);
-            }
-            bl->seg_of[w] = o;
-        }
-    }
-    lds_barrier();
-    return nb;
+    int32_t rel = lo - (int32_t)R.ip0;
+    if (rel < 0) rel += R.npr;
+    const int32_t e = rel + np, w = R.width, back = e - R.npr;     /* pixels [0, back) after coming round */
+    c = d = 0;
+    if (rel >= w) { a = 0; len = back > 0 ? (back < w ? back : w) : 0; return len; }
+    if (back <= 0) { a = rel; len = (e < w ? e : w) - rel; return len; }
+    a = 0; len = w;
+    if (back >= rel) return w;
+    c = back; d = rel;
+    return w - (d - c);
 }
+
+/* Which segment a wave's pixel belongs to: the wave's pixels are numbered
+ * segment by segment (start: this lane's first pixel, len of them, the
+ * segments without pixels left out of the numbering), and bit p of a bitmap is
+ * set if a segment starts at pixel p + 1, so that pixel p's segment is the number
+ * of bits below p.  Returns this lane's 64 bits of the window of WPIX pixels
+ * from base: pixels base + 64 c .. are the bits of lane c. */
+__device__ static inline unsigned long long start_bits(unsigned long long *bits, uint32_t base, uint32_t start, bool has)
+{
+    const int lane = __lane_id();
+    bits[lane] = 0ULL;
+    wave_lds_fence();
+    const uint32_t at = start - 1u - base;         /* wraps below the window */
+    if (has && start > 0u && at < WPIX) atomicOr(reinterpret_cast<uint32_t *>(bits) + (at >> 5), 1u << (at & 31u));
+    wave_lds_fence();
+    return bits[lane];
+}
+
+/* where wave w of nw (1 to 8) starts in n pairs: equal shares, the last ones
+ * shorter; no division but by constants */
+__device__ static inline uint32_t wave_share(uint32_t n, int w, int nw)
+{
+    uint32_t c;
+    switch (nw) {
+    case 1: c = n; break;
+    case 2: c = (n + 1) / 2; break;
+    case 3: c = (n + 2) / 3; break;
+    case 4: c = (n + 3) / 4; break;
+    default: c = n / (uint32_t)nw + 1; break;
+    }
+    const uint32_t s = c * (uint32_t)w;
+    return s < n ? s : n;
+}
+
+/* Tiles come from one queue per XCD: workgroup b runs on XCD b % 8 and
+ * claims the next tile of that XCD's contiguous eighth of the tiles (sector
+ * by sector along a band, so the tiles in flight on an XCD share halos and
+ * map lines in its L2) from the XCD's counter.  A workgroup that becomes
+ * resident late, or whose tiles run long, leaves the remaining tiles to the
+ * others. */
+struct TileQueue {
+    unsigned int *ctr;
+    int64_t xb, xe;
+    __device__ TileQueue(const TileArgs &A)
+    {
+        const bool xq = (gridDim.x % 8) == 0 && A.n_tiles >= 8;
+        const int xcd = xq ? (int)(blockIdx.x % 8) : 0;
+        xb = xq ? (int64_t)xcd * A.n_tiles / 8 : 0;
+        xe = xq ? (int64_t)(xcd + 1) * A.n_tiles / 8 : A.n_tiles;
+        ctr = A.tile_next + xcd * P2M_TQ_STRIDE;
+    }
+    __device__ int32_t claim() const { return (int32_t)(xb + (int64_t)atomicAdd(ctr, 1u)); }
+};
 
 /* ------------------------------------------------------------------ */
 /* FP64 tiled painter                                                   */
@@ -1115,13 +933,14 @@ __device__ static inline int batch_prepare(BatchLDS *bl, uint32_t len, int nstag
 /* tile (ds_add_f64) and reduced to the FP64 map.                        */
 /* ------------------------------------------------------------------ */
 
-/* the per-halo values the exact per-pixel code reads, staged per segment */
-struct ExactSeg {
-    BatchLDS b;
-    double hx[FSEG], hy[FSEG], hz[FSEG], dth[FSEG], vh[FSEG], chir[FSEG], fc[FSEG], fm[FSEG];
-    unsigned long long hash[FSEG];
-    uint32_t lo[FSEG];
-    int32_t imh[FSEG], ichi[FSEG], cout[FSEG];
+/* the per-segment values the exact per-pixel code reads, one set per wave */
+struct ExactWave {
+    double hx[WSEG], hy[WSEG], hz[WSEG], dth[WSEG], vh[WSEG], chir[WSEG], fc[WSEG], fm[WSEG];
+    unsigned long long hash[WSEG];
+    unsigned long long bits[WPIX / 64];   /* segment starts */
+    int32_t col[WSEG];             /* in-row pixel minus the wave's pixel number */
+    int32_t imh[WSEG], ichi[WSEG], cout[WSEG], row[WSEG];
+    int32_t hole[WSEG];            /* in-row pixels the run leaves out: first | end << 16 */
 };
 
 /* interpolate_table (maptable.f90:176-216) on staged per-halo values, the
@@ -1156,105 +975,149 @@ __device__ static inline double interp_staged(int chi_out, double chi_r, double 
     return v;
 }
 
+/* per-thread statistics of a painter */
+struct PaintStats {
+    unsigned long long listed, upd, segs, err;
+};
+
 template <int NM>
-__global__ void __launch_bounds__(512) k_tile_exact(TileArgs A)
+__global__ void __launch_bounds__(512) k_tile_exact(TileArgs A, const TileDesc *__restrict__ tdesc,
+                                                    const unsigned long long *__restrict__ toff,
+                                                    const RingDesc *__restrict__ rdesc)
 {
     extern __shared__ unsigned char smem_raw[];
-    const int W = 1 << A.log2w;
-    /* LDS: acc (NM*W doubles) | hash (W u64) count (W u32) if membership | ExactSeg */
+    const int W = 1 << A.log2w, log2c = A.shape.log2c;
+    /* LDS: acc (NM*W doubles) | hash (W u64) count (W u32) if membership | TileCtl | ExactWave per wave */
     double *acc = (double *)smem_raw;
     const size_t acc_bytes = (size_t)NM * W * 8;
     unsigned long long *lhash = (unsigned long long *)(smem_raw + acc_bytes);
     uint32_t *lcount = (uint32_t *)(smem_raw + acc_bytes + (A.count ? (size_t)W * 8 : 0));
     const size_t mem_bytes = A.count ? (size_t)W * 12 : 0;
-    ExactSeg *sl = (ExactSeg *)(smem_raw + ((acc_bytes + mem_bytes + 15) & ~(size_t)15));
-    __shared__ unsigned long long lds16[16];
-    const int tid = threadIdx.x;
-    unsigned long long n_upd = 0, n_err = 0;
+    TileCtl *ctl = (TileCtl *)(smem_raw + ((acc_bytes + mem_bytes + 15) & ~(size_t)15));
+    const int tid = threadIdx.x, lane = __lane_id(), wv = tid >> 6, nwv = (int)(blockDim.x >> 6);
+    ExactWave *ew = (ExactWave *)(ctl + 1) + wv;
+    PaintStats st = {0, 0, 0, 0};
     __amdgpu_buffer_rsrc_t trs[NM];
     for (int m = 0; m < NM; ++m)
         trs[m] = __builtin_amdgcn_make_buffer_rsrc((void *)A.tab_flat[m], (short)0, (int)(A.n_flat * 4), 0x00020000);
-    int64_t tbeg, tend, tstep;
-    tile_range(A, tbeg, tend, tstep);
-    for (int64_t t = tbeg; t < tend; t += tstep) {
-        const TileDesc G = A.desc[t];
-        const uint64_t sbeg = A.tile_off[t], send = A.tile_off[t + 1];
-        for (int q = tid; q < G.width; q += blockDim.x) {
-            for (int m = 0; m < NM; ++m) acc[m * W + q] = 0.0;
-            if (A.count) { lcount[q] = 0; lhash[q] = 0ULL; }
-        }
-        for (uint64_t b0 = sbeg; b0 < send;) {
-            lds_barrier();
-            int nstage = (int)(send - b0 < FSEG ? send - b0 : FSEG);
-            if (nstage > (int)blockDim.x) nstage = (int)blockDim.x;
-            uint32_t len = 0;
-            if (tid < nstage) {
-                const uint2 sg = A.segs[b0 + tid];
-                /* a segment must name a record and lie inside the tile */
-                const uint32_t slo = sg.y >> 16, slen = sg.y & 0xffffu;
-                const bool ok = sg.x < (uint64_t)A.n_halo && slo + slen <= (uint32_t)G.width;
-                if (!ok) n_err++;
-                const HaloRec &h = A.halos[ok ? sg.x : 0u];
-                sl->lo[tid] = slo;
-                len = ok ? slen : 0u;
-                sl->hx[tid] = h.hx; sl->hy[tid] = h.hy; sl->hz[tid] = h.hz; sl->dth[tid] = h.dtheta;
-                sl->vh[tid] = h.vh; sl->chir[tid] = h.chi_r; sl->fc[tid] = h.fc; sl->fm[tid] = h.fm;
-                sl->imh[tid] = h.imh; sl->ichi[tid] = h.ichi; sl->cout[tid] = h.chi_out;
-                if (A.count) sl->hash[tid] = halo_hash(h.cat);
-            }
-            uint32_t P;
-            const int nb = batch_prepare(&sl->b, len, nstage, P);
-            b0 += (uint64_t)nb;
-            const unsigned char *segb = (const unsigned char *)sl->b.seg_of;
-            for (uint32_t p = tid; p < P; p += blockDim.x) {
-                const int s = segb[p];
-                const int q = (int)(sl->lo[s] + (p - sl->b.pre[s]));
-                const double phi = (((double)(G.ip0 + q) + G.off) * HPX_HALFPI) / G.den;
-                double sn, cs;
-                p2m_sincos(phi, &sn, &cs);
-                const double angle = angdist(sl->hx[s], sl->hy[s], sl->hz[s], G.sth * cs, G.sth * sn, G.zr);
-                if (!(angle < sl->dth[s])) continue;
-                n_upd++;
-                for (int m = 0; m < NM; ++m)
-                    atomicAdd(&acc[m * W + q], sl->vh[s] * interp_staged(sl->cout[s], sl->chir[s], sl->fc[s], sl->fm[s],
-                                                                         sl->imh[s], sl->ichi[s], A.g, trs[m],
-                                                                         A.profile, angle));
-                if (A.count) {
-                    atomicAdd(&lcount[q], 1u);
-                    atomicAdd(&lhash[q], sl->hash[s]);
-                }
-            }
-        }
-        lds_barrier();
-        const int64_t pix0 = G.first + G.ip0;
-        /* branch on accumulate outside the loops (no speculative map loads) */
-        if (A.accumulate) {
-            for (int q = tid; q < G.width; q += blockDim.x) {
-                for (int m = 0; m < NM; ++m) A.map64[m][pix0 + q] += acc[m * W + q];
-                if (A.count) {
-                    A.count[pix0 + q] += lcount[q];
-                    A.hash[pix0 + q] += lhash[q];
-                }
-            }
-        } else {
-            for (int q = tid; q < G.width; q += blockDim.x) {
-                for (int m = 0; m < NM; ++m) A.map64[m][pix0 + q] = acc[m * W + q];
-                if (A.count) {
-                    A.count[pix0 + q] = lcount[q];
-                    A.hash[pix0 + q] = lhash[q];
-                }
-            }
-        }
-        lds_barrier();
+    const TileQueue q(A);
+    if (tid == 0) ctl->next_tile[0] = q.claim();
+    for (int p = tid; p < W; p += blockDim.x) {
+        for (int m = 0; m < NM; ++m) acc[m * W + p] = 0.0;
+        if (A.count) { lcount[p] = 0; lhash[p] = 0ULL; }
     }
-    block_count(&A.counters[1], n_upd, lds16);
-    block_count(A.err, n_err, lds16);
+    lds_barrier();
+    for (int par = 0;; par ^= 1) {
+        const int64_t t = (int64_t)__builtin_amdgcn_readfirstlane(ctl->next_tile[par]);
+        if (t >= q.xe) break;
+        const TileDesc G = tdesc[t];
+        const uint64_t sbeg = toff[t], send = toff[t + 1];
+        const TileRow *rows = ctl->rows[par];
+        if (tid < G.rows) stage_row(ctl->rows[par][tid], rdesc[G.ring0 - 1 + tid], G.K, G.k);
+        if (tid == 0) ctl->next_tile[par ^ 1] = q.claim();
+        lds_barrier();
+        const uint32_t cnt = (uint32_t)(send - sbeg);
+        const int wv_u = __builtin_amdgcn_readfirstlane(wv);
+        uint64_t pos = sbeg + wave_share(cnt, wv_u, nwv);
+        const uint64_t end = sbeg + wave_share(cnt, wv_u + 1, nwv);
+        while (pos < end) {
+            const bool has = pos + (uint64_t)lane < end;
+            const uint64_t at = has ? pos + (uint64_t)lane : end - 1;
+            Seg g;
+            pos += (uint64_t)wave_segments(A.keys[at], A.vals[at], has, g);
+            uint32_t slot = g.val;
+            /* a pair must name a record and rows of the tile; one that does
+             * not is counted as an error and painted empty */
+            if (g.act && !((uint64_t)slot < (uint64_t)A.n_halo && g.row < G.rows)) { st.err++; g.act = false; }
+            if (!g.act) { slot = 0; g.row = 0; }
+            const HaloRec &h = A.halos[slot];
+            const TileRow &R = rows[g.row];
+            const int32_t ring = G.ring0 + g.row;
+            int32_t lo = 0, np = 0, a = 0, len = 0, c = 0, d = 0;
+            if (g.act) np = disc_ring_run_fast(disc_rec(h), ring2z(A.nside, ring), R.npr, R.kshift(), lo);
+            if (np > 0) st.listed += (unsigned long long)clip_run(lo, np, R, a, len, c, d);
+            st.segs += len > 0;
+            const uint32_t incl = wave_incl_scan((uint32_t)len), start = incl - (uint32_t)len;
+            const uint32_t P = (uint32_t)__builtin_amdgcn_readlane((int)incl, 63);
+            wave_lds_fence();
+            const unsigned long long some = __ballot(len > 0);
+            if (len > 0) {
+                const int k = (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(some >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)some, 0u));
+                ew->hx[k] = h.hx; ew->hy[k] = h.hy; ew->hz[k] = h.hz; ew->dth[k] = h.dtheta;
+                ew->vh[k] = h.vh; ew->chir[k] = h.chi_r; ew->fc[k] = h.fc; ew->fm[k] = h.fm;
+                ew->imh[k] = h.imh; ew->ichi[k] = h.ichi; ew->cout[k] = h.chi_out;
+                ew->row[k] = g.row; ew->col[k] = a - (int32_t)start; ew->hole[k] = c | (d << 16);
+                if (A.count) ew->hash[k] = halo_hash(h.cat);
+            }
+            uint32_t before = 0;
+            for (uint32_t base = 0; base < P; base += WPIX) {
+                const unsigned long long sb = start_bits(ew->bits, base, start, len > 0);
+                const uint32_t pe = P - base < WPIX ? P : base + WPIX;
+                for (uint32_t p0 = base; p0 < pe; p0 += 64) {
+                    const int ch = (int)((p0 - base) >> 6);
+                    const uint32_t mlo = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)sb, ch);
+                    const uint32_t mhi = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(sb >> 32), ch);
+                    const int s = (int)__builtin_amdgcn_mbcnt_hi(mhi, __builtin_amdgcn_mbcnt_lo(mlo, before));
+                    before += (uint32_t)(__builtin_popcount(mlo) + __builtin_popcount(mhi));
+                    const uint32_t p = p0 + (uint32_t)lane;
+                    if (p >= pe) continue;
+                    const int row = ew->row[s], col = ew->col[s] + (int)p, hole = ew->hole[s];
+                    if (col >= (hole & 0xffff) && col < (hole >> 16)) continue;
+                    const TileRow &Q = rows[row];
+                    const double phi = (((double)((int)Q.ip0 + col) + (double)Q.off) * HPX_HALFPI) / Q.den();
+                    double sn, cs;
+                    p2m_sincos(phi, &sn, &cs);
+                    const double angle = angdist(ew->hx[s], ew->hy[s], ew->hz[s], Q.sth * cs, Q.sth * sn, Q.zr);
+                    if (!(angle < ew->dth[s])) continue;
+                    st.upd++;
+                    const int o = (row << log2c) + col;
+                    for (int m = 0; m < NM; ++m)
+                        atomicAdd(&acc[m * W + o], ew->vh[s] * interp_staged(ew->cout[s], ew->chir[s], ew->fc[s], ew->fm[s],
+                                                                             ew->imh[s], ew->ichi[s], A.g, trs[m],
+                                                                             A.profile, angle));
+                    if (A.count) {
+                        atomicAdd(&lcount[o], 1u);
+                        atomicAdd(&lhash[o], ew->hash[s]);
+                    }
+                }
+            }
+        }
+        lds_barrier();
+        /* every thread writes its pixels and clears them for the next tile;
+         * branch on accumulate outside the loops (no speculative map loads) */
+        const int npx = G.rows << log2c;
+        auto out = [&](auto add) {
+            for (int p = tid; p < npx; p += blockDim.x) {
+                const TileRow &R = rows[p >> log2c];
+                const int col = p & ((1 << log2c) - 1);
+                if (col < (int)R.width) {
+                    const int64_t pix = R.pix0 + col;
+                    for (int m = 0; m < NM; ++m) {
+                        if constexpr (decltype(add)::value) A.map64[m][pix] += acc[m * W + p];
+                        else A.map64[m][pix] = acc[m * W + p];
+                    }
+                    if (A.count) {
+                        if constexpr (decltype(add)::value) { A.count[pix] += lcount[p]; A.hash[pix] += lhash[p]; }
+                        else { A.count[pix] = lcount[p]; A.hash[pix] = lhash[p]; }
+                    }
+                }
+                for (int m = 0; m < NM; ++m) acc[m * W + p] = 0.0;
+                if (A.count) { lcount[p] = 0; lhash[p] = 0ULL; }
+            }
+        };
+        if (A.accumulate) out(std::true_type{}); else out(std::false_type{});
+    }
+    unsigned long long *red = (unsigned long long *)ctl->fb;
+    block_count(&A.counters[0], st.listed, red);
+    block_count(&A.counters[1], st.upd, red);
+    block_count(&A.counters[4], st.segs, red);
+    block_count(A.err, st.err, red);
 }
 
 /* --------------------------------------------------------------------- */
 /* FP32 tiled painter                                                      */
 /*                                                                         */
-/* Per pixel: one FP64 FMA for the azimuth offset from the halo centre,    */
+/* Per pixel: the azimuth offset from the halo centre,                     */
 /* then FP32: chord^2 = A + B sin^2(dphi/2) with the per-(halo,ring)       */
 /* constants A = (z-z0)^2 + (sth-s0)^2, B = 4 sth s0 staged in LDS;        */
 /* tan^2(theta) = 4h(1-h)/(1-2h)^2 with h = chord^2/4; the cell coordinate */
@@ -1265,30 +1128,35 @@ __global__ void __launch_bounds__(512) k_tile_exact(TileArgs A)
 /* `band` of a cell boundary, the r cut-off or the r clamp, are deferred   */
 /* to k_fallback, which decides them with the exact FP64 arithmetic of the */
 /* reference.                                                              */
+/*                                                                         */
+/* The waves of a workgroup share the tile's accumulator and nothing else: */
+/* each takes its part of the tile's pairs and works through them alone,   */
+/* staging up to 64 (halo, row) segments at a time in LDS of its own (their */
+/* runs, a bitmap of where each starts, then the pixels), with no barrier   */
+/* between the tile's first and its last.                                  */
+/*                                                                         */
+/* Bound: VALU issue (80% busy at six waves a SIMD).  A pixel takes about   */
+/* 90 instructions, a batch of 64 segments about 250 before them (the       */
+/* runs, which the binning no longer computes).  2e7 halos at nside 4096:   */
+/* 1.25 ms -> 1.44 ms for 1.35 -> 0.39 ms of binning; 2e7 heavy halos at    */
+/* nside 2048 3.1 -> 2.5 ms; 4e7 at nside 4096 14.7 -> 12.9 ms.  Rows by    */
+/* columns of a tile: 8 x 128 instead of 16 x 64 takes 0.1 ms off the first  */
+/* and adds as much to its binning, and is 2% slower on the last two.       */
 /* --------------------------------------------------------------------- */
 
 /* One array per constant: a wave's pixels read a few consecutive segments,
- * and 4-byte reads of one array (paired by the compiler into read2st64)
+ * and 4-byte reads of one array (paired by the compiler into read2)
  * broadcast in one pass, where 16-byte reads of a struct keep the LDS unit
  * several times busier. */
-struct FastSeg {
-    uint32_t nb_s, P_s;            /* the batch's segment and pixel counts (set between its barriers) */
-    uint32_t seg_of[PMAX / 4];     /* batch pixel -> segment (bytes) */
-    uint32_t wsum[16];             /* per wave: staged lengths [0, 8), segments that fit [8, 16) */
-    /* the per-tile control words come in two slots, used by alternate
-     * tiles, so that a tile's end needs no barrier before the next begins */
-    uint32_t nfb[2];               /* deferred pixels of the tile */
-    uint32_t lost[2];              /* a deferred pixel of the tile found the list full */
-    int32_t next_tile[2];          /* the tile this workgroup paints next */
-    unsigned long long fb_base;    /* list slot of the tile's deferred pixels */
-    uint4 fb[FB_LDS];
-    uint32_t halo[FSEG];
-    int16_t qoff[FSEG];            /* in-tile pixel minus batch pixel: lo - pre (-3072 .. 2047) */
-    float A[FSEG], B[FSEG], thr_hi[FSEG], chi2[FSEG];   /* chord^2 = A + B sin^2(x); its band top; chi^2 */
-    float w00[FSEG], w10[FSEG], w01[FSEG], w11[FSEG];   /* corner weights times the velocity factor */
-    float xc[FSEG];                /* azimuth origin x_c */
-    int32_t cidx[FSEG];            /* batch pixel of the azimuth origin: p - cidx = ip - ip_c */
-    int32_t colbase[FSEG];
+struct FastWave {
+    unsigned long long bits[WPIX / 64];   /* segment starts */
+    float A[WSEG], B[WSEG], thr_hi[WSEG], chi2[WSEG];   /* chord^2 = A + B sin^2(x); its band top; chi^2 */
+    float w00[WSEG], w10[WSEG], w01[WSEG], w11[WSEG];   /* corner weights times the velocity factor */
+    float xc[WSEG], hphi[WSEG];    /* azimuth origin x_c; x step per pixel along the ring */
+    int32_t cidx[WSEG];            /* wave's pixel number of the azimuth origin: p - cidx = ip - ip_c */
+    int32_t colbase[WSEG];
+    uint32_t slot[WSEG];           /* halo; ASK_RUN: its deferred pixels must lie in the exact run */
+    int16_t qoff[WSEG];            /* in-tile pixel minus the wave's pixel number (-4096 .. 2047) */
 };
 
 /* sin^2(x) for |x| <= 2: the odd Taylor polynomial of sin to x^15 (the
@@ -1328,99 +1196,32 @@ __device__ static inline void load_floats(__amdgpu_buffer_rsrc_t r, int vo, int 
     for (; k < NF; ++k) f[k] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(r, vo + 4 * k, so, 0));
 }
 
-/* Scan of the staged lengths: start receives this thread's first batch
- * pixel and fit whether its segment belongs to the batch, i.e. lies within
- * the first PMAX pixels (a segment is at most W <= PMAX pixels, so at least
- * one does; the prefix is non-decreasing, so the batch is a leading run of
- * the staged segments).  The batch's segment and pixel counts reach
- * fs->nb_s and fs->P_s through LDS atomics, readable after the caller's next
- * barrier.  Every thread calls; one barrier. */
-__device__ static inline void batch_prefix(FastSeg *fs, uint32_t len, int nstage, uint32_t &start, bool &fit)
-{
-    const int tid = threadIdx.x, lane = __lane_id(), wv = tid >> 6;
-    uint32_t v = wave_incl_scan(len);
-    if (lane == 63) fs->wsum[wv] = v;
-    if (tid == 0) { fs->nb_s = 0; fs->P_s = 0; }
-    lds_barrier();
-    uint32_t add = 0;
-    for (int k = 0; k < wv; ++k) add += fs->wsum[k];
-    v += add;
-    start = v - len;
-    fit = tid < nstage && v <= PMAX;
-    const unsigned long long fm = __ballot(fit);
-    if (fm) {
-        /* the wave's fitting lanes are lanes 0 .. last */
-        const int last = 63 - __clzll((long long)fm);
-        if (lane == 0) atomicAdd(&fs->nb_s, (uint32_t)__popcll(fm));
-        if (lane == last) atomicMax(&fs->P_s, v);
-    }
-}
-
-/* The batch's pixel -> segment byte map, written by the segments
- * themselves: thread s (in the batch) owns pixels [a, a + len).  A segment of at
- * most 64 pixels is written by its own thread (bytes up to a word boundary,
- * whole words, the tail bytes); a longer one by its whole wave, 64 words a
- * round, its head and tail bytes by six lanes.  Every byte belongs to one
- * segment and whole-word writes only cover words inside one, so the writes
- * never overlap; there are no reads.  Every lane of the wave must be
- * active.  The caller's barrier publishes the map. */
-__device__ static inline void build_seg_map_direct(FastSeg *fs, bool in_batch, uint32_t a, uint32_t len)
-{
-    unsigned char *mb = reinterpret_cast<unsigned char *>(fs->seg_of);
-    uint32_t *mw = fs->seg_of;
-    const int tid = threadIdx.x, lane = __lane_id();
-    const bool mine = in_batch && len > 0;
-    const bool lng = mine && len > 64;
-    if (mine && !lng) {
-        const uint32_t e = a + len, fill = (uint32_t)tid * 0x01010101u;
-        uint32_t p = a;
-        for (; p < e && (p & 3u); ++p) mb[p] = (unsigned char)tid;
-        for (; p + 4 <= e; p += 4) mw[p >> 2] = fill;
-        for (; p < e; ++p) mb[p] = (unsigned char)tid;
-    }
-    unsigned long long lm = __ballot(lng);
-    while (lm) {
-        const int L = __ffsll((long long)lm) - 1;
-        lm &= lm - 1;
-        const uint32_t aL = (uint32_t)__builtin_amdgcn_readlane((int)a, L);
-        const uint32_t eL = aL + (uint32_t)__builtin_amdgcn_readlane((int)len, L);
-        const uint32_t sL = (uint32_t)((tid & ~63) + L), fL = sL * 0x01010101u;
-        const uint32_t w0 = (aL + 3u) >> 2, w1 = eL >> 2;     /* whole words [w0, w1): len > 64, so w0 < w1 */
-        for (uint32_t w = w0 + (uint32_t)lane; w < w1; w += 64) mw[w] = fL;
-        if (lane < 3) {
-            const uint32_t p = aL + (uint32_t)lane;             /* head bytes below 4 w0 */
-            if (p < 4u * w0) mb[p] = (unsigned char)sL;
-        } else if (lane < 6) {
-            const uint32_t p = 4u * w1 + (uint32_t)(lane - 3);   /* tail bytes from 4 w1 */
-            if (p < eL) mb[p] = (unsigned char)sL;
-        }
-    }
-}
-
-
 template <int NM>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NM == 1 ? 6 : 1))) k_tile_fast(TileArgs A, const TileDesc *__restrict__ tdesc,
-                                                   const unsigned long long *__restrict__ toff)
+                                                   const unsigned long long *__restrict__ toff,
+                                                   const RingDesc *__restrict__ rdesc)
 {
     extern __shared__ unsigned char smem_raw[];
-    const int W = 1 << A.log2w;
-    /* LDS: acc (NM*W doubles) | hash (W u64) count (W u32) if membership | FastSeg | hashes (FSEG u64) if
-     * membership | 1/r_node^2 (nrt+2 floats) */
+    const int W = 1 << A.log2w, log2c = A.shape.log2c;
+    /* LDS: acc (NM*W doubles) | hash (W u64) count (W u32) if membership | TileCtl | FastWave per wave |
+     * hashes (WSEG u64 per wave) if membership | 1/r_node^2 (nrt+2 floats) */
     double *acc = (double *)smem_raw;
     const size_t acc_bytes = (size_t)NM * W * 8;
     unsigned long long *lhash = (unsigned long long *)(smem_raw + acc_bytes);
     uint32_t *lcount = (uint32_t *)(smem_raw + acc_bytes + (A.count ? (size_t)W * 8 : 0));
     const size_t mem_bytes = A.count ? (size_t)W * 12 : 0;
-    FastSeg *sl = (FastSeg *)(smem_raw + ((acc_bytes + mem_bytes + 15) & ~(size_t)15));
-    unsigned long long *hh = (unsigned long long *)(sl + 1);   /* membership hashes, if counted */
-    float *invn = (float *)(hh + (A.count ? FSEG : 0));
+    TileCtl *ctl = (TileCtl *)(smem_raw + ((acc_bytes + mem_bytes + 15) & ~(size_t)15));
+    const int tid = threadIdx.x, lane = __lane_id(), wv = tid >> 6, nwv = (int)(blockDim.x >> 6);
+    FastWave *fw = (FastWave *)(ctl + 1) + wv;
+    unsigned long long *hh = (unsigned long long *)((FastWave *)(ctl + 1) + nwv) + wv * WSEG;
+    float *invn = (float *)((unsigned long long *)((FastWave *)(ctl + 1) + nwv) + (A.count ? nwv * WSEG : 0));
     /* inner edge of the deferral band, relative to the outer one */
     const float lo_band = (float)((1.0 - (double)A.band_c) / (1.0 + (double)A.band_c));
     const float u_zero = A.u_max + A.band;
     /* constants of the pixel loop that an instruction needs in a vector
      * register (a second scalar operand, a select), pinned there once */
     float v_k0 = A.u_k0, v_frc = A.fr_clamp;
-    int v_irc = A.ir_clamp;
+    int v_irc = A.ir_clamp - 1;
     asm volatile("" : "+v"(v_k0), "+v"(v_frc), "+v"(v_irc));
 
     const int nrt = A.g.nrt;
@@ -1428,293 +1229,299 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NM == 
      * reads past its end return 0 */
     const __amdgpu_buffer_rsrc_t trs =
         __builtin_amdgcn_make_buffer_rsrc((void *)A.tab_q, (short)0, (int)(A.n_quad * 4), 0x00020000);
-    const int tid = threadIdx.x;
-    unsigned long long n_upd = 0, n_fb = 0, n_err = 0;
+    uint32_t n_upd = 0, n_fb = 0, n_list = 0, n_seg = 0, n_err = 0;     /* this thread's, see flush below */
     const int64_t fbs = A.fb_cap / P2M_SHARDS;
     unsigned long long *const fbc = A.fb_count + (blockIdx.x % P2M_SHARDS) * P2M_CTR_STRIDE;
     uint4 *const fbr = A.fb + (blockIdx.x % P2M_SHARDS) * fbs;
-    if (tid == 0) { sl->nfb[0] = sl->nfb[1] = 0; sl->lost[0] = sl->lost[1] = 0; }
+    const TileQueue q(A);
+    if (tid == 0) {
+        ctl->nfb[0] = ctl->nfb[1] = 0; ctl->lost[0] = ctl->lost[1] = 0;
+        ctl->next_tile[0] = q.claim();
+        ctl->next_tile[1] = q.claim();
+    }
     for (int k = tid; k < nrt + 2; k += blockDim.x) invn[k] = A.inv_node2f[k];
+    for (int p = tid; p < W; p += blockDim.x) {
+        for (int m = 0; m < NM; ++m) acc[m * W + p] = 0.0;
+        if (A.count) { lcount[p] = 0; lhash[p] = 0ULL; }
+    }
     lds_barrier();
 
-    /* Tiles come from one queue per XCD: workgroup b runs on XCD b % 8 and
-     * claims the next tile of that XCD's contiguous eighth of the tiles
-     * (ring-major, so the tiles in flight on an XCD share halos in its L2)
-     * from the XCD's counter.  A workgroup that becomes resident late, or
-     * whose tiles run long, leaves the remaining tiles to the others.
-     * Thread 0 claims the following tile with the tile's first segment
-     * loads and writes it to the other slot, which the tile's next barrier
-     * publishes.
-     *
-     * Tile k uses slot par = k & 1.  Its end needs no barrier: the next
-     * tile's first writes to shared words come after that tile's own
-     * barriers, its clear of the accumulator touches only the pixels each
-     * thread itself wrote back, and slot par ^ 1 is cleared by thread 0
-     * after tile k's post-loop barrier, when tile k-1's readers of it are
-     * done. */
-    const bool xq = (gridDim.x % 8) == 0 && A.n_tiles >= 8;
-    const int xcd = xq ? (int)(blockIdx.x % 8) : 0;
-    const int64_t xb = xq ? (int64_t)xcd * A.n_tiles / 8 : 0;
-    const int64_t xe = xq ? (int64_t)(xcd + 1) * A.n_tiles / 8 : A.n_tiles;
-    unsigned int *const qctr = A.tile_next + xcd * P2M_TQ_STRIDE;
-    if (tid == 0) sl->next_tile[0] = (int32_t)(xb + (int64_t)atomicAdd(qctr, 1u));
-    lds_barrier();
+    /* A tile's descriptor, pair range and first pairs are loaded, and its
+     * rows staged, while the tile before it is painted: every thread reads
+     * the same tile, so the descriptor and range are scalar loads.  Tile k
+     * uses slot par = k & 1 of the rows and control words, and next_tile[par ^ 1]
+     * is the tile after it.  Between tile k's two barriers the waves paint;
+     * after the second every thread writes out and clears its own pixels.  The
+     * next tile's rows and words go to the other slot, whose readers of tile
+     * k-1 were done at tile k's first barrier. */
+    int64_t t = (int64_t)__builtin_amdgcn_readfirstlane(ctl->next_tile[0]);
+    if (t < q.xe) {
+    TileDesc G = tdesc[t];
+    uint64_t sbeg = toff[t];
+    uint32_t cnt = (uint32_t)(toff[t + 1] - sbeg);
+    bool skip = A.redo && !A.lost[t];            /* repaint pass: only the tiles that lost pixels */
+    if (tid < G.rows) stage_row(ctl->rows[0][tid], rdesc[G.ring0 - 1 + tid], G.K, G.k);
+    uint32_t key = 0, val = 0;
+    auto load_pairs = [&](uint64_t base, uint32_t i, uint32_t e) {
+        if (i >= e) return;
+        const uint64_t at = base + (i + (uint32_t)lane < e ? i + (uint32_t)lane : e - 1);
+        key = A.keys[at]; val = A.vals[at];
+    };
+    const int wv_u = __builtin_amdgcn_readfirstlane(wv);
+    auto wave_from = [&](uint32_t n, int w) { return wave_share(n, w, nwv); };
+    load_pairs(sbeg, wave_from(cnt, wv_u), wave_from(cnt, wv_u + 1));
     for (int par = 0;; par ^= 1) {
-        /* every thread reads the same tile: taken as uniform, its descriptor
-         * and segment range are scalar loads */
-        const int64_t t = (int64_t)__builtin_amdgcn_readfirstlane(sl->next_tile[par]);
-        if (t >= xe) break;
-        bool claimed = false;
-        const TileDesc G = tdesc[t];
-        const uint64_t sbeg = toff[t], send = toff[t + 1];
-        if (A.redo && !A.lost[t]) {      /* repaint pass: only the tiles that lost pixels */
-            lds_barrier();
-            if (tid == 0) {
-                sl->nfb[par ^ 1] = 0; sl->lost[par ^ 1] = 0;
-                sl->next_tile[par ^ 1] = (int32_t)(xb + (int64_t)atomicAdd(qctr, 1u));
+        lds_barrier();
+        const int64_t tn = (int64_t)__builtin_amdgcn_readfirstlane(ctl->next_tile[par ^ 1]);
+        const bool more = tn < q.xe;
+        int32_t after = 0;
+        if (tid == 0) after = q.claim();
+        const TileDesc Gn = tdesc[more ? tn : t];
+        const uint64_t sbeg_n = toff[more ? tn : t];
+        const uint32_t cnt_n = (uint32_t)(toff[(more ? tn : t) + 1] - sbeg_n);
+        const TileRow *rows = ctl->rows[par];
+        uint32_t tu = 0, tf = 0, tl = 0, ts = 0;     /* this tile's updates, deferrals, listed, segments */
+        uint32_t i = wave_from(cnt, wv_u);
+        const uint32_t e = skip ? i : wave_from(cnt, wv_u + 1);
+        bool fetched = false;
+        while (i < e) {
+            Seg g;
+            i += (uint32_t)wave_segments(key, val, i + (uint32_t)lane < e, g);
+            uint32_t slot = g.val;
+            /* a pair must name a record and rows of the tile; one that does
+             * not is counted as an error and painted empty */
+            if (g.act && !((uint64_t)slot < (uint64_t)A.n_halo && g.row < G.rows)) { n_err++; g.act = false; }
+            if (!g.act) { slot = 0; g.row = 0; }
+            const TileHalo &h = A.hot[slot];
+            /* the record's fields, all requested before the first is used
+             * (one memory round trip; the empty asm keeps them together) */
+            const double zz0 = h.zz0, s0 = h.s0, phi0 = h.phi0, thr = h.thr;
+            const float thr_h = h.thr_hi, chi2 = h.chi2, w00h = h.w00, w10h = h.w10, w01h = h.w01, w11h = h.w11;
+            const int32_t colbase = h.colbase;
+            /* the next pairs (the next tile's after the last of this one) */
+            if (i < e) load_pairs(sbeg, i, e);
+            else if (more) { load_pairs(sbeg_n, wave_from(cnt_n, wv_u), wave_from(cnt_n, wv_u + 1)); fetched = true; }
+            asm volatile("" :: "v"(zz0), "v"(s0), "v"(phi0), "v"(thr), "v"(thr_h), "v"(chi2), "v"(w00h), "v"(w10h), "v"(w01h), "v"(w11h), "v"(colbase));
+            const TileRow R = rows[g.row];
+            const double off = (double)R.off, ik = R.ik();
+            const double dz = R.zr - zz0, ds = R.sth - s0, chA = dz * dz + ds * ds;
+            const float chB = (float)((4.0 * R.sth) * s0);
+            /* azimuth origin: the ring pixel ip_c nearest the halo centre's
+             * azimuth, with x_c = ((ip_c + off) kphi - phi0) / 2
+             * (|x_c| <= kphi / 4) in FP64; a pixel's x is then x_c plus
+             * n = ip - ip_c steps of kphi / 2 in FP32.  n may move by npr
+             * (x by pi: sin^2 has period pi): the segment's middle step is
+             * moved into [-npr/2, npr/2] here, and a segment is at most a
+             * quarter of its ring, so every n of it is within 5/8 npr and
+             * |x| <= pi/2 + pi/8 + kphi/4.  So the FP32 error of x stays
+             * relative to x. */
+            const double ipcd = __builtin_rint(phi0 * ik - off);
+            const float xc = (float)(0.5 * ((ipcd + off) * R.kphi - phi0));
+            int32_t ipc = (int32_t)ipcd;
+            if (ipc < 0) ipc += R.npr;
+            if (ipc >= R.npr) ipc -= R.npr;
+            /* the halo's run on this ring.  Where that is left open, every
+             * pixel that may belong to it is deferred (B = 0, its chord^2 the
+             * disc edge's) for k_fallback to ask the exact run, and to count.
+             * A row that the run leaves and comes back to is tested whole,
+             * and its deferred pixels are asked the exact run too. */
+            int32_t lo = 0, np = 0, np_max = 0, a = 0, len = 0, c = 0, d = 0;
+            if (g.act) np = disc_ring_run_chord(thr, chA, chB, R.e_row, xc, (float)(2.0 * ik), ipc, R.npr, lo, np_max);
+            const int32_t in_row = np != 0 && np_max > 0 ? clip_run(lo, np_max, R, a, len, c, d) : 0;
+            const bool open = np < 0;
+            if (!open) tl += (uint32_t)in_row;
+            ts += len > 0;
+            const uint32_t incl = wave_incl_scan((uint32_t)len), start = incl - (uint32_t)len;
+            const uint32_t P = (uint32_t)__builtin_amdgcn_readlane((int)incl, 63);
+            const unsigned long long some = __ballot(len > 0);
+            wave_lds_fence();
+            if (len > 0) {
+                const int k = (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(some >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)some, 0u));
+                const int32_t half_npr = R.npr >> 1;
+                fw->slot[k] = slot | (open || d > c ? ASK_RUN : 0u);
+                fw->qoff[k] = (int16_t)((g.row << log2c) + a - (int32_t)start);
+                fw->A[k] = open ? (float)thr : (float)chA;
+                fw->B[k] = open ? 0.0f : chB;
+                fw->thr_hi[k] = thr_h;
+                fw->chi2[k] = chi2;
+                fw->w00[k] = w00h; fw->w10[k] = w10h; fw->w01[k] = w01h; fw->w11[k] = w11h;
+                fw->colbase[k] = colbase;
+                fw->xc[k] = xc;
+                fw->hphi[k] = (float)(0.5 * R.kphi);
+                const int32_t nmid = (int32_t)R.ip0 + a + (len >> 1) - ipc;
+                fw->cidx[k] = ipc - (int32_t)R.ip0 - (a - (int32_t)start) +
+                              (nmid > half_npr ? R.npr : (nmid < -half_npr ? -R.npr : 0));
+                if (A.count) hh[k] = halo_hash(A.halos[slot].cat);
             }
-            lds_barrier();
-            continue;
-        }
-        const double kphi = G.kphi;
-        const double inv_kphi = G.den * (2.0 / HPX_PI);   /* 1 / kphi */
-        const float hphi = (float)(0.5 * kphi);          /* x step per pixel along the ring */
-        const int32_t mr = G.ring < A.nside ? G.ring : (G.ring < 3 * A.nside ? A.nside : 4 * A.nside - G.ring);
-        const int32_t npr = 4 * mr, half_npr = npr / 2;
-        uint32_t tu = 0, tf = 0;             /* this tile's updates and deferrals */
-        for (int q = tid; q < G.width; q += blockDim.x) {
-            for (int m = 0; m < NM; ++m) acc[m * W + q] = 0.0;
-            if (A.count) { lcount[q] = 0; lhash[q] = 0ULL; }
-        }
-        for (uint64_t b0 = sbeg; b0 < send;) {
-            /* a later batch restages what the previous one's pixels read
-             * (the first batch is ordered after the previous tile's reads by
-             * that tile's post-loop barrier) */
-            if (b0 != sbeg) lds_barrier();
-            int nstage = (int)(send - b0 < FSEG ? send - b0 : FSEG);
-            if (nstage > (int)blockDim.x) nstage = (int)blockDim.x;
-            uint32_t len = 0;
-            /* unconditional (the last staged entry for the idle lanes), so
-             * that its wait can move down to the first use */
-            /* a streaming load: the segment list is read once */
-            const unsigned long long sgw = __builtin_nontemporal_load(
-                reinterpret_cast<const unsigned long long *>(A.segs) + b0 + (uint64_t)(tid < nstage ? tid : nstage - 1));
-            const uint2 sg = make_uint2((uint32_t)sgw, (uint32_t)(sgw >> 32));
-            /* the claim of the following tile is made with the first
-             * batch's segment loads, so that one wait covers both */
-            if (!claimed) {
-                if (tid == 0) sl->next_tile[par ^ 1] = (int32_t)(xb + (int64_t)atomicAdd(qctr, 1u));
-                claimed = true;
-            }
-            uint32_t slo = 0;
-            if (tid < nstage) {
-                /* a segment must name a record and lie inside the tile; one
-                 * that does not is counted as an error and painted empty */
-                slo = sg.y >> 16;
-                const uint32_t slen = sg.y & 0xffffu;
-                const bool ok = sg.x < (uint64_t)A.n_halo && slo + slen <= (uint32_t)G.width;
-                if (!ok) n_err++;
-                len = ok ? slen : 0u;
-            }
-            uint32_t start;
-            bool fit;
-            batch_prefix(sl, len, nstage, start, fit);
-            if (fit) {
-                const TileHalo &h = A.hot[sg.x < (uint64_t)A.n_halo ? sg.x : 0u];
-                /* the record's fields, all requested before the first is used
-                 * (one memory round trip; the empty asm keeps them together) */
-                const double zz0 = h.zz0, s0 = h.s0, phi0 = h.phi0, thr = h.thr;
-                const float chi2 = h.chi2, fc = h.fc, fm = h.fm, vh = h.vh;
-                const int32_t colbase = h.colbase;
-                asm volatile("" :: "v"(zz0), "v"(s0), "v"(phi0), "v"(thr), "v"(chi2), "v"(fc), "v"(fm), "v"(vh), "v"(colbase));
-                sl->halo[tid] = sg.x;
-                sl->qoff[tid] = (int16_t)((int32_t)slo - (int32_t)start);
-                const double dz = G.zr - zz0, ds = G.sth - s0;
-                sl->A[tid] = (float)(dz * dz + ds * ds);
-                sl->B[tid] = (float)((4.0 * G.sth) * s0);
-                sl->thr_hi[tid] = (float)(thr * (1.0 + (double)A.band_c));
-                sl->chi2[tid] = chi2;
-                sl->w00[tid] = vh * ((1.0f - fc) * (1.0f - fm));
-                sl->w10[tid] = vh * (fc * (1.0f - fm));
-                sl->w01[tid] = vh * ((1.0f - fc) * fm);
-                sl->w11[tid] = vh * (fc * fm);
-                sl->colbase[tid] = colbase;
-                /* azimuth origin: the ring pixel ip_c nearest the halo centre's
-                 * azimuth, with x_c = ((ip_c + off) kphi - phi0) / 2 folded by
-                 * pi (|x_c| <= kphi / 4) in FP64; a pixel's x is then x_c plus
-                 * n = ip - ip_c steps of kphi / 2 in FP32.  n may move by npr
-                 * (x by pi: sin^2 has period pi): the segment's middle step is
-                 * moved into [-npr/2, npr/2] here, so on rings of at least 4 W
-                 * pixels every n of the segment is within npr/2 + W/2 and
-                 * |x| <= pi/2 + pi/8 + kphi/4; on shorter rings each pixel's n
-                 * is folded into [-npr/2, npr/2] as well.  Either way the FP32
-                 * error of x stays relative to x. */
-                double ipc = __builtin_rint(phi0 * inv_kphi - G.off);
-                if (ipc < 0.0) ipc += (double)npr;
-                if (ipc >= (double)npr) ipc -= (double)npr;
-                double xc = 0.5 * ((ipc + G.off) * kphi - phi0);
-                xc -= HPX_PI * __builtin_rint(xc * (1.0 / HPX_PI));
-                sl->xc[tid] = (float)xc;
-                const int32_t nmid = G.ip0 + (int32_t)slo + (int32_t)(len >> 1) - (int32_t)ipc;
-                sl->cidx[tid] = (int32_t)ipc - G.ip0 - ((int32_t)slo - (int32_t)start) +
-                                (nmid > half_npr ? npr : (nmid < -half_npr ? -npr : 0));
-                if (A.count) hh[tid] = h.hash;
-            }
-            build_seg_map_direct(sl, fit, start, len);
-            lds_barrier();
-            const int nb = (int)sl->nb_s;
-            const uint32_t P = sl->P_s;
-            b0 += (uint64_t)nb;
-            const unsigned char *segb = (const unsigned char *)sl->seg_of;
-            /* the pixel loop, with or without the per-pixel fold of n (a
-             * tile-uniform choice: two copies of the loop) */
-            auto paint_pixels = [&](auto fold) {
-            for (uint32_t p = tid; p < P; p += blockDim.x) {
-                const int s = segb[p];
-                /* every per-segment constant the accepted path needs is read
-                 * here, in one round of LDS reads: the empty asm below keeps
-                 * the compiler from moving the later ones behind the disc test,
-                 * where each would cost a round trip of its own */
-                const int cix = sl->cidx[s];
-                const float xcs = sl->xc[s], As = sl->A[s], Bs = sl->B[s], thr_hi = sl->thr_hi[s];
-                const float chi2 = sl->chi2[s];
-                const int qo = sl->qoff[s], cb = sl->colbase[s];
-                int n = (int)p - cix;
-                if constexpr (decltype(fold)::value) n = n > half_npr ? n - npr : (n < -half_npr ? n + npr : n);
-                const float x = __builtin_fmaf((float)n, hphi, xcs);
-                const float s2 = sin2f(x);
-                const float c2 = __builtin_fmaf(Bs, s2, As);
-                asm volatile("" :: "v"(chi2), "v"(qo), "v"(cb));
-                if (!(c2 < thr_hi)) continue;                     /* outside the disc */
-                const int q = (int)p + qo;
-                /* tan^2(theta) = 4h(1-h)/(1-2h)^2 with h = chord^2/4 */
-                const float dd = __builtin_fmaf(c2, -0.5f, 1.0f);
-                const float rd = __builtin_amdgcn_rcpf(dd);
-                const float t2 = __builtin_fmaf(-0.25f * c2, c2, c2) * (rd * rd);
-                const float r2 = chi2 * t2;
-                const float u = __builtin_fmaf(__builtin_amdgcn_logf(r2), A.u_k1, -v_k0);
-                const bool zero = u > u_zero;                     /* r > rmaxt: value 0 */
-                /* deferred: near the disc edge, a degenerate chord, or u within
-                 * the band of a cell boundary 0..u_max (u clamped to that range,
-                 * then its nearest boundary) */
-                const float ub = __builtin_amdgcn_fmed3f(u, 0.0f, A.u_max);
-                const bool defer = (c2 > thr_hi * lo_band) | !(dd > 1e-3f) | (__builtin_fabsf(u - __builtin_rintf(ub)) <= A.band);
-                if (defer) {
-                    const uint32_t slot = atomicAdd(&sl->nfb[par], 1u);
-                    const uint4 e = make_uint4((uint32_t)G.ring, (uint32_t)(G.ip0 + q), sl->halo[s], 0u);
-                    if (slot < FB_LDS) sl->fb[slot] = e;
-                    else {
-                        const unsigned long long gs = atomicAdd(fbc, 1ULL);
-                        if (gs < (unsigned long long)fbs) fbr[gs] = e;
-                        else sl->lost[par] = 1u;
+            uint32_t before = 0;
+            for (uint32_t base = 0; base < P; base += WPIX) {
+                const unsigned long long sb = start_bits(fw->bits, base, start, len > 0);
+                const uint32_t pe = P - base < WPIX ? P : base + WPIX;
+                for (uint32_t p0 = base; p0 < pe; p0 += 64) {
+                    const int ch = (int)((p0 - base) >> 6);
+                    const uint32_t mlo = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)sb, ch);
+                    const uint32_t mhi = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(sb >> 32), ch);
+                    const int s = (int)__builtin_amdgcn_mbcnt_hi(mhi, __builtin_amdgcn_mbcnt_lo(mlo, before));
+                    before += (uint32_t)(__builtin_popcount(mlo) + __builtin_popcount(mhi));
+                    const uint32_t p = p0 + (uint32_t)lane;
+                    if (p >= pe) continue;
+                    /* every per-segment constant the accepted path needs is read
+                     * here, in one round of LDS reads: the empty asm below keeps
+                     * the compiler from moving the later ones behind the disc test,
+                     * where each would cost a round trip of its own */
+                    const int cix = fw->cidx[s];
+                    const float xcs = fw->xc[s], hphi = fw->hphi[s], As = fw->A[s], Bs = fw->B[s], thr_hi = fw->thr_hi[s];
+                    const float chi2s = fw->chi2[s];
+                    const int qo = fw->qoff[s], cb = fw->colbase[s];
+                    const int n = (int)p - cix;
+                    const float x = __builtin_fmaf((float)n, hphi, xcs);
+                    const float s2 = sin2f(x);
+                    const float c2 = __builtin_fmaf(Bs, s2, As);
+                    asm volatile("" :: "v"(chi2s), "v"(qo), "v"(cb));
+                    if (!(c2 < thr_hi)) continue;                     /* outside the disc */
+                    const int o = (int)p + qo;
+                    /* tan^2(theta) = 4h(1-h)/(1-2h)^2 with h = chord^2/4 */
+                    const float dd = __builtin_fmaf(c2, -0.5f, 1.0f);
+                    const float rd = __builtin_amdgcn_rcpf(dd);
+                    const float t2 = __builtin_fmaf(-0.25f * c2, c2, c2) * (rd * rd);
+                    const float r2 = chi2s * t2;
+                    const float u = __builtin_fmaf(__builtin_amdgcn_logf(r2), A.u_k1, -v_k0);
+                    const bool zero = u > u_zero;                     /* r > rmaxt: value 0 */
+                    /* deferred: near the disc edge, a degenerate chord, or u within
+                     * the band of a cell boundary 0..u_max (u clamped to that range,
+                     * then its nearest boundary) */
+                    const float ub = __builtin_amdgcn_fmed3f(u, 0.0f, A.u_max);
+                    const bool defer = (c2 > thr_hi * lo_band) | !(dd > 1e-3f) | (__builtin_fabsf(u - __builtin_rintf(ub)) <= A.band);
+                    if (defer) {
+                        const uint32_t at = atomicAdd(&ctl->nfb[par], 1u);
+                        const bool is_open = Bs == 0.0f;
+                        const uint4 e = make_uint4((uint32_t)(o >> log2c) | (is_open ? COUNT_LISTED : 0u),
+                                                   (uint32_t)(o & ((1 << log2c) - 1)), fw->slot[s], (uint32_t)t);
+                        if (at < FB_LDS) ctl->fb[at] = e;
+                        else {
+                            const unsigned long long gs = atomicAdd(fbc, 1ULL);
+                            if (gs < (unsigned long long)fbs) fbr[gs] = e;
+                            else ctl->lost[par] = 1u;
+                        }
+                        tf += !is_open;
+                        continue;
                     }
-                    tf++;
-                    continue;
-                }
-                const bool clampr = u < 0.0f;                     /* r < rmint: r = rmint + 1e-5 */
-                /* floor(u) + 1 clamped to [1, nrt-1] (u >= 0 here unless clamped:
-                 * truncation is floor); a clamped r (r = rmint + 1e-5) has the cell
-                 * and fraction the host computed for it */
-                const int ir_u = min(max((int)u + 1, 1), nrt - 1);
-                const int ir = clampr ? v_irc : ir_u;
-                /* nodes ir-1 and ir of the cell: 4 corners of every map each,
-                 * 32 NM contiguous bytes, requested before the radial fraction
-                 * so that their latency covers its LDS read and log */
-                const int vo = (cb + (ir - 1)) * (16 * NM);
-                float tq[8 * NM];
-                load_floats<8 * NM>(trs, vo, 0, tq);
-                const float w00 = sl->w00[s], w10 = sl->w10[s], w01 = sl->w01[s], w11 = sl->w11[s];
-                /* fr = ln(r / r_node) = (ln 2 / 2) log2(r^2 / r_node^2): the ratio is
-                 * in [1, 1.08), where the hardware log2 is within one ulp
-                 * (7e-9); both sides evaluated, then selected */
-                float fr_in = 0.34657359f * __builtin_amdgcn_logf(r2 * invn[ir - 1]);
-                asm volatile("" : "+v"(fr_in));   /* computed on every lane: a select, not a branch */
-                const float fr = clampr ? v_frc : fr_in;
-                tu++;
+                    const bool clampr = u < 0.0f;                     /* r < rmint: r = rmint + 1e-5 */
+                    /* cell floor(u) clamped to [0, nrt-2] (u >= 0 here unless clamped:
+                     * truncation is floor); a clamped r (r = rmint + 1e-5) has the cell
+                     * and fraction the host computed for it */
+                    const int cell = clampr ? v_irc : min((int)ub, nrt - 2);
+                    /* nodes `cell` and cell + 1: 4 corners of every map each,
+                     * 32 NM contiguous bytes, requested before the radial fraction
+                     * so that their latency covers its LDS read and log */
+                    const int vo = (cb + cell) * (16 * NM);
+                    float tq[8 * NM];
+                    load_floats<8 * NM>(trs, vo, 0, tq);
+                    const float w00 = fw->w00[s], w10 = fw->w10[s], w01 = fw->w01[s], w11 = fw->w11[s];
+                    /* fr = ln(r / r_node) = (ln 2 / 2) log2(r^2 / r_node^2): the ratio is
+                     * in [1, 1.08), where the hardware log2 is within one ulp
+                     * (7e-9); both sides evaluated, then selected */
+                    float fr_in = 0.34657359f * __builtin_amdgcn_logf(r2 * invn[cell]);
+                    asm volatile("" : "+v"(fr_in));   /* computed on every lane: a select, not a branch */
+                    const float fr = clampr ? v_frc : fr_in;
+                    tu++;
 #pragma unroll
-                for (int m = 0; m < NM; ++m) {
-                    const float *c0v = tq + 4 * m, *c1v = tq + 4 * (NM + m);
-                    /* the corners combined at each node, then one lerp in r */
-                    float v0 = w00 * c0v[0];
-                    v0 = __builtin_fmaf(w10, c0v[1], v0);
-                    v0 = __builtin_fmaf(w01, c0v[2], v0);
-                    v0 = __builtin_fmaf(w11, c0v[3], v0);
-                    float v1 = w00 * c1v[0];
-                    v1 = __builtin_fmaf(w10, c1v[1], v1);
-                    v1 = __builtin_fmaf(w01, c1v[2], v1);
-                    v1 = __builtin_fmaf(w11, c1v[3], v1);
-                    const float val = __builtin_fmaf(fr, v1 - v0, v0);
-                    atomicAdd(&acc[m * W + q], (double)(zero ? 0.0f : val));
-                }
-                if (A.count) {
-                    atomicAdd(&lcount[q], 1u);
-                    atomicAdd(&lhash[q], hh[s]);
+                    for (int m = 0; m < NM; ++m) {
+                        const float *c0v = tq + 4 * m, *c1v = tq + 4 * (NM + m);
+                        /* the corners combined at each node, then one lerp in r */
+                        float v0 = w00 * c0v[0];
+                        v0 = __builtin_fmaf(w10, c0v[1], v0);
+                        v0 = __builtin_fmaf(w01, c0v[2], v0);
+                        v0 = __builtin_fmaf(w11, c0v[3], v0);
+                        float v1 = w00 * c1v[0];
+                        v1 = __builtin_fmaf(w10, c1v[1], v1);
+                        v1 = __builtin_fmaf(w01, c1v[2], v1);
+                        v1 = __builtin_fmaf(w11, c1v[3], v1);
+                        const float fv = __builtin_fmaf(fr, v1 - v0, v0);
+                        atomicAdd(&acc[m * W + o], (double)(zero ? 0.0f : fv));
+                    }
+                    if (A.count) {
+                        atomicAdd(&lcount[o], 1u);
+                        atomicAdd(&lhash[o], hh[s]);
+                    }
                 }
             }
-            };
-            if (npr < 4 * W) paint_pixels(std::true_type{});
-            else paint_pixels(std::false_type{});
         }
-        if (!claimed && tid == 0)        /* a tile without segments */
-            sl->next_tile[par ^ 1] = (int32_t)(xb + (int64_t)atomicAdd(qctr, 1u));
+        if (!fetched && more) load_pairs(sbeg_n, wave_from(cnt_n, wv_u), wave_from(cnt_n, wv_u + 1));
+        if (more && wv == nwv - 1 && lane < Gn.rows)
+            stage_row(ctl->rows[par ^ 1][lane], rdesc[Gn.ring0 - 1 + lane], Gn.K, Gn.k);
+        if (tid == 0) ctl->next_tile[par] = after;
         lds_barrier();
         /* the tile's deferred pixels still in LDS join the list before the
          * tile is written: a tile whose deferred pixels do not all fit in the
          * list writes nothing and is marked for the repaint pass */
-        const uint32_t nfb = sl->nfb[par];
+        const uint32_t nfb = ctl->nfb[par];
         const uint32_t nfl = nfb < FB_LDS ? nfb : FB_LDS;
         if (nfl) {
-            if (tid == 0) sl->fb_base = atomicAdd(fbc, (unsigned long long)nfl);
+            if (tid == 0) ctl->fb_base = atomicAdd(fbc, (unsigned long long)nfl);
             lds_barrier();
             for (uint32_t k = tid; k < nfl; k += blockDim.x)
-                if (sl->fb_base + k < (unsigned long long)fbs) fbr[sl->fb_base + k] = sl->fb[k];
+                if (ctl->fb_base + k < (unsigned long long)fbs) fbr[ctl->fb_base + k] = ctl->fb[k];
         }
-        const bool lost = sl->lost[par] != 0u || (nfl && sl->fb_base + nfl > (unsigned long long)fbs);
+        const bool lost = ctl->lost[par] != 0u || (nfl && ctl->fb_base + nfl > (unsigned long long)fbs);
         if (tid == 0) {
             if (lost) { A.lost[t] = 1; atomicAdd(A.n_lost + (blockIdx.x % P2M_SHARDS) * P2M_CTR_STRIDE, 1ULL); }
             else if (A.redo) A.lost[t] = 0;
         }
-        if (!lost) { n_upd += (unsigned long long)tu; n_fb += (unsigned long long)tf; }
-        const int64_t pix0 = G.first + G.ip0;
+        if (!lost) { n_upd += tu; n_fb += tf; n_list += tl; n_seg += ts; }
+        const bool keep = lost || skip;
         /* the branch on accumulate is taken outside the loops: a select
          * inside lets the compiler load the map speculatively (a map read and
          * a wait on it per tile) even when the tile only stores */
-        if (lost) {
-        } else if (A.accumulate) {
-            for (int q = tid; q < G.width; q += blockDim.x) {
-                for (int m = 0; m < NM; ++m) {
-                    float *dst = A.map32[m] + pix0 + q;
-                    *dst = (float)((double)*dst + acc[m * W + q]);
+        const int npx = G.rows << log2c;
+        auto out = [&](auto add) {
+            for (int p = tid; p < npx; p += blockDim.x) {
+                const TileRow &R = rows[p >> log2c];
+                const int col = p & ((1 << log2c) - 1);
+                if (col < (int)R.width && !keep) {
+                    const int64_t pix = R.pix0 + col;
+                    for (int m = 0; m < NM; ++m) {
+                        float *dst = A.map32[m] + pix;
+                        if constexpr (decltype(add)::value) *dst = (float)((double)*dst + acc[m * W + p]);
+                        else __builtin_nontemporal_store((float)acc[m * W + p], dst);    /* not read again in the pass */
+                    }
+                    if (A.count) {
+                        if constexpr (decltype(add)::value) { A.count[pix] += lcount[p]; A.hash[pix] += lhash[p]; }
+                        else { A.count[pix] = lcount[p]; A.hash[pix] = lhash[p]; }
+                    }
                 }
-                if (A.count) {
-                    A.count[pix0 + q] += lcount[q];
-                    A.hash[pix0 + q] += lhash[q];
-                }
+                for (int m = 0; m < NM; ++m) acc[m * W + p] = 0.0;
+                if (A.count) { lcount[p] = 0; lhash[p] = 0ULL; }
             }
-        } else {
-            for (int q = tid; q < G.width; q += blockDim.x) {
-                /* streaming stores: the map is not read again in the pass, so
-                 * it should not displace halo records and table rows in L2 */
-                for (int m = 0; m < NM; ++m) __builtin_nontemporal_store((float)acc[m * W + q], A.map32[m] + pix0 + q);
-                if (A.count) {
-                    A.count[pix0 + q] = lcount[q];
-                    A.hash[pix0 + q] = lhash[q];
-                }
-            }
+        };
+        if (A.accumulate) out(std::true_type{}); else out(std::false_type{});
+        if (tid == 0) { ctl->nfb[par ^ 1] = 0; ctl->lost[par ^ 1] = 0; }   /* the next tile's slot */
+        if (!more) break;
+        /* the thread's 32-bit counts go out long before they could wrap (a
+         * tile adds at most its pairs' pixels over the lanes) */
+        if (n_upd >= 1u << 30 || n_list >= 1u << 30) {
+            atomicAdd(&A.counters[0], (unsigned long long)n_list); n_list = 0;
+            atomicAdd(&A.counters[1], (unsigned long long)n_upd); n_upd = 0;
         }
-        if (tid == 0) { sl->nfb[par ^ 1] = 0; sl->lost[par ^ 1] = 0; }   /* the next tile's slot */
+        t = tn; G = Gn; sbeg = sbeg_n; cnt = cnt_n;
+        skip = A.redo && !A.lost[t];
     }
-    /* the staged constants are dead: their space takes the block sums (the
+    }
+    lds_barrier();
+    /* the deferred pixels' buffer is free: its space takes the block sums (the
      * kernel has no static LDS, so its occupancy is what its launch asks) */
-    unsigned long long *red = (unsigned long long *)sl->fb;
+    unsigned long long *red = (unsigned long long *)ctl->fb;
+    block_count(&A.counters[0], n_list, red);
     block_count(&A.counters[1], n_upd, red);
+    block_count(&A.counters[4], n_seg, red);
     block_count(&A.counters[5], n_fb, red);
     block_count(A.err, n_err, red);
 }
 
-/* Deferred pixels of k_tile_fast, decided and valued with the exact FP64
- * arithmetic of the reference (pix2vec_ring, angdist, interpolate_table),
- * added to the FP32 map with one atomic each. */
+/* Deferred pixels of k_tile_fast -- (row, in-row pixel, halo, tile) --
+ * decided and valued with the exact FP64 arithmetic of the reference
+ * (pix2vec_ring, angdist, interpolate_table), added to the FP32 map with one
+ * atomic each; ASK_RUN, COUNT_LISTED: see k_tile_fast. */
 __global__ void __launch_bounds__(256) k_fallback(FallbackArgs A)
 {
     __shared__ unsigned long long lds16[16];
@@ -1723,21 +1530,25 @@ __global__ void __launch_bounds__(256) k_fallback(FallbackArgs A)
     unsigned long long n = A.fb_count[blockIdx.y * P2M_CTR_STRIDE];
     if (n > fbs) n = fbs;
     const uint4 *fbr = A.fb + blockIdx.y * fbs;
-    unsigned long long n_upd = 0, n_err = 0;
+    unsigned long long n_upd = 0, n_list = 0, n_err = 0;
     for (unsigned long long i = blockIdx.x * (unsigned long long)blockDim.x + threadIdx.x; i < n;
          i += (unsigned long long)gridDim.x * blockDim.x) {
         const uint4 e = fbr[i];
-        const int32_t ring = (int32_t)e.x, ip = (int32_t)e.y;
-        if (!(e.z < (uint64_t)A.n_halo && ring >= 1 && ring <= 4 * A.nside - 1 && ip >= 0)) { n_err++; continue; }
+        const uint32_t slot = e.z & ~ASK_RUN, row = e.x & ~COUNT_LISTED;
+        if (!(slot < (uint64_t)A.n_halo && e.w < (uint64_t)A.n_tiles && row < MAXROWS)) { n_err++; continue; }
         /* the entries of a tile that lost some of its deferred pixels: the
          * repaint pass decides that tile again */
-        if (A.lost[A.tile_base[ring - 1] + (ip >> A.log2w)]) continue;
+        if (A.lost[e.w]) continue;
+        const TileDesc G = A.desc[e.w];
+        if ((int32_t)row >= G.rows) { n_err++; continue; }
+        const int32_t ring = G.ring0 + (int32_t)row;
         /* bytes [0, 32), [80, 112) and [128, 160) of the record: the fields
          * of the exact test and value, requested before the ring geometry */
-        const uint4 *hs = reinterpret_cast<const uint4 *>(A.halos + A.order[e.z]);
+        const uint4 *hs = reinterpret_cast<const uint4 *>(A.halos + slot);
         const uint4 c0 = hs[0], c1 = hs[1], c5 = hs[5], c6 = hs[6], c8 = hs[8], c9 = hs[9];
         int32_t npr, kshift; int64_t first;
         ring_info(A.nside, ring, npr, kshift, first);
+        const int32_t ip = sector_start(npr, G.K, G.k) + (int32_t)e.y;
         double zr, sth, off, den;
         ring_zsth(A.nside, ring, zr, sth);
         ring_phi_param(A.nside, ring, off, den);
@@ -1752,6 +1563,14 @@ __global__ void __launch_bounds__(256) k_fallback(FallbackArgs A)
         const int64_t cat = (int64_t)(((unsigned long long)c8.y << 32) | c8.x);
         const int32_t ichi = (int32_t)c8.z, imh = (int32_t)c8.w, chi_out = (int32_t)c9.z;
         const double angle = angdist(hx, hy, hz, sth * cs, sth * sn, zr);
+        if (e.z & ASK_RUN) {
+            int32_t lo = 0;
+            const int32_t np = disc_ring_run_z(disc_rec(A.halos[slot]), ring2z(A.nside, ring), npr, kshift, lo);
+            int32_t rel = ip - lo;
+            if (rel < 0) rel += npr;
+            if (rel >= np) continue;
+            n_list += (e.x & COUNT_LISTED) != 0u;
+        }
         if (!(angle < dtheta)) continue;
         n_upd++;
         const int64_t pix = first + ip;
@@ -1768,6 +1587,7 @@ __global__ void __launch_bounds__(256) k_fallback(FallbackArgs A)
             atomicAdd(&A.hash[pix], (unsigned long long)halo_hash(cat));
         }
     }
+    block_count(&A.counters[0], n_list, lds16);
     block_count(&A.counters[1], n_upd, lds16);
     block_count(A.err, n_err, lds16);
 }
@@ -1819,23 +1639,18 @@ void p2m_launch_build_quad(const float *slice, int64_t n_slice, int32_t nrt, int
                        slot, quad);
 }
 
-/* widest tile the painters take: a segment (at most one tile wide) must fit
- * in one batch of PMAX pixels */
-int p2m_tile_max_log2w(void)
-{
-    int l = 6;
-    while ((2 << l) <= PMAX) ++l;
-    return l;
-}
+/* widest tile the painters take (in-tile pixel numbers and the wave's
+ * 64 segments of at most a row, 128 pixels, must fit 16 bits) */
+int p2m_tile_max_log2w(void) { return 11; }
 
-size_t p2m_tile_lds_bytes(int mode, int n_maps, int log2w, int membership, int nrt)
+size_t p2m_tile_lds_bytes(int mode, int n_maps, int log2w, int membership, int nrt, int wg)
 {
-    size_t W = (size_t)1 << log2w;
+    const size_t W = (size_t)1 << log2w, nw = (size_t)(wg / 64);
     size_t b = (size_t)n_maps * W * 8;
     if (membership) b += W * 12;
-    b = (b + 15) & ~(size_t)15;
-    if (mode == 2) b += sizeof(FastSeg) + (membership ? 8 * FSEG : 0) + sizeof(float) * (size_t)(nrt + 2);
-    else b += sizeof(ExactSeg);
+    b = ((b + 15) & ~(size_t)15) + sizeof(TileCtl);
+    if (mode == 2) b += nw * (sizeof(FastWave) + (membership ? 8 * WSEG : 0)) + sizeof(float) * (size_t)(nrt + 2);
+    else b += nw * sizeof(ExactWave);
     return b;
 }
 
@@ -1860,14 +1675,12 @@ int p2m_tile_occupancy(int mode, int n_maps, int wg, size_t lds)
 
 int p2m_launch_tile_paint(const TileArgs &a, int mode, int n_maps, int grid, int wg, hipStream_t s)
 {
-    size_t lds = p2m_tile_lds_bytes(mode, n_maps, a.log2w, a.count != nullptr, a.g.nrt);
+    size_t lds = p2m_tile_lds_bytes(mode, n_maps, a.log2w, a.count != nullptr, a.g.nrt, wg);
     if (lds > 160 * 1024 || wg > 512 || (mode == 2 && wg > 256)) return -1;
-    if (mode == 2) {
-        if (!a.tile_next) return -1;
-        p2m_launch_fill_u32(a.tile_next, 8 * P2M_TQ_STRIDE, 0u, s);   /* empty tile queues */
-    }
-#define P2M_TE(NMv) case NMv: hipLaunchKernelGGL((k_tile_exact<NMv>), dim3(grid), dim3(wg), lds, s, a); break;
-#define P2M_TF(NMv) case NMv: hipLaunchKernelGGL((k_tile_fast<NMv>), dim3(grid), dim3(wg), lds, s, a, a.desc, a.tile_off); break;
+    if (!a.tile_next) return -1;
+    p2m_launch_fill_u32(a.tile_next, 8 * P2M_TQ_STRIDE, 0u, s);   /* empty tile queues */
+#define P2M_TE(NMv) case NMv: hipLaunchKernelGGL((k_tile_exact<NMv>), dim3(grid), dim3(wg), lds, s, a, a.desc, a.tile_off, a.ring); break;
+#define P2M_TF(NMv) case NMv: hipLaunchKernelGGL((k_tile_fast<NMv>), dim3(grid), dim3(wg), lds, s, a, a.desc, a.tile_off, a.ring); break;
     if (mode == 1) {
         switch (n_maps) { P2M_TE(1) P2M_TE(2) P2M_TE(3) P2M_TE(4) P2M_TE(5) P2M_TE(6) default: return -1; }
     } else {
