@@ -106,13 +106,13 @@ struct p2m_ctx {
     float hdr_f[6] = {0, 0, 0, 0, 0, 0};
     TabGeom g;
     float *d_flat[P2M_MAXMAPS] = {nullptr};
-    float *d_prof[P2M_MAXMAPS] = {nullptr};    /* the profile's slice, zero-padded (FP32 painter) */
-    float *d_quad = nullptr;                    /* corner-quad table of all maps (FP32 painter) */
-    int64_t n_flat = 0, n_prof = 0, n_quad = 0;
+    float *d_quad = nullptr;                    /* corner-quad table of all maps (tiled painters) */
+    int64_t n_flat = 0, n_quad = 0;
     double *d_inv_node2 = nullptr;
     float *d_inv_node2f = nullptr;
     uint4 *d_fb = nullptr;
     int64_t fb_cap = 0;
+    double fr_clamp64 = 0.0;
     float fr_clamp = 0.f, u_k1 = 0.f, u_k0 = 0.f, u_max = 0.f;
     int32_t ir_clamp = 1;
     float u_band = 2.5e-4f;     /* half-width of the deferral band around cell boundaries, in cells */
@@ -173,7 +173,7 @@ struct p2m_ctx {
     /* the FP32 painter's last launch, kept for the repaint pass */
     TileArgs last_t;
     FallbackArgs last_f;
-    int last_grid = 0;
+    int last_grid = 0, last_wg = 0;
     bool last_fast = false;
     uint32_t *d_cand = nullptr;
     int64_t cand_cap = 0;
@@ -389,7 +389,7 @@ void p2m_destroy(p2m_ctx *c)
     if (c->ev_h2d_end) (void)hipEventDestroy(c->ev_h2d_end);
     if (c->h2d_stream) (void)hipStreamDestroy(c->h2d_stream);
     for (int m = 0; m < P2M_MAXMAPS; ++m) {
-        dfree(c->d_hp64[m]); dfree(c->d_hp32[m]); dfree(c->d_fs64[m]); dfree(c->d_flat[m]); dfree(c->d_prof[m]);
+        dfree(c->d_hp64[m]); dfree(c->d_hp32[m]); dfree(c->d_fs64[m]); dfree(c->d_flat[m]);
     }
     dfree(c->d_quad);
     dfree(c->d_count); dfree(c->d_hash); dfree(c->d_fs_count); dfree(c->d_fs_hash);
@@ -529,8 +529,8 @@ int p2m_load_table(p2m_ctx *c, int slot, const int32_t hdr_i[3], const float hdr
          * fits goes back to the library's choice */
         const int ml = c->cfg.precision == P2M_PREC_FP64 ? 1 : 2;
         const int mem = c->d_count != nullptr;
-        if (p2m_tile_lds_bytes(ml, c->cfg.n_maps, 10, mem, hdr_i[2], 256) > 160 * 1024) return P2M_E_SIZE;
-        if (c->tuned && c->log2w && p2m_tile_lds_bytes(ml, c->cfg.n_maps, c->log2w, mem, hdr_i[2], c->wg) > 160 * 1024)
+        if (p2m_tile_lds_bytes(ml, c->cfg.n_maps, 10, mem, hdr_i[2], 64) > 160 * 1024) return P2M_E_SIZE;
+        if (c->tuned && c->log2w && p2m_tile_lds_bytes(ml, c->cfg.n_maps, c->log2w, mem, hdr_i[2], 64) > 160 * 1024)
             c->tuned = false;
     }
     TabGeom &g = c->g;
@@ -553,19 +553,11 @@ int p2m_load_table(p2m_ctx *c, int slot, const int32_t hdr_i[3], const float hdr
     std::vector<float> flat(c->n_flat, 0.f);
     memcpy(flat.data(), table, sizeof(float) * nt);
     HIPCHK(hipMemcpy(c->d_flat[slot], flat.data(), sizeof(float) * c->n_flat, hipMemcpyHostToDevice));
-    if (c->cfg.precision == P2M_PREC_FP32_COMP) {
-        /* the profile's slice (column-major ir, imh, ichi), with the same
-         * zero padding past the end for the upper-edge aliasing (Q6) */
-        c->n_prof = nt / 2 + pad / 2;
-        std::vector<float> prof((size_t)c->n_prof, 0.f);
-        const int p = c->cfg.profile;
-        for (int64_t i = 0; i < nt / 2; ++i) prof[(size_t)i] = table[(p - 1) + 2 * i];
-        if (!c->d_prof[slot] && dmalloc((void **)&c->d_prof[slot], sizeof(float) * c->n_prof)) return P2M_E_NOMEM;
-        HIPCHK(hipMemcpy(c->d_prof[slot], prof.data(), sizeof(float) * c->n_prof, hipMemcpyHostToDevice));
+    if (c->cfg.precision != P2M_PREC_PLAIN_FP64) {
         c->n_quad = (int64_t)g.nchit * g.nmht * g.nrt * 4 * c->cfg.n_maps;
         if (!c->d_quad && dmalloc((void **)&c->d_quad, sizeof(float) * c->n_quad)) return P2M_E_NOMEM;
-        p2m_launch_build_quad(c->d_prof[slot], c->n_prof, g.nrt, g.nmht, g.nchit, c->cfg.n_maps, slot, c->d_quad,
-                              c->stream);
+        p2m_launch_build_quad(c->d_flat[slot], c->n_flat, c->cfg.profile, g.nrt, g.nmht, g.nchit, c->cfg.n_maps, slot,
+                              c->d_quad, c->stream);
         HIPCHK(hipGetLastError());
         HIPCHK(hipStreamSynchronize(c->stream));
     }
@@ -590,7 +582,8 @@ int p2m_load_table(p2m_ctx *c, int slot, const int32_t hdr_i[3], const float hdr
          * and fraction as interpolate_table forms them (:196, :200), in FP64 */
         const double lrc = p2m_log(g.rmint + 1e-5);
         c->ir_clamp = (int)((lrc - g.lr0) / g.drt) + 1;
-        c->fr_clamp = (float)(lrc - (g.lr0 + (double)(c->ir_clamp - 1) * g.drt));
+        c->fr_clamp64 = lrc - (g.lr0 + (double)(c->ir_clamp - 1) * g.drt);
+        c->fr_clamp = (float)c->fr_clamp64;
     }
     c->have_table[slot] = true;
     return 0;
@@ -607,7 +600,7 @@ int p2m_set_tile(p2m_ctx *c, int32_t tile_w, int32_t tile_wg)
     int l = 0;
     while ((1 << l) < tile_w) ++l;
     if (p2m_tile_lds_bytes(c->cfg.precision == P2M_PREC_FP64 ? 1 : 2, c->cfg.n_maps, l, c->d_count != nullptr,
-                           c->have_table[0] ? c->g.nrt : 200, tile_wg) > 160 * 1024)
+                           c->have_table[0] ? c->g.nrt : 200, 64) > 160 * 1024)
         return P2M_E_INVALID;
     HIPCHK(hipSetDevice(c->cfg.device));
     int rc = build_tiles(c, l);
@@ -836,6 +829,9 @@ static int paint_halos(p2m_ctx *c, int64_t n_halo, int64_t n_flat, unsigned long
         t.u_k1 = c->u_k1; t.u_k0 = c->u_k0; t.u_max = c->u_max; t.band = c->u_band; t.fr_clamp = c->fr_clamp; t.ir_clamp = c->ir_clamp;
         t.band_c = (float)CHORD_BAND;
         t.inv_node2f = c->d_inv_node2f;
+        t.inv_drt = 1.0 / c->g.drt; t.u_max64 = (double)(c->g.nrt - 1); t.fr_clamp64 = c->fr_clamp64;
+        /* ln r is off by a few 1e-12 at most for discs above 1e-4 rad */
+        t.band64 = std::max(1e-7, 1e-11 * t.inv_drt);
         t.n_quad = c->n_quad; t.tab_q = c->d_quad;
         t.fb = c->d_fb; t.fb_count = pc + 6; t.fb_cap = c->fb_cap;
         t.lost = c->d_lost; t.tile_next = c->d_tile_next; t.redo = 0; t.n_halo = n_halo; t.err = c->d_ctr + Ctr::ERR; t.n_lost = c->d_ctr + Ctr::LOST;
@@ -846,15 +842,16 @@ static int paint_halos(p2m_ctx *c, int64_t n_halo, int64_t n_flat, unsigned long
         /* persistent grid of exactly the resident workgroups (a multiple
          * of 8 for the XCD-aware tile order): no partial last round */
         int grid = (int)std::min<int64_t>(c->n_tiles, 8192);
+        const int wg = p2m_tile_wg(mode, c->cfg.n_maps, c->log2w, c->d_count != nullptr, c->g.nrt, c->wg);
         {
-            const size_t lds = p2m_tile_lds_bytes(mode, c->cfg.n_maps, c->log2w, c->d_count != nullptr, c->g.nrt, c->wg);
-            const int occ = p2m_tile_occupancy(mode, c->cfg.n_maps, c->wg, lds);
+            const size_t lds = p2m_tile_lds_bytes(mode, c->cfg.n_maps, c->log2w, c->d_count != nullptr, c->g.nrt, wg);
+            const int occ = p2m_tile_occupancy(mode, c->cfg.n_maps, wg, lds);
             if (occ > 0 && c->n_cu > 0) {
                 const int64_t res = ((int64_t)occ * c->n_cu) & ~(int64_t)7;
                 if (res >= 8) grid = (int)std::min<int64_t>(c->n_tiles, res);
             }
         }
-        if (p2m_launch_tile_paint(t, mode, c->cfg.n_maps, grid, c->wg, c->stream)) return P2M_E_INVALID;
+        if (p2m_launch_tile_paint(t, mode, c->cfg.n_maps, grid, wg, c->stream)) return P2M_E_INVALID;
         HIPCHK(hipGetLastError());
         HIPCHK(hipEventRecord(c->ev[7], c->stream));
         if (mode == P2M_PREC_FP32_COMP) {
@@ -868,7 +865,7 @@ static int paint_halos(p2m_ctx *c, int64_t n_halo, int64_t n_flat, unsigned long
             f.lost = c->d_lost; f.desc = c->d_tile_desc; f.n_tiles = c->n_tiles; f.n_halo = n_halo;
             f.err = c->d_ctr + Ctr::ERR;
             if (p2m_launch_fallback(f, (int64_t)(n_pix / 256) + 1024, c->stream)) return P2M_E_HIP;
-            c->last_t = t; c->last_f = f; c->last_grid = grid; 
+            c->last_t = t; c->last_f = f; c->last_grid = grid; c->last_wg = wg; 
         }
         c->last_fast = mode == P2M_PREC_FP32_COMP;
         HIPCHK(hipEventRecord(c->ev[4], c->stream));
@@ -947,7 +944,7 @@ static int repaint_lost(p2m_ctx *c, unsigned long long h[Ctr::TOTAL], unsigned l
         p2m_launch_clear_ctr(c->d_ctr, Ctr::LOST, 1, c->stream);
         TileArgs t = c->last_t;
         t.fb = c->d_fb; t.fb_cap = cap; t.redo = 1;
-        if (p2m_launch_tile_paint(t, P2M_PREC_FP32_COMP, c->cfg.n_maps, c->last_grid, c->wg, c->stream))
+        if (p2m_launch_tile_paint(t, P2M_PREC_FP32_COMP, c->cfg.n_maps, c->last_grid, c->last_wg, c->stream))
             return P2M_E_INVALID;
         HIPCHK(hipGetLastError());
         FallbackArgs f = c->last_f;
@@ -1327,7 +1324,7 @@ static int autotune(p2m_ctx *c, int64_t n_halo, int64_t n_flat, unsigned long lo
     float best_ms = 1e30f;
     for (auto &cd : cand) {
         if (cd[0] > p2m_tile_max_log2w()) continue;
-        if (p2m_tile_lds_bytes(mode_ld, c->cfg.n_maps, cd[0], c->d_count != nullptr, c->g.nrt, cd[1]) > 160 * 1024) continue;
+        if (p2m_tile_lds_bytes(mode_ld, c->cfg.n_maps, cd[0], c->d_count != nullptr, c->g.nrt, 64) > 160 * 1024) continue;
         int rc = build_tiles(c, cd[0]); if (rc) return rc;
         c->wg = cd[1]; c->tuned = true;
         c->hp_zero = true;

@@ -113,6 +113,8 @@ struct TileArgs {
     const double *inv_node2;      /* exp(-2 (lr0 + k drt)), k = 0..nrt */
     const float *inv_node2f;      /* the same in float */
     float u_k1, u_k0, u_max, band, fr_clamp;
+    double inv_drt, u_max64, band64, fr_clamp64;     /* the FP64 painter's: 1/drt, nrt - 1, the band around cell
+                                                        boundaries (in cells) that takes the exact arithmetic */
     int32_t ir_clamp;             /* cell and fraction of r = rmint + 1e-5 (maptable.f90:190, 196, 200) */
     float band_c;                 /* CHORD_BAND */
     double *map64[P2M_MAXMAPS];
@@ -175,9 +177,10 @@ void p2m_launch_ring_desc(int32_t nside, RingDesc *out, hipStream_t s);
 void p2m_launch_tile_desc(const TileShape &g, const int32_t *band_tile, TileDesc *desc, hipStream_t s);
 int p2m_scan_u32(const uint32_t *cnt, unsigned long long *off, int64_t n, void *tmp, size_t *tmp_bytes, hipStream_t s);
 int p2m_tile_max_log2w(void);
-void p2m_launch_build_quad(const float *slice, int64_t n_slice, int32_t nrt, int32_t nmht, int32_t nchit,
+void p2m_launch_build_quad(const float *flat, int64_t n_flat, int32_t profile, int32_t nrt, int32_t nmht, int32_t nchit,
                            int32_t n_maps, int32_t slot, float *quad, hipStream_t s);
 size_t p2m_tile_lds_bytes(int mode, int n_maps, int log2w, int membership, int nrt, int wg);
+int p2m_tile_wg(int mode, int n_maps, int log2w, int membership, int nrt, int wg);
 int p2m_tile_occupancy(int mode, int n_maps, int wg, size_t lds);
 int p2m_launch_tile_paint(const TileArgs &a, int mode, int n_maps, int grid, int wg, hipStream_t s);
 int p2m_launch_fallback(const FallbackArgs &a, int64_t n_max, hipStream_t s);

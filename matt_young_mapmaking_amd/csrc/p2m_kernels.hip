@@ -17,7 +17,7 @@
  *  k_fallback        the exact FP64 decision and value (haloproject.f90:60-75,
  *                    maptable.f90:176-216)
  *  k_tile_exact      FP64 painter over the same tiles, the reference's
- *                    arithmetic per pixel, FP64 LDS tile
+ *                    arithmetic where it decides, FP64 LDS tile
  *  k_paint_plain_hp  baseline: one work item per halo, naive query_disc loop,
  *                    pix2vec_ring/angdist/interpolate_table per pixel, FP64
  *                    global atomics (haloproject.f90:55-75)
@@ -28,6 +28,7 @@
  *  k_moments         map moments and the dP/dy histogram (pks2map.f90:321-357)
  */
 #include "p2m_kernels.h"
+#include "p2m_fast64.h"
 
 #include <hipcub/hipcub.hpp>
 #include <type_traits>
@@ -927,21 +928,41 @@ struct TileQueue {
 /* ------------------------------------------------------------------ */
 /* FP64 tiled painter                                                   */
 /*                                                                      */
-/* The exact arithmetic of the reference per pixel: pix2vec_ring from    */
-/* the ring's z and sin(theta) and the pixel's phi, angdist against the  */
-/* disc radius, interpolate_table in FP64, accumulated in an FP64 LDS    */
-/* tile (ds_add_f64) and reduced to the FP64 map.                        */
+/* Each tile's pixel vectors are formed once, in LDS, with the            */
+/* reference's arithmetic (pix2vec_ring from the ring's z and sin(theta)   */
+/* and the pixel's phi); per pixel and halo sin^2(theta) is the squared     */
+/* cross product, the same bits as the reference's, the table cell and      */
+/* fraction follow from its logarithm, the value from the corner-quad table; */
+/* it is accumulated in an FP64 LDS tile (ds_add_f64) and written to the    */
+/* FP64 map.  Where a decision could differ from the reference's -- sin^2     */
+/* within rounding of the disc edge's, the radial coordinate of a cell       */
+/* boundary -- and for wide discs, the reference's arithmetic is carried    */
+/* out in place: angdist against the disc radius, interpolate_table.        */
+/*                                                                      */
+/* Bound: FP64 VALU.  Carrying that out for every pixel took five times     */
+/* the operations (a sine, a cosine, an arc tangent, a tangent and a        */
+/* logarithm with their quotients, eight table loads): 2e6 halos at nside  */
+/* 2048 1.85 ms, 1.22 ms now.  (The chord relation of the FP32 painter needs */
+/* no vectors and was as fast, but its rounding is another than the cross   */
+/* product's: 1e-16 of the chord, 1.3e-12 of a value near a halo's centre.)  */
 /* ------------------------------------------------------------------ */
 
-/* the per-segment values the exact per-pixel code reads, one set per wave */
+/* the per-segment values, one set per wave */
 struct ExactWave {
-    double hx[WSEG], hy[WSEG], hz[WSEG], dth[WSEG], vh[WSEG], chir[WSEG], fc[WSEG], fm[WSEG];
-    unsigned long long hash[WSEG];
     unsigned long long bits[WPIX / 64];   /* segment starts */
-    int32_t col[WSEG];             /* in-row pixel minus the wave's pixel number */
-    int32_t imh[WSEG], ichi[WSEG], cout[WSEG], row[WSEG];
-    int32_t hole[WSEG];            /* in-row pixels the run leaves out: first | end << 16 */
+    double hx[WSEG], hy[WSEG], hz[WSEG];
+    double edge[WSEG];             /* sin^2(dtheta) (1 + EDGE_BAND) */
+    double l0[WSEG];               /* (ln chi - ln rmin) / drt */
+    double w00[WSEG], w10[WSEG], w01[WSEG], w11[WSEG];     /* corner weights times the velocity factor */
+    int32_t qoff[WSEG];            /* in-tile pixel minus the wave's pixel number */
+    int32_t colbase[WSEG];
+    uint32_t slot[WSEG];           /* halo; SLOW: every pixel takes the reference's arithmetic */
+    uint32_t hole[WSEG];           /* in-tile pixels the run leaves out: first | end << 12 | row << 24 */
 };
+/* relative half-width of the band around the disc edge: sin^2 and the edge's are
+ * rounded a few times */
+#define EDGE_BAND 1e-13
+#define SLOW 0x80000000u
 
 /* interpolate_table (maptable.f90:176-216) on staged per-halo values, the
  * same operations in the same order as interp_exact; the table through a
@@ -975,19 +996,41 @@ __device__ static inline double interp_staged(int chi_out, double chi_r, double 
     return v;
 }
 
+/* NF consecutive floats of a raw buffer at byte offset vo + so, in loads of
+ * 16 and 8 bytes (dword alignment is enough for buffer loads) */
+template <int NF>
+__device__ static inline void load_floats(__amdgpu_buffer_rsrc_t r, int vo, int so, float *f)
+{
+    int k = 0;
+#pragma unroll
+    for (; k + 4 <= NF; k += 4) {
+        const auto v = __builtin_amdgcn_raw_buffer_load_b128(r, vo + 4 * k, so, 0);
+        f[k] = __uint_as_float((uint32_t)v[0]); f[k + 1] = __uint_as_float((uint32_t)v[1]);
+        f[k + 2] = __uint_as_float((uint32_t)v[2]); f[k + 3] = __uint_as_float((uint32_t)v[3]);
+    }
+#pragma unroll
+    for (; k + 2 <= NF; k += 2) {
+        const auto v = __builtin_amdgcn_raw_buffer_load_b64(r, vo + 4 * k, so, 0);
+        f[k] = __uint_as_float((uint32_t)v[0]); f[k + 1] = __uint_as_float((uint32_t)v[1]);
+    }
+#pragma unroll
+    for (; k < NF; ++k) f[k] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(r, vo + 4 * k, so, 0));
+}
+
 /* per-thread statistics of a painter */
 struct PaintStats {
     unsigned long long listed, upd, segs, err;
 };
 
 template <int NM>
-__global__ void __launch_bounds__(512) k_tile_exact(TileArgs A, const TileDesc *__restrict__ tdesc,
+__global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(NM == 1 ? 3 : 2))) k_tile_exact(TileArgs A, const TileDesc *__restrict__ tdesc,
                                                     const unsigned long long *__restrict__ toff,
                                                     const RingDesc *__restrict__ rdesc)
 {
     extern __shared__ unsigned char smem_raw[];
     const int W = 1 << A.log2w, log2c = A.shape.log2c;
-    /* LDS: acc (NM*W doubles) | hash (W u64) count (W u32) if membership | TileCtl | ExactWave per wave */
+    /* LDS: acc (NM*W doubles) | hash (W u64) count (W u32) if membership | TileCtl | pixel vectors (2W doubles) |
+     * ExactWave per wave */
     double *acc = (double *)smem_raw;
     const size_t acc_bytes = (size_t)NM * W * 8;
     unsigned long long *lhash = (unsigned long long *)(smem_raw + acc_bytes);
@@ -995,13 +1038,14 @@ __global__ void __launch_bounds__(512) k_tile_exact(TileArgs A, const TileDesc *
     const size_t mem_bytes = A.count ? (size_t)W * 12 : 0;
     TileCtl *ctl = (TileCtl *)(smem_raw + ((acc_bytes + mem_bytes + 15) & ~(size_t)15));
     const int tid = threadIdx.x, lane = __lane_id(), wv = tid >> 6, nwv = (int)(blockDim.x >> 6);
-    ExactWave *ew = (ExactWave *)(ctl + 1) + wv;
+    /* x and y of the tile's pixel vectors */
+    double *vx = (double *)(ctl + 1), *vy = vx + W;
+    ExactWave *ew = (ExactWave *)(vy + W) + wv;
     PaintStats st = {0, 0, 0, 0};
-    __amdgpu_buffer_rsrc_t trs[NM];
-    for (int m = 0; m < NM; ++m)
-        trs[m] = __builtin_amdgcn_make_buffer_rsrc((void *)A.tab_flat[m], (short)0, (int)(A.n_flat * 4), 0x00020000);
-    const TileQueue q(A);
-    if (tid == 0) ctl->next_tile[0] = q.claim();
+    const __amdgpu_buffer_rsrc_t tab =
+        __builtin_amdgcn_make_buffer_rsrc((void *)A.tab_q, (short)0, (int)(A.n_quad * 4), 0x00020000);
+    const TileQueue queue(A);
+    if (tid == 0) ctl->next_tile[0] = queue.claim();
     for (int p = tid; p < W; p += blockDim.x) {
         for (int m = 0; m < NM; ++m) acc[m * W + p] = 0.0;
         if (A.count) { lcount[p] = 0; lhash[p] = 0ULL; }
@@ -1009,13 +1053,24 @@ __global__ void __launch_bounds__(512) k_tile_exact(TileArgs A, const TileDesc *
     lds_barrier();
     for (int par = 0;; par ^= 1) {
         const int64_t t = (int64_t)__builtin_amdgcn_readfirstlane(ctl->next_tile[par]);
-        if (t >= q.xe) break;
+        if (t >= queue.xe) break;
         const TileDesc G = tdesc[t];
         const uint64_t sbeg = toff[t], send = toff[t + 1];
         const TileRow *rows = ctl->rows[par];
         if (tid < G.rows) stage_row(ctl->rows[par][tid], rdesc[G.ring0 - 1 + tid], G.K, G.k);
-        if (tid == 0) ctl->next_tile[par ^ 1] = q.claim();
+        if (tid == 0) ctl->next_tile[par ^ 1] = queue.claim();
         lds_barrier();
+        if (send > sbeg) {
+            for (int p = tid; p < G.rows << log2c; p += blockDim.x) {
+                const TileRow &Q = rows[p >> log2c];
+                const double phi = (((double)((int)Q.ip0 + (p & ((1 << log2c) - 1))) + (double)Q.off) * HPX_HALFPI) / Q.den();
+                double sn, cs;
+                p2m_sincos(phi, &sn, &cs);
+                vx[p] = Q.sth * cs;
+                vy[p] = Q.sth * sn;
+            }
+            lds_barrier();
+        }
         const uint32_t cnt = (uint32_t)(send - sbeg);
         const int wv_u = __builtin_amdgcn_readfirstlane(wv);
         uint64_t pos = sbeg + wave_share(cnt, wv_u, nwv);
@@ -1031,23 +1086,43 @@ __global__ void __launch_bounds__(512) k_tile_exact(TileArgs A, const TileDesc *
             if (g.act && !((uint64_t)slot < (uint64_t)A.n_halo && g.row < G.rows)) { st.err++; g.act = false; }
             if (!g.act) { slot = 0; g.row = 0; }
             const HaloRec &h = A.halos[slot];
-            const TileRow &R = rows[g.row];
+            const TileRow R = rows[g.row];
             const int32_t ring = G.ring0 + g.row;
             int32_t lo = 0, np = 0, a = 0, len = 0, c = 0, d = 0;
-            if (g.act) np = disc_ring_run_fast(disc_rec(h), ring2z(A.nside, ring), R.npr, R.kshift(), lo);
+            const double thr = h.thr;
+            if (g.act) {
+                /* the run as in k_tile_fast, the exact one in place where that is open */
+                const double off = (double)R.off, ik = R.ik(), phi0 = h.phi0;
+                const double dz = R.zr - h.zz0, ds = R.sth - h.s0;
+                const double ipcd = __builtin_rint(phi0 * ik - off);
+                int32_t ipc = (int32_t)ipcd, np_max;
+                if (ipc < 0) ipc += R.npr;
+                if (ipc >= R.npr) ipc -= R.npr;
+                np = disc_ring_run_chord(thr, dz * dz + ds * ds, (float)((4.0 * R.sth) * h.s0), R.e_row,
+                                         (float)(0.5 * ((ipcd + off) * R.kphi - phi0)), (float)(2.0 * ik), ipc, R.npr, lo, np_max);
+                if (np < 0) np = disc_ring_run_z(disc_rec(h), ring2z(A.nside, ring), R.npr, R.kshift(), lo);
+            }
             if (np > 0) st.listed += (unsigned long long)clip_run(lo, np, R, a, len, c, d);
             st.segs += len > 0;
             const uint32_t incl = wave_incl_scan((uint32_t)len), start = incl - (uint32_t)len;
             const uint32_t P = (uint32_t)__builtin_amdgcn_readlane((int)incl, 63);
-            wave_lds_fence();
             const unsigned long long some = __ballot(len > 0);
+            wave_lds_fence();
             if (len > 0) {
                 const int k = (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(some >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)some, 0u));
-                ew->hx[k] = h.hx; ew->hy[k] = h.hy; ew->hz[k] = h.hz; ew->dth[k] = h.dtheta;
-                ew->vh[k] = h.vh; ew->chir[k] = h.chi_r; ew->fc[k] = h.fc; ew->fm[k] = h.fm;
-                ew->imh[k] = h.imh; ew->ichi[k] = h.ichi; ew->cout[k] = h.chi_out;
-                ew->row[k] = g.row; ew->col[k] = a - (int32_t)start; ew->hole[k] = c | (d << 16);
-                if (A.count) ew->hash[k] = halo_hash(h.cat);
+                const bool slow = h.chi_out || !(thr < F64_SMALL_Q) || !(h.chi_r > 1e-30);
+                const double gm = 1.0 - h.fm, gc = 1.0 - h.fc;
+                ew->hx[k] = h.hx; ew->hy[k] = h.hy; ew->hz[k] = h.hz;
+                /* sin^2(dtheta) from the chord^2 of the edge */
+                ew->edge[k] = (thr * (1.0 - 0.25 * thr)) * (1.0 + EDGE_BAND);
+                ew->l0[k] = slow ? 0.0 : (f64_log(h.chi_r) - A.g.lr0) * A.inv_drt;
+                ew->w00[k] = h.vh * (gc * gm); ew->w10[k] = h.vh * (h.fc * gm);
+                ew->w01[k] = h.vh * (gc * h.fm); ew->w11[k] = h.vh * (h.fc * h.fm);
+                const int32_t o0 = g.row << log2c;
+                ew->qoff[k] = o0 + a - (int32_t)start;
+                ew->colbase[k] = A.g.nrt * ((h.imh - 1) + A.g.nmht * (h.ichi - 1));
+                ew->slot[k] = slot | (slow ? SLOW : 0u);
+                ew->hole[k] = (uint32_t)(d > c ? o0 + c : 0) | ((uint32_t)(d > c ? o0 + d : 0) << 12) | ((uint32_t)g.row << 24);
             }
             uint32_t before = 0;
             for (uint32_t base = 0; base < P; base += WPIX) {
@@ -1060,24 +1135,64 @@ __global__ void __launch_bounds__(512) k_tile_exact(TileArgs A, const TileDesc *
                     const int s = (int)__builtin_amdgcn_mbcnt_hi(mhi, __builtin_amdgcn_mbcnt_lo(mlo, before));
                     before += (uint32_t)(__builtin_popcount(mlo) + __builtin_popcount(mhi));
                     const uint32_t p = p0 + (uint32_t)lane;
-                    if (p >= pe) continue;
-                    const int row = ew->row[s], col = ew->col[s] + (int)p, hole = ew->hole[s];
-                    if (col >= (hole & 0xffff) && col < (hole >> 16)) continue;
-                    const TileRow &Q = rows[row];
-                    const double phi = (((double)((int)Q.ip0 + col) + (double)Q.off) * HPX_HALFPI) / Q.den();
-                    double sn, cs;
-                    p2m_sincos(phi, &sn, &cs);
-                    const double angle = angdist(ew->hx[s], ew->hy[s], ew->hz[s], Q.sth * cs, Q.sth * sn, Q.zr);
-                    if (!(angle < ew->dth[s])) continue;
-                    st.upd++;
-                    const int o = (row << log2c) + col;
-                    for (int m = 0; m < NM; ++m)
-                        atomicAdd(&acc[m * W + o], ew->vh[s] * interp_staged(ew->cout[s], ew->chir[s], ew->fc[s], ew->fm[s],
-                                                                             ew->imh[s], ew->ichi[s], A.g, trs[m],
-                                                                             A.profile, angle));
-                    if (A.count) {
+                    const bool in = p < pe;
+                    /* every lane computes (those past the end on the wave's last
+                     * segment's values), the decisions are masks: the step is
+                     * one stretch of code but for the stores and the rare
+                     * pixels that take the reference's arithmetic */
+                    const uint32_t hole = ew->hole[s], sl = ew->slot[s];
+                    const int row = (int)(hole >> 24), o = in ? (int)p + ew->qoff[s] : 0;
+                    const bool far = (int32_t)sl >= 0;                 /* not SLOW */
+                    /* the cross product of angdist */
+                    const double ax = ew->hx[s], ay = ew->hy[s], az = ew->hz[s], bx = vx[o], by = vy[o], bz = rows[row].zr;
+                    const double v0 = ay * bz - az * by, v1 = az * bx - ax * bz, v2 = ax * by - ay * bx;
+                    const double q = (v0 * v0 + v1 * v1) + v2 * v2, edge = ew->edge[s];
+                    const double u = __builtin_fma(__builtin_fma(0.5, f64_log(q), f64_lntan_sin2(q)), A.inv_drt, ew->l0[s]);
+                    const double ub = __builtin_fmin(__builtin_fmax(u, 0.0), A.u_max64);
+                    const bool gap = (o >= (int)(hole & 0xfffu)) & (o < (int)((hole >> 12) & 0xfffu));
+                    const bool cand = in & !gap & !(far & (q > edge));
+                    const bool plain = cand & far & (q < edge * (1.0 - 2.0 * EDGE_BAND)) & (q > 1e-60) &
+                                       (__builtin_fabs(u - __builtin_rint(ub)) > A.band64);
+                    bool taken = plain;
+                    if (plain) {
+                        const bool clampr = u < 0.0;                  /* r < rmint: r = rmint + 1e-5 */
+                        const int cl = min((int)ub, A.g.nrt - 2), cell = clampr ? A.ir_clamp - 1 : cl;
+                        const double fr = clampr ? A.fr_clamp64 : (u - (double)cl) * A.g.drt;
+                        const double gr = 1.0 - fr;
+                        float tq[8 * NM];
+                        load_floats<8 * NM>(tab, (ew->colbase[s] + cell) * (16 * NM), 0, tq);
+                        const double w00 = ew->w00[s], w10 = ew->w10[s], w01 = ew->w01[s], w11 = ew->w11[s];
+                        const bool zero = u > A.u_max64;               /* r > rmaxt */
+#pragma unroll
+                        for (int m = 0; m < NM; ++m) {
+                            const float *c0v = tq + 4 * m, *c1v = tq + 4 * (NM + m);
+                            double v0m = w00 * (double)c0v[0], v1m = w00 * (double)c1v[0];
+                            v0m = __builtin_fma(w10, (double)c0v[1], v0m); v1m = __builtin_fma(w10, (double)c1v[1], v1m);
+                            v0m = __builtin_fma(w01, (double)c0v[2], v0m); v1m = __builtin_fma(w01, (double)c1v[2], v1m);
+                            v0m = __builtin_fma(w11, (double)c0v[3], v0m); v1m = __builtin_fma(w11, (double)c1v[3], v1m);
+                            atomicAdd(&acc[m * W + o], zero ? 0.0 : __builtin_fma(fr, v1m, gr * v0m));
+                        }
+                    }
+                    if (__ballot(cand & !plain)) {
+                        if (cand & !plain) {
+                            /* the reference's arithmetic */
+                            const HaloRec &hr = A.halos[sl & ~SLOW];
+                            const double angle = angdist(hr.hx, hr.hy, hr.hz, bx, by, bz);
+                            if (angle < hr.dtheta) {
+                                taken = true;
+                                for (int m = 0; m < NM; ++m) {
+                                    const __amdgpu_buffer_rsrc_t tr =
+                                        __builtin_amdgcn_make_buffer_rsrc((void *)A.tab_flat[m], (short)0, (int)(A.n_flat * 4), 0x00020000);
+                                    atomicAdd(&acc[m * W + o], hr.vh * interp_staged(hr.chi_out, hr.chi_r, hr.fc, hr.fm, hr.imh, hr.ichi,
+                                                                                     A.g, tr, A.profile, angle));
+                                }
+                            }
+                        }
+                    }
+                    st.upd += taken;
+                    if (A.count && taken) {
                         atomicAdd(&lcount[o], 1u);
-                        atomicAdd(&lhash[o], ew->hash[s]);
+                        atomicAdd(&lhash[o], (unsigned long long)halo_hash(A.halos[sl & ~SLOW].cat));
                     }
                 }
             }
@@ -1173,27 +1288,6 @@ __device__ static inline float sin2f(float x)
     p = __builtin_fmaf(z, p, -1.6666667e-1f);
     const float sn = __builtin_fmaf(x * z, p, x);
     return sn * sn;
-}
-
-/* NF consecutive floats of a raw buffer at byte offset vo + so, in loads of
- * 16 and 8 bytes (dword alignment is enough for buffer loads) */
-template <int NF>
-__device__ static inline void load_floats(__amdgpu_buffer_rsrc_t r, int vo, int so, float *f)
-{
-    int k = 0;
-#pragma unroll
-    for (; k + 4 <= NF; k += 4) {
-        const auto v = __builtin_amdgcn_raw_buffer_load_b128(r, vo + 4 * k, so, 0);
-        f[k] = __uint_as_float((uint32_t)v[0]); f[k + 1] = __uint_as_float((uint32_t)v[1]);
-        f[k + 2] = __uint_as_float((uint32_t)v[2]); f[k + 3] = __uint_as_float((uint32_t)v[3]);
-    }
-#pragma unroll
-    for (; k + 2 <= NF; k += 2) {
-        const auto v = __builtin_amdgcn_raw_buffer_load_b64(r, vo + 4 * k, so, 0);
-        f[k] = __uint_as_float((uint32_t)v[0]); f[k + 1] = __uint_as_float((uint32_t)v[1]);
-    }
-#pragma unroll
-    for (; k < NF; ++k) f[k] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(r, vo + 4 * k, so, 0));
 }
 
 template <int NM>
@@ -1601,16 +1695,16 @@ int p2m_launch_fallback(const FallbackArgs &a, int64_t n_max, hipStream_t s)
     return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 
-/* The FP32 painter's table: for every (mass, chi) cell and radial node k,
+/* The tiled painters' table: for every (mass, chi) cell and radial node k,
  * the values of the four corners the pixel weights combine -- (imh, ichi),
  * (imh+1, ichi), (imh, ichi+1), (imh+1, ichi+1) -- for every map, so that a
  * pixel's two nodes k = ir-1, ir are 32 NM contiguous bytes:
  *   quad[((cell * nrt + k) * n_maps + m) * 4 + corner],
  *   cell = (imh-1) + nmht (ichi-1).
- * Corner values come from the profile slice by the reference's flat index
+ * Corner values come from the (zero-padded) table by the reference's flat index
  * (maptable.f90:204-212), so the aliasing past the upper mass or chi edge
  * (Q6) reads the next column or the zero padding as the flat table does. */
-__global__ void k_build_quad(const float *slice, int64_t n_slice, int32_t nrt, int32_t nmht, int32_t nchit,
+__global__ void k_build_quad(const float *flat, int64_t n_flat, int32_t profile, int32_t nrt, int32_t nmht, int32_t nchit,
                              int32_t n_maps, int32_t slot, float *quad)
 {
     const int64_t n = (int64_t)nrt * nmht * nchit;
@@ -1621,21 +1715,22 @@ __global__ void k_build_quad(const float *slice, int64_t n_slice, int32_t nrt, i
         float v[4];
         for (int cr = 0; cr < 4; ++cr) {
             const int64_t idx = (int64_t)k + (int64_t)nrt * ((int64_t)(imh0 + (cr & 1)) + (int64_t)nmht * (ichi0 + (cr >> 1)));
-            v[cr] = idx < n_slice ? slice[idx] : 0.0f;
+            const int64_t at = 2 * idx + (profile - 1);
+            v[cr] = at < n_flat ? flat[at] : 0.0f;
         }
         float *q = quad + (e * n_maps + slot) * 4;
         q[0] = v[0]; q[1] = v[1]; q[2] = v[2]; q[3] = v[3];
     }
 }
 
-void p2m_launch_build_quad(const float *slice, int64_t n_slice, int32_t nrt, int32_t nmht, int32_t nchit,
+void p2m_launch_build_quad(const float *flat, int64_t n_flat, int32_t profile, int32_t nrt, int32_t nmht, int32_t nchit,
                            int32_t n_maps, int32_t slot, float *quad, hipStream_t s)
 {
     const int64_t n = (int64_t)nrt * nmht * nchit;
     if (n <= 0) return;
     int64_t g = (n + 255) / 256;
     if (g > 16384) g = 16384;
-    hipLaunchKernelGGL(k_build_quad, dim3((unsigned)g), dim3(256), 0, s, slice, n_slice, nrt, nmht, nchit, n_maps,
+    hipLaunchKernelGGL(k_build_quad, dim3((unsigned)g), dim3(256), 0, s, flat, n_flat, profile, nrt, nmht, nchit, n_maps,
                        slot, quad);
 }
 
@@ -1650,8 +1745,17 @@ size_t p2m_tile_lds_bytes(int mode, int n_maps, int log2w, int membership, int n
     if (membership) b += W * 12;
     b = ((b + 15) & ~(size_t)15) + sizeof(TileCtl);
     if (mode == 2) b += nw * (sizeof(FastWave) + (membership ? 8 * WSEG : 0)) + sizeof(float) * (size_t)(nrt + 2);
-    else b += nw * sizeof(ExactWave);
+    else b += 2 * W * sizeof(double) + nw * sizeof(ExactWave);
     return b;
+}
+
+/* The workgroup size to launch for an asked one: every wave has its own
+ * staging, so a wide tile of many maps takes fewer waves than asked (down to
+ * one) where all of them do not fit the CU's 160 KB of LDS. */
+int p2m_tile_wg(int mode, int n_maps, int log2w, int membership, int nrt, int wg)
+{
+    while (wg > 64 && p2m_tile_lds_bytes(mode, n_maps, log2w, membership, nrt, wg) > 160 * 1024) wg -= 64;
+    return wg;
 }
 
 /* workgroups of the tile painter resident per CU at this shape (0 on error) */

@@ -17,6 +17,7 @@
 
 #include "../../include/pks2map_gpu.h"
 #include "p2m_kernels.h"
+#include "p2m_fast64.h"
 
 namespace {
 
@@ -171,69 +172,6 @@ __global__ void __launch_bounds__(64) k_gram_rules(double *rules)
     rules[2 * i + 1] = w;
 }
 
-/* square root, ln x and e^x of normal arguments (x > 0 for the first two):
- * a refined reciprocal square root, and the series of p2m_log and p2m_exp with
- * fused multiply-adds and the quotient by a refined reciprocal; a few 1e-16
- * relative, as those */
-__device__ static inline double mt_sqrt(double x)
-{
-    const double r = __builtin_amdgcn_rsq(x);
-    double g = x * r, h = 0.5 * r;
-    const double e = __builtin_fma(-h, g, 0.5);
-    g = __builtin_fma(g, e, g);
-    h = __builtin_fma(h, e, h);
-    return __builtin_fma(__builtin_fma(-g, g, x), h, g);
-}
-
-__device__ static inline double mt_log(double x)
-{
-    double m = __builtin_amdgcn_frexp_mant(x);
-    int e = __builtin_amdgcn_frexp_exp(x);
-    const bool low = m < 0x1.6a09e667f3bcdp-1;
-    m = low ? 2.0 * m : m;
-    e = low ? e - 1 : e;
-    const double d = m + 1.0, nn = m - 1.0;
-    double r = __builtin_amdgcn_rcp(d);
-    r = __builtin_fma(r, __builtin_fma(-d, r, 1.0), r);
-    r = __builtin_fma(r, __builtin_fma(-d, r, 1.0), r);
-    double s = nn * r;
-    s = __builtin_fma(r, __builtin_fma(-s, d, nn), s);
-    const double z = s * s;
-    double p = 0x1.642c8590b2164p-4;
-    p = __builtin_fma(z, p, 0x1.8618618618618p-4);
-    p = __builtin_fma(z, p, 0x1.af286bca1af28p-4);
-    p = __builtin_fma(z, p, 0x1.e1e1e1e1e1e1ep-4);
-    p = __builtin_fma(z, p, 0x1.1111111111111p-3);
-    p = __builtin_fma(z, p, 0x1.3b13b13b13b14p-3);
-    p = __builtin_fma(z, p, 0x1.745d1745d1746p-3);
-    p = __builtin_fma(z, p, 0x1.c71c71c71c71cp-3);
-    p = __builtin_fma(z, p, 0x1.2492492492492p-2);
-    p = __builtin_fma(z, p, 0x1.999999999999ap-2);
-    p = __builtin_fma(z, p, 0x1.5555555555555p-1);
-    const double k = (double)e;
-    return __builtin_fma(k, P2M_LN2_HI, __builtin_fma(k, P2M_LN2_LO, __builtin_fma(s * z, p, 2.0 * s)));
-}
-
-__device__ static inline double mt_exp(double x)
-{
-    const double k = __builtin_rint(x * P2M_INVLN2);
-    double r = __builtin_fma(-k, P2M_LN2_HI, x);
-    r = __builtin_fma(-k, P2M_LN2_LO, r);
-    double p = 0x1.6124613a86d09p-33;
-    p = __builtin_fma(r, p, 0x1.1eed8eff8d898p-29);
-    p = __builtin_fma(r, p, 0x1.ae64567f544e4p-26);
-    p = __builtin_fma(r, p, 0x1.27e4fb7789f5cp-22);
-    p = __builtin_fma(r, p, 0x1.71de3a556c734p-19);
-    p = __builtin_fma(r, p, 0x1.a01a01a01a01ap-16);
-    p = __builtin_fma(r, p, 0x1.a01a01a01a01ap-13);
-    p = __builtin_fma(r, p, 0x1.6c16c16c16c17p-10);
-    p = __builtin_fma(r, p, 0x1.1111111111111p-7);
-    p = __builtin_fma(r, p, 0x1.5555555555555p-5);
-    p = __builtin_fma(r, p, 0x1.5555555555555p-3);
-    p = __builtin_fma(r, p, 0.5);
-    return __builtin_amdgcn_ldexp(1.0 + __builtin_fma(r * r, p, r), (int)k);
-}
-
 /* per (chi, M): the fit parameters and prefactors; per (chi, r): chi times
  * the sine of the angle.  One work item each. */
 __global__ void __launch_bounds__(64) k_maptable_cells(MTArgs A)
@@ -317,14 +255,14 @@ __global__ void __launch_bounds__(256) k_make_maptable(MTArgs A)
     double ysum = 0.0, rsum = 0.0;
     auto rho = [&](double lx) {
         const double l = lx + lhalf;
-        return mt_exp(__builtin_fma(c.er, mt_log(1.0 + mt_exp(c.alr * l)), -MT_GAMMA_RHO * l));
+        return f64_exp(__builtin_fma(c.er, f64_log(1.0 + f64_exp(c.alr * l)), -MT_GAMMA_RHO * l));
     };
     /* both integrands at s = (pos + t) ds with weights wy and wr */
     auto both = [&](double q, double wy, double wr) {
         const double s = q * MT_DS;
         const double s2 = __builtin_fma(s, s, b2);
-        const double lx = 0.5 * mt_log(s2), x = mt_sqrt(s2);
-        const double y = mt_exp(__builtin_fma(MT_GAMMA, lx, c.gl) - c.beta * mt_log(__builtin_fma(x, c.ixc, 1.0)));
+        const double lx = 0.5 * f64_log(s2), x = f64_sqrt(s2);
+        const double y = f64_exp(__builtin_fma(MT_GAMMA, lx, c.gl) - c.beta * f64_log(__builtin_fma(x, c.ixc, 1.0)));
         ysum = __builtin_fma(wy, y, ysum);
         rsum = __builtin_fma(wr, rho(lx), rsum);
     };
@@ -348,7 +286,7 @@ __global__ void __launch_bounds__(256) k_make_maptable(MTArgs A)
         const double *h = A.rules + 2 * MT_N * (rest - 1);
         for (int j = 0; j < MT_N; ++j) {
             const double s = ((double)edge + h[2 * j]) * MT_DS;
-            rsum = __builtin_fma(h[2 * j + 1], rho(0.5 * mt_log(__builtin_fma(s, s, b2))), rsum);
+            rsum = __builtin_fma(h[2 * j + 1], rho(0.5 * f64_log(__builtin_fma(s, s, b2))), rsum);
         }
     }
     const double yint = in ? (c.P0 * ysum) * MT_DS : 0.0;
