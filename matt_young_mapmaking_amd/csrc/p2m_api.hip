@@ -144,8 +144,10 @@ struct p2m_ctx {
     int n_cu = 0;                   /* compute units of the device */
     TileDesc *d_tile_desc = nullptr;
     RingDesc *d_ring = nullptr;     /* geometry of every ring */
-    uint32_t *d_fs_cnt = nullptr;   /* flat-sky box pixels per listed halo, and their scan */
+    uint32_t *d_fs_cnt = nullptr;   /* flat-sky pairs per tile (0 between calls), and their scan */
     unsigned long long *d_fs_off = nullptr;
+    uint2 *d_fs_pairs = nullptr;
+    unsigned long long flat_pairs = 0;      /* the decode's count of them */
     int64_t fs_cap = 0;
     int64_t n_tiles = 0;
     unsigned long long *d_tile_off = nullptr;
@@ -396,7 +398,7 @@ void p2m_destroy(p2m_ctx *c)
     dfree(c->d_rofz); dfree(c->d_zofr); dfree(c->d_inv_node2); dfree(c->d_inv_node2f); dfree(c->d_fb);
     dfree(c->d_halo); dfree(c->d_flat_idx); dfree(c->d_n_pairs); dfree(c->d_pair_off); dfree(c->d_ctr);
     dfree(c->d_band_tile); dfree(c->d_tile_off); dfree(c->d_scan_tmp); dfree(c->d_scan_tmp_fs);
-    dfree(c->d_tile_desc); dfree(c->d_ring); dfree(c->d_fs_cnt); dfree(c->d_fs_off);
+    dfree(c->d_tile_desc); dfree(c->d_ring); dfree(c->d_fs_cnt); dfree(c->d_fs_off); dfree(c->d_fs_pairs);
     dfree(c->d_cand);
     dfree(c->d_hot); dfree(c->d_pair_halo); dfree(c->d_keys); dfree(c->d_vals); dfree(c->d_sort_tmp);
     for (int i = 0; i < 10; ++i) if (c->ev[i]) (void)hipEventDestroy(c->ev[i]);
@@ -684,6 +686,7 @@ static int decode_chunk(p2m_ctx *c, const float *d_src, int64_t n, int64_t base)
     a.dpix = c->cfg.npix_fs > 0 ? a.fov / (double)c->cfg.npix_fs : 1.0;
     a.out = c->d_halo; a.cap = c->halo_cap;
     a.flat_idx = c->d_flat_idx;
+    a.flat_tiles = c->cfg.precision != P2M_PREC_PLAIN_FP64;
     a.cand = c->d_cand;
     a.n_cand = c->d_ctr + Ctr::N_CAND;
     a.n_cand0 = c->d_ctr + Ctr::N_CAND0;
@@ -696,13 +699,28 @@ static int decode_chunk(p2m_ctx *c, const float *d_src, int64_t n, int64_t base)
 
 static int autotune(p2m_ctx *c, int64_t n_halo, int64_t n_flat, unsigned long long n_pix);
 
-static int launch_flat(p2m_ctx *c, PaintArgs &pa, int64_t n_flat, hipStream_t s);
+static int launch_flat(p2m_ctx *c, int64_t n_flat, hipStream_t s);
 
 /* the main stream waits for whatever the flat-sky stream has enqueued */
 static void fs_join(p2m_ctx *c)
 {
     if (hipEventRecord(c->ev_fs, c->fs_stream) == hipSuccess) (void)hipStreamWaitEvent(c->stream, c->ev_fs, 0);
     (void)hipGetLastError();
+}
+
+/* the painters' table arguments */
+static void table_args(const p2m_ctx *c, TileArgs &t)
+{
+    t.n_maps = c->cfg.n_maps; t.profile = c->cfg.profile;
+    t.g = c->g; t.n_flat = c->n_flat; t.inv_node2 = c->d_inv_node2;
+    t.u_k1 = c->u_k1; t.u_k0 = c->u_k0; t.u_max = c->u_max; t.band = c->u_band; t.fr_clamp = c->fr_clamp; t.ir_clamp = c->ir_clamp;
+    t.band_c = (float)CHORD_BAND;
+    t.inv_node2f = c->d_inv_node2f;
+    t.inv_drt = 1.0 / c->g.drt; t.u_max64 = (double)(c->g.nrt - 1); t.fr_clamp64 = c->fr_clamp64;
+    /* ln r is off by a few 1e-12 at most for discs above 1e-4 rad */
+    t.band64 = std::max(1e-7, 1e-11 * t.inv_drt);
+    t.n_quad = c->n_quad; t.tab_q = c->d_quad;
+    for (int m = 0; m < c->cfg.n_maps; ++m) t.tab_flat[m] = c->d_flat[m];
 }
 
 /* n_pix: the pixels of the painted discs, about */
@@ -714,7 +732,6 @@ static int paint_halos(p2m_ctx *c, int64_t n_halo, int64_t n_flat, unsigned long
     PaintArgs pa;
     memset(&pa, 0, sizeof(pa));
     pa.halos = c->d_halo; pa.n_halo = n_halo; pa.nside = c->cfg.nside; pa.npix_fs = c->cfg.npix_fs;
-    pa.flat_idx = c->d_flat_idx; pa.n_flat_dev = c->d_ctr + Ctr::N_FLAT; pa.n_flat_host = n_flat;
     pa.n_maps = c->cfg.n_maps; pa.profile = c->cfg.profile;
     pa.fov = ((c->cfg.fov_deg / 360.0) * 2.0) * c->mypi;
     pa.dpix = c->cfg.npix_fs > 0 ? pa.fov / (double)c->cfg.npix_fs : 1.0;
@@ -735,7 +752,7 @@ static int paint_halos(p2m_ctx *c, int64_t n_halo, int64_t n_flat, unsigned long
         if (c->cfg.nside > 0) p2m_launch_paint_plain_hp(pa, c->stream);
         HIPCHK(hipGetLastError());
         HIPCHK(hipEventRecord(c->ev[3], c->stream));
-        if (c->cfg.npix_fs > 0) p2m_launch_paint_fs(pa, 1, c->stream);
+        if (c->cfg.npix_fs > 0) p2m_launch_paint_fs(pa, c->stream);
         HIPCHK(hipGetLastError());
         HIPCHK(hipEventRecord(c->ev[4], c->stream));
         HIPCHK(hipEventRecord(c->ev[5], c->stream));
@@ -747,7 +764,7 @@ static int paint_halos(p2m_ctx *c, int64_t n_halo, int64_t n_flat, unsigned long
          * its own stream beside the binning and the tile painter */
         HIPCHK(hipEventRecord(c->ev_dec, c->stream));
         HIPCHK(hipStreamWaitEvent(c->fs_stream, c->ev_dec, 0));
-        { int rc = launch_flat(c, pa, n_flat, c->fs_stream); if (rc) { fs_join(c); return rc; } }
+        { int rc = launch_flat(c, n_flat, c->fs_stream); if (rc) { fs_join(c); return rc; } }
         HIPCHK(hipEventRecord(c->ev_fs, c->fs_stream));
         /* every return from here on, error or not, first orders the work
          * that follows on the main stream after the flat-sky painter */
@@ -822,21 +839,14 @@ static int paint_halos(p2m_ctx *c, int64_t n_halo, int64_t n_flat, unsigned long
         memset(&t, 0, sizeof(t));
         t.halos = c->d_halo; t.hot = c->d_hot; t.shape = c->shape; t.nside = c->cfg.nside;
         t.log2w = c->log2w;
-        t.n_maps = c->cfg.n_maps; t.profile = c->cfg.profile; t.accumulate = c->hp_zero ? 0 : 1;
+        t.accumulate = c->hp_zero ? 0 : 1;
         t.n_tiles = c->n_tiles; t.desc = c->d_tile_desc; t.ring = c->d_ring; t.tile_off = c->d_tile_off;
         t.keys = keys; t.vals = vals;
-        t.g = c->g; t.n_flat = c->n_flat; t.inv_node2 = c->d_inv_node2;
-        t.u_k1 = c->u_k1; t.u_k0 = c->u_k0; t.u_max = c->u_max; t.band = c->u_band; t.fr_clamp = c->fr_clamp; t.ir_clamp = c->ir_clamp;
-        t.band_c = (float)CHORD_BAND;
-        t.inv_node2f = c->d_inv_node2f;
-        t.inv_drt = 1.0 / c->g.drt; t.u_max64 = (double)(c->g.nrt - 1); t.fr_clamp64 = c->fr_clamp64;
-        /* ln r is off by a few 1e-12 at most for discs above 1e-4 rad */
-        t.band64 = std::max(1e-7, 1e-11 * t.inv_drt);
-        t.n_quad = c->n_quad; t.tab_q = c->d_quad;
+        table_args(c, t);
         t.fb = c->d_fb; t.fb_count = pc + 6; t.fb_cap = c->fb_cap;
         t.lost = c->d_lost; t.tile_next = c->d_tile_next; t.redo = 0; t.n_halo = n_halo; t.err = c->d_ctr + Ctr::ERR; t.n_lost = c->d_ctr + Ctr::LOST;
         for (int m = 0; m < c->cfg.n_maps; ++m) {
-            t.tab_flat[m] = c->d_flat[m]; t.map64[m] = c->d_hp64[m]; t.map32[m] = c->d_hp32[m];
+            t.map64[m] = c->d_hp64[m]; t.map32[m] = c->d_hp32[m];
         }
         t.count = c->d_count; t.hash = c->d_hash; t.counters = pc;
         /* persistent grid of exactly the resident workgroups (a multiple
@@ -874,36 +884,66 @@ static int paint_halos(p2m_ctx *c, int64_t n_halo, int64_t n_flat, unsigned long
     } else {
         HIPCHK(hipEventRecord(c->ev[3], c->stream));
         HIPCHK(hipEventRecord(c->ev[4], c->stream));
-        { int rc = launch_flat(c, pa, n_flat, c->stream); if (rc) return rc; }
+        { int rc = launch_flat(c, n_flat, c->stream); if (rc) return rc; }
     }
     HIPCHK(hipEventRecord(c->ev[5], c->stream));
     c->hp_zero = false;
     return 0;
 }
 
-/* flat-sky painter over the flattened box pixels on stream s, between
- * events 8 and 9 */
-static int launch_flat(p2m_ctx *c, PaintArgs &pa, int64_t n_flat, hipStream_t s)
+/* Most pairs of the flat-sky painter's list (2 GiB): more are painted in
+ * parts of the halo list that cannot hold more. */
+#define FS_MAX_PAIRS (1LL << 28)
+
+/* flat-sky painter on stream s, between events 8 and 9 */
+static int launch_flat(p2m_ctx *c, int64_t n_flat, hipStream_t s)
 {
     HIPCHK(hipEventRecord(c->ev[8], s));
     if (c->cfg.npix_fs > 0 && n_flat > 0) {
-        if (n_flat + 1 > c->fs_cap || !c->d_fs_cnt) {
-            dfree(c->d_fs_cnt); dfree(c->d_fs_off); c->d_fs_cnt = nullptr; c->d_fs_off = nullptr; c->fs_cap = 0;
-            const int64_t cap = n_flat + 1 + 1024;
-            if (dmalloc((void **)&c->d_fs_cnt, sizeof(uint32_t) * cap)) return P2M_E_NOMEM;
+        FlatArgs f;
+        memset(&f, 0, sizeof(f));
+        f.halos = c->d_halo; f.npix = c->cfg.npix_fs;
+        f.fov = ((c->cfg.fov_deg / 360.0) * 2.0) * c->mypi;
+        f.dpix = f.fov / (double)c->cfg.npix_fs;
+        f.n_tiles = p2m_flat_tiles(f.npix, &f.nj);
+        for (int m = 0; m < c->cfg.n_maps; ++m) f.map[m] = c->d_fs64[m];
+        f.count = c->d_fs_count; f.hash = c->d_fs_hash; f.counters = c->d_ctr + Ctr::PAINT;
+        TileArgs t;
+        memset(&t, 0, sizeof(t));
+        table_args(c, t);
+        int64_t most = FS_MAX_PAIRS, part = n_flat, pairs = (int64_t)c->flat_pairs;
+        if (const char *e = getenv("P2M_FS_PAIRS")) { if (atoll(e) > 0) most = atoll(e); }
+        if (pairs > most) { part = std::max<int64_t>(1, most / f.n_tiles); pairs = part * f.n_tiles; }
+        f.slices = p2m_flat_slices(f.n_tiles, pairs);
+        const int64_t n_lists = f.n_tiles * f.slices;
+        if (!c->d_fs_cnt) {
+            const int64_t cap = f.n_tiles * p2m_flat_slices(f.n_tiles, INT64_MAX) + 1;
+            dfree(c->d_fs_off); c->d_fs_off = nullptr;
             if (dmalloc((void **)&c->d_fs_off, sizeof(unsigned long long) * cap)) return P2M_E_NOMEM;
+            if (dmalloc((void **)&c->d_fs_cnt, sizeof(uint32_t) * cap)) return P2M_E_NOMEM;
+            p2m_launch_fill_u32(c->d_fs_cnt, cap, 0u, s);
+        }
+        if (pairs > c->fs_cap || !c->d_fs_pairs) {
+            dfree(c->d_fs_pairs); c->d_fs_pairs = nullptr; c->fs_cap = 0;
+            const int64_t cap = pairs + pairs / 8 + 1024;
+            if (dmalloc((void **)&c->d_fs_pairs, sizeof(uint2) * cap)) return P2M_E_NOMEM;
             c->fs_cap = cap;
         }
-        pa.fs_cnt = c->d_fs_cnt; pa.fs_off = c->d_fs_off;
-        p2m_launch_fs_counts(pa, s);
-        {
-            /* its own scan storage when beside the binning */
-            const bool own = s != c->stream;
-            int rc = scan_counts_on(c->d_fs_cnt, c->d_fs_off, n_flat + 1, own ? &c->d_scan_tmp_fs : &c->d_scan_tmp,
-                                    own ? &c->scan_tmp_fs_bytes : &c->scan_tmp_bytes, s);
-            if (rc) return rc;
+        f.cnt = c->d_fs_cnt; f.off = c->d_fs_off; f.pairs = c->d_fs_pairs; f.pair_cap = (unsigned long long)c->fs_cap;
+        for (int64_t i = 0; i < n_flat; i += part) {
+            f.list = c->d_flat_idx + i; f.n_list = std::min(part, n_flat - i);
+            f.first = i == 0;
+            p2m_launch_flat_pairs(f, 0, s);
+            {
+                /* its own scan storage when beside the binning */
+                const bool own = s != c->stream;
+                int rc = scan_counts_on(c->d_fs_cnt, c->d_fs_off, n_lists + 1, own ? &c->d_scan_tmp_fs : &c->d_scan_tmp,
+                                        own ? &c->scan_tmp_fs_bytes : &c->scan_tmp_bytes, s);
+                if (rc) { p2m_launch_fill_u32(c->d_fs_cnt, n_lists + 1, 0u, s); return rc; }
+            }
+            p2m_launch_flat_pairs(f, 1, s);
+            if (p2m_launch_flat_paint(t, f, s)) return P2M_E_INVALID;
         }
-        p2m_launch_fs_paint(pa, s);
     }
     HIPCHK(hipGetLastError());
     HIPCHK(hipEventRecord(c->ev[9], s));
@@ -1136,6 +1176,7 @@ static int pass_finish(p2m_ctx *c, bool allow_tune)
     int64_t n_halo = (int64_t)std::min<unsigned long long>(hc[Ctr::N_CAND], (unsigned long long)c->halo_cap);
     int64_t n_flat = (int64_t)std::min<unsigned long long>(hc[Ctr::N_FLAT], (unsigned long long)c->halo_cap);
     c->counted_pairs = hc[Ctr::PAIRS];
+    c->flat_pairs = hc[Ctr::PAINT + 2];
     c->ask_gaps = hc[Ctr::GAPS] != 0;
     rc = paint_halos(c, n_halo, n_flat, hc[Ctr::PIX], allow_tune);
     if (rc) {

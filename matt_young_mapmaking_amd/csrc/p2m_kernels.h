@@ -37,18 +37,14 @@ struct DecodeArgs {
     PairHalo *pair_halo;         /* the binning's records (tiled painters, or NULL) */
     uint32_t *n_pairs;           /* tiles each of them reaches, at shape */
     TileShape shape;
+    int32_t flat_tiles;          /* count the flat-sky painter's pairs */
     unsigned long long *counters;/* sharded: [0] passed radial cut, [2] radius errors, [3] (halo, tile) pairs,
-                                    [10] halos that may have a ring gap, [14] pixels of the discs, about */
+                                    [9] the flat-sky painter's, [10] halos that may have a ring gap, [14] pixels of the discs, about */
 };
 
 struct PaintArgs {
     const HaloRec *halos;
     int64_t n_halo;
-    const uint32_t *flat_idx;     /* flat-sky halo list (tiled painters) */
-    const unsigned long long *n_flat_dev;
-    int64_t n_flat_host;          /* its length, known on the host */
-    uint32_t *fs_cnt;             /* box pixels per listed halo (n_flat_host + 1) */
-    unsigned long long *fs_off;   /* their exclusive scan */
     int32_t nside, npix_fs, n_maps, profile;
     double fov, dpix;
     TabGeom g;
@@ -136,6 +132,26 @@ struct TileArgs {
     unsigned long long *n_lost;   /* sharded: tiles marked lost */
 };
 
+/* the flat-sky painter's (halo, tile) pairs and maps; its tables are TileArgs' */
+struct FlatArgs {
+    const HaloRec *halos;
+    const uint32_t *list;         /* halos to paint */
+    int64_t n_list;
+    int32_t first;                /* the first part of a call's list: the count starts anew */
+    int32_t npix, nj;             /* the map's pixels a side, its tiles in a row of tiles */
+    int64_t n_tiles;
+    int32_t slices;               /* lists per tile: list k of tile t is k n_tiles + t */
+    double fov, dpix;
+    uint32_t *cnt;                /* pairs per list while they are listed, 0 before and after; one more 0 */
+    unsigned long long *off;      /* their exclusive scan */
+    uint2 *pairs;                 /* by list: first row << 4 | rows - 1, halo */
+    unsigned long long pair_cap;
+    double *map[P2M_MAXMAPS];
+    uint32_t *count;
+    unsigned long long *hash;
+    unsigned long long *counters; /* [2] updates */
+};
+
 struct FallbackArgs {
     const HaloRec *halos;
     const uint4 *fb;
@@ -163,9 +179,11 @@ void p2m_launch_fill_f32(float *p, int64_t n, hipStream_t s);
 void p2m_launch_clear_ctr(unsigned long long *ctr, int first, int count, hipStream_t s);
 void p2m_launch_decode(const DecodeArgs &a, hipStream_t s);
 void p2m_launch_paint_plain_hp(const PaintArgs &a, hipStream_t s);
-void p2m_launch_paint_fs(const PaintArgs &a, int plain, hipStream_t s);
-void p2m_launch_fs_counts(const PaintArgs &a, hipStream_t s);
-void p2m_launch_fs_paint(const PaintArgs &a, hipStream_t s);
+void p2m_launch_paint_fs(const PaintArgs &a, hipStream_t s);
+int64_t p2m_flat_tiles(int32_t npix, int32_t *nj);
+int p2m_flat_slices(int64_t n_tiles, int64_t n_pairs);
+void p2m_launch_flat_pairs(const FlatArgs &f, int emit, hipStream_t s);
+int p2m_launch_flat_paint(const TileArgs &a, const FlatArgs &f, hipStream_t s);
 void p2m_launch_pair_count(const BinArgs &b, hipStream_t s);
 void p2m_launch_ring_gaps(const BinArgs &b, hipStream_t s);
 void p2m_launch_pair_emit(const BinArgs &b, hipStream_t s);

@@ -21,10 +21,9 @@
  *  k_paint_plain_hp  baseline: one work item per halo, naive query_disc loop,
  *                    pix2vec_ring/angdist/interpolate_table per pixel, FP64
  *                    global atomics (haloproject.f90:55-75)
- *  k_fs_counts, k_fs_paint, k_paint_fs
- *                    flat-sky painter over the flattened (halo, box pixel)
- *                    space; one work item per halo for the baseline
- *                    (haloproject.f90:136-152)
+ *  k_fs_pairs, k_fs_paint, k_paint_fs
+ *                    flat-sky painter over (halo, tile) pairs; one work item
+ *                    per halo for the baseline (haloproject.f90:136-152)
  *  k_moments         map moments and the dP/dy histogram (pks2map.f90:321-357)
  */
 #include "p2m_kernels.h"
@@ -145,6 +144,19 @@ __device__ static inline uint32_t wave_incl_scan(uint32_t v)
     return v;
 }
 
+/* tiles of the flat-sky map (64 columns j by 16 rows k) that a halo's box meets */
+#define FS_LOG2C 6
+#define FS_LOG2R 4
+struct FlatBox {
+    int32_t j0, nj, k0, nk;
+    __device__ uint32_t n() const { return (uint32_t)nj * (uint32_t)nk; }
+};
+__device__ static inline FlatBox flat_box(const HaloRec &h)
+{
+    const int32_t j0 = (h.jmin - 1) >> FS_LOG2C, k0 = (h.kmin - 1) >> FS_LOG2R;
+    return {j0, ((h.jmax - 1) >> FS_LOG2C) - j0 + 1, k0, ((h.kmax - 1) >> FS_LOG2R) - k0 + 1};
+}
+
 /* ===================================================================== */
 /* decode                                                                 */
 /* ===================================================================== */
@@ -227,7 +239,7 @@ __global__ void __launch_bounds__(256) k_setup(DecodeArgs A)
     const CosmoDev &c = A.c;
     const TabGeom &g = A.g;
     __shared__ unsigned long long lds16[16];
-    unsigned long long tot_rad = 0, tot_pairs = 0, tot_pix = 0, tot_gaps = 0;
+    unsigned long long tot_rad = 0, tot_pairs = 0, tot_pix = 0, tot_gaps = 0, tot_flat = 0;
     const unsigned long long kbeg = *A.n_cand0, kend = *A.n_cand;
     for (unsigned long long k0 = kbeg + blockIdx.x * (unsigned long long)blockDim.x; k0 < kend;
          k0 += (unsigned long long)gridDim.x * blockDim.x) {
@@ -365,12 +377,16 @@ __global__ void __launch_bounds__(256) k_setup(DecodeArgs A)
             }
         }
         const unsigned long long fs = wave_append(A.n_flat_out, flat);
-        if (flat) A.flat_idx[fs] = (uint32_t)k;
+        if (flat) {
+            A.flat_idx[fs] = (uint32_t)k;
+            if (A.flat_tiles) tot_flat += flat_box(h).n();
+        }
     }
     block_count(&A.counters[2], tot_rad, lds16);
     block_count(&A.counters[3], tot_pairs, lds16);
     block_count(&A.counters[14], tot_pix, lds16);
     block_count(&A.counters[10], tot_gaps, lds16);
+    block_count(&A.counters[9], tot_flat, lds16);
 }
 
 /* n_cand0 <- n_cand: the first candidate slot of the next chunk */
@@ -444,128 +460,45 @@ void p2m_launch_paint_plain_hp(const PaintArgs &a, hipStream_t s)
 }
 
 /* ===================================================================== */
-/* flat-sky painter: one wave per halo, FP64, global atomics              */
+/* baseline flat-sky painter: one work item per halo, FP64, global atomics */
 /* ===================================================================== */
 
-__global__ void __launch_bounds__(256) k_paint_fs(PaintArgs A, int plain)
+__global__ void __launch_bounds__(256) k_paint_fs(PaintArgs A)
 {
     unsigned long long n_upd = 0;
-    if (plain) {
-        /* baseline: one work item per halo */
-        const int64_t hidx = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-        if (hidx < A.n_halo) {
-            const HaloRec &hr = A.halos[hidx];
-            if (hr.flat) {
-                HaloRec h = hr;
-                double hf = A.fov / 2.0;
-                for (int k = h.kmin; k <= h.kmax; ++k) {
-                    double phip = -hf + ((double)k - 0.5) * A.dpix;
-                    for (int j = h.jmin; j <= h.jmax; ++j) {
-                        double thetap = -hf + ((double)j - 0.5) * A.dpix;
-                        double dphi = phip - h.ph, dth = thetap - h.th;
-                        double angle = p2m_sqrt(dphi * dphi + dth * dth);
-                        if (angle < h.dtheta) {
-                            int64_t pix = (int64_t)(j - 1) + (int64_t)A.npix_fs * (k - 1);
-                            n_upd++;
-                            for (int m = 0; m < A.n_maps; ++m)
-                                atomicAdd(&A.fs64[m][pix], h.vh * interp_exact(h, A.g, A.tab_flat[m], A.n_flat, A.profile, angle));
-                            if (A.fs_count) {
-                                atomicAdd(&A.fs_count[pix], 1u);
-                                atomicAdd(&A.fs_hash[pix], (unsigned long long)halo_hash(h.cat));
-                            }
+    const int64_t hidx = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
+    if (hidx < A.n_halo) {
+        const HaloRec &hr = A.halos[hidx];
+        if (hr.flat) {
+            HaloRec h = hr;
+            double hf = A.fov / 2.0;
+            for (int k = h.kmin; k <= h.kmax; ++k) {
+                double phip = -hf + ((double)k - 0.5) * A.dpix;
+                for (int j = h.jmin; j <= h.jmax; ++j) {
+                    double thetap = -hf + ((double)j - 0.5) * A.dpix;
+                    double dphi = phip - h.ph, dth = thetap - h.th;
+                    double angle = p2m_sqrt(dphi * dphi + dth * dth);
+                    if (angle < h.dtheta) {
+                        int64_t pix = (int64_t)(j - 1) + (int64_t)A.npix_fs * (k - 1);
+                        n_upd++;
+                        for (int m = 0; m < A.n_maps; ++m)
+                            atomicAdd(&A.fs64[m][pix], h.vh * interp_exact(h, A.g, A.tab_flat[m], A.n_flat, A.profile, angle));
+                        if (A.fs_count) {
+                            atomicAdd(&A.fs_count[pix], 1u);
+                            atomicAdd(&A.fs_hash[pix], (unsigned long long)halo_hash(h.cat));
                         }
                     }
                 }
-            }
-        }
-        wave_count(&A.counters[2], n_upd);
-        return;
-    }
-}
-
-/* box pixels of each listed flat-sky halo (haloproject.f90:124-135) */
-__global__ void __launch_bounds__(256) k_fs_counts(PaintArgs A)
-{
-    for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i <= A.n_flat_host; i += (int64_t)gridDim.x * blockDim.x) {
-        uint32_t n = 0;
-        if (i < A.n_flat_host) {
-            const HaloRec &h = A.halos[A.flat_idx[i]];
-            n = (uint32_t)((h.jmax - h.jmin + 1) * (h.kmax - h.kmin + 1));
-        }
-        A.fs_cnt[i] = n;
-    }
-}
-
-/* Flat-sky painter over the flattened (halo, box pixel) space: every wave
- * takes 64 consecutive box pixels, so a few large boxes do not serialise
- * on one wave.  FP64 angle and value (haloproject.f90:130-150), global
- * FP64 atomics into the map. */
-__global__ void __launch_bounds__(256) k_fs_paint(PaintArgs A)
-{
-    const int lane = __lane_id();
-    const int64_t nfl = A.n_flat_host;
-    const unsigned long long total = A.fs_off[nfl];
-    const unsigned long long ngroup = (total + 63) >> 6;
-    const unsigned long long nw = ((unsigned long long)gridDim.x * blockDim.x) >> 6;
-    const double hf = A.fov / 2.0;
-    unsigned long long n_upd = 0;
-    for (unsigned long long g = (blockIdx.x * (unsigned long long)blockDim.x + threadIdx.x) >> 6; g < ngroup; g += nw) {
-        const unsigned long long c = g << 6;
-        int64_t lo = 0, hi = nfl - 1;           /* halo holding pixel c (wave-uniform) */
-        while (lo < hi) {
-            const int64_t mid = (lo + hi + 1) >> 1;
-            if (A.fs_off[mid] <= c) lo = mid; else hi = mid - 1;
-        }
-        const unsigned long long item = c + lane;
-        const int64_t hl = lo + lane;
-        const unsigned long long my_off = hl <= nfl ? A.fs_off[hl] : ~0ULL;
-        int jj = 0;
-        for (int step = 32; step > 0; step >>= 1) {
-            const unsigned long long o = __shfl(my_off, jj + step);
-            if (o <= item) jj += step;
-        }
-        const unsigned long long hoff = __shfl(my_off, jj);
-        if (item >= total) continue;
-        const HaloRec &h = A.halos[A.flat_idx[lo + jj]];
-        const int nj = h.jmax - h.jmin + 1;
-        const int q = (int)(item - hoff);
-        const int k = h.kmin + q / nj, j = h.jmin + q % nj;
-        const double phip = -hf + ((double)k - 0.5) * A.dpix;
-        const double thetap = -hf + ((double)j - 0.5) * A.dpix;
-        const double dphi = phip - h.ph, dth = thetap - h.th;
-        const double angle = p2m_sqrt(dphi * dphi + dth * dth);
-        if (angle < h.dtheta) {
-            const int64_t pix = (int64_t)(j - 1) + (int64_t)A.npix_fs * (k - 1);
-            n_upd++;
-            for (int m = 0; m < A.n_maps; ++m)
-                atomicAdd(&A.fs64[m][pix], h.vh * interp_exact(h, A.g, A.tab_flat[m], A.n_flat, A.profile, angle));
-            if (A.fs_count) {
-                atomicAdd(&A.fs_count[pix], 1u);
-                atomicAdd(&A.fs_hash[pix], (unsigned long long)halo_hash(h.cat));
             }
         }
     }
     wave_count(&A.counters[2], n_upd);
 }
 
-void p2m_launch_paint_fs(const PaintArgs &a, int plain, hipStream_t s)
+void p2m_launch_paint_fs(const PaintArgs &a, hipStream_t s)
 {
     if (a.n_halo <= 0 || a.npix_fs <= 0) return;
-    if (plain) hipLaunchKernelGGL(k_paint_fs, dim3((unsigned)((a.n_halo + 255) / 256)), dim3(256), 0, s, a, 1);
-}
-
-void p2m_launch_fs_counts(const PaintArgs &a, hipStream_t s)
-{
-    if (a.n_flat_host <= 0 || a.npix_fs <= 0) return;
-    int64_t g = (a.n_flat_host + 1 + 255) / 256;
-    if (g > 8192) g = 8192;
-    hipLaunchKernelGGL(k_fs_counts, dim3((unsigned)g), dim3(256), 0, s, a);
-}
-
-void p2m_launch_fs_paint(const PaintArgs &a, hipStream_t s)
-{
-    if (a.n_flat_host <= 0 || a.npix_fs <= 0) return;
-    hipLaunchKernelGGL(k_fs_paint, dim3(2048), dim3(256), 0, s, a);
+    hipLaunchKernelGGL(k_paint_fs, dim3((unsigned)((a.n_halo + 255) / 256)), dim3(256), 0, s, a);
 }
 
 /* ===================================================================== */
@@ -1017,6 +950,32 @@ __device__ static inline void load_floats(__amdgpu_buffer_rsrc_t r, int vo, int 
     for (; k < NF; ++k) f[k] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(r, vo + 4 * k, so, 0));
 }
 
+/* The value of a pixel at cell coordinate u (ub: u kept within the table) of
+ * segment s's halo, for every map: the cell and fraction of interpolate_table
+ * (r < rmint clamped, r > rmaxt 0), a lerp of the two radial columns. */
+template <int NM, typename Wave, typename F>
+__device__ static inline void quad_value(const TileArgs &A, __amdgpu_buffer_rsrc_t tab, const Wave &w, int s, double u,
+                                         double ub, F add)
+{
+    const bool clampr = u < 0.0;                  /* r < rmint: r = rmint + 1e-5 */
+    const int cl = min((int)ub, A.g.nrt - 2), cell = clampr ? A.ir_clamp - 1 : cl;
+    const double fr = clampr ? A.fr_clamp64 : (u - (double)cl) * A.g.drt;
+    const double gr = 1.0 - fr;
+    float tq[8 * NM];
+    load_floats<8 * NM>(tab, (w.colbase[s] + cell) * (16 * NM), 0, tq);
+    const double w00 = w.w00[s], w10 = w.w10[s], w01 = w.w01[s], w11 = w.w11[s];
+    const bool zero = u > A.u_max64;               /* r > rmaxt */
+#pragma unroll
+    for (int m = 0; m < NM; ++m) {
+        const float *c0v = tq + 4 * m, *c1v = tq + 4 * (NM + m);
+        double v0m = w00 * (double)c0v[0], v1m = w00 * (double)c1v[0];
+        v0m = __builtin_fma(w10, (double)c0v[1], v0m); v1m = __builtin_fma(w10, (double)c1v[1], v1m);
+        v0m = __builtin_fma(w01, (double)c0v[2], v0m); v1m = __builtin_fma(w01, (double)c1v[2], v1m);
+        v0m = __builtin_fma(w11, (double)c0v[3], v0m); v1m = __builtin_fma(w11, (double)c1v[3], v1m);
+        add(m, zero ? 0.0 : __builtin_fma(fr, v1m, gr * v0m));
+    }
+}
+
 /* per-thread statistics of a painter */
 struct PaintStats {
     unsigned long long listed, upd, segs, err;
@@ -1154,25 +1113,7 @@ __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(NM == 
                     const bool plain = cand & far & (q < edge * (1.0 - 2.0 * EDGE_BAND)) & (q > 1e-60) &
                                        (__builtin_fabs(u - __builtin_rint(ub)) > A.band64);
                     bool taken = plain;
-                    if (plain) {
-                        const bool clampr = u < 0.0;                  /* r < rmint: r = rmint + 1e-5 */
-                        const int cl = min((int)ub, A.g.nrt - 2), cell = clampr ? A.ir_clamp - 1 : cl;
-                        const double fr = clampr ? A.fr_clamp64 : (u - (double)cl) * A.g.drt;
-                        const double gr = 1.0 - fr;
-                        float tq[8 * NM];
-                        load_floats<8 * NM>(tab, (ew->colbase[s] + cell) * (16 * NM), 0, tq);
-                        const double w00 = ew->w00[s], w10 = ew->w10[s], w01 = ew->w01[s], w11 = ew->w11[s];
-                        const bool zero = u > A.u_max64;               /* r > rmaxt */
-#pragma unroll
-                        for (int m = 0; m < NM; ++m) {
-                            const float *c0v = tq + 4 * m, *c1v = tq + 4 * (NM + m);
-                            double v0m = w00 * (double)c0v[0], v1m = w00 * (double)c1v[0];
-                            v0m = __builtin_fma(w10, (double)c0v[1], v0m); v1m = __builtin_fma(w10, (double)c1v[1], v1m);
-                            v0m = __builtin_fma(w01, (double)c0v[2], v0m); v1m = __builtin_fma(w01, (double)c1v[2], v1m);
-                            v0m = __builtin_fma(w11, (double)c0v[3], v0m); v1m = __builtin_fma(w11, (double)c1v[3], v1m);
-                            atomicAdd(&acc[m * W + o], zero ? 0.0 : __builtin_fma(fr, v1m, gr * v0m));
-                        }
-                    }
+                    if (plain) quad_value<NM>(A, tab, *ew, s, u, ub, [&](int m, double v) { atomicAdd(&acc[m * W + o], v); });
                     if (__ballot(cand & !plain)) {
                         if (cand & !plain) {
                             /* the reference's arithmetic */
@@ -1227,6 +1168,242 @@ __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(NM == 
     block_count(&A.counters[1], st.upd, red);
     block_count(&A.counters[4], st.segs, red);
     block_count(A.err, st.err, red);
+}
+
+/* --------------------------------------------------------------------- */
+/* flat-sky painter                                                        */
+/*                                                                         */
+/* (halo, tile) pairs of the boxes (haloproject.f90:101-135), grouped by     */
+/* tile of 64 columns by 16 rows with a counting sort: k_fs_pairs counts     */
+/* them per tile, the counts are scanned, k_fs_pairs lists them.  A workgroup */
+/* takes a tile (or a slice of its pairs, where the map has few), its waves work as  */
+/* those of the FP64 tiled painter do, on rows of the discs instead of ring    */
+/* runs: theta^2 is formed with the reference's operations and gives the same  */
+/* bits, the value follows from its logarithm, the reference's own arithmetic  */
+/* (haloproject.f90:136-150) is carried out within rounding of the disc edge    */
+/* and of a cell boundary and for wide discs.  Pixels are summed in LDS.         */
+/*                                                                         */
+/* Bound: FP64 VALU.  Before, a wave took 64 box pixels (35% of them outside   */
+/* their disc), each with a search for its halo, the reference's arithmetic     */
+/* and an atomic into the map: 6e4 halos on 4096 x 4096 pixels (2.7e8 updates)   */
+/* 8.2 ms, of which the values 3.5 ms and the atomics 1.5 ms; 1.17 ms now, pairs  */
+/* included.  2e4 halos on 1024 x 1024 0.23 -> 0.083 ms.  Five waves a SIMD or    */
+/* four, 1024 to 4096 workgroups where a map has few tiles: the same time.        */
+/* --------------------------------------------------------------------- */
+
+/* Counts (EMIT false) or lists the pairs of the listed halos, `per` halos a
+ * wave, the lanes over the flattened (halo, tile) pairs so that a box of
+ * many tiles is shared out.  The listing takes the counts down again to 0,
+ * as they are found by the next call. */
+template <bool EMIT>
+__global__ void __launch_bounds__(256) k_fs_pairs(FlatArgs F, int per)
+{
+    const int lane = __lane_id();
+    if (!EMIT && F.first && blockIdx.x == 0)
+        for (int i = threadIdx.x; i < P2M_SHARDS; i += blockDim.x) F.counters[i * P2M_CTR_STRIDE + 2] = 0ULL;
+    const int64_t w = (blockIdx.x * (int64_t)blockDim.x + threadIdx.x) >> 6, first = w * per;
+    if (first >= F.n_list) return;
+    const int64_t at = first + lane;
+    const bool has = lane < per && at < F.n_list;
+    const uint32_t slot = F.list[has ? at : first];
+    const HaloRec &h = F.halos[slot];
+    const FlatBox b = flat_box(h);
+    const uint32_t n = has ? b.n() : 0u;
+    const uint32_t incl = wave_incl_scan(n), excl = incl - n;
+    const uint32_t total = (uint32_t)__builtin_amdgcn_readlane((int)incl, 63);
+    const int32_t kmin = h.kmin - 1, kmax = h.kmax - 1;
+    for (uint32_t base = 0; base < total; base += 64) {
+        const uint32_t item = base + (uint32_t)lane;
+        int o = 0;                          /* the last lane whose pairs start at or before item */
+        for (int step = 32; step > 0; step >>= 1)
+            if (__shfl(excl, o + step) <= item) o += step;
+        const uint32_t q = item - __shfl(excl, o);
+        const int32_t nj = __shfl(b.nj, o), j0 = __shfl(b.j0, o), k0 = __shfl(b.k0, o);
+        const int32_t klo = __shfl(kmin, o), khi = __shfl(kmax, o);
+        const uint32_t sl = __shfl(slot, o);
+        if (item < total) {
+            const int32_t dk = (int32_t)(q / (uint32_t)nj), tk = k0 + dk, tj = j0 + (int32_t)(q - (uint32_t)dk * (uint32_t)nj);
+            /* the slice: another for every wave */
+            const int64_t t = (int64_t)tk * F.nj + tj + F.n_tiles * (int64_t)((uint32_t)w % (uint32_t)F.slices);
+            if constexpr (EMIT) {
+                const int32_t r0 = max(klo - (tk << FS_LOG2R), 0), r1 = min(khi - (tk << FS_LOG2R), (1 << FS_LOG2R) - 1);
+                const unsigned long long pos = F.off[t] + (atomicSub(&F.cnt[t], 1u) - 1u);
+                if (pos < F.pair_cap) F.pairs[pos] = make_uint2((uint32_t)(r0 << 4 | (r1 - r0)), sl);
+            } else {
+                atomicAdd(&F.cnt[t], 1u);
+            }
+        }
+    }
+}
+
+/* the per-segment values, one set per wave */
+struct FlatWave {
+    unsigned long long bits[WPIX / 64];   /* segment starts */
+    double th[WSEG], dphi2[WSEG];
+    double edge[WSEG];             /* dtheta^2 (1 + EDGE_BAND) */
+    double l0[WSEG];               /* (ln chi - ln rmin) / drt */
+    double w00[WSEG], w10[WSEG], w01[WSEG], w11[WSEG];     /* corner weights times the velocity factor */
+    int32_t qoff[WSEG];            /* in-tile pixel minus the wave's pixel number */
+    int32_t colbase[WSEG];
+    uint32_t slot[WSEG];           /* halo; SLOW: every pixel takes the reference's arithmetic */
+};
+
+template <int NM>
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NM == 1 ? 5 : 3))) k_fs_paint(TileArgs A, FlatArgs F)
+{
+    extern __shared__ unsigned char smem_raw[];
+    const int W = 1 << (FS_LOG2C + FS_LOG2R);
+    __shared__ unsigned long long lds16[16];
+    double *acc = (double *)smem_raw;                       /* NM * W */
+    const int tid = threadIdx.x, lane = __lane_id(), wv = __builtin_amdgcn_readfirstlane(tid >> 6), nwv = (int)(blockDim.x >> 6);
+    FlatWave *fw = (FlatWave *)(acc + NM * W) + wv;
+    const int32_t t = (int32_t)(blockIdx.x % (unsigned)F.n_tiles), tk = t / F.nj, tj = t - tk * F.nj;
+    const uint64_t sbeg = F.off[blockIdx.x];
+    const uint32_t cnt = (uint32_t)(F.off[blockIdx.x + 1] - sbeg);
+    if (cnt == 0) return;
+    for (int p = tid; p < NM * W; p += blockDim.x) acc[p] = 0.0;
+    __syncthreads();
+    const __amdgpu_buffer_rsrc_t tab =
+        __builtin_amdgcn_make_buffer_rsrc((void *)A.tab_q, (short)0, (int)(A.n_quad * 4), 0x00020000);
+    const int32_t j1 = (tj << FS_LOG2C) + 1, k1 = (tk << FS_LOG2R) + 1;       /* the tile's first column and row */
+    const double hf = F.fov / 2.0, inv_dpix = 1.0 / F.dpix;
+    unsigned long long upd = 0;
+    uint64_t pos = sbeg + wave_share(cnt, wv, nwv);
+    const uint64_t end = sbeg + wave_share(cnt, wv + 1, nwv);
+    while (pos < end) {
+        const bool has = pos + (uint64_t)lane < end;
+        const uint2 pr = F.pairs[has ? pos + (uint64_t)lane : end - 1];
+        Seg g;
+        pos += (uint64_t)wave_segments(pr.x, pr.y, has, g);
+        const uint32_t slot = g.act ? g.val : 0u;
+        const HaloRec &h = F.halos[slot];
+        const int32_t k = k1 + (g.act ? g.row : 0);
+        /* the row's columns that may lie in the disc, a hundredth of a
+         * pixel wider than it */
+        const double phip = -hf + ((double)k - 0.5) * F.dpix, dphi = phip - h.ph, d2 = dphi * dphi;
+        const double r2 = h.dtheta * h.dtheta, rem = r2 - d2;
+        const double half = f64_sqrt(__builtin_fmax(rem, 1e-300)) * inv_dpix * (1.0 + 1e-9) + 0.01;
+        const double jc = (h.th + hf) * inv_dpix + 0.5;
+        const int32_t lo = (int32_t)__builtin_fmax(__builtin_ceil(jc - half), (double)max(h.jmin, j1));
+        const int32_t hi = (int32_t)__builtin_fmin(__builtin_floor(jc + half), (double)min(h.jmax, j1 + (1 << FS_LOG2C) - 1));
+        const int32_t len = g.act && !(rem < -1e-12 * r2) && hi >= lo ? hi - lo + 1 : 0;
+        const uint32_t incl = wave_incl_scan((uint32_t)len), start = incl - (uint32_t)len;
+        const uint32_t P = (uint32_t)__builtin_amdgcn_readlane((int)incl, 63);
+        const unsigned long long some = __ballot(len > 0);
+        wave_lds_fence();
+        if (len > 0) {
+            const int s = (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(some >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)some, 0u));
+            const bool slow = h.chi_out || !(r2 < F64_SMALL_Q) || !(h.chi_r > 1e-30);
+            const double gm = 1.0 - h.fm, gc = 1.0 - h.fc;
+            fw->th[s] = h.th; fw->dphi2[s] = d2;
+            fw->edge[s] = r2 * (1.0 + EDGE_BAND);
+            fw->l0[s] = slow ? 0.0 : (f64_log(h.chi_r) - A.g.lr0) * A.inv_drt;
+            fw->w00[s] = h.vh * (gc * gm); fw->w10[s] = h.vh * (h.fc * gm);
+            fw->w01[s] = h.vh * (gc * h.fm); fw->w11[s] = h.vh * (h.fc * h.fm);
+            fw->qoff[s] = (g.row << FS_LOG2C) + (lo - j1) - (int32_t)start;
+            fw->colbase[s] = A.g.nrt * ((h.imh - 1) + A.g.nmht * (h.ichi - 1));
+            fw->slot[s] = slot | (slow ? SLOW : 0u);
+        }
+        /* at most WSEG segments of a row each: all in one window of start bits */
+        const unsigned long long sb = start_bits(fw->bits, 0u, start, len > 0);
+        uint32_t before = 0;
+        for (uint32_t p0 = 0; p0 < P; p0 += 64) {
+            const int ch = (int)(p0 >> 6);
+            const uint32_t mlo = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)sb, ch);
+            const uint32_t mhi = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(sb >> 32), ch);
+            const int s = (int)__builtin_amdgcn_mbcnt_hi(mhi, __builtin_amdgcn_mbcnt_lo(mlo, before));
+            before += (uint32_t)(__builtin_popcount(mlo) + __builtin_popcount(mhi));
+            const uint32_t p = p0 + (uint32_t)lane;
+            const bool in = p < P;
+            const uint32_t sl = fw->slot[s];
+            const int o = in ? (int)p + fw->qoff[s] : 0;
+            const bool far = (int32_t)sl >= 0;                 /* not SLOW */
+            const double thetap = -hf + ((double)(j1 + (o & ((1 << FS_LOG2C) - 1))) - 0.5) * F.dpix;
+            const double dth = thetap - fw->th[s], edge = fw->edge[s];
+            const double q = fw->dphi2[s] + dth * dth;
+            const double u = __builtin_fma(__builtin_fma(0.5, f64_log(q), f64_lntan_angle(q)), A.inv_drt, fw->l0[s]);
+            const double ub = __builtin_fmin(__builtin_fmax(u, 0.0), A.u_max64);
+            const bool cand = in & !(far & (q > edge));
+            const bool plain = cand & far & (q < edge * (1.0 - 2.0 * EDGE_BAND)) & (q > 1e-60) &
+                               (__builtin_fabs(u - __builtin_rint(ub)) > A.band64);
+            bool taken = plain;
+            if (plain) quad_value<NM>(A, tab, *fw, s, u, ub, [&](int m, double v) { atomicAdd(&acc[m * W + o], v); });
+            if (__ballot(cand & !plain)) {
+                if (cand & !plain) {
+                    /* the reference's arithmetic */
+                    const HaloRec &hr = F.halos[sl & ~SLOW];
+                    const double angle = p2m_sqrt(q);
+                    if (angle < hr.dtheta) {
+                        taken = true;
+                        for (int m = 0; m < NM; ++m) {
+                            const __amdgpu_buffer_rsrc_t tr =
+                                __builtin_amdgcn_make_buffer_rsrc((void *)A.tab_flat[m], (short)0, (int)(A.n_flat * 4), 0x00020000);
+                            atomicAdd(&acc[m * W + o], hr.vh * interp_staged(hr.chi_out, hr.chi_r, hr.fc, hr.fm, hr.imh, hr.ichi,
+                                                                             A.g, tr, A.profile, angle));
+                        }
+                    }
+                }
+            }
+            upd += taken;
+            if (F.count && taken) {
+                const int64_t pix = (int64_t)(j1 - 1 + (o & ((1 << FS_LOG2C) - 1))) + (int64_t)F.npix * (k1 - 1 + (o >> FS_LOG2C));
+                atomicAdd(&F.count[pix], 1u);
+                atomicAdd(&F.hash[pix], (unsigned long long)halo_hash(F.halos[sl & ~SLOW].cat));
+            }
+        }
+    }
+    block_count(&F.counters[2], upd, lds16);           /* its barriers order the sums before the stores too */
+    for (int p = tid; p < W; p += blockDim.x) {
+        const int64_t j = j1 - 1 + (p & ((1 << FS_LOG2C) - 1)), k = k1 - 1 + (p >> FS_LOG2C);
+        if (j >= F.npix || k >= F.npix) continue;
+#pragma unroll
+        for (int m = 0; m < NM; ++m) {
+            const double v = acc[m * W + p];
+            if (v != 0.0) {
+                if (F.slices > 1) atomicAdd(&F.map[m][j + F.npix * k], v);
+                else F.map[m][j + F.npix * k] += v;
+            }
+        }
+    }
+}
+
+int64_t p2m_flat_tiles(int32_t npix, int32_t *nj)
+{
+    const int64_t c = ((int64_t)npix + (1 << FS_LOG2C) - 1) >> FS_LOG2C, r = ((int64_t)npix + (1 << FS_LOG2R) - 1) >> FS_LOG2R;
+    *nj = (int32_t)c;
+    return c * r;
+}
+
+/* A map of few tiles has each tile's pairs in several slices, a workgroup
+ * each: 2048 workgroups fill the GPU, of at least 8 pairs so that a tile's
+ * clearing and adding up pays (32 is up to 1.6 times slower, 4 no faster),
+ * and the slices' counters keep the listing's atomics apart (6e4 halos on
+ * 200 x 200 pixels, 52 tiles: in one list per tile 307 us, 44 us in 39). */
+int p2m_flat_slices(int64_t n_tiles, int64_t n_pairs)
+{
+    const int64_t s = std::min<int64_t>(2048 / n_tiles, n_pairs / (8 * n_tiles));
+    return (int)std::max<int64_t>(1, std::min<int64_t>(s, 64));
+}
+
+void p2m_launch_flat_pairs(const FlatArgs &f, int emit, hipStream_t s)
+{
+    /* few halos: a wave each, so that wide boxes are spread out */
+    int64_t per = f.n_list / 8192 + 1;
+    if (per > 64) per = 64;
+    const int64_t waves = (f.n_list + per - 1) / per;
+    const dim3 grid((unsigned)((waves + 3) / 4));
+    if (emit) hipLaunchKernelGGL((k_fs_pairs<true>), grid, dim3(256), 0, s, f, (int)per);
+    else hipLaunchKernelGGL((k_fs_pairs<false>), grid, dim3(256), 0, s, f, (int)per);
+}
+
+int p2m_launch_flat_paint(const TileArgs &a, const FlatArgs &f, hipStream_t s)
+{
+    const dim3 grid((unsigned)(f.n_tiles * f.slices));
+    const size_t lds = (size_t)a.n_maps * (sizeof(double) << (FS_LOG2C + FS_LOG2R)) + 4 * sizeof(FlatWave);
+#define P2M_FS(NMv) case NMv: hipLaunchKernelGGL((k_fs_paint<NMv>), grid, dim3(256), lds, s, a, f); break;
+    switch (a.n_maps) { P2M_FS(1) P2M_FS(2) P2M_FS(3) P2M_FS(4) P2M_FS(5) P2M_FS(6) default: return -1; }
+#undef P2M_FS
+    return 0;
 }
 
 /* --------------------------------------------------------------------- */
