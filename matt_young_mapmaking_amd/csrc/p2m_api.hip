@@ -251,7 +251,7 @@ static int build_tiles(p2m_ctx *c, int log2w)
     c->log2w = 0;
     int rc = 0;
     rc |= dmalloc((void **)&c->d_lost, (size_t)((acc + 3) / 4) * 4);
-    if (!c->d_tile_next) rc |= dmalloc((void **)&c->d_tile_next, sizeof(unsigned int) * 8 * P2M_TQ_STRIDE);
+    if (!c->d_tile_next) rc |= dmalloc((void **)&c->d_tile_next, sizeof(unsigned int) * P2M_TQ_MAX * P2M_TQ_STRIDE);
     rc |= dmalloc((void **)&c->d_tile_desc, sizeof(TileDesc) * acc);
     rc |= dmalloc((void **)&c->d_band_tile, sizeof(int32_t) * (size_t)(nb + 1));
     rc |= dmalloc((void **)&c->d_tile_off, sizeof(unsigned long long) * (c->n_tiles + 1));
@@ -851,14 +851,14 @@ static int paint_halos(p2m_ctx *c, int64_t n_halo, int64_t n_flat, unsigned long
         t.count = c->d_count; t.hash = c->d_hash; t.counters = pc;
         /* persistent grid of exactly the resident workgroups (a multiple
          * of 8 for the XCD-aware tile order): no partial last round */
-        int grid = (int)std::min<int64_t>(c->n_tiles, 8192);
+        int grid = (int)std::min<int64_t>(c->n_tiles, P2M_TQ_MAX);
         const int wg = p2m_tile_wg(mode, c->cfg.n_maps, c->log2w, c->d_count != nullptr, c->g.nrt, c->wg);
         {
             const size_t lds = p2m_tile_lds_bytes(mode, c->cfg.n_maps, c->log2w, c->d_count != nullptr, c->g.nrt, wg);
             const int occ = p2m_tile_occupancy(mode, c->cfg.n_maps, wg, lds);
             if (occ > 0 && c->n_cu > 0) {
                 const int64_t res = ((int64_t)occ * c->n_cu) & ~(int64_t)7;
-                if (res >= 8) grid = (int)std::min<int64_t>(c->n_tiles, res);
+                if (res >= 8) grid = (int)std::min<int64_t>(grid, res);
             }
         }
         if (p2m_launch_tile_paint(t, mode, c->cfg.n_maps, grid, wg, c->stream)) return P2M_E_INVALID;

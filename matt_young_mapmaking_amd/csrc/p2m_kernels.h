@@ -89,6 +89,7 @@ struct __attribute__((aligned(16))) TileDesc {
 };
 
 #define P2M_TQ_STRIDE 32           /* tile-queue counters one 128-byte line apart */
+#define P2M_TQ_MAX 8192            /* of them, and workgroups of a tile painter */
 
 struct TileArgs {
     const HaloRec *halos;
@@ -125,7 +126,7 @@ struct TileArgs {
     int32_t redo;                 /* paint only the tiles marked lost, clearing the mark of each
                                      that now fits */
     int64_t n_halo;               /* records in hot / halos */
-    unsigned int *tile_next;      /* the tile queues: one counter per XCD, P2M_TQ_STRIDE
+    unsigned int *tile_next;      /* the tile queues: one counter per XCD or workgroup, P2M_TQ_STRIDE
                                      apart (zeroed by p2m_launch_tile_paint) */
     unsigned long long *counters; /* [0] listed, [1] hp updates, [4] segments, [5] FP64 fallbacks */
     unsigned long long *err;      /* sharded: pairs whose halo or rows are out of bounds */
