@@ -175,6 +175,7 @@ struct p2m_ctx {
     /* the FP32 painter's last launch, kept for the repaint pass */
     TileArgs last_t;
     FallbackArgs last_f;
+    int64_t n_chunks = 0;                   /* chunks of the call decoded */
     int last_grid = 0, last_wg = 0;
     bool last_fast = false;
     uint32_t *d_cand = nullptr;
@@ -639,10 +640,10 @@ static int scan_counts(p2m_ctx *c, const uint32_t *cnt, unsigned long long *off,
 /* counter block summed over its shards (blocks until the stream is idle) */
 static int read_counters(p2m_ctx *c, unsigned long long out[Ctr::TOTAL], unsigned long long *raw = nullptr)
 {
-    unsigned long long hbuf[Ctr::ALL];
-    unsigned long long *h = raw ? raw : hbuf;
-    HIPCHK(hipMemcpyAsync(h, c->d_ctr, sizeof(hbuf), hipMemcpyDeviceToHost, c->stream));
+    unsigned long long hbuf[Ctr::ALL], *h = c->h_pin ? c->h_pin : hbuf;
+    HIPCHK(hipMemcpyAsync(h, c->d_ctr, sizeof(*h) * Ctr::ALL, hipMemcpyDeviceToHost, c->stream));
     HIPCHK(hipStreamSynchronize(c->stream));
+    if (raw) memcpy(raw, h, sizeof(*h) * Ctr::ALL);
     for (int k = 0; k < Ctr::TOTAL; ++k) {
         out[k] = 0;
         for (int sh = 0; sh < P2M_SHARDS; ++sh) out[k] += h[sh * Ctr::TOTAL + k];
@@ -676,7 +677,7 @@ static int ensure_halo_cap(p2m_ctx *c, int64_t n)
 static int decode_chunk(p2m_ctx *c, const float *d_src, int64_t n, int64_t base)
 {
     DecodeArgs a;
-    a.halos = d_src; a.n = n; a.index_base = base;
+    a.halos = d_src; a.n = n; a.index_base = base; a.first = c->n_chunks++ == 0;
     a.c = c->cdev; a.g = c->g;
     a.cut_low = c->cut_low; a.cut_high = c->cut_high; a.chihview = c->run.chihview; a.mmin = c->run.mmin;
     a.precut = (c->run.flags & P2M_RUN_PRECUT) ? 1 : 0;
@@ -760,19 +761,7 @@ static int paint_halos(p2m_ctx *c, int64_t n_halo, int64_t n_flat, unsigned long
         return 0;
     }
     if (c->cfg.nside > 0) {
-        /* the flat-sky painter needs only the decoded records: it runs on
-         * its own stream beside the binning and the tile painter */
         HIPCHK(hipEventRecord(c->ev_dec, c->stream));
-        HIPCHK(hipStreamWaitEvent(c->fs_stream, c->ev_dec, 0));
-        { int rc = launch_flat(c, n_flat, c->fs_stream); if (rc) { fs_join(c); return rc; } }
-        HIPCHK(hipEventRecord(c->ev_fs, c->fs_stream));
-        /* every return from here on, error or not, first orders the work
-         * that follows on the main stream after the flat-sky painter */
-        struct FsJoin {
-            p2m_ctx *c;
-            bool armed;
-            ~FsJoin() { if (armed) (void)hipStreamWaitEvent(c->stream, c->ev_fs, 0); }
-        } fs_guard{c, true};
         /* (halo, tile) pairs: counted by the decode at the shape it knew,
          * listed in halo order, sorted by tile */
         BinArgs b;
@@ -879,7 +868,13 @@ static int paint_halos(p2m_ctx *c, int64_t n_halo, int64_t n_flat, unsigned long
         }
         c->last_fast = mode == P2M_PREC_FP32_COMP;
         HIPCHK(hipEventRecord(c->ev[4], c->stream));
-        fs_guard.armed = false;
+        /* the flat-sky painter needs only the decoded records: it runs on
+         * its own stream beside the binning and the tile painter.  It is the
+         * shorter chain of launches, so it is queued last: a small call's
+         * painting does not wait for the host to have queued it */
+        HIPCHK(hipStreamWaitEvent(c->fs_stream, c->ev_dec, 0));
+        { int rc = launch_flat(c, n_flat, c->fs_stream); if (rc) { fs_join(c); return rc; } }
+        HIPCHK(hipEventRecord(c->ev_fs, c->fs_stream));
         HIPCHK(hipStreamWaitEvent(c->stream, c->ev_fs, 0));
     } else {
         HIPCHK(hipEventRecord(c->ev[3], c->stream));
@@ -1086,6 +1081,7 @@ static int pass_begin(p2m_ctx *c, int64_t n_total)
     c->stream_h2d_bytes = 0;
     c->n_host_push = 0;
     c->n_pieces = 0;
+    c->n_chunks = 0;
     c->stream_pinned = true;
     return 0;
 }

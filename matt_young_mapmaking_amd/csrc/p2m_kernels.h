@@ -20,6 +20,7 @@
 struct DecodeArgs {
     const float *halos;          /* 7 float32 per halo */
     int64_t n, index_base;
+    int32_t first;               /* the call's first chunk */
     CosmoDev c;
     TabGeom g;
     double cut_low, cut_high, chihview, mmin, dmodel;

@@ -402,7 +402,7 @@ void p2m_launch_decode(const DecodeArgs &a, hipStream_t s)
     if (gc > 2048) gc = 2048;
     int64_t g = (a.n + 255) / 256;
     if (g > 8192) g = 8192;
-    hipLaunchKernelGGL(k_mark_cand, dim3(1), dim3(64), 0, s, a);
+    if (!a.first) hipLaunchKernelGGL(k_mark_cand, dim3(1), dim3(64), 0, s, a);      /* 0 and 0 before the first */
     hipLaunchKernelGGL(k_cull, dim3((unsigned)gc), dim3(256), 0, s, a);
     hipLaunchKernelGGL(k_setup, dim3((unsigned)g), dim3(256), 0, s, a);
 }
@@ -611,8 +611,39 @@ int p2m_sort_pairs(uint32_t *keys, uint32_t *vals, unsigned long long n, int64_t
 }
 
 /* exclusive scan of uint32 counts into uint64 offsets with a 64-bit accumulator */
+/* Exclusive scan of up to 16384 counts by one workgroup, consecutive ones a
+ * thread: one launch instead of two (2569 counts: 5 us instead of 6 us and the
+ * gap between them). */
+#define SCAN_SMALL 16384
+__global__ void __launch_bounds__(1024) k_scan_small(const uint32_t *__restrict__ cnt, unsigned long long *__restrict__ off, int n)
+{
+    __shared__ uint32_t sums[16];
+    const int per = (n + 1023) / 1024, i0 = (int)threadIdx.x * per, wv = (int)threadIdx.x >> 6;
+    uint32_t v[SCAN_SMALL / 1024], t = 0;
+#pragma unroll
+    for (int k = 0; k < SCAN_SMALL / 1024; ++k) {
+        v[k] = k < per && i0 + k < n ? cnt[i0 + k] : 0u;
+        t += v[k];
+    }
+    const uint32_t incl = wave_incl_scan(t);
+    if (__lane_id() == 63) sums[wv] = incl;
+    __syncthreads();
+    unsigned long long o = incl - t;
+    for (int w = 0; w < wv; ++w) o += sums[w];
+#pragma unroll
+    for (int k = 0; k < SCAN_SMALL / 1024; ++k) {
+        if (k < per && i0 + k < n) off[i0 + k] = o;
+        o += v[k];
+    }
+}
+
 int p2m_scan_u32(const uint32_t *cnt, unsigned long long *off, int64_t n, void *tmp, size_t *tmp_bytes, hipStream_t s)
 {
+    if (n <= SCAN_SMALL) {
+        if (!tmp) *tmp_bytes = 0;
+        else if (n > 0) hipLaunchKernelGGL(k_scan_small, dim3(1), dim3(1024), 0, s, cnt, off, (int)n);
+        return 0;
+    }
     hipError_t e = hipcub::DeviceScan::ExclusiveScan(tmp, *tmp_bytes, cnt, off, hipcub::Sum(), 0ULL, (int)n, s);
     return e == hipSuccess ? 0 : -1;
 }
