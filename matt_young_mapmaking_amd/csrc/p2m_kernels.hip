@@ -898,9 +898,8 @@ struct TileQueue {
 /* ------------------------------------------------------------------ */
 /* FP64 tiled painter                                                   */
 /*                                                                      */
-/* Each tile's pixel vectors are formed once, in LDS, with the            */
-/* reference's arithmetic (pix2vec_ring from the ring's z and sin(theta)   */
-/* and the pixel's phi); per pixel and halo sin^2(theta) is the squared     */
+/* A tile's pixel vectors are formed once, and kept in LDS, with the reference's arithmetic (pix2vec_ring from the    */
+/* ring's z and sin(theta) and the pixel's phi); per pixel and halo sin^2(theta) is the squared     */
 /* cross product, the same bits as the reference's, the table cell and      */
 /* fraction follow from its logarithm, the value from the corner-quad table; */
 /* it is accumulated in an FP64 LDS tile (ds_add_f64) and written to the    */
@@ -933,6 +932,11 @@ struct ExactWave {
  * rounded a few times */
 #define EDGE_BAND 1e-13
 #define SLOW 0x80000000u
+/* Pairs above which a tile's pixel vectors are all formed at its start; fewer
+ * do not reach most of its pixels, and each is formed when a disc first meets
+ * it.  Nside 2048, ms all at the start / all on demand: 7 pairs a tile 0.27 /
+ * 0.24, 11: 0.62 / 0.54, 21: 0.70 / 0.63, 35: 0.81 / 0.77, 70: 1.24 / 1.28. */
+#define MANY_PAIRS 40u
 
 /* interpolate_table (maptable.f90:176-216) on staged per-halo values, the
  * same operations in the same order as interp_exact; the table through a
@@ -1034,7 +1038,7 @@ __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(NM == 
     const size_t mem_bytes = A.count ? (size_t)W * 12 : 0;
     TileCtl *ctl = (TileCtl *)(smem_raw + ((acc_bytes + mem_bytes + 15) & ~(size_t)15));
     const int tid = threadIdx.x, lane = __lane_id(), wv = tid >> 6, nwv = (int)(blockDim.x >> 6);
-    /* x and y of the tile's pixel vectors */
+    /* x and y of the tile's pixel vectors, NaN until a wave has needed one (several may form it: the same bits) */
     double *vx = (double *)(ctl + 1), *vy = vx + W;
     ExactWave *ew = (ExactWave *)(vy + W) + wv;
     PaintStats st = {0, 0, 0, 0};
@@ -1044,6 +1048,7 @@ __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(NM == 
     if (tid == 0) ctl->next_tile[0] = queue.claim();
     for (int p = tid; p < W; p += blockDim.x) {
         for (int m = 0; m < NM; ++m) acc[m * W + p] = 0.0;
+        vx[p] = vy[p] = __builtin_nan("");
         if (A.count) { lcount[p] = 0; lhash[p] = 0ULL; }
     }
     lds_barrier();
@@ -1056,18 +1061,20 @@ __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(NM == 
         if (tid < G.rows) stage_row(ctl->rows[par][tid], rdesc[G.ring0 - 1 + tid], G.K, G.k);
         if (tid == 0) ctl->next_tile[par ^ 1] = queue.claim();
         lds_barrier();
-        if (send > sbeg) {
-            for (int p = tid; p < G.rows << log2c; p += blockDim.x) {
-                const TileRow &Q = rows[p >> log2c];
-                const double phi = (((double)((int)Q.ip0 + (p & ((1 << log2c) - 1))) + (double)Q.off) * HPX_HALFPI) / Q.den();
-                double sn, cs;
-                p2m_sincos(phi, &sn, &cs);
-                vx[p] = Q.sth * cs;
-                vy[p] = Q.sth * sn;
-            }
+        const uint32_t cnt = (uint32_t)(send - sbeg);
+        /* x and y of an in-tile pixel's vector */
+        auto vector_of = [&](int o, double &x, double &y) {
+            const TileRow &Q = rows[o >> log2c];
+            const double phi = (((double)((int)Q.ip0 + (o & ((1 << log2c) - 1))) + (double)Q.off) * HPX_HALFPI) / Q.den();
+            double sn, cs;
+            p2m_sincos(phi, &sn, &cs);
+            x = Q.sth * cs;
+            y = Q.sth * sn;
+        };
+        if (cnt > MANY_PAIRS) {
+            for (int p = tid; p < G.rows << log2c; p += blockDim.x) vector_of(p, vx[p], vy[p]);
             lds_barrier();
         }
-        const uint32_t cnt = (uint32_t)(send - sbeg);
         const int wv_u = __builtin_amdgcn_readfirstlane(wv);
         uint64_t pos = sbeg + wave_share(cnt, wv_u, nwv);
         const uint64_t end = sbeg + wave_share(cnt, wv_u + 1, nwv);
@@ -1140,7 +1147,15 @@ __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(NM == 
                     const int row = (int)(hole >> 24), o = in ? (int)p + ew->qoff[s] : 0;
                     const bool far = (int32_t)sl >= 0;                 /* not SLOW */
                     /* the cross product of angdist */
-                    const double ax = ew->hx[s], ay = ew->hy[s], az = ew->hz[s], bx = vx[o], by = vy[o], bz = rows[row].zr;
+                    const double ax = ew->hx[s], ay = ew->hy[s], az = ew->hz[s], bz = rows[row].zr;
+                    double bx = vx[o], by = vy[o];
+                    if (__ballot(in & ((bx != bx) | (by != by)))) {
+                        if (in & ((bx != bx) | (by != by))) {
+                            vector_of(o, bx, by);
+                            vx[o] = bx;
+                            vy[o] = by;
+                        }
+                    }
                     const double v0 = ay * bz - az * by, v1 = az * bx - ax * bz, v2 = ax * by - ay * bx;
                     const double q = (v0 * v0 + v1 * v1) + v2 * v2, edge = ew->edge[s];
                     const double u = __builtin_fma(__builtin_fma(0.5, f64_log(q), f64_lntan_sin2(q)), A.inv_drt, ew->l0[s]);
@@ -1195,6 +1210,7 @@ __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(NM == 
                     }
                 }
                 for (int m = 0; m < NM; ++m) acc[m * W + p] = 0.0;
+                vx[p] = vy[p] = __builtin_nan("");
                 if (A.count) { lcount[p] = 0; lhash[p] = 0ULL; }
             }
         };
