@@ -116,8 +116,22 @@ P2M_HD void p2m_sincos(double x, double *s, double *c)
     }
 }
 
-P2M_HD double p2m_sin(double x) { double s, c; p2m_sincos(x, &s, &c); return s; }
-P2M_HD double p2m_cos(double x) { double s, c; p2m_sincos(x, &s, &c); return c; }
+/* one of the two only: a wave whose lanes need the same polynomial skips the other */
+P2M_HD double p2m_sin(double x)
+{
+    double r;
+    const int q = p2m_rem_pio2(x, &r);
+    const double v = (q & 1) ? p2m_cos_poly(r) : p2m_sin_poly(r);
+    return (q & 2) ? -v : v;
+}
+
+P2M_HD double p2m_cos(double x)
+{
+    double r;
+    const int q = p2m_rem_pio2(x, &r);
+    const double v = (q & 1) ? p2m_sin_poly(r) : p2m_cos_poly(r);
+    return ((q + 1) & 2) ? -v : v;
+}
 
 P2M_HD double p2m_tan(double x)
 {
@@ -162,20 +176,16 @@ P2M_HD double p2m_atan01(double t)
 P2M_HD double p2m_atan2(double y, double x)
 {
     if (x != x || y != y) return x + y;
-    double ax = p2m_fabs(x), ay = p2m_fabs(y);
-    int ysign = (int)(p2m_dbits(y) >> 63);
-    double a;
-    if (ay == 0.0) {
-        a = (p2m_dbits(x) >> 63) ? P2M_PI_HI : 0.0;
-    } else if (ax == 0.0) {
-        a = P2M_PIO2_HI;
-    } else if (ay <= ax) {
-        a = p2m_atan01(ay / ax);
-        if (x < 0.0) a = (P2M_PI_HI - a) + P2M_PI_LO;
-    } else {
-        a = (P2M_PIO2_HI - p2m_atan01(ax / ay)) + P2M_PIO2_LO;
-        if (x < 0.0) a = (P2M_PI_HI - a) + P2M_PI_LO;
-    }
+    /* one quotient and one arc tangent for either octant, and selects: the
+     * lanes of a wave stay together (the quotient of a zero is exact, its arc
+     * tangent 0 or pi/2 to the bit; 0 / 0 is put right by the last select) */
+    const double ax = p2m_fabs(x), ay = p2m_fabs(y);
+    const int ysign = (int)(p2m_dbits(y) >> 63), xsign = (int)(p2m_dbits(x) >> 63);
+    const int low = ay <= ax;
+    const double at = p2m_atan01((low ? ay : ax) / (ay == 0.0 ? 1.0 : (low ? ax : ay)));
+    double a = low ? at : (P2M_PIO2_HI - at) + P2M_PIO2_LO;
+    a = x < 0.0 ? (P2M_PI_HI - a) + P2M_PI_LO : a;
+    a = ay == 0.0 ? (xsign ? P2M_PI_HI : 0.0) : a;
     return ysign ? -a : a;
 }
 
