@@ -35,7 +35,7 @@ extern "C" {
 #define P2M_E_STATE      -6   /* call out of order (no cosmology / table loaded) */
 #define P2M_E_IO         -7   /* file could not be written */
 #define P2M_E_NODEVICE   -8   /* no GPU visible */
-#define P2M_E_INTERNAL   -9   /* a device-side consistency check failed (segment or tile out of range);
+#define P2M_E_INTERNAL   -9   /* a device-side consistency check failed (pair or tile out of range);
                                  the maps of that call are not valid */
 
 /* precision / algorithm of the painter */
@@ -79,12 +79,12 @@ typedef struct {
     int64_t n_in, n_cut, n_painted;
     int64_t n_listed_hp, n_upd_hp, n_upd_fs;
     int64_t n_fallback;     /* FP32 path pixels recomputed in FP64 near cell/edge boundaries */
-    int64_t n_segments;     /* (halo, ring, tile) work items */
+    int64_t n_segments;     /* (halo, ring, tile) runs with pixels */
     int64_t n_ring_gaps;    /* empty rings between non-empty rings (quirk Q15); expect 0 */
     int64_t n_radius_err;   /* halos with disc radius outside [0, pi] (skipped) */
     double  cut_low, cut_high;
-    /* device time of the last p2m_paint* call: total, decode, binning (spatial
-     * sort to segment lists), healpix painting, flat-sky painting (the tiled
+    /* device time of the last p2m_paint* call: total, decode, binning (the list
+     * of (halo, tile) pairs, sorted by tile), healpix painting, flat-sky painting (the tiled
      * modes run it on a second stream beside the binning) */
     double  ms_total, ms_decode, ms_bin, ms_paint, ms_finish;
     int32_t tile_w, tile_wg;  /* tile shape used (autotuned or set) */
@@ -160,9 +160,10 @@ int p2m_fetch_membership(p2m_ctx *ctx, uint32_t *hp_count, uint64_t *hp_hash,
                          uint32_t *fs_count, uint64_t *fs_hash);
 int p2m_get_stats(p2m_ctx *ctx, p2m_stats *st);
 
-/* Tile shape of the tiled painter: width in pixels along a ring (power of 2,
- * 64..2048) and workgroup size (a multiple of 64, 64..512; 64..256 for
- * P2M_PREC_FP32_COMP).
+/* Tile shape of the tiled painter: pixels of a tile (power of 2, 64..2048: up
+ * to 16 rings by a sector of azimuth) and workgroup size (a multiple of 64,
+ * 64..512; 64..256 for P2M_PREC_FP32_COMP).  Where the waves' own storage does
+ * not fit LDS beside a wide tile of many maps, fewer waves are launched.
  * 0,0 (and a context that never calls this) = the library picks the shape on
  * the next paint call: with at least 2e5 halos past the cuts and cleared maps
  * it times each candidate shape on those halos (painting, then clearing the

@@ -528,9 +528,9 @@ void p2m_launch_paint_fs(const PaintArgs &a, hipStream_t s)
  * Before, the (halo, ring) runs of every disc were cut at ring tiles,
  * counted per tile through an LDS hash and scattered: 13 items a halo, two
  * passes bound by load latency and LDS atomics.  Binning time, scans and sort
- * included: 2e7 halos at nside 4096, 2.2e6 painted, 1.35 -> 0.39 ms; 2e7
- * heavy halos at nside 2048, 1.7e7 painted, 6.0 -> 1.4 ms; 4e7 at nside 4096
- * 17.9 -> 3.5 ms. */
+ * included: 2e7 halos at nside 4096, 2.2e6 painted, 1.35 -> 0.33 ms; 2e7
+ * heavy halos at nside 2048, 1.7e7 painted, 6.0 -> 1.0 ms; 4e7 at nside 4096
+ * 17.9 -> 2.75 ms. */
 /* the fields of a record that the exact disc query reads */
 struct DiscRec { double cosang, zz0, a, phi0; };
 __device__ static inline DiscRec disc_rec(const HaloRec &h) { return {h.cosang, h.zz0, h.a, h.phi0}; }
@@ -922,7 +922,7 @@ struct TileQueue {
 /* Bound: FP64 VALU.  Carrying that out for every pixel took five times     */
 /* the operations (a sine, a cosine, an arc tangent, a tangent and a        */
 /* logarithm with their quotients, eight table loads): 2e6 halos at nside  */
-/* 2048 1.85 ms, 1.22 ms now.  (The chord relation of the FP32 painter needs */
+/* 2048 1.85 ms, 1.25 ms now.  (The chord relation of the FP32 painter needs */
 /* no vectors and was as fast, but its rounding is another than the cross   */
 /* product's: 1e-16 of the chord, 1.3e-12 of a value near a halo's centre.)  */
 /* ------------------------------------------------------------------ */
@@ -1494,7 +1494,7 @@ int p2m_launch_flat_paint(const TileArgs &a, const FlatArgs &f, hipStream_t s)
 /* Bound: VALU issue (80% busy at six waves a SIMD).  A pixel takes about   */
 /* 90 instructions, a batch of 64 segments about 250 before them (the       */
 /* runs, which the binning no longer computes).  2e7 halos at nside 4096:   */
-/* 1.25 ms -> 1.44 ms for 1.35 -> 0.39 ms of binning; 2e7 heavy halos at    */
+/* 1.25 ms -> 1.45 ms for 1.35 -> 0.33 ms of binning; 2e7 heavy halos at    */
 /* nside 2048 3.1 -> 2.5 ms; 4e7 at nside 4096 14.7 -> 12.9 ms.  Rows by    */
 /* columns of a tile: 8 x 128 instead of 16 x 64 takes 0.1 ms off the first  */
 /* and adds as much to its binning, and is 2% slower on the last two.       */
