@@ -628,16 +628,21 @@ int p2m_sort_pairs(uint32_t *keys, uint32_t *vals, unsigned long long n, int64_t
 #define SCAN_SMALL 16384
 __global__ void __launch_bounds__(1024) k_scan_small(const uint32_t *__restrict__ cnt, unsigned long long *__restrict__ off, int n)
 {
-    __shared__ uint32_t sums[16];
-    const int per = (n + 1023) / 1024, i0 = (int)threadIdx.x * per, wv = (int)threadIdx.x >> 6;
-    uint32_t v[SCAN_SMALL / 1024], t = 0;
+    __shared__ unsigned long long sums[16];
+    const int per = (n + 1023) / 1024, i0 = (int)threadIdx.x * per, wv = (int)threadIdx.x >> 6, lane = __lane_id();
+    uint32_t v[SCAN_SMALL / 1024];
+    unsigned long long t = 0;
 #pragma unroll
     for (int k = 0; k < SCAN_SMALL / 1024; ++k) {
         v[k] = k < per && i0 + k < n ? cnt[i0 + k] : 0u;
         t += v[k];
     }
-    const uint32_t incl = wave_incl_scan(t);
-    if (__lane_id() == 63) sums[wv] = incl;
+    unsigned long long incl = t;
+    for (int step = 1; step < 64; step <<= 1) {
+        const unsigned long long u = __shfl_up(incl, step);
+        if (lane >= step) incl += u;
+    }
+    if (lane == 63) sums[wv] = incl;
     __syncthreads();
     unsigned long long o = incl - t;
     for (int w = 0; w < wv; ++w) o += sums[w];
