@@ -130,7 +130,7 @@ struct p2m_ctx {
     TileHalo *d_hot = nullptr;                    /* what the FP32 painter stages of it */
     uint32_t *d_n_pairs = nullptr;                /* tiles per halo, and their scan */
     unsigned long long *d_pair_off = nullptr;
-    uint32_t *d_keys = nullptr, *d_vals = nullptr;  /* (halo, tile) pairs: as listed, then sorted by tile */
+    uint32_t *d_keys = nullptr, *d_vals = nullptr;  /* (halo, tile) pairs: as listed, then sorted by tile (one allocation) */
     int64_t pair_cap = 0;
     int counted_log2w = 0;                        /* the tile shape that n_pairs were counted at, and their sum */
     unsigned long long counted_pairs = 0;
@@ -171,6 +171,8 @@ struct p2m_ctx {
      * (the tile then wrote nothing and is painted again) */
     uint8_t *d_lost = nullptr;
     unsigned int *d_tile_next = nullptr;   /* tile-queue counters */
+    unsigned char *d_split = nullptr;      /* slices of split tiles: count, units, states, parts */
+    size_t split_bytes = 0;
     int n_redo = 0;
     /* the FP32 painter's last launch, kept for the repaint pass */
     TileArgs last_t;
@@ -383,7 +385,7 @@ void p2m_destroy(p2m_ctx *c)
     if (c->stream) (void)hipStreamSynchronize(c->stream);
     if (c->fs_stream) (void)hipStreamSynchronize(c->fs_stream);
     if (c->h2d_stream) (void)hipStreamSynchronize(c->h2d_stream);
-    dfree(c->d_slot[0]); dfree(c->d_slot[1]); dfree(c->d_lost); dfree(c->d_tile_next);
+    dfree(c->d_slot[0]); dfree(c->d_slot[1]); dfree(c->d_lost); dfree(c->d_tile_next); dfree(c->d_split);
     for (int i = 0; i < 2; ++i) {
         if (c->ev_copy[i]) (void)hipEventDestroy(c->ev_copy[i]);
         if (c->ev_free[i]) (void)hipEventDestroy(c->ev_free[i]);
@@ -401,7 +403,7 @@ void p2m_destroy(p2m_ctx *c)
     dfree(c->d_band_tile); dfree(c->d_tile_off); dfree(c->d_scan_tmp); dfree(c->d_scan_tmp_fs);
     dfree(c->d_tile_desc); dfree(c->d_ring); dfree(c->d_fs_cnt); dfree(c->d_fs_off); dfree(c->d_fs_pairs);
     dfree(c->d_cand);
-    dfree(c->d_hot); dfree(c->d_pair_halo); dfree(c->d_keys); dfree(c->d_vals); dfree(c->d_sort_tmp);
+    dfree(c->d_hot); dfree(c->d_pair_halo); dfree(c->d_keys); dfree(c->d_sort_tmp);
     for (int i = 0; i < 10; ++i) if (c->ev[i]) (void)hipEventDestroy(c->ev[i]);
     if (c->h_pin) (void)hipHostFree(c->h_pin);
     if (c->h_prod) (void)hipHostFree(c->h_prod);
@@ -724,6 +726,42 @@ static void table_args(const p2m_ctx *c, TileArgs &t)
     for (int m = 0; m < c->cfg.n_maps; ++m) t.tab_flat[m] = c->d_flat[m];
 }
 
+/* Splitting of tiles with many pairs (k_tile_bounds) for a launch of `grid`
+ * workgroups, and its storage.  A tile is split above the mean of the
+ * workgroups, but not below twice the mean tile (an even sky is never split)
+ * nor below 1024 pairs, about 10 us of a workgroup; a call of up to 4096 pairs
+ * is not worth the second launch.  At most n_pairs / above tiles have more
+ * than `above` pairs, at most `grid`, and their slices are fewer than twice as
+ * many.  Without memory for it no tile is split.  (1e6 halos of a 10-degree
+ * field, tile kernel: split above 512 / 1024 / 2048 pairs nside 512 0.19 / 0.12 /
+ * 0.11 ms, nside 4096 0.98 / 0.99 / 1.03; 1e5 of a 1-degree field at nside 4096
+ * 0.54 / 0.56 / 0.68.  Half or twice the mean of the workgroups: 4096 1.14, 1.11.) */
+static SplitArgs split_args(p2m_ctx *c, unsigned long long n_pairs, int grid, size_t part_bytes)
+{
+    SplitArgs s;
+    memset(&s, 0, sizeof(s));
+    const unsigned long long above = std::max<unsigned long long>(
+        1024, std::max<unsigned long long>((n_pairs + grid - 1) / grid, 2 * n_pairs / c->n_tiles));
+    if (n_pairs <= 4096 || n_pairs <= above) return s;
+    const size_t o_units = 256, o_state = o_units + sizeof(SplitUnit) * 2 * P2M_TQ_MAX,
+                 o_part = o_state + sizeof(SplitState) * P2M_TQ_MAX;
+    const size_t parts = (size_t)(n_pairs / above), bytes = o_part + parts * part_bytes;
+    if (bytes > c->split_bytes) {
+        dfree(c->d_split); c->d_split = nullptr; c->split_bytes = 0;
+        const size_t cap = (bytes + bytes / 8 + 255) & ~(size_t)255;
+        if (dmalloc((void **)&c->d_split, cap)) return s;
+        c->split_bytes = cap;
+        p2m_launch_fill_u32((uint32_t *)c->d_split, (int64_t)(cap / 4), 0u, c->stream);
+    }
+    s.above = (uint32_t)above;
+    s.unit_cap = 2 * P2M_TQ_MAX; s.part_cap = (uint32_t)parts;
+    s.n = (uint32_t *)c->d_split;
+    s.units = (SplitUnit *)(c->d_split + o_units);
+    s.state = (SplitState *)(c->d_split + o_state);
+    s.part = c->d_split + o_part;
+    return s;
+}
+
 /* n_pix: the pixels of the painted discs, about */
 static int paint_halos(p2m_ctx *c, int64_t n_halo, int64_t n_flat, unsigned long long n_pix, bool allow_tune)
 {
@@ -779,14 +817,29 @@ static int paint_halos(p2m_ctx *c, int64_t n_halo, int64_t n_flat, unsigned long
         }
         c->counted_log2w = c->log2w;
         const unsigned long long n_pairs = c->counted_pairs;
-        if ((int64_t)n_pairs > c->pair_cap || !c->d_keys || !c->d_vals) {
-            dfree(c->d_keys); dfree(c->d_vals); c->d_keys = nullptr; c->d_vals = nullptr; c->pair_cap = 0;
-            const int64_t cap = (int64_t)(n_pairs * 1.125) + 1024;
-            if (dmalloc((void **)&c->d_keys, sizeof(uint32_t) * 2 * cap)) return P2M_E_NOMEM;
-            if (dmalloc((void **)&c->d_vals, sizeof(uint32_t) * 2 * cap)) return P2M_E_NOMEM;
+        if ((int64_t)n_pairs > c->pair_cap || !c->d_keys) {
+            dfree(c->d_keys); c->d_keys = nullptr; c->d_vals = nullptr; c->pair_cap = 0;
+            const int64_t cap = ((int64_t)(n_pairs * 1.125) + 1024 + 63) & ~(int64_t)63;
+            if (dmalloc((void **)&c->d_keys, sizeof(uint32_t) * 4 * cap)) return P2M_E_NOMEM;
+            c->d_vals = c->d_keys + 2 * cap;
             c->pair_cap = cap;
         }
         b.keys = c->d_keys; b.vals = c->d_vals; b.pair_cap = n_pairs;
+        /* persistent grid of exactly the resident workgroups (a multiple
+         * of 8 for the XCD-aware tile order): no partial last round */
+        int grid = (int)std::min<int64_t>(c->n_tiles, P2M_TQ_MAX);
+        const int wg = p2m_tile_wg(mode, c->cfg.n_maps, c->log2w, c->d_count != nullptr, c->g.nrt, c->wg);
+        {
+            const size_t lds = p2m_tile_lds_bytes(mode, c->cfg.n_maps, c->log2w, c->d_count != nullptr, c->g.nrt, wg);
+            const int occ = p2m_tile_occupancy(mode, c->cfg.n_maps, wg, lds);
+            if (occ > 0 && c->n_cu > 0) {
+                const int64_t res = ((int64_t)occ * c->n_cu) & ~(int64_t)7;
+                if (res >= 8) grid = (int)std::min<int64_t>(grid, res);
+            }
+        }
+        const SplitArgs split = split_args(c, n_pairs, grid, (size_t)c->cfg.n_maps * ((size_t)8 << c->log2w) +
+                                                             (c->d_count ? (size_t)12 << c->log2w : 0));
+        b.n_split = split.n;
         if (n_pairs > 0) {
             if (c->ask_gaps) {
                 /* in the place of the decode's count of such halos */
@@ -805,7 +858,7 @@ static int paint_halos(p2m_ctx *c, int64_t n_halo, int64_t n_flat, unsigned long
             if (p2m_sort_pairs(c->d_keys, c->d_vals, n_pairs, c->n_tiles, c->d_sort_tmp, &bytes, c->stream)) return P2M_E_HIP;
         }
         const uint32_t *keys = c->d_keys + n_pairs, *vals = c->d_vals + n_pairs;     /* sorted */
-        p2m_launch_tile_bounds(keys, n_pairs, c->n_tiles, c->d_tile_off, c->stream);
+        p2m_launch_tile_bounds(keys, n_pairs, c->n_tiles, c->d_tile_off, split, c->d_ctr + Ctr::ERR, c->stream);
         HIPCHK(hipGetLastError());
         if (mode == P2M_PREC_FP32_COMP) {
             /* deferred FP64 pixels: ~5e-4 of the listed pixels in practice;
@@ -833,23 +886,11 @@ static int paint_halos(p2m_ctx *c, int64_t n_halo, int64_t n_flat, unsigned long
         t.keys = keys; t.vals = vals;
         table_args(c, t);
         t.fb = c->d_fb; t.fb_count = pc + 6; t.fb_cap = c->fb_cap;
-        t.lost = c->d_lost; t.tile_next = c->d_tile_next; t.redo = 0; t.n_halo = n_halo; t.err = c->d_ctr + Ctr::ERR; t.n_lost = c->d_ctr + Ctr::LOST;
+        t.lost = c->d_lost; t.tile_next = c->d_tile_next; t.split = split; t.redo = 0; t.n_halo = n_halo; t.err = c->d_ctr + Ctr::ERR; t.n_lost = c->d_ctr + Ctr::LOST;
         for (int m = 0; m < c->cfg.n_maps; ++m) {
             t.map64[m] = c->d_hp64[m]; t.map32[m] = c->d_hp32[m];
         }
         t.count = c->d_count; t.hash = c->d_hash; t.counters = pc;
-        /* persistent grid of exactly the resident workgroups (a multiple
-         * of 8 for the XCD-aware tile order): no partial last round */
-        int grid = (int)std::min<int64_t>(c->n_tiles, P2M_TQ_MAX);
-        const int wg = p2m_tile_wg(mode, c->cfg.n_maps, c->log2w, c->d_count != nullptr, c->g.nrt, c->wg);
-        {
-            const size_t lds = p2m_tile_lds_bytes(mode, c->cfg.n_maps, c->log2w, c->d_count != nullptr, c->g.nrt, wg);
-            const int occ = p2m_tile_occupancy(mode, c->cfg.n_maps, wg, lds);
-            if (occ > 0 && c->n_cu > 0) {
-                const int64_t res = ((int64_t)occ * c->n_cu) & ~(int64_t)7;
-                if (res >= 8) grid = (int)std::min<int64_t>(grid, res);
-            }
-        }
         if (p2m_launch_tile_paint(t, mode, c->cfg.n_maps, grid, wg, c->stream)) return P2M_E_INVALID;
         HIPCHK(hipGetLastError());
         HIPCHK(hipEventRecord(c->ev[7], c->stream));

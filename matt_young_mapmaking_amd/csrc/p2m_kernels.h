@@ -70,6 +70,7 @@ struct BinArgs {
     uint32_t *keys, *vals;        /* the pairs, see k_pair_count */
     unsigned long long pair_cap;
     const HaloRec *recs;          /* the full records */
+    uint32_t *n_split;            /* SplitArgs::n, cleared here */
     unsigned long long *counters; /* [3] ring gaps */
 };
 
@@ -91,6 +92,27 @@ struct __attribute__((aligned(16))) TileDesc {
 
 #define P2M_TQ_STRIDE 32           /* tile-queue counters one 128-byte line apart */
 #define P2M_TQ_MAX 8192            /* of them, and workgroups of a tile painter */
+
+/* Tiles of more than split_above pairs are painted in slices by several
+ * workgroups, see k_tile_bounds: each slice adds its pixels to the tile's
+ * part, the one that is done last writes the tile.  Parts and states are 0
+ * between calls. */
+struct __attribute__((aligned(16))) SplitUnit {
+    uint32_t tile, part, from, cnt;        /* its pairs, counted from the tile's first */
+    uint32_t slices, pad[3];
+};
+struct __attribute__((aligned(64))) SplitState {
+    uint32_t arrived, lost;        /* slices done; one of them lost deferred pixels */
+    unsigned long long stat[4];    /* the FP32 painter's counts: listed, updates, segments, deferrals */
+};
+struct SplitArgs {
+    uint32_t above;                /* pairs of a tile above which it is split; 0: never */
+    uint32_t unit_cap, part_cap;
+    uint32_t *n;                   /* [0] units, [1] split tiles (0 before k_tile_bounds) */
+    SplitUnit *units;
+    SplitState *state;             /* per split tile */
+    unsigned char *part;           /* per split tile, as the LDS tile: n_maps W doubles, then the membership hashes and counts */
+};
 
 struct TileArgs {
     const HaloRec *halos;
@@ -129,6 +151,7 @@ struct TileArgs {
     int64_t n_halo;               /* records in hot / halos */
     unsigned int *tile_next;      /* the tile queues: one counter per XCD or workgroup, P2M_TQ_STRIDE
                                      apart (zeroed by p2m_launch_tile_paint) */
+    SplitArgs split;
     unsigned long long *counters; /* [0] listed, [1] hp updates, [4] segments, [5] FP64 fallbacks */
     unsigned long long *err;      /* sharded: pairs whose halo or rows are out of bounds */
     unsigned long long *n_lost;   /* sharded: tiles marked lost */
@@ -190,7 +213,7 @@ void p2m_launch_pair_count(const BinArgs &b, hipStream_t s);
 void p2m_launch_ring_gaps(const BinArgs &b, hipStream_t s);
 void p2m_launch_pair_emit(const BinArgs &b, hipStream_t s);
 void p2m_launch_tile_bounds(const uint32_t *keys, unsigned long long n, int64_t n_tiles, unsigned long long *tile_off,
-                            hipStream_t s);
+                            const SplitArgs &split, unsigned long long *err, hipStream_t s);
 int p2m_sort_pairs(uint32_t *keys, uint32_t *vals, unsigned long long n, int64_t n_tiles, void *tmp, size_t *tmp_bytes,
                    hipStream_t s);
 void p2m_launch_ring_desc(int32_t nside, RingDesc *out, hipStream_t s);

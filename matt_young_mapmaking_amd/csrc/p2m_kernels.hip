@@ -560,6 +560,7 @@ __global__ void __launch_bounds__(256) k_pair_count(BinArgs B)
 
 __global__ void __launch_bounds__(256) k_pair_emit(BinArgs B)
 {
+    if (B.n_split && blockIdx.x == 0 && threadIdx.x < 2) B.n_split[threadIdx.x] = 0u;
     for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < B.n_halo; i += (int64_t)gridDim.x * blockDim.x) {
         const PairHalo h = B.halos[i];
         unsigned long long o = B.pair_off[i];
@@ -574,17 +575,41 @@ __global__ void __launch_bounds__(256) k_pair_emit(BinArgs B)
 }
 
 /* tile_off[t] = the first sorted pair of tile t or a later one, by binary
- * search (empty stretches of the sky leave long runs of equal offsets) */
+ * search (empty stretches of the sky leave long runs of equal offsets).
+ *
+ * A tile of more than S.above pairs is listed for painting in slices: a
+ * catalogue of a small field has all its pairs in a few tiles, and a
+ * workgroup for each leaves the rest of the GPU idle.  Tile kernel, unsplit
+ * and split: 1e6 halos of a 10 x 10 degree field, nside 512 0.97 -> 0.12 ms
+ * (FP64 3.29 -> 0.19), nside 1024 1.56 -> 0.20 (FP64 2.76 -> 0.34), nside 4096 2.08 ->
+ * 0.99 (FP64 4.79 -> 2.53); 1e5 of a 1 x 1 degree field at nside 4096 2.41 -> 0.56. */
+__device__ static inline unsigned long long first_of_tile(const uint32_t *__restrict__ keys, unsigned long long lo,
+                                                          unsigned long long hi, int64_t t)
+{
+    while (lo < hi) {
+        const unsigned long long mid = (lo + hi) >> 1;
+        if ((int64_t)(keys[mid] >> 8) < t) lo = mid + 1; else hi = mid;
+    }
+    return lo;
+}
+
 __global__ void __launch_bounds__(256) k_tile_bounds(const uint32_t *__restrict__ keys, unsigned long long n, int64_t n_tiles,
-                                                     unsigned long long *tile_off)
+                                                     unsigned long long *tile_off, SplitArgs S, unsigned long long *err)
 {
     for (int64_t t = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; t <= n_tiles; t += (int64_t)gridDim.x * blockDim.x) {
-        unsigned long long lo = 0, hi = n;
-        while (lo < hi) {
-            const unsigned long long mid = (lo + hi) >> 1;
-            if ((int64_t)(keys[mid] >> 8) < t) lo = mid + 1; else hi = mid;
-        }
+        const unsigned long long lo = first_of_tile(keys, 0, n, t);
         tile_off[t] = lo;
+        if (S.above && t < n_tiles && lo + S.above < n && (int64_t)(keys[lo + S.above] >> 8) == t) {
+            const uint32_t cnt = (uint32_t)(first_of_tile(keys, lo, n, t + 1) - lo), slices = (cnt - 1) / S.above + 1;
+            const uint32_t at = atomicAdd(&S.n[0], slices), part = atomicAdd(&S.n[1], 1u);
+            const uint32_t per = cnt / slices, more = cnt - per * slices;
+            /* both fit by the choice of `above` */
+            if ((uint64_t)at + slices <= S.unit_cap && part < S.part_cap)
+                for (uint32_t k = 0; k < slices; ++k)
+                    S.units[at + k] = {(uint32_t)t, part, k * per + (k < more ? k : more), per + (k < more ? 1u : 0u), slices, {0, 0, 0}};
+            else
+                atomicAdd(err, 1ULL);
+        }
     }
 }
 
@@ -601,9 +626,10 @@ void p2m_launch_pair_emit(const BinArgs &b, hipStream_t s)
 {
     if (b.n_halo > 0) hipLaunchKernelGGL(k_pair_emit, dim3(bin_grid(b.n_halo)), dim3(256), 0, s, b);
 }
-void p2m_launch_tile_bounds(const uint32_t *keys, unsigned long long n, int64_t n_tiles, unsigned long long *tile_off, hipStream_t s)
+void p2m_launch_tile_bounds(const uint32_t *keys, unsigned long long n, int64_t n_tiles, unsigned long long *tile_off,
+                            const SplitArgs &split, unsigned long long *err, hipStream_t s)
 {
-    hipLaunchKernelGGL(k_tile_bounds, dim3(bin_grid(n_tiles + 1)), dim3(256), 0, s, keys, n, n_tiles, tile_off);
+    hipLaunchKernelGGL(k_tile_bounds, dim3(bin_grid(n_tiles + 1)), dim3(256), 0, s, keys, n, n_tiles, tile_off, split, err);
 }
 
 /* stable radix sort of the pairs by their tile: keys and vals hold 2n
@@ -768,6 +794,8 @@ struct TileCtl {
     uint32_t lost[2];              /* a deferred pixel of the tile found the list full */
     int32_t next_tile[2];          /* the tile this workgroup paints next */
     unsigned long long fb_base;    /* list slot of the tile's deferred pixels */
+    uint32_t last;                 /* a slice's end: SLICE_LAST, SLICE_LOST */
+    uint32_t stat[4];              /* its counts */
     uint4 fb[FB_LDS];
 };
 
@@ -893,6 +921,7 @@ __device__ static inline uint32_t wave_share(uint32_t n, int w, int nw)
  * others.  Where there is a workgroup for every tile, each has a queue of its
  * own that holds one: claims from shared ones, by all workgroups at once, took
  * 30 us of the launch (3000 halos at nside 64: 48 -> 18 us). */
+#define NO_UNIT 0x7fffffff         /* past the end of every queue */
 struct TileQueue {
     unsigned int *ctr;
     int64_t xb, xe;
@@ -908,8 +937,112 @@ struct TileQueue {
         }
         ctr = A.tile_next + (all ? (int)blockIdx.x : xcd) * P2M_TQ_STRIDE;
     }
+    __device__ int32_t first() const { return claim(); }
     __device__ int32_t claim() const { return (int32_t)(xb + (int64_t)atomicAdd(ctr, 1u)); }
 };
+
+/* The slices of split tiles, in eighths likewise; a workgroup's first is its
+ * own number, so that not all of them claim at once. */
+struct SliceQueue {
+    unsigned int *ctr;
+    int64_t xb, xe;
+    int32_t own, wgs;
+    __device__ SliceQueue(const TileArgs &A)
+    {
+        const uint32_t n_units = *A.split.n, n = n_units < A.split.unit_cap ? n_units : A.split.unit_cap;
+        const bool xq = (gridDim.x % 8) == 0;
+        const int xcd = xq ? (int)(blockIdx.x % 8) : 0, queues = xq ? 8 : 1;
+        xb = (int64_t)xcd * n / queues;
+        xe = (int64_t)(xcd + 1) * n / queues;
+        own = (int32_t)(blockIdx.x / queues);
+        wgs = (int32_t)(gridDim.x / queues);
+        ctr = A.tile_next + xcd * P2M_TQ_STRIDE + P2M_TQ_STRIDE / 2;
+    }
+    __device__ int32_t first() const { return (int32_t)xb + own; }
+    __device__ int32_t claim() const { return (int32_t)xb + wgs + (int32_t)atomicAdd(ctr, 1u); }
+};
+
+/* Number u of a queue: tile u, or slice u of the split tiles.  Its tile and
+ * pairs, the same in every lane. */
+struct PaintUnit {
+    int64_t t;
+    uint64_t sbeg;
+    uint32_t cnt;
+};
+template <bool SLICES>
+__device__ static inline PaintUnit paint_unit(const TileArgs &A, const unsigned long long *__restrict__ toff, int64_t u)
+{
+    if constexpr (SLICES) {
+        const SplitUnit &s = A.split.units[u];
+        const int64_t t = (int64_t)__builtin_amdgcn_readfirstlane((int)s.tile);
+        return {t, toff[t] + (uint32_t)__builtin_amdgcn_readfirstlane((int)s.from), (uint32_t)__builtin_amdgcn_readfirstlane((int)s.cnt)};
+    }
+    const uint64_t b = toff[u];
+    return {u, b, (uint32_t)(toff[u + 1] - b)};
+}
+
+/* The end of a slice, by every thread of the workgroup after the barrier
+ * that follows its painting: the LDS tile is added to the tile's part, and
+ * the workgroup that is the last of them takes the sums back into its LDS tile
+ * (its own pixels, as it will write and clear them) and leaves the part 0.
+ * Returns SLICE_LAST if the caller is it, SLICE_LOST if any slice was lost.
+ * The additions are device-scope atomics; the fences order them before the
+ * arrival, and the last one's reads after it.  No workgroup waits for
+ * another. */
+#define SLICE_LAST 1u
+#define SLICE_LOST 2u
+template <int NM>
+__device__ static inline uint32_t join_slice(const TileArgs &A, TileCtl *ctl, int64_t unit, int npx, bool lost,
+                                             double *acc, unsigned long long *lhash, uint32_t *lcount)
+{
+    const int W = 1 << A.log2w;
+    const SplitUnit su = A.split.units[unit];
+    unsigned char *base = A.split.part + (size_t)su.part * ((size_t)NM * W * 8 + (A.count ? (size_t)W * 12 : 0));
+    double *sum = (double *)base;
+    unsigned long long *hsum = (unsigned long long *)(sum + (size_t)NM * W);
+    uint32_t *csum = (uint32_t *)(hsum + W);
+    SplitState *st = A.split.state + su.part;
+#pragma unroll 1
+    for (int p = threadIdx.x; p < npx; p += blockDim.x) {
+#pragma unroll 1
+        for (int m = 0; m < NM; ++m) {
+            const double v = acc[m * W + p];
+            if (v != 0.0) atomicAdd(&sum[m * W + p], v);
+        }
+        if (A.count && lcount[p]) {
+            atomicAdd(&csum[p], lcount[p]);
+            atomicAdd(&hsum[p], lhash[p]);
+        }
+    }
+    if (lost && threadIdx.x == 0) atomicOr(&st->lost, 1u);
+    __threadfence();
+    lds_barrier();
+    if (threadIdx.x == 0) {
+        uint32_t r = 0;
+        if (atomicAdd(&st->arrived, 1u) + 1u == su.slices) {
+            __threadfence();
+            r = SLICE_LAST | (atomicExch(&st->lost, 0u) ? SLICE_LOST : 0u);
+            (void)atomicExch(&st->arrived, 0u);
+        }
+        ctl->last = r;
+    }
+    lds_barrier();
+    const uint32_t r = ctl->last;
+    if (r & SLICE_LAST) {
+        __threadfence();
+#pragma unroll 1
+        for (int p = threadIdx.x; p < npx; p += blockDim.x) {
+#pragma unroll 1
+            for (int m = 0; m < NM; ++m)
+                acc[m * W + p] = __longlong_as_double((long long)atomicExch((unsigned long long *)&sum[m * W + p], 0ULL));
+            if (A.count) {
+                lcount[p] = atomicExch(&csum[p], 0u);
+                lhash[p] = atomicExch(&hsum[p], 0ULL);
+            }
+        }
+    }
+    return r;
+}
 
 /* ------------------------------------------------------------------ */
 /* FP64 tiled painter                                                   */
@@ -1042,10 +1175,9 @@ struct PaintStats {
     unsigned long long listed, upd, segs, err;
 };
 
-template <int NM>
-__global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(NM == 1 ? 3 : 2))) k_tile_exact(TileArgs A, const TileDesc *__restrict__ tdesc,
-                                                    const unsigned long long *__restrict__ toff,
-                                                    const RingDesc *__restrict__ rdesc)
+template <int NM, bool SLICES>
+__device__ static __forceinline__ void paint_exact(const TileArgs &A, const TileDesc *__restrict__ tdesc,
+                                                   const unsigned long long *__restrict__ toff, const RingDesc *__restrict__ rdesc)
 {
     extern __shared__ unsigned char smem_raw[];
     const int W = 1 << A.log2w, log2c = A.shape.log2c;
@@ -1064,8 +1196,8 @@ __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(NM == 
     PaintStats st = {0, 0, 0, 0};
     const __amdgpu_buffer_rsrc_t tab =
         __builtin_amdgcn_make_buffer_rsrc((void *)A.tab_q, (short)0, (int)(A.n_quad * 4), 0x00020000);
-    const TileQueue queue(A);
-    if (tid == 0) ctl->next_tile[0] = queue.claim();
+    const std::conditional_t<SLICES, SliceQueue, TileQueue> queue(A);
+    if (tid == 0) ctl->next_tile[0] = queue.first();
     for (int p = tid; p < W; p += blockDim.x) {
         for (int m = 0; m < NM; ++m) acc[m * W + p] = 0.0;
         vx[p] = vy[p] = __builtin_nan("");
@@ -1073,15 +1205,18 @@ __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(NM == 
     }
     lds_barrier();
     for (int par = 0;; par ^= 1) {
-        const int64_t t = (int64_t)__builtin_amdgcn_readfirstlane(ctl->next_tile[par]);
-        if (t >= queue.xe) break;
-        const TileDesc G = tdesc[t];
-        const uint64_t sbeg = toff[t], send = toff[t + 1];
+        const int64_t unit = (int64_t)__builtin_amdgcn_readfirstlane(ctl->next_tile[par]);
+        if (unit >= queue.xe) break;
+        const PaintUnit U = paint_unit<SLICES>(A, toff, unit);
+        const TileDesc G = tdesc[U.t];
+        const uint64_t sbeg = U.sbeg;
         const TileRow *rows = ctl->rows[par];
         if (tid < G.rows) stage_row(ctl->rows[par][tid], rdesc[G.ring0 - 1 + tid], G.K, G.k);
-        if (tid == 0) ctl->next_tile[par ^ 1] = queue.claim();
+        if (!SLICES && tid == 0) ctl->next_tile[par ^ 1] = queue.claim();
         lds_barrier();
-        const uint32_t cnt = (uint32_t)(send - sbeg);
+        /* a split tile is painted in slices: not here */
+        const bool split = !SLICES && A.split.above && U.cnt > A.split.above;
+        const uint32_t cnt = split ? 0u : U.cnt;
         /* x and y of an in-tile pixel's vector */
         auto vector_of = [&](int o, double &x, double &y) {
             const TileRow &Q = rows[o >> log2c];
@@ -1215,11 +1350,13 @@ __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(NM == 
         /* every thread writes its pixels and clears them for the next tile;
          * branch on accumulate outside the loops (no speculative map loads) */
         const int npx = G.rows << log2c;
+        bool keep = split;
+        if constexpr (SLICES) keep = !(join_slice<NM>(A, ctl, unit, npx, false, acc, lhash, lcount) & SLICE_LAST);
         auto out = [&](auto add) {
             for (int p = tid; p < npx; p += blockDim.x) {
                 const TileRow &R = rows[p >> log2c];
                 const int col = p & ((1 << log2c) - 1);
-                if (col < (int)R.width) {
+                if (col < (int)R.width && !keep) {
                     const int64_t pix = R.pix0 + col;
                     for (int m = 0; m < NM; ++m) {
                         if constexpr (decltype(add)::value) A.map64[m][pix] += acc[m * W + p];
@@ -1236,12 +1373,26 @@ __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(NM == 
             }
         };
         if (A.accumulate) out(std::true_type{}); else out(std::false_type{});
+        if constexpr (SLICES) {        /* one at a time: a slice claimed ahead is one that no idle workgroup takes */
+            lds_barrier();
+            if (tid == 0) ctl->next_tile[par ^ 1] = queue.claim();
+            lds_barrier();
+        }
     }
     unsigned long long *red = (unsigned long long *)ctl->fb;
     block_count(&A.counters[0], st.listed, red);
     block_count(&A.counters[1], st.upd, red);
     block_count(&A.counters[4], st.segs, red);
     block_count(A.err, st.err, red);
+}
+
+template <int NM>
+__global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(NM == 1 ? 3 : 2))) k_tile_exact(TileArgs A, const TileDesc *__restrict__ tdesc,
+                                                    const unsigned long long *__restrict__ toff,
+                                                    const RingDesc *__restrict__ rdesc)
+{
+    paint_exact<NM, false>(A, tdesc, toff, rdesc);
+    if (A.split.above && *A.split.n != 0u) paint_exact<NM, true>(A, tdesc, toff, rdesc);
 }
 
 /* --------------------------------------------------------------------- */
@@ -1542,10 +1693,9 @@ __device__ static inline float sin2f(float x)
     return sn * sn;
 }
 
-template <int NM>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NM == 1 ? 6 : 1))) k_tile_fast(TileArgs A, const TileDesc *__restrict__ tdesc,
-                                                   const unsigned long long *__restrict__ toff,
-                                                   const RingDesc *__restrict__ rdesc)
+template <int NM, bool SLICES>
+__device__ static __forceinline__ void paint_fast(const TileArgs &A, const TileDesc *__restrict__ tdesc,
+                                                  const unsigned long long *__restrict__ toff, const RingDesc *__restrict__ rdesc)
 {
     extern __shared__ unsigned char smem_raw[];
     const int W = 1 << A.log2w, log2c = A.shape.log2c;
@@ -1579,11 +1729,11 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NM == 
     const int64_t fbs = A.fb_cap / P2M_SHARDS;
     unsigned long long *const fbc = A.fb_count + (blockIdx.x % P2M_SHARDS) * P2M_CTR_STRIDE;
     uint4 *const fbr = A.fb + (blockIdx.x % P2M_SHARDS) * fbs;
-    const TileQueue q(A);
+    const std::conditional_t<SLICES, SliceQueue, TileQueue> q(A);
     if (tid == 0) {
         ctl->nfb[0] = ctl->nfb[1] = 0; ctl->lost[0] = ctl->lost[1] = 0;
-        ctl->next_tile[0] = q.claim();
-        ctl->next_tile[1] = q.claim();
+        ctl->next_tile[0] = q.first();
+        ctl->next_tile[1] = SLICES ? NO_UNIT : q.claim();
     }
     for (int k = tid; k < nrt + 2; k += blockDim.x) invn[k] = A.inv_node2f[k];
     for (int p = tid; p < W; p += blockDim.x) {
@@ -1600,12 +1750,15 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NM == 
      * after the second every thread writes out and clears its own pixels.  The
      * next tile's rows and words go to the other slot, whose readers of tile
      * k-1 were done at tile k's first barrier. */
-    int64_t t = (int64_t)__builtin_amdgcn_readfirstlane(ctl->next_tile[0]);
-    if (t < q.xe) {
-    TileDesc G = tdesc[t];
-    uint64_t sbeg = toff[t];
-    uint32_t cnt = (uint32_t)(toff[t + 1] - sbeg);
-    bool skip = A.redo && !A.lost[t];            /* repaint pass: only the tiles that lost pixels */
+    for (;;) {                     /* once, or slice by slice */
+    int64_t unit = (int64_t)__builtin_amdgcn_readfirstlane(ctl->next_tile[0]);
+    if (unit >= q.xe) break;
+    PaintUnit U = paint_unit<SLICES>(A, toff, unit);
+    TileDesc G = tdesc[U.t];
+    /* not painted: a split tile here, where its slices are painted, and in
+     * the repaint pass a tile that lost no pixels */
+    auto skipped = [&]() { return (!SLICES && A.split.above && U.cnt > A.split.above) || (A.redo && !A.lost[U.t]); };
+    bool skip = skipped();
     if (tid < G.rows) stage_row(ctl->rows[0][tid], rdesc[G.ring0 - 1 + tid], G.K, G.k);
     uint32_t key = 0, val = 0;
     auto load_pairs = [&](uint64_t base, uint32_t i, uint32_t e) {
@@ -1615,16 +1768,20 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NM == 
     };
     const int wv_u = __builtin_amdgcn_readfirstlane(wv);
     auto wave_from = [&](uint32_t n, int w) { return wave_share(n, w, nwv); };
-    load_pairs(sbeg, wave_from(cnt, wv_u), wave_from(cnt, wv_u + 1));
+    load_pairs(U.sbeg, wave_from(U.cnt, wv_u), wave_from(U.cnt, wv_u + 1));
     for (int par = 0;; par ^= 1) {
         lds_barrier();
         const int64_t tn = (int64_t)__builtin_amdgcn_readfirstlane(ctl->next_tile[par ^ 1]);
         const bool more = tn < q.xe;
-        int32_t after = 0;
-        if (tid == 0) after = q.claim();
-        const TileDesc Gn = tdesc[more ? tn : t];
-        const uint64_t sbeg_n = toff[more ? tn : t];
-        const uint32_t cnt_n = (uint32_t)(toff[(more ? tn : t) + 1] - sbeg_n);
+        int32_t after = NO_UNIT;
+        if (!SLICES && tid == 0) after = q.claim();
+        const int64_t t = U.t;
+        const uint64_t sbeg = U.sbeg;
+        const uint32_t cnt = U.cnt;
+        const PaintUnit Un = paint_unit<SLICES>(A, toff, more ? tn : unit);
+        const TileDesc Gn = tdesc[Un.t];
+        const uint64_t sbeg_n = Un.sbeg;
+        const uint32_t cnt_n = Un.cnt;
         const TileRow *rows = ctl->rows[par];
         uint32_t tu = 0, tf = 0, tl = 0, ts = 0;     /* this tile's updates, deferrals, listed, segments */
         uint32_t i = wave_from(cnt, wv_u);
@@ -1809,13 +1966,36 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NM == 
             for (uint32_t k = tid; k < nfl; k += blockDim.x)
                 if (ctl->fb_base + k < (unsigned long long)fbs) fbr[ctl->fb_base + k] = ctl->fb[k];
         }
-        const bool lost = ctl->lost[par] != 0u || (nfl && ctl->fb_base + nfl > (unsigned long long)fbs);
-        if (tid == 0) {
+        bool lost = ctl->lost[par] != 0u || (nfl && ctl->fb_base + nfl > (unsigned long long)fbs);
+        bool write = !skip;
+        if constexpr (SLICES) {
+            if (!skip) {
+                /* the slice's counts go to the tile's, which the last slice adds
+                 * up unless one was lost */
+                unsigned long long *st = A.split.state[A.split.units[unit].part].stat;
+                if (tid < 4) ctl->stat[tid] = 0;
+                lds_barrier();
+                atomicAdd(&ctl->stat[0], tl); atomicAdd(&ctl->stat[1], tu);
+                atomicAdd(&ctl->stat[2], ts); atomicAdd(&ctl->stat[3], tf);
+                lds_barrier();
+                if (tid < 4) atomicAdd(&st[tid], (unsigned long long)ctl->stat[tid]);
+                const uint32_t r = join_slice<NM>(A, ctl, unit, G.rows << log2c, lost, acc, lhash, lcount);
+                write = (r & SLICE_LAST) != 0u;
+                lost = (r & SLICE_LOST) != 0u;
+                if (write && tid < 4) {
+                    const unsigned long long v = atomicExch(&st[tid], 0ULL);
+                    const int at = tid < 2 ? tid : tid + 2;           /* counters 0, 1, 4, 5 */
+                    if (!lost) atomicAdd(&A.counters[at + (blockIdx.x % P2M_SHARDS) * P2M_CTR_STRIDE], v);
+                }
+            }
+            tu = tf = tl = ts = 0;
+        }
+        if (tid == 0 && write) {
             if (lost) { A.lost[t] = 1; atomicAdd(A.n_lost + (blockIdx.x % P2M_SHARDS) * P2M_CTR_STRIDE, 1ULL); }
             else if (A.redo) A.lost[t] = 0;
         }
         if (!lost) { n_upd += tu; n_fb += tf; n_list += tl; n_seg += ts; }
-        const bool keep = lost || skip;
+        const bool keep = lost || !write;
         /* the branch on accumulate is taken outside the loops: a select
          * inside lets the compiler load the map speculatively (a map read and
          * a wait on it per tile) even when the tile only stores */
@@ -1849,9 +2029,17 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NM == 
             atomicAdd(&A.counters[0], (unsigned long long)n_list); n_list = 0;
             atomicAdd(&A.counters[1], (unsigned long long)n_upd); n_upd = 0;
         }
-        t = tn; G = Gn; sbeg = sbeg_n; cnt = cnt_n;
-        skip = A.redo && !A.lost[t];
+        unit = tn; U = Un; G = Gn;
+        skip = skipped();
     }
+    if constexpr (!SLICES) break;
+    lds_barrier();
+    if (tid == 0) {
+        ctl->nfb[0] = 0; ctl->lost[0] = 0;
+        ctl->next_tile[0] = q.claim();
+        ctl->next_tile[1] = NO_UNIT;
+    }
+    lds_barrier();
     }
     lds_barrier();
     /* the deferred pixels' buffer is free: its space takes the block sums (the
@@ -1862,6 +2050,19 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NM == 
     block_count(&A.counters[4], n_seg, red);
     block_count(&A.counters[5], n_fb, red);
     block_count(A.err, n_err, red);
+}
+
+/* The tiles, then the slices of split ones: a loop of their own, since in
+ * the tiles' loop a tile's descriptor would be two loads behind its number (2e7
+ * halos at nside 4096 1.45 -> 1.52 ms), and in the same launch, since an empty
+ * one of as many workgroups takes 20 us. */
+template <int NM>
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NM == 1 ? 6 : 1))) k_tile_fast(TileArgs A, const TileDesc *__restrict__ tdesc,
+                                                   const unsigned long long *__restrict__ toff,
+                                                   const RingDesc *__restrict__ rdesc)
+{
+    paint_fast<NM, false>(A, tdesc, toff, rdesc);
+    if (A.split.above && *A.split.n != 0u) paint_fast<NM, true>(A, tdesc, toff, rdesc);
 }
 
 /* Deferred pixels of k_tile_fast -- (row, in-row pixel, halo, tile) --
@@ -2034,7 +2235,7 @@ int p2m_launch_tile_paint(const TileArgs &a, int mode, int n_maps, int grid, int
     size_t lds = p2m_tile_lds_bytes(mode, n_maps, a.log2w, a.count != nullptr, a.g.nrt, wg);
     if (lds > 160 * 1024 || wg > 512 || (mode == 2 && wg > 256)) return -1;
     if (!a.tile_next || grid > P2M_TQ_MAX) return -1;
-    /* the tile queues' counters */
+    /* the queues' counters (the slices' between the first two of the tiles') */
     p2m_launch_fill_u32(a.tile_next, (grid >= a.n_tiles ? std::max(grid, 8) : 8) * P2M_TQ_STRIDE, 0u, s);
 #define P2M_TE(NMv) case NMv: hipLaunchKernelGGL((k_tile_exact<NMv>), dim3(grid), dim3(wg), lds, s, a, a.desc, a.tile_off, a.ring); break;
 #define P2M_TF(NMv) case NMv: hipLaunchKernelGGL((k_tile_fast<NMv>), dim3(grid), dim3(wg), lds, s, a, a.desc, a.tile_off, a.ring); break;
