@@ -1616,11 +1616,14 @@ int64_t p2m_flat_tiles(int32_t npix, int32_t *nj)
  * each: 2048 workgroups fill the GPU, of at least 8 pairs so that a tile's
  * clearing and adding up pays (32 is up to 1.6 times slower, 4 no faster),
  * and the slices' counters keep the listing's atomics apart (6e4 halos on
- * 200 x 200 pixels, 52 tiles: in one list per tile 307 us, 44 us in 39). */
+ * 200 x 200 pixels, 52 tiles: in one list per tile 307 us, 44 us in 39).  The
+ * fewer the tiles, the more slices each (1e5 halos on 64 x 64 pixels, 4 tiles: 64
+ * slices a tile 150 us, 128 84, 256 54, 512 42; on 16 x 16, one tile: 64 850 us,
+ * 2048 60). */
 int p2m_flat_slices(int64_t n_tiles, int64_t n_pairs)
 {
     const int64_t s = std::min<int64_t>(2048 / n_tiles, n_pairs / (8 * n_tiles));
-    return (int)std::max<int64_t>(1, std::min<int64_t>(s, 64));
+    return (int)std::max<int64_t>(1, s);
 }
 
 void p2m_launch_flat_pairs(const FlatArgs &f, int emit, hipStream_t s)
