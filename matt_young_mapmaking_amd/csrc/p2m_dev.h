@@ -260,38 +260,61 @@ P2M_HD float disc_half_turn(double thr, double s0)
     return asinf(sd / s) * (1.00001f / 6.2831853f) + 1e-6f;
 }
 
+/* The tiles of a band that a halo's disc may reach: n of its K sectors from
+ * k0 (past the last one comes the first), `rows` rows from `row`. */
+struct BandTiles { int32_t K, k0, n, row, rows; };
+P2M_HD BandTiles band_tiles(const TileShape &g, int32_t band, float turn, float half, int32_t ra, int32_t rb)
+{
+    int32_t r0, r1;
+    const int32_t K = band_sectors(g, band, r0, r1);
+    const int32_t first = ra > r0 ? ra : r0, last = rb < r1 ? rb : r1;
+    int32_t n = K, k0 = 0;
+    if (half < 0.5f) {
+        /* a pixel ip of a ring lies at (ip + off) / npr turns, off 0 or
+         * 1/2, in the sector ceil((ip + 1) K / npr) - 1: not below the
+         * floor of its turn times K, at most a pixel's K / npr above */
+        const int32_t m0 = r0 < 4 * g.nside - r1 ? r0 : 4 * g.nside - r1;
+        const int32_t nmin = 4 * (m0 < g.nside ? m0 : g.nside);
+        const float fk = (float)K;
+        const double lo = ((double)turn - (double)half) * fk, hi = ((double)turn + (double)half) * fk + (double)(fk / (float)nmin);
+        k0 = (int32_t)p2m_floor(lo);
+        n = (int32_t)p2m_floor(hi + 1e-6) - k0 + 1;
+        if (n >= K) { n = K; k0 = 0; }
+        else if (k0 < 0) k0 += K;
+    }
+    return {K, k0, n, first - r0, last - first + 1};
+}
+
+/* the bands [b0, b1] of the rings of a PairHalo; none: b0 > b1 */
+P2M_HD void halo_bands(const TileShape &g, uint32_t rings, int32_t &ra, int32_t &rb, int32_t &b0, int32_t &b1)
+{
+    ra = (int32_t)(rings & 0xffffu);
+    rb = (int32_t)((rings >> 16) & 0x7fffu);
+    b0 = (ra - 1) >> g.log2r;
+    b1 = ra > rb ? b0 - 1 : (rb - 1) >> g.log2r;
+}
+
 /* The tiles a halo's disc may reach, in band order: f(band, sector, first
  * row, rows), every tile once. */
 template <typename F>
 P2M_HD void halo_tiles(const TileShape &g, float turn, float half, uint32_t rings, F f)
 {
-    const int32_t ra = (int32_t)(rings & 0xffffu), rb = (int32_t)((rings >> 16) & 0x7fffu);
-    if (ra > rb) return;
-    const int32_t b0 = (ra - 1) >> g.log2r, b1 = (rb - 1) >> g.log2r;
+    int32_t ra, rb, b0, b1;
+    halo_bands(g, rings, ra, rb, b0, b1);
     for (int32_t band = b0; band <= b1; ++band) {
-        int32_t r0, r1;
-        const int32_t K = band_sectors(g, band, r0, r1);
-        const int32_t first = ra > r0 ? ra : r0, last = rb < r1 ? rb : r1;
-        int32_t n = K, k0 = 0;
-        if (half < 0.5f) {
-            /* a pixel ip of a ring lies at (ip + off) / npr turns, off 0 or
-             * 1/2, in the sector ceil((ip + 1) K / npr) - 1: not below the
-             * floor of its turn times K, at most a pixel's K / npr above */
-            const int32_t m0 = r0 < 4 * g.nside - r1 ? r0 : 4 * g.nside - r1;
-            const int32_t nmin = 4 * (m0 < g.nside ? m0 : g.nside);
-            const float fk = (float)K;
-            const double lo = ((double)turn - (double)half) * fk, hi = ((double)turn + (double)half) * fk + (double)(fk / (float)nmin);
-            k0 = (int32_t)p2m_floor(lo);
-            n = (int32_t)p2m_floor(hi + 1e-6) - k0 + 1;
-            if (n >= K) { n = K; k0 = 0; }
-            else if (k0 < 0) k0 += K;
-        }
-        for (int32_t j = 0; j < n; ++j) {
-            int32_t k = k0 + j;
-            if (k >= K) k -= K;
-            f(band, k, first - r0, last - first + 1);
-        }
+        const BandTiles t = band_tiles(g, band, turn, half, ra, rb);
+        for (int32_t j = 0; j < t.n; ++j) f(band, t.k0 + j < t.K ? t.k0 + j : t.k0 + j - t.K, t.row, t.rows);
     }
+}
+
+/* how many */
+P2M_HD uint32_t halo_tile_count(const TileShape &g, float turn, float half, uint32_t rings)
+{
+    int32_t ra, rb, b0, b1;
+    halo_bands(g, rings, ra, rb, b0, b1);
+    uint32_t n = 0;
+    for (int32_t band = b0; band <= b1; ++band) n += (uint32_t)band_tiles(g, band, turn, half, ra, rb).n;
+    return n;
 }
 
 /* Pixel-centre z and sin(theta) of ring `ring`, exactly as pix2vec_ring

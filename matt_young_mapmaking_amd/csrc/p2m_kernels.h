@@ -152,6 +152,7 @@ struct TileArgs {
     unsigned int *tile_next;      /* the tile queues: one counter per XCD or workgroup, P2M_TQ_STRIDE
                                      apart (zeroed by p2m_launch_tile_paint) */
     SplitArgs split;
+    int32_t wide;                 /* pairs are mostly the insides of wide discs (paint_exact) */
     unsigned long long *counters; /* [0] listed, [1] hp updates, [4] segments, [5] FP64 fallbacks */
     unsigned long long *err;      /* sharded: pairs whose halo or rows are out of bounds */
     unsigned long long *n_lost;   /* sharded: tiles marked lost */

@@ -379,8 +379,7 @@ __global__ void __launch_bounds__(256) k_setup(DecodeArgs A)
                 q.rings = rings;
                 if (gaps_possible(A.nside, ztop, zbot, h.a, q.half, rings)) { q.rings |= RINGS_ASK_GAPS; tot_gaps++; }
                 A.pair_halo[k] = q;
-                uint32_t np = 0;
-                halo_tiles(A.shape, q.turn, q.half, rings, [&](int32_t, int32_t, int32_t, int32_t) { ++np; });
+                const uint32_t np = halo_tile_count(A.shape, q.turn, q.half, rings);
                 A.n_pairs[k] = np;
                 tot_pairs += np;
                 /* pixels of the disc, about: its share of the sphere is chord^2 / 4 */
@@ -552,25 +551,55 @@ __global__ void __launch_bounds__(256) k_pair_count(BinArgs B)
 {
     for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < B.n_halo; i += (int64_t)gridDim.x * blockDim.x) {
         const PairHalo h = B.halos[i];
-        uint32_t n = 0;
-        halo_tiles(B.shape, h.turn, h.half, h.rings, [&](int32_t, int32_t, int32_t, int32_t) { ++n; });
-        B.n_pairs[i] = n;
+        B.n_pairs[i] = halo_tile_count(B.shape, h.turn, h.half, h.rings);
     }
 }
 
-__global__ void __launch_bounds__(256) k_pair_emit(BinArgs B)
+/* Lists the pairs, `per` halos a wave.  A lane lists its halo's, unless they
+ * are more than 64: a disc over hundreds of tiles is listed by the whole wave,
+ * the bands' geometry over the lanes, then band by band the sectors (100 discs
+ * of 0.27 rad at nside 1024, 430 tiles each: 158 us by their lanes alone, 15
+ * now). */
+#define WIDE_PAIRS 64
+__global__ void __launch_bounds__(256) k_pair_emit(BinArgs B, int per)
 {
     if (B.n_split && blockIdx.x == 0 && threadIdx.x < 2) B.n_split[threadIdx.x] = 0u;
-    for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < B.n_halo; i += (int64_t)gridDim.x * blockDim.x) {
-        const PairHalo h = B.halos[i];
-        unsigned long long o = B.pair_off[i];
-        halo_tiles(B.shape, h.turn, h.half, h.rings, [&](int32_t band, int32_t k, int32_t row, int32_t rows) {
-            if (o < B.pair_cap) {
-                B.keys[o] = ((uint32_t)(B.band_tile[band] + k) << 8) | ((uint32_t)row << 4) | (uint32_t)(rows - 1);
-                B.vals[o] = (uint32_t)i;
+    const int lane = __lane_id();
+    const int64_t waves = ((int64_t)gridDim.x * blockDim.x) >> 6;
+    for (int64_t w = (blockIdx.x * (int64_t)blockDim.x + threadIdx.x) >> 6; w * per < B.n_halo; w += waves) {
+        const int64_t i = w * per + lane;
+        PairHalo h = {0.0f, 0.0f, 1u};
+        unsigned long long o = 0;
+        uint32_t n = 0;
+        if (lane < per && i < B.n_halo) { h = B.halos[i]; o = B.pair_off[i]; n = B.n_pairs[i]; }
+        auto list = [&](unsigned long long at, int64_t halo, int32_t band, int32_t k, int32_t row, int32_t rows) {
+            if (at < B.pair_cap) {
+                B.keys[at] = ((uint32_t)(B.band_tile[band] + k) << 8) | ((uint32_t)row << 4) | (uint32_t)(rows - 1);
+                B.vals[at] = (uint32_t)halo;
             }
-            ++o;
-        });
+        };
+        if (n <= WIDE_PAIRS)
+            halo_tiles(B.shape, h.turn, h.half, h.rings, [&](int32_t band, int32_t k, int32_t row, int32_t rows) {
+                list(o++, i, band, k, row, rows);
+            });
+        for (unsigned long long wide = __ballot(n > WIDE_PAIRS); wide; wide &= wide - 1) {
+            const int l = __ffsll((long long)wide) - 1;
+            const float turn = __shfl(h.turn, l), half = __shfl(h.half, l);
+            unsigned long long at = __shfl(o, l);
+            int32_t ra, rb, b0, b1;
+            halo_bands(B.shape, (uint32_t)__shfl((int)h.rings, l), ra, rb, b0, b1);
+            for (int32_t band = b0; band <= b1; band += 64) {
+                BandTiles t = {1, 0, 0, 0, 0};
+                if (band + lane <= b1) t = band_tiles(B.shape, band + lane, turn, half, ra, rb);
+                const int bands = b1 - band < 63 ? b1 - band + 1 : 64;
+                for (int b = 0; b < bands; ++b) {
+                    const int32_t K = __shfl(t.K, b), k0 = __shfl(t.k0, b), m = __shfl(t.n, b);
+                    const int32_t row = __shfl(t.row, b), rows = __shfl(t.rows, b);
+                    for (int32_t k = lane; k < m; k += 64) list(at + k, w * per + l, band + b, k0 + k < K ? k0 + k : k0 + k - K, row, rows);
+                    at += m;
+                }
+            }
+        }
     }
 }
 
@@ -624,7 +653,10 @@ void p2m_launch_ring_gaps(const BinArgs &b, hipStream_t s)
 }
 void p2m_launch_pair_emit(const BinArgs &b, hipStream_t s)
 {
-    if (b.n_halo > 0) hipLaunchKernelGGL(k_pair_emit, dim3(bin_grid(b.n_halo)), dim3(256), 0, s, b);
+    if (b.n_halo <= 0) return;
+    /* few halos: a wave each, so that wide discs are spread out */
+    const int64_t per = std::min<int64_t>(b.n_halo / 8192 + 1, 64);
+    hipLaunchKernelGGL(k_pair_emit, dim3(bin_grid((b.n_halo + per - 1) / per * 64)), dim3(256), 0, s, b, (int)per);
 }
 void p2m_launch_tile_bounds(const uint32_t *keys, unsigned long long n, int64_t n_tiles, unsigned long long *tile_off,
                             const SplitArgs &split, unsigned long long *err, hipStream_t s)
@@ -913,6 +945,19 @@ __device__ static inline uint32_t wave_share(uint32_t n, int w, int nw)
     return s < n ? s : n;
 }
 
+/* Where most pairs are whole tiles (the insides of wide discs), a tile has few
+ * of them: the FP64 painter's waves then share each by rows (WIDE), every wave
+ * goes over all pairs and takes its part of a pair's rows, if the pair has
+ * eight or more; the others are the first wave's. */
+__device__ static inline bool narrow_pair(uint32_t &key, int part, int parts)
+{
+    const int rows = (int)(key & 15u) + 1;
+    if (rows < 8) return part == 0;
+    const int r0 = rows * part / parts, r1 = rows * (part + 1) / parts;
+    key = (key & ~255u) | ((((key >> 4) & 15u) + (uint32_t)r0) << 4) | (uint32_t)(r1 - r0 - 1);
+    return true;
+}
+
 /* Tiles come from one queue per XCD: workgroup b runs on XCD b % 8 and
  * claims the next tile of that XCD's contiguous eighth of the tiles (sector
  * by sector along a band, so the tiles in flight on an XCD share halos and
@@ -1186,7 +1231,12 @@ struct PaintStats {
     unsigned long long listed, upd, segs, err;
 };
 
-template <int NM, bool SLICES>
+/* WIDE: for calls whose pairs are mostly the insides of wide discs.  Their
+ * pixels all take the reference's arithmetic, so a step of such pixels alone
+ * leaves out the quick one, and the waves share the pairs by rows.  100 discs
+ * of 0.27 rad at nside 1024: 0.94 -> 0.61 ms.  An instantiation of its own: as
+ * branches of the other it costs that 4% (2e6 halos at nside 2048). */
+template <int NM, bool SLICES, bool WIDE>
 __device__ static __forceinline__ void paint_exact(const TileArgs &A, const TileDesc *__restrict__ tdesc,
                                                    const unsigned long long *__restrict__ toff, const RingDesc *__restrict__ rdesc)
 {
@@ -1242,13 +1292,15 @@ __device__ static __forceinline__ void paint_exact(const TileArgs &A, const Tile
             lds_barrier();
         }
         const int wv_u = __builtin_amdgcn_readfirstlane(wv);
-        uint64_t pos = sbeg + wave_share(cnt, wv_u, nwv);
-        const uint64_t end = sbeg + wave_share(cnt, wv_u + 1, nwv);
+        uint64_t pos = sbeg + (WIDE ? 0u : wave_share(cnt, wv_u, nwv));
+        const uint64_t end = sbeg + (WIDE ? cnt : wave_share(cnt, wv_u + 1, nwv));
         while (pos < end) {
-            const bool has = pos + (uint64_t)lane < end;
-            const uint64_t at = has ? pos + (uint64_t)lane : end - 1;
+            const bool has = WIDE ? lane == 0 : pos + (uint64_t)lane < end;
+            const uint64_t at = WIDE ? pos : (has ? pos + (uint64_t)lane : end - 1);
             Seg g;
-            pos += (uint64_t)wave_segments(A.keys[at], A.vals[at], has, g);
+            uint32_t key = A.keys[at];
+            if (WIDE && !narrow_pair(key, wv_u, nwv)) { ++pos; continue; }
+            pos += (uint64_t)wave_segments(key, A.vals[at], has, g);
             uint32_t slot = g.val;
             /* a pair must name a record and rows of the tile; one that does
              * not is counted as an error and painted empty */
@@ -1322,17 +1374,20 @@ __device__ static __forceinline__ void paint_exact(const TileArgs &A, const Tile
                             vy[o] = by;
                         }
                     }
-                    const double v0 = ay * bz - az * by, v1 = az * bx - ax * bz, v2 = ax * by - ay * bx;
-                    const double q = (v0 * v0 + v1 * v1) + v2 * v2, edge = ew->edge[s];
-                    const double lr = __builtin_fma(0.5, f64_log(q * ew->chi2[s]), f64_lntan_sin2(q));
-                    const double u = (lr - A.g.lr0) * A.inv_drt;
-                    const double ub = __builtin_fmin(__builtin_fmax(u, 0.0), A.u_max64);
                     const bool gap = (o >= (int)(hole & 0xfffu)) & (o < (int)((hole >> 12) & 0xfffu));
-                    const bool cand = in & !gap & !(far & (q > edge));
-                    const bool plain = cand & far & (q < edge * (1.0 - 2.0 * EDGE_BAND)) & (q > 1e-60) &
-                                       (__builtin_fabs(u - __builtin_rint(ub)) > A.band64);
+                    bool cand = in & !gap, plain = false;
+                    if (!WIDE || __ballot(in & far)) {
+                        const double v0 = ay * bz - az * by, v1 = az * bx - ax * bz, v2 = ax * by - ay * bx;
+                        const double q = (v0 * v0 + v1 * v1) + v2 * v2, edge = ew->edge[s];
+                        const double lr = __builtin_fma(0.5, f64_log(q * ew->chi2[s]), f64_lntan_sin2(q));
+                        const double u = (lr - A.g.lr0) * A.inv_drt;
+                        const double ub = __builtin_fmin(__builtin_fmax(u, 0.0), A.u_max64);
+                        cand = cand & !(far & (q > edge));
+                        plain = cand & far & (q < edge * (1.0 - 2.0 * EDGE_BAND)) & (q > 1e-60) &
+                                (__builtin_fabs(u - __builtin_rint(ub)) > A.band64);
+                        if (plain) quad_value<NM>(A, tab, *ew, s, lr, u, ub, [&](int m, double v) { atomicAdd(&acc[m * W + o], v); });
+                    }
                     bool taken = plain;
-                    if (plain) quad_value<NM>(A, tab, *ew, s, lr, u, ub, [&](int m, double v) { atomicAdd(&acc[m * W + o], v); });
                     if (__ballot(cand & !plain)) {
                         if (cand & !plain) {
                             /* the reference's arithmetic */
@@ -1397,14 +1452,14 @@ __device__ static __forceinline__ void paint_exact(const TileArgs &A, const Tile
     block_count(A.err, st.err, red);
 }
 
-template <int NM>
+template <int NM, bool WIDE>
 __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(NM == 1 ? 3 : 2))) k_tile_exact(TileArgs A, const TileDesc *__restrict__ tdesc,
                                                     const unsigned long long *__restrict__ toff,
                                                     const RingDesc *__restrict__ rdesc)
 {
-    paint_exact<NM, false>(A, tdesc, toff, rdesc);
+    paint_exact<NM, false, WIDE>(A, tdesc, toff, rdesc);
     const TileArgs &B = launch_args();
-    if (B.split.above && *B.split.n != 0u) paint_exact<NM, true>(B, B.desc, B.tile_off, B.ring);
+    if (B.split.above && *B.split.n != 0u) paint_exact<NM, true, WIDE>(B, B.desc, B.tile_off, B.ring);
 }
 
 /* --------------------------------------------------------------------- */
@@ -2234,9 +2289,9 @@ int p2m_tile_occupancy(int mode, int n_maps, int wg, size_t lds)
     hipError_t e = hipErrorInvalidValue;
 #define P2M_OC(K) e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, K, wg, lds)
     switch (mode * 8 + n_maps) {
-    case 9: P2M_OC(k_tile_exact<1>); break;   case 10: P2M_OC(k_tile_exact<2>); break;
-    case 11: P2M_OC(k_tile_exact<3>); break;  case 12: P2M_OC(k_tile_exact<4>); break;
-    case 13: P2M_OC(k_tile_exact<5>); break;  case 14: P2M_OC(k_tile_exact<6>); break;
+    case 9: P2M_OC((k_tile_exact<1, false>)); break;   case 10: P2M_OC((k_tile_exact<2, false>)); break;
+    case 11: P2M_OC((k_tile_exact<3, false>)); break;  case 12: P2M_OC((k_tile_exact<4, false>)); break;
+    case 13: P2M_OC((k_tile_exact<5, false>)); break;  case 14: P2M_OC((k_tile_exact<6, false>)); break;
     case 17: P2M_OC(k_tile_fast<1>); break;   case 18: P2M_OC(k_tile_fast<2>); break;
     case 19: P2M_OC(k_tile_fast<3>); break;   case 20: P2M_OC(k_tile_fast<4>); break;
     case 21: P2M_OC(k_tile_fast<5>); break;   case 22: P2M_OC(k_tile_fast<6>); break;
@@ -2253,7 +2308,11 @@ int p2m_launch_tile_paint(const TileArgs &a, int mode, int n_maps, int grid, int
     if (!a.tile_next || grid > P2M_TQ_MAX) return -1;
     /* the queues' counters (the slices' between the first two of the tiles') */
     p2m_launch_fill_u32(a.tile_next, (grid >= a.n_tiles ? std::max(grid, 8) : 8) * P2M_TQ_STRIDE, 0u, s);
-#define P2M_TE(NMv) case NMv: hipLaunchKernelGGL((k_tile_exact<NMv>), dim3(grid), dim3(wg), lds, s, a, a.desc, a.tile_off, a.ring); break;
+#define P2M_TE(NMv) \
+    case NMv: \
+        if (a.wide) hipLaunchKernelGGL((k_tile_exact<NMv, true>), dim3(grid), dim3(wg), lds, s, a, a.desc, a.tile_off, a.ring); \
+        else hipLaunchKernelGGL((k_tile_exact<NMv, false>), dim3(grid), dim3(wg), lds, s, a, a.desc, a.tile_off, a.ring); \
+        break;
 #define P2M_TF(NMv) case NMv: hipLaunchKernelGGL((k_tile_fast<NMv>), dim3(grid), dim3(wg), lds, s, a, a.desc, a.tile_off, a.ring); break;
     if (mode == 1) {
         switch (n_maps) { P2M_TE(1) P2M_TE(2) P2M_TE(3) P2M_TE(4) P2M_TE(5) P2M_TE(6) default: return -1; }
