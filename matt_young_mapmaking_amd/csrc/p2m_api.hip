@@ -886,11 +886,13 @@ static int paint_halos(p2m_ctx *c, int64_t n_halo, int64_t n_flat, unsigned long
         t.keys = keys; t.vals = vals;
         table_args(c, t);
         t.fb = c->d_fb; t.fb_count = pc + 6; t.fb_cap = c->fb_cap;
-        t.lost = c->d_lost; t.tile_next = c->d_tile_next; t.split = split; t.wide = 2 * n_pix > (n_pairs << (c->shape.log2r + c->shape.log2c)); t.redo = 0; t.n_halo = n_halo; t.err = c->d_ctr + Ctr::ERR; t.n_lost = c->d_ctr + Ctr::LOST;
+        t.lost = c->d_lost; t.tile_next = c->d_tile_next; t.split = split; t.redo = 0; t.n_halo = n_halo; t.err = c->d_ctr + Ctr::ERR; t.n_lost = c->d_ctr + Ctr::LOST;
         for (int m = 0; m < c->cfg.n_maps; ++m) {
             t.map64[m] = c->d_hp64[m]; t.map32[m] = c->d_hp32[m];
         }
         t.count = c->d_count; t.hash = c->d_hash; t.counters = pc;
+        t.wide = 2 * n_pix > (n_pairs << (c->shape.log2r + c->shape.log2c));      /* half a tile a pair */
+        t.vectors = p2m_exact_vectors(c->cfg.n_maps, c->log2w, c->d_count != nullptr, wg);
         if (p2m_launch_tile_paint(t, mode, c->cfg.n_maps, grid, wg, c->stream)) return P2M_E_INVALID;
         HIPCHK(hipGetLastError());
         HIPCHK(hipEventRecord(c->ev[7], c->stream));

@@ -153,6 +153,7 @@ struct TileArgs {
                                      apart (zeroed by p2m_launch_tile_paint) */
     SplitArgs split;
     int32_t wide;                 /* pairs are mostly the insides of wide discs (paint_exact) */
+    int32_t vectors;              /* the FP64 painter keeps pixel vectors (p2m_exact_vectors) */
     unsigned long long *counters; /* [0] listed, [1] hp updates, [4] segments, [5] FP64 fallbacks */
     unsigned long long *err;      /* sharded: pairs whose halo or rows are out of bounds */
     unsigned long long *n_lost;   /* sharded: tiles marked lost */
@@ -224,6 +225,7 @@ int p2m_tile_max_log2w(void);
 void p2m_launch_build_quad(const float *flat, int64_t n_flat, int32_t profile, int32_t nrt, int32_t nmht, int32_t nchit,
                            int32_t n_maps, int32_t slot, float *quad, hipStream_t s);
 size_t p2m_tile_lds_bytes(int mode, int n_maps, int log2w, int membership, int nrt, int wg);
+int p2m_exact_vectors(int n_maps, int log2w, int membership, int wg);
 int p2m_tile_wg(int mode, int n_maps, int log2w, int membership, int nrt, int wg);
 int p2m_tile_occupancy(int mode, int n_maps, int wg, size_t lds);
 int p2m_launch_tile_paint(const TileArgs &a, int mode, int n_maps, int grid, int wg, hipStream_t s);

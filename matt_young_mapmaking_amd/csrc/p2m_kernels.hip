@@ -946,7 +946,7 @@ __device__ static inline uint32_t wave_share(uint32_t n, int w, int nw)
 }
 
 /* Where most pairs are whole tiles (the insides of wide discs), a tile has few
- * of them: the FP64 painter's waves then share each by rows (WIDE), every wave
+ * of them: the FP64 painter's waves then share each by rows, every wave
  * goes over all pairs and takes its part of a pair's rows, if the pair has
  * eight or more; the others are the first wave's. */
 __device__ static inline bool narrow_pair(uint32_t &key, int part, int parts)
@@ -1231,12 +1231,17 @@ struct PaintStats {
     unsigned long long listed, upd, segs, err;
 };
 
-/* WIDE: for calls whose pairs are mostly the insides of wide discs.  Their
- * pixels all take the reference's arithmetic, so a step of such pixels alone
- * leaves out the quick one, and the waves share the pairs by rows.  100 discs
- * of 0.27 rad at nside 1024: 0.94 -> 0.61 ms.  An instantiation of its own: as
- * branches of the other it costs that 4% (2e6 halos at nside 2048). */
-template <int NM, bool SLICES, bool WIDE>
+/* SPECIAL: an instantiation of its own for two kinds of calls, as their
+ * branches cost the other one 4% (2e6 halos at nside 2048).
+ *  - Pairs are mostly the insides of wide discs (A.wide).  Their pixels all
+ *    take the reference's arithmetic, so a step of such pixels alone leaves out
+ *    the quick one, and the waves share the pairs by rows.  100 discs of 0.27
+ *    rad at nside 1024: 0.94 -> 0.61 ms.
+ *  - Tiles of many pixels and maps (exact_vectors): a tile's pixel vectors take
+ *    the LDS that the waves need for their own values, so each is formed as it
+ *    is used.  1e6 halos at nside 1024, six maps with membership, tiles of 2048
+ *    pixels: one wave a CU 2.02, six 0.63 ms. */
+template <int NM, bool SLICES, bool SPECIAL>
 __device__ static __forceinline__ void paint_exact(const TileArgs &A, const TileDesc *__restrict__ tdesc,
                                                    const unsigned long long *__restrict__ toff, const RingDesc *__restrict__ rdesc)
 {
@@ -1253,7 +1258,8 @@ __device__ static __forceinline__ void paint_exact(const TileArgs &A, const Tile
     const int tid = threadIdx.x, lane = __lane_id(), wv = tid >> 6, nwv = (int)(blockDim.x >> 6);
     /* x and y of the tile's pixel vectors, NaN until a wave has needed one (several may form it: the same bits) */
     double *vx = (double *)(ctl + 1), *vy = vx + W;
-    ExactWave *ew = (ExactWave *)(vy + W) + wv;
+    const bool vectors = !SPECIAL || A.vectors, by_rows = SPECIAL && A.wide;
+    ExactWave *ew = (ExactWave *)(vectors ? vy + W : vx) + wv;
     PaintStats st = {0, 0, 0, 0};
     const __amdgpu_buffer_rsrc_t tab =
         __builtin_amdgcn_make_buffer_rsrc((void *)A.tab_q, (short)0, (int)(A.n_quad * 4), 0x00020000);
@@ -1261,7 +1267,7 @@ __device__ static __forceinline__ void paint_exact(const TileArgs &A, const Tile
     if (tid == 0) ctl->next_tile[0] = queue.first();
     for (int p = tid; p < W; p += blockDim.x) {
         for (int m = 0; m < NM; ++m) acc[m * W + p] = 0.0;
-        vx[p] = vy[p] = __builtin_nan("");
+        if (vectors) vx[p] = vy[p] = __builtin_nan("");
         if (A.count) { lcount[p] = 0; lhash[p] = 0ULL; }
     }
     lds_barrier();
@@ -1287,19 +1293,19 @@ __device__ static __forceinline__ void paint_exact(const TileArgs &A, const Tile
             x = Q.sth * cs;
             y = Q.sth * sn;
         };
-        if (cnt > MANY_PAIRS) {
+        if (vectors && cnt > MANY_PAIRS) {
             for (int p = tid; p < G.rows << log2c; p += blockDim.x) vector_of(p, vx[p], vy[p]);
             lds_barrier();
         }
         const int wv_u = __builtin_amdgcn_readfirstlane(wv);
-        uint64_t pos = sbeg + (WIDE ? 0u : wave_share(cnt, wv_u, nwv));
-        const uint64_t end = sbeg + (WIDE ? cnt : wave_share(cnt, wv_u + 1, nwv));
+        uint64_t pos = sbeg + (by_rows ? 0u : wave_share(cnt, wv_u, nwv));
+        const uint64_t end = sbeg + (by_rows ? cnt : wave_share(cnt, wv_u + 1, nwv));
         while (pos < end) {
-            const bool has = WIDE ? lane == 0 : pos + (uint64_t)lane < end;
-            const uint64_t at = WIDE ? pos : (has ? pos + (uint64_t)lane : end - 1);
+            const bool has = by_rows ? lane == 0 : pos + (uint64_t)lane < end;
+            const uint64_t at = by_rows ? pos : (has ? pos + (uint64_t)lane : end - 1);
             Seg g;
             uint32_t key = A.keys[at];
-            if (WIDE && !narrow_pair(key, wv_u, nwv)) { ++pos; continue; }
+            if (by_rows && !narrow_pair(key, wv_u, nwv)) { ++pos; continue; }
             pos += (uint64_t)wave_segments(key, A.vals[at], has, g);
             uint32_t slot = g.val;
             /* a pair must name a record and rows of the tile; one that does
@@ -1366,17 +1372,23 @@ __device__ static __forceinline__ void paint_exact(const TileArgs &A, const Tile
                     const bool far = (int32_t)sl >= 0;                 /* not SLOW */
                     /* the cross product of angdist */
                     const double ax = ew->hx[s], ay = ew->hy[s], az = ew->hz[s], bz = rows[row].zr;
-                    double bx = vx[o], by = vy[o];
-                    if (__ballot(in & ((bx != bx) | (by != by)))) {
-                        if (in & ((bx != bx) | (by != by))) {
-                            vector_of(o, bx, by);
-                            vx[o] = bx;
-                            vy[o] = by;
+                    double bx, by;
+                    if (vectors) {
+                        bx = vx[o];
+                        by = vy[o];
+                        if (__ballot(in & ((bx != bx) | (by != by)))) {
+                            if (in & ((bx != bx) | (by != by))) {
+                                vector_of(o, bx, by);
+                                vx[o] = bx;
+                                vy[o] = by;
+                            }
                         }
+                    } else {
+                        vector_of(o, bx, by);
                     }
                     const bool gap = (o >= (int)(hole & 0xfffu)) & (o < (int)((hole >> 12) & 0xfffu));
                     bool cand = in & !gap, plain = false;
-                    if (!WIDE || __ballot(in & far)) {
+                    if (!SPECIAL || __ballot(in & far)) {
                         const double v0 = ay * bz - az * by, v1 = az * bx - ax * bz, v2 = ax * by - ay * bx;
                         const double q = (v0 * v0 + v1 * v1) + v2 * v2, edge = ew->edge[s];
                         const double lr = __builtin_fma(0.5, f64_log(q * ew->chi2[s]), f64_lntan_sin2(q));
@@ -1434,7 +1446,7 @@ __device__ static __forceinline__ void paint_exact(const TileArgs &A, const Tile
                     }
                 }
                 for (int m = 0; m < NM; ++m) acc[m * W + p] = 0.0;
-                vx[p] = vy[p] = __builtin_nan("");
+                if (vectors) vx[p] = vy[p] = __builtin_nan("");
                 if (A.count) { lcount[p] = 0; lhash[p] = 0ULL; }
             }
         };
@@ -1452,14 +1464,14 @@ __device__ static __forceinline__ void paint_exact(const TileArgs &A, const Tile
     block_count(A.err, st.err, red);
 }
 
-template <int NM, bool WIDE>
+template <int NM, bool SPECIAL>
 __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(NM == 1 ? 3 : 2))) k_tile_exact(TileArgs A, const TileDesc *__restrict__ tdesc,
                                                     const unsigned long long *__restrict__ toff,
                                                     const RingDesc *__restrict__ rdesc)
 {
-    paint_exact<NM, false, WIDE>(A, tdesc, toff, rdesc);
+    paint_exact<NM, false, SPECIAL>(A, tdesc, toff, rdesc);
     const TileArgs &B = launch_args();
-    if (B.split.above && *B.split.n != 0u) paint_exact<NM, true, WIDE>(B, B.desc, B.tile_off, B.ring);
+    if (B.split.above && *B.split.n != 0u) paint_exact<NM, true, SPECIAL>(B, B.desc, B.tile_off, B.ring);
 }
 
 /* --------------------------------------------------------------------- */
@@ -2262,6 +2274,15 @@ void p2m_launch_build_quad(const float *flat, int64_t n_flat, int32_t profile, i
  * 64 segments of at most a row, 128 pixels, must fit 16 bits) */
 int p2m_tile_max_log2w(void) { return 11; }
 
+/* Whether the FP64 painter keeps a tile's pixel vectors in LDS: not where
+ * fewer waves than asked, and than four, fit beside them. */
+int p2m_exact_vectors(int n_maps, int log2w, int membership, int wg)
+{
+    const size_t W = (size_t)1 << log2w, b = (size_t)n_maps * W * 8 + (membership ? W * 12 : 0) + sizeof(TileCtl) + 2 * W * 8;
+    const int waves = b > 160 * 1024 ? 0 : (int)((160 * 1024 - b) / sizeof(ExactWave));
+    return waves >= std::min(wg / 64, 4);
+}
+
 size_t p2m_tile_lds_bytes(int mode, int n_maps, int log2w, int membership, int nrt, int wg)
 {
     const size_t W = (size_t)1 << log2w, nw = (size_t)(wg / 64);
@@ -2269,13 +2290,13 @@ size_t p2m_tile_lds_bytes(int mode, int n_maps, int log2w, int membership, int n
     if (membership) b += W * 12;
     b = ((b + 15) & ~(size_t)15) + sizeof(TileCtl);
     if (mode == 2) b += nw * (sizeof(FastWave) + (membership ? 8 * WSEG : 0)) + sizeof(float) * (size_t)(nrt + 2);
-    else b += 2 * W * sizeof(double) + nw * sizeof(ExactWave);
+    else b += (p2m_exact_vectors(n_maps, log2w, membership, wg) ? 2 * W * sizeof(double) : 0) + nw * sizeof(ExactWave);
     return b;
 }
 
 /* The workgroup size to launch for an asked one: every wave has its own
- * staging, so a wide tile of many maps takes fewer waves than asked (down to
- * one) where all of them do not fit the CU's 160 KB of LDS. */
+ * staging, so a wide tile of many maps takes fewer waves than asked where all
+ * of them do not fit the CU's 160 KB of LDS. */
 int p2m_tile_wg(int mode, int n_maps, int log2w, int membership, int nrt, int wg)
 {
     while (wg > 64 && p2m_tile_lds_bytes(mode, n_maps, log2w, membership, nrt, wg) > 160 * 1024) wg -= 64;
@@ -2310,7 +2331,7 @@ int p2m_launch_tile_paint(const TileArgs &a, int mode, int n_maps, int grid, int
     p2m_launch_fill_u32(a.tile_next, (grid >= a.n_tiles ? std::max(grid, 8) : 8) * P2M_TQ_STRIDE, 0u, s);
 #define P2M_TE(NMv) \
     case NMv: \
-        if (a.wide) hipLaunchKernelGGL((k_tile_exact<NMv, true>), dim3(grid), dim3(wg), lds, s, a, a.desc, a.tile_off, a.ring); \
+        if (a.wide || !a.vectors) hipLaunchKernelGGL((k_tile_exact<NMv, true>), dim3(grid), dim3(wg), lds, s, a, a.desc, a.tile_off, a.ring); \
         else hipLaunchKernelGGL((k_tile_exact<NMv, false>), dim3(grid), dim3(wg), lds, s, a, a.desc, a.tile_off, a.ring); \
         break;
 #define P2M_TF(NMv) case NMv: hipLaunchKernelGGL((k_tile_fast<NMv>), dim3(grid), dim3(wg), lds, s, a, a.desc, a.tile_off, a.ring); break;
