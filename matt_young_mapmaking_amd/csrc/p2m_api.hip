@@ -20,6 +20,7 @@
 #include <vector>
 
 #include "../../include/pks2map_gpu.h"
+#include "p2m_convert.h"
 #include "p2m_kernels.h"
 
 /* Scratch of the map products: the 10000-bin dP/dy histogram (u64), then the
@@ -198,6 +199,18 @@ static int dmalloc(void **p, size_t bytes)
 }
 static void dfree(void *p) { if (p) (void)hipFree(p); }
 
+/* the same for a context that may hold memory it can do without: the
+ * conversion buffer of p2m_fetch_maps, given back where device memory is short */
+static int grow(p2m_ctx *c, void **p, size_t bytes)
+{
+    const int rc = dmalloc(p, bytes);
+    if (!rc || !c->d_conv) return rc;
+    dfree(c->d_conv);
+    c->d_conv = nullptr;
+    c->conv_cap = 0;
+    return dmalloc(p, bytes);
+}
+
 /* cosmology.f90:123-133 (dzdr) and 109-119 (drdz), FP64 */
 static double dzdr(double h, double om, double z)
 {
@@ -253,18 +266,18 @@ static int build_tiles(p2m_ctx *c, int log2w)
     c->d_band_tile = nullptr; c->d_tile_off = nullptr; c->d_tile_desc = nullptr; c->d_lost = nullptr;
     c->log2w = 0;
     int rc = 0;
-    rc |= dmalloc((void **)&c->d_lost, (size_t)((acc + 3) / 4) * 4);
-    if (!c->d_tile_next) rc |= dmalloc((void **)&c->d_tile_next, sizeof(unsigned int) * P2M_TQ_MAX * P2M_TQ_STRIDE);
-    rc |= dmalloc((void **)&c->d_tile_desc, sizeof(TileDesc) * acc);
-    rc |= dmalloc((void **)&c->d_band_tile, sizeof(int32_t) * (size_t)(nb + 1));
-    rc |= dmalloc((void **)&c->d_tile_off, sizeof(unsigned long long) * (c->n_tiles + 1));
+    rc |= grow(c, (void **)&c->d_lost, (size_t)((acc + 3) / 4) * 4);
+    if (!c->d_tile_next) rc |= grow(c, (void **)&c->d_tile_next, sizeof(unsigned int) * P2M_TQ_MAX * P2M_TQ_STRIDE);
+    rc |= grow(c, (void **)&c->d_tile_desc, sizeof(TileDesc) * acc);
+    rc |= grow(c, (void **)&c->d_band_tile, sizeof(int32_t) * (size_t)(nb + 1));
+    rc |= grow(c, (void **)&c->d_tile_off, sizeof(unsigned long long) * (c->n_tiles + 1));
     if (rc) return P2M_E_NOMEM;
     HIPCHK(hipMemcpy(c->d_band_tile, band_tile.data(), sizeof(int32_t) * (size_t)(nb + 1), hipMemcpyHostToDevice));
     p2m_launch_tile_desc(g, c->d_band_tile, c->d_tile_desc, c->stream);
     p2m_launch_fill_u32((uint32_t *)c->d_lost, (acc + 3) / 4, 0u, c->stream);
     HIPCHK(hipGetLastError());
     if (!c->d_ring) {
-        if (dmalloc((void **)&c->d_ring, sizeof(RingDesc) * (size_t)(4 * ns - 1))) return P2M_E_NOMEM;
+        if (grow(c, (void **)&c->d_ring, sizeof(RingDesc) * (size_t)(4 * ns - 1))) return P2M_E_NOMEM;
         p2m_launch_ring_desc(ns, c->d_ring, c->stream);
         HIPCHK(hipGetLastError());
     }
@@ -477,8 +490,8 @@ int p2m_set_run(p2m_ctx *c, const p2m_run *r)
         double z = c->zofr[i - 2];
         c->zofr[i - 1] = c->zofr[i - 2] + dzdr(r->h, r->omegam, z) * dr;
     }
-    if (!c->d_rofz && dmalloc((void **)&c->d_rofz, sizeof(double) * n)) return P2M_E_NOMEM;
-    if (!c->d_zofr && dmalloc((void **)&c->d_zofr, sizeof(double) * n)) return P2M_E_NOMEM;
+    if (!c->d_rofz && grow(c, (void **)&c->d_rofz, sizeof(double) * n)) return P2M_E_NOMEM;
+    if (!c->d_zofr && grow(c, (void **)&c->d_zofr, sizeof(double) * n)) return P2M_E_NOMEM;
     HIPCHK(hipMemcpy(c->d_rofz, c->rofz.data(), sizeof(double) * n, hipMemcpyHostToDevice));
     HIPCHK(hipMemcpy(c->d_zofr, c->zofr.data(), sizeof(double) * n, hipMemcpyHostToDevice));
     c->mypi = 4.0 * p2m_atan(1.0);                         /* pks2map.f90:88 */
@@ -554,13 +567,13 @@ int p2m_load_table(p2m_ctx *c, int slot, const int32_t hdr_i[3], const float hdr
      * bytes per map and node of each cell), must each stay below 2 GiB */
     if ((nt + pad) * 4 > INT32_MAX || (nt / 2) * 16 * c->cfg.n_maps > INT32_MAX) return P2M_E_SIZE;
     c->n_flat = nt + pad;
-    if (!c->d_flat[slot] && dmalloc((void **)&c->d_flat[slot], sizeof(float) * c->n_flat)) return P2M_E_NOMEM;
+    if (!c->d_flat[slot] && grow(c, (void **)&c->d_flat[slot], sizeof(float) * c->n_flat)) return P2M_E_NOMEM;
     std::vector<float> flat(c->n_flat, 0.f);
     memcpy(flat.data(), table, sizeof(float) * nt);
     HIPCHK(hipMemcpy(c->d_flat[slot], flat.data(), sizeof(float) * c->n_flat, hipMemcpyHostToDevice));
     if (c->cfg.precision != P2M_PREC_PLAIN_FP64) {
         c->n_quad = (int64_t)g.nchit * g.nmht * g.nrt * 4 * c->cfg.n_maps;
-        if (!c->d_quad && dmalloc((void **)&c->d_quad, sizeof(float) * c->n_quad)) return P2M_E_NOMEM;
+        if (!c->d_quad && grow(c, (void **)&c->d_quad, sizeof(float) * c->n_quad)) return P2M_E_NOMEM;
         p2m_launch_build_quad(c->d_flat[slot], c->n_flat, c->cfg.profile, g.nrt, g.nmht, g.nchit, c->cfg.n_maps, slot,
                               c->d_quad, c->stream);
         HIPCHK(hipGetLastError());
@@ -571,8 +584,8 @@ int p2m_load_table(p2m_ctx *c, int slot, const int32_t hdr_i[3], const float hdr
     for (int k = 0; k < g.nrt + 2; ++k) inv[k] = p2m_exp(-2.0 * (g.lr0 + (double)k * g.drt));
     std::vector<float> invf(g.nrt + 2);
     for (int k = 0; k < g.nrt + 2; ++k) invf[k] = (float)inv[k];
-    if (!c->d_inv_node2 && dmalloc((void **)&c->d_inv_node2, sizeof(double) * (g.nrt + 2))) return P2M_E_NOMEM;
-    if (!c->d_inv_node2f && dmalloc((void **)&c->d_inv_node2f, sizeof(float) * (g.nrt + 2))) return P2M_E_NOMEM;
+    if (!c->d_inv_node2 && grow(c, (void **)&c->d_inv_node2, sizeof(double) * (g.nrt + 2))) return P2M_E_NOMEM;
+    if (!c->d_inv_node2f && grow(c, (void **)&c->d_inv_node2f, sizeof(float) * (g.nrt + 2))) return P2M_E_NOMEM;
     HIPCHK(hipMemcpy(c->d_inv_node2, inv.data(), sizeof(double) * (g.nrt + 2), hipMemcpyHostToDevice));
     HIPCHK(hipMemcpy(c->d_inv_node2f, invf.data(), sizeof(float) * (g.nrt + 2), hipMemcpyHostToDevice));
     c->u_k1 = (float)(0.5 * 0.6931471805599453 / g.drt);   /* log2(r^2) -> (ln r)/drt */
@@ -663,13 +676,13 @@ static int ensure_halo_cap(p2m_ctx *c, int64_t n)
     dfree(c->d_hot); c->d_hot = nullptr;
     dfree(c->d_pair_halo); c->d_pair_halo = nullptr;
     int64_t cap = std::max<int64_t>(n, 1024);
-    if (dmalloc((void **)&c->d_halo, sizeof(HaloRec) * cap)) return P2M_E_NOMEM;
-    if (dmalloc((void **)&c->d_flat_idx, sizeof(uint32_t) * cap)) return P2M_E_NOMEM;
+    if (grow(c, (void **)&c->d_halo, sizeof(HaloRec) * cap)) return P2M_E_NOMEM;
+    if (grow(c, (void **)&c->d_flat_idx, sizeof(uint32_t) * cap)) return P2M_E_NOMEM;
     if (c->cfg.precision != P2M_PREC_PLAIN_FP64 && c->cfg.nside > 0) {
-        if (dmalloc((void **)&c->d_pair_halo, sizeof(PairHalo) * cap)) return P2M_E_NOMEM;
-        if (dmalloc((void **)&c->d_n_pairs, sizeof(uint32_t) * (cap + 1))) return P2M_E_NOMEM;
-        if (dmalloc((void **)&c->d_pair_off, sizeof(unsigned long long) * (cap + 1))) return P2M_E_NOMEM;
-        if (c->cfg.precision == P2M_PREC_FP32_COMP && dmalloc((void **)&c->d_hot, sizeof(TileHalo) * cap))
+        if (grow(c, (void **)&c->d_pair_halo, sizeof(PairHalo) * cap)) return P2M_E_NOMEM;
+        if (grow(c, (void **)&c->d_n_pairs, sizeof(uint32_t) * (cap + 1))) return P2M_E_NOMEM;
+        if (grow(c, (void **)&c->d_pair_off, sizeof(unsigned long long) * (cap + 1))) return P2M_E_NOMEM;
+        if (c->cfg.precision == P2M_PREC_FP32_COMP && grow(c, (void **)&c->d_hot, sizeof(TileHalo) * cap))
             return P2M_E_NOMEM;
     }
     c->halo_cap = cap;
@@ -749,7 +762,7 @@ static SplitArgs split_args(p2m_ctx *c, unsigned long long n_pairs, int grid, si
     if (bytes > c->split_bytes) {
         dfree(c->d_split); c->d_split = nullptr; c->split_bytes = 0;
         const size_t cap = (bytes + bytes / 8 + 255) & ~(size_t)255;
-        if (dmalloc((void **)&c->d_split, cap)) return s;
+        if (grow(c, (void **)&c->d_split, cap)) return s;
         c->split_bytes = cap;
         p2m_launch_fill_u32((uint32_t *)c->d_split, (int64_t)(cap / 4), 0u, c->stream);
     }
@@ -820,7 +833,7 @@ static int paint_halos(p2m_ctx *c, int64_t n_halo, int64_t n_flat, unsigned long
         if ((int64_t)n_pairs > c->pair_cap || !c->d_keys) {
             dfree(c->d_keys); c->d_keys = nullptr; c->d_vals = nullptr; c->pair_cap = 0;
             const int64_t cap = ((int64_t)(n_pairs * 1.125) + 1024 + 63) & ~(int64_t)63;
-            if (dmalloc((void **)&c->d_keys, sizeof(uint32_t) * 4 * cap)) return P2M_E_NOMEM;
+            if (grow(c, (void **)&c->d_keys, sizeof(uint32_t) * 4 * cap)) return P2M_E_NOMEM;
             c->d_vals = c->d_keys + 2 * cap;
             c->pair_cap = cap;
         }
@@ -851,7 +864,7 @@ static int paint_halos(p2m_ctx *c, int64_t n_halo, int64_t n_flat, unsigned long
             if (p2m_sort_pairs(c->d_keys, c->d_vals, n_pairs, c->n_tiles, nullptr, &need, c->stream)) return P2M_E_HIP;
             if (need > c->sort_tmp_bytes || !c->d_sort_tmp) {
                 dfree(c->d_sort_tmp); c->d_sort_tmp = nullptr; c->sort_tmp_bytes = 0;
-                if (dmalloc(&c->d_sort_tmp, need + 256)) return P2M_E_NOMEM;
+                if (grow(c, &c->d_sort_tmp, need + 256)) return P2M_E_NOMEM;
                 c->sort_tmp_bytes = need + 256;
             }
             size_t bytes = c->sort_tmp_bytes;
@@ -872,7 +885,7 @@ static int paint_halos(p2m_ctx *c, int64_t n_halo, int64_t n_flat, unsigned long
             }
             if (need != c->fb_cap && (need > c->fb_cap || getenv("P2M_FB_CAP"))) {
                 dfree(c->d_fb); c->d_fb = nullptr; c->fb_cap = 0;
-                if (dmalloc((void **)&c->d_fb, sizeof(uint4) * need)) return P2M_E_NOMEM;
+                if (grow(c, (void **)&c->d_fb, sizeof(uint4) * need)) return P2M_E_NOMEM;
                 c->fb_cap = need;
             }
         }
@@ -957,14 +970,14 @@ static int launch_flat(p2m_ctx *c, int64_t n_flat, hipStream_t s)
         if (!c->d_fs_cnt) {
             const int64_t cap = f.n_tiles * p2m_flat_slices(f.n_tiles, INT64_MAX) + 1;
             dfree(c->d_fs_off); c->d_fs_off = nullptr;
-            if (dmalloc((void **)&c->d_fs_off, sizeof(unsigned long long) * cap)) return P2M_E_NOMEM;
-            if (dmalloc((void **)&c->d_fs_cnt, sizeof(uint32_t) * cap)) return P2M_E_NOMEM;
+            if (grow(c, (void **)&c->d_fs_off, sizeof(unsigned long long) * cap)) return P2M_E_NOMEM;
+            if (grow(c, (void **)&c->d_fs_cnt, sizeof(uint32_t) * cap)) return P2M_E_NOMEM;
             p2m_launch_fill_u32(c->d_fs_cnt, cap, 0u, s);
         }
         if (pairs > c->fs_cap || !c->d_fs_pairs) {
             dfree(c->d_fs_pairs); c->d_fs_pairs = nullptr; c->fs_cap = 0;
             const int64_t cap = pairs + pairs / 8 + 1024;
-            if (dmalloc((void **)&c->d_fs_pairs, sizeof(uint2) * cap)) return P2M_E_NOMEM;
+            if (grow(c, (void **)&c->d_fs_pairs, sizeof(uint2) * cap)) return P2M_E_NOMEM;
             c->fs_cap = cap;
         }
         f.cnt = c->d_fs_cnt; f.off = c->d_fs_off; f.pairs = c->d_fs_pairs; f.pair_cap = (unsigned long long)c->fs_cap;
@@ -1016,7 +1029,7 @@ static int repaint_lost(p2m_ctx *c, unsigned long long h[Ctr::TOTAL], unsigned l
         }
         const int64_t cap = (int64_t)P2M_SHARDS * (int64_t)(demand + 64);
         dfree(c->d_fb); c->d_fb = nullptr; c->fb_cap = 0;
-        if (dmalloc((void **)&c->d_fb, sizeof(uint4) * cap)) return P2M_E_NOMEM;
+        if (grow(c, (void **)&c->d_fb, sizeof(uint4) * cap)) return P2M_E_NOMEM;
         c->fb_cap = cap;
         p2m_launch_clear_ctr(pc, 6, 1, c->stream);
         p2m_launch_clear_ctr(c->d_ctr, Ctr::LOST, 1, c->stream);
@@ -1112,7 +1125,7 @@ static int pass_begin(p2m_ctx *c, int64_t n_total)
     }
     if (n_total > 0 && n_total > c->cand_cap) {
         dfree(c->d_cand); c->d_cand = nullptr; c->cand_cap = 0;
-        if (dmalloc((void **)&c->d_cand, sizeof(uint32_t) * n_total)) return P2M_E_NOMEM;
+        if (grow(c, (void **)&c->d_cand, sizeof(uint32_t) * n_total)) return P2M_E_NOMEM;
         c->cand_cap = n_total;
     }
     p2m_launch_fill_u64(c->d_ctr, Ctr::ALL, c->stream);
@@ -1148,8 +1161,8 @@ static int pass_push_impl(p2m_ctx *c, const float *src, bool on_device, int64_t 
             dfree(c->d_slot[0]); dfree(c->d_slot[1]);
             c->d_slot[0] = c->d_slot[1] = nullptr; c->slot_cap = 0;
             const int64_t cap = std::max<int64_t>(piece, 1 << 16);
-            if (dmalloc((void **)&c->d_slot[0], sizeof(float) * 7 * cap)) return P2M_E_NOMEM;
-            if (dmalloc((void **)&c->d_slot[1], sizeof(float) * 7 * cap)) return P2M_E_NOMEM;
+            if (grow(c, (void **)&c->d_slot[0], sizeof(float) * 7 * cap)) return P2M_E_NOMEM;
+            if (grow(c, (void **)&c->d_slot[1], sizeof(float) * 7 * cap)) return P2M_E_NOMEM;
             c->slot_cap = cap;
             c->n_pieces = 0;
         }
@@ -1316,26 +1329,51 @@ static int copy_out(p2m_ctx *c, void *dst, const void *src, size_t bytes)
 
 /* A device map to host memory in the other precision: converted on the
  * device, 2^24 values at a time through a buffer that the context keeps, and
- * copied straight to the caller's memory.  (Copied to a host vector first and
- * converted there, a 4096 x 4096 flat map took 36 ms; 1.2 ms now, the copy.) */
-static int copy_converted(p2m_ctx *c, void *dst, const void *src, int64_t n, bool to_double)
-{
-    const int64_t piece = std::min<int64_t>(n, 1 << 24);
-    if (piece > c->conv_cap) {
+ * copied straight to the caller's memory; less at a time, or by the host, where
+ * device memory is short.  (Copied to a host vector first and converted there,
+ * a 4096 x 4096 flat map took 36 ms; 1.2 ms now, the copy.) */
+namespace {
+struct ConvertOps {
+    p2m_ctx *c;
+    char *dst;
+    const char *src;
+    bool to_double;
+    size_t in() const { return to_double ? sizeof(float) : sizeof(double); }
+    size_t out() const { return to_double ? sizeof(double) : sizeof(float); }
+    bool buffer(int64_t k)
+    {
+        if (k <= c->conv_cap) return true;
         dfree(c->d_conv); c->d_conv = nullptr; c->conv_cap = 0;
-        if (dmalloc(&c->d_conv, sizeof(double) * piece)) return P2M_E_NOMEM;
-        c->conv_cap = piece;
+        if (dmalloc(&c->d_conv, sizeof(double) * k)) return false;
+        c->conv_cap = k;
+        return true;
     }
-    const size_t size = to_double ? sizeof(double) : sizeof(float);
-    for (int64_t i = 0; i < n; i += piece) {
-        const int64_t k = std::min(piece, n - i);
+    int on_device(int64_t i, int64_t k)
+    {
         if (to_double) p2m_launch_f32_to_f64((const float *)src + i, (double *)c->d_conv, k, c->stream);
         else p2m_launch_f64_to_f32((const double *)src + i, (float *)c->d_conv, k, c->stream);
         HIPCHK(hipGetLastError());
-        int rc = copy_out(c, (char *)dst + size * i, c->d_conv, size * k);
-        if (rc) return rc;
+        return copy_out(c, dst + out() * i, c->d_conv, out() * k);
     }
-    return 0;
+    int on_host(int64_t i, int64_t k)
+    {
+        void *h = malloc(in() * k);
+        if (!h) return P2M_E_NOMEM;
+        const int rc = copy_out(c, h, src + in() * i, in() * k);
+        for (int64_t j = 0; !rc && j < k; ++j) {
+            if (to_double) ((double *)dst)[i + j] = (double)((const float *)h)[j];
+            else ((float *)dst)[i + j] = (float)((const double *)h)[j];
+        }
+        free(h);
+        return rc;
+    }
+};
+}  // namespace
+
+static int copy_converted(p2m_ctx *c, void *dst, const void *src, int64_t n, bool to_double)
+{
+    ConvertOps o = {c, (char *)dst, (const char *)src, to_double};
+    return convert_out(o, n, 1 << 24, 1 << 16);
 }
 
 static int fetch_map(p2m_ctx *c, const float *d32, const double *d64, int64_t n, float *h32, double *h64)
@@ -1615,7 +1653,7 @@ static int write_fits_dev(p2m_ctx *c, int slot, const char *path)
         (void)hipGetLastError();
         rc = P2M_E_NOMEM;
     }
-    if (!rc && c->d_hp64[slot] && dmalloc((void **)&d32, sizeof(float) * 2 * piece)) rc = P2M_E_NOMEM;
+    if (!rc && c->d_hp64[slot] && grow(c, (void **)&d32, sizeof(float) * 2 * piece)) rc = P2M_E_NOMEM;
     if (!rc && (hipEventCreateWithFlags(&ev[0], hipEventDisableTiming) != hipSuccess ||
                 hipEventCreateWithFlags(&ev[1], hipEventDisableTiming) != hipSuccess)) {
         (void)hipGetLastError();
