@@ -906,6 +906,7 @@ static int paint_halos(p2m_ctx *c, int64_t n_halo, int64_t n_flat, unsigned long
         t.count = c->d_count; t.hash = c->d_hash; t.counters = pc;
         t.wide = 2 * n_pix > (n_pairs << (c->shape.log2r + c->shape.log2c));      /* half a tile a pair */
         t.vectors = p2m_exact_vectors(c->cfg.n_maps, c->log2w, c->d_count != nullptr, wg);
+        c->last_wg = wg;
         if (p2m_launch_tile_paint(t, mode, c->cfg.n_maps, grid, wg, c->stream)) return P2M_E_INVALID;
         HIPCHK(hipGetLastError());
         HIPCHK(hipEventRecord(c->ev[7], c->stream));
@@ -920,7 +921,7 @@ static int paint_halos(p2m_ctx *c, int64_t n_halo, int64_t n_flat, unsigned long
             f.lost = c->d_lost; f.desc = c->d_tile_desc; f.n_tiles = c->n_tiles; f.n_halo = n_halo;
             f.err = c->d_ctr + Ctr::ERR;
             if (p2m_launch_fallback(f, (int64_t)(n_pix / 256) + 1024, c->stream)) return P2M_E_HIP;
-            c->last_t = t; c->last_f = f; c->last_grid = grid; c->last_wg = wg; 
+            c->last_t = t; c->last_f = f; c->last_grid = grid;
         }
         c->last_fast = mode == P2M_PREC_FP32_COMP;
         HIPCHK(hipEventRecord(c->ev[4], c->stream));
@@ -1111,7 +1112,8 @@ static int finish_stats(p2m_ctx *c)
         (void)hipEventElapsedTime(&ms, c->ev[3], c->ev[7]); s.ms_tile = ms;
     }
     s.tile_w = c->log2w ? (1 << c->log2w) : 0;
-    s.tile_wg = c->wg;
+    /* as launched: fewer waves than set where no more fit (p2m_tile_wg) */
+    s.tile_wg = c->cfg.precision != P2M_PREC_PLAIN_FP64 && c->cfg.nside > 0 ? c->last_wg : c->wg;
     return 0;
 }
 
@@ -1444,7 +1446,7 @@ int p2m_fetch_membership(p2m_ctx *c, uint32_t *hc, uint64_t *hh, uint32_t *fc, u
  * halos already decoded, keeps the fastest, and restores the maps. */
 static int autotune(p2m_ctx *c, int64_t n_halo, int64_t n_flat, unsigned long long n_pix)
 {
-    static const int cand[][2] = {{9, 256}, {10, 256}, {11, 256}, {11, 128}, {12, 256}};
+    static const int cand[][2] = {{9, 256}, {10, 256}, {11, 256}, {11, 128}};
     int mode_ld = c->cfg.precision == P2M_PREC_FP64 ? 1 : 2;
     int best_l = 10, best_wg = 256;
     /* small problems: the default shape */
@@ -1463,20 +1465,24 @@ static int autotune(p2m_ctx *c, int64_t n_halo, int64_t n_flat, unsigned long lo
         return 0;
     }
     float best_ms = 1e30f;
+    int tried_l = 0, tried_wg = 0;
     for (auto &cd : cand) {
-        if (cd[0] > p2m_tile_max_log2w()) continue;
         if (p2m_tile_lds_bytes(mode_ld, c->cfg.n_maps, cd[0], c->d_count != nullptr, c->g.nrt, 64) > 160 * 1024) continue;
+        /* the workgroup that would be launched; the same as the last trial's
+         * where LDS holds no more waves */
+        const int wg = p2m_tile_wg(mode_ld, c->cfg.n_maps, cd[0], c->d_count != nullptr, c->g.nrt, cd[1]);
+        if (cd[0] == tried_l && wg == tried_wg) continue;
+        tried_l = cd[0]; tried_wg = wg;
         int rc = build_tiles(c, cd[0]); if (rc) return rc;
-        c->wg = cd[1]; c->tuned = true;
+        c->wg = wg; c->tuned = true;
         c->hp_zero = true;
         /* each trial starts from zero paint counters, as a call does: the
          * deferred-pixel and overflow lists are appended at their counters */
         p2m_launch_clear_ctr(c->d_ctr, Ctr::PAINT, Ctr::TOTAL - Ctr::PAINT, c->stream);
         rc = paint_halos(c, n_halo, n_flat, n_pix, false);
         if (rc == P2M_E_INVALID) {
-            /* a shape the painter rejects at launch: the trial's flat-sky
-             * paint is still on its stream, so the clear waits for it */
-            HIPCHK(hipStreamWaitEvent(c->stream, c->ev_fs, 0));
+            /* a shape the painter rejects at launch, before the trial's
+             * flat-sky paint is queued */
             (void)p2m_clear(c);
             continue;
         }
@@ -1484,7 +1490,7 @@ static int autotune(p2m_ctx *c, int64_t n_halo, int64_t n_flat, unsigned long lo
         HIPCHK(hipStreamSynchronize(c->stream));
         float ms = 0;
         (void)hipEventElapsedTime(&ms, c->ev[2], c->ev[4]);
-        if (ms < best_ms) { best_ms = ms; best_l = cd[0]; best_wg = cd[1]; }
+        if (ms < best_ms) { best_ms = ms; best_l = cd[0]; best_wg = wg; }
         rc = p2m_clear(c); if (rc) return rc;
         /* a trial's tiles that lost deferred pixels are not repainted: the
          * maps are cleared anyway, and so are the marks */
