@@ -94,7 +94,8 @@ struct p2m_ctx {
     hipStream_t fs_stream = nullptr;            /* the flat-sky painter, beside the binning */
     hipEvent_t ev_dec = nullptr, ev_fs = nullptr;
     unsigned long long *h_pin = nullptr;   /* pinned host words for mid-call readbacks */
-    char *h_prod = nullptr;                /* pinned host copy of the products' scratch */
+    char *h_prod = nullptr;                /* host copy of the products' scratch, pinned if that is to be had */
+    bool prod_pinned = true;
     char *d_prod = nullptr;                /* the products' scratch */
     bool have_run = false;
     bool have_table[P2M_MAXMAPS] = {false};
@@ -360,7 +361,9 @@ int p2m_create(p2m_ctx **out, const p2m_config *cfg)
     }
     if (hipHostMalloc((void **)&c->h_prod, P2M_PROD_BYTES + P2M_PROD_PART_BYTES, hipHostMallocDefault) != hipSuccess) {
         (void)hipGetLastError();
-        c->h_prod = nullptr;
+        c->prod_pinned = false;
+        c->h_prod = (char *)malloc(P2M_PROD_BYTES + P2M_PROD_PART_BYTES);
+        if (!c->h_prod) { p2m_destroy(c); return P2M_E_NOMEM; }
     }
     c->hpnpix = cfg->nside > 0 ? 12LL * cfg->nside * cfg->nside : 0;
     c->fsnpix = (int64_t)cfg->npix_fs * cfg->npix_fs;
@@ -419,7 +422,8 @@ void p2m_destroy(p2m_ctx *c)
     dfree(c->d_hot); dfree(c->d_pair_halo); dfree(c->d_keys); dfree(c->d_sort_tmp);
     for (int i = 0; i < 10; ++i) if (c->ev[i]) (void)hipEventDestroy(c->ev[i]);
     if (c->h_pin) (void)hipHostFree(c->h_pin);
-    if (c->h_prod) (void)hipHostFree(c->h_prod);
+    if (c->h_prod && c->prod_pinned) (void)hipHostFree(c->h_prod);
+    if (!c->prod_pinned) free(c->h_prod);
     dfree(c->d_prod); dfree(c->d_conv);
     if (c->ev_dec) (void)hipEventDestroy(c->ev_dec);
     if (c->ev_fs) (void)hipEventDestroy(c->ev_fs);
@@ -1516,8 +1520,7 @@ static int products(p2m_ctx *c, int slot, char *scratch, double moments[6], doub
     if (slot < 0 || slot >= c->cfg.n_maps) return P2M_E_INVALID;
     HIPCHK(hipSetDevice(c->cfg.device));
     { int rc = ensure_hp_valid(c); if (rc) return rc; }
-    char hbuf[P2M_PROD_BYTES + P2M_PROD_PART_BYTES];
-    char *h = c->h_prod ? c->h_prod : hbuf;
+    char *h = c->h_prod;
     unsigned long long *d_hist = (unsigned long long *)scratch;
     double *d_part = (double *)(scratch + P2M_PROD_PART_OFF);
     const float dy = 1e-4f / (float)P2M_NDPDY;                 /* pks2map.f90:39-40 */
