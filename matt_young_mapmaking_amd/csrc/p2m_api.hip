@@ -233,18 +233,6 @@ static double host_lookup(const std::vector<double> &t, double tmin, double dt, 
 
 static bool is_pow2(int32_t x) { return x > 0 && (x & (x - 1)) == 0; }
 
-/* Rows and columns of a tile of up to 2^log2w pixels: at most 16 rings, 64
- * pixels along each at the default 1024.  A map of few tiles (nside 128 and
- * below at that size) takes fewer rings per tile, so that there are tiles for
- * the CUs. */
-static TileShape tile_shape(int32_t nside, int log2w)
-{
-    TileShape g = {nside, log2w / 2 - 1 < 4 ? log2w / 2 - 1 : 4, 0};
-    g.log2c = log2w - g.log2r;
-    while (g.log2r > 0 && (12LL * nside * nside) >> (g.log2r + g.log2c) < 2048) --g.log2r;
-    return g;
-}
-
 static int build_tiles(p2m_ctx *c, int log2w)
 {
     int32_t ns = c->cfg.nside;

@@ -207,6 +207,18 @@ struct TileShape {
     int32_t nside, log2r, log2c;
 };
 
+/* Rows and columns of a tile of up to 2^log2w pixels: at most 16 rings, 64
+ * pixels along each at the default 1024.  A map of few tiles (nside 128 and
+ * below at that size) takes fewer rings per tile, so that there are tiles for
+ * the CUs. */
+P2M_HD TileShape tile_shape(int32_t nside, int log2w)
+{
+    TileShape g = {nside, log2w / 2 - 1 < 4 ? log2w / 2 - 1 : 4, 0};
+    g.log2c = log2w - g.log2r;
+    while (g.log2r > 0 && (12LL * nside * nside) >> (g.log2r + g.log2c) < 2048) --g.log2r;
+    return g;
+}
+
 P2M_HD int32_t n_bands(const TileShape &g) { return ((4 * g.nside - 1) + (1 << g.log2r) - 1) >> g.log2r; }
 
 /* first and last ring of band `band` and its number of sectors */
