@@ -2,10 +2,10 @@
  * p2m_api.hip -- host runtime behind the C ABI of include/pks2map_gpu.h.
  *
  * Owns the device state of one pks2map run: distance tables, profile tables,
- * maps, per-halo records, tile bins.  A paint call decodes the catalogue in
- * chunks (appending painted halos to one device array), bins every
- * (halo, ring) pixel run into ring tiles, and paints all tiles in one launch,
- * so each map pixel is written once per call.
+ * maps, per-halo records, (halo, tile) pairs.  A paint call decodes the
+ * catalogue in chunks (appending painted halos to one device array), lists
+ * the tiles that every disc may reach, sorted by tile, and paints all tiles
+ * in one launch, so each map pixel is written once per call.
  */
 #include <hip/hip_runtime.h>
 
@@ -110,7 +110,6 @@ struct p2m_ctx {
     float *d_flat[P2M_MAXMAPS] = {nullptr};
     float *d_quad = nullptr;                    /* corner-quad table of all maps (tiled painters) */
     int64_t n_flat = 0, n_quad = 0;
-    double *d_inv_node2 = nullptr;
     float *d_inv_node2f = nullptr;
     uint4 *d_fb = nullptr;
     int64_t fb_cap = 0;
@@ -402,7 +401,7 @@ void p2m_destroy(p2m_ctx *c)
     }
     dfree(c->d_quad);
     dfree(c->d_count); dfree(c->d_hash); dfree(c->d_fs_count); dfree(c->d_fs_hash);
-    dfree(c->d_rofz); dfree(c->d_zofr); dfree(c->d_inv_node2); dfree(c->d_inv_node2f); dfree(c->d_fb);
+    dfree(c->d_rofz); dfree(c->d_zofr); dfree(c->d_inv_node2f); dfree(c->d_fb);
     dfree(c->d_halo); dfree(c->d_flat_idx); dfree(c->d_n_pairs); dfree(c->d_pair_off); dfree(c->d_ctr);
     dfree(c->d_band_tile); dfree(c->d_tile_off); dfree(c->d_scan_tmp); dfree(c->d_scan_tmp_fs);
     dfree(c->d_tile_desc); dfree(c->d_ring); dfree(c->d_fs_cnt); dfree(c->d_fs_off); dfree(c->d_fs_pairs);
@@ -572,13 +571,9 @@ int p2m_load_table(p2m_ctx *c, int slot, const int32_t hdr_i[3], const float hdr
         HIPCHK(hipStreamSynchronize(c->stream));
     }
     /* FP32 path constants: node radii, ln r -> cell coordinate */
-    std::vector<double> inv(g.nrt + 2);
-    for (int k = 0; k < g.nrt + 2; ++k) inv[k] = p2m_exp(-2.0 * (g.lr0 + (double)k * g.drt));
     std::vector<float> invf(g.nrt + 2);
-    for (int k = 0; k < g.nrt + 2; ++k) invf[k] = (float)inv[k];
-    if (!c->d_inv_node2 && grow(c, (void **)&c->d_inv_node2, sizeof(double) * (g.nrt + 2))) return P2M_E_NOMEM;
+    for (int k = 0; k < g.nrt + 2; ++k) invf[k] = (float)p2m_exp(-2.0 * (g.lr0 + (double)k * g.drt));
     if (!c->d_inv_node2f && grow(c, (void **)&c->d_inv_node2f, sizeof(float) * (g.nrt + 2))) return P2M_E_NOMEM;
-    HIPCHK(hipMemcpy(c->d_inv_node2, inv.data(), sizeof(double) * (g.nrt + 2), hipMemcpyHostToDevice));
     HIPCHK(hipMemcpy(c->d_inv_node2f, invf.data(), sizeof(float) * (g.nrt + 2), hipMemcpyHostToDevice));
     c->u_k1 = (float)(0.5 * 0.6931471805599453 / g.drt);   /* log2(r^2) -> (ln r)/drt */
     c->u_k0 = (float)(g.lr0 / g.drt);
@@ -720,7 +715,7 @@ static void fs_join(p2m_ctx *c)
 static void table_args(const p2m_ctx *c, TileArgs &t)
 {
     t.n_maps = c->cfg.n_maps; t.profile = c->cfg.profile;
-    t.g = c->g; t.n_flat = c->n_flat; t.inv_node2 = c->d_inv_node2;
+    t.g = c->g; t.n_flat = c->n_flat;
     t.u_k1 = c->u_k1; t.u_k0 = c->u_k0; t.u_max = c->u_max; t.band = c->u_band; t.fr_clamp = c->fr_clamp; t.ir_clamp = c->ir_clamp;
     t.band_c = (float)CHORD_BAND;
     t.inv_node2f = c->d_inv_node2f;
@@ -1071,7 +1066,7 @@ static int finish_stats(p2m_ctx *c)
     }
     if (h[Ctr::ERR]) {
         snprintf(g_hip_detail, sizeof(g_hip_detail),
-                 "%llu device-side range checks failed (segment, tile slot or deferred entry out of range)",
+                 "%llu device-side range checks failed (pair, tile or deferred entry out of range)",
                  h[Ctr::ERR]);
         return P2M_E_INTERNAL;
     }

@@ -176,8 +176,8 @@ P2M_HD void ring_info(int32_t nside, int32_t ring, int32_t &npr, int32_t &kshift
 /* Ring tiles: ring `ring` is cut into ceil(npr / W) tiles of W = 2^log2w
  * consecutive RING pixels, the last one narrower.  Tile `col` starts at
  * in-ring pixel ip0 = col W, holds `width` pixels, and its first map pixel is
- * first + ip0 (first: the ring's first pixel).  The painters' own tiles are
- * bands of rings by sectors, below. */
+ * first + ip0 (first: the ring's first pixel).  Host checks of the ring
+ * geometry use them; the painters' tiles are bands of rings by sectors, below. */
 P2M_HD int32_t ring_tiles(int32_t nside, int32_t ring, int32_t log2w)
 {
     int32_t npr, kshift;

@@ -130,8 +130,7 @@ struct TileArgs {
                                      cell, 4 corners of every map, are 8 n_maps contiguous floats */
     int64_t n_quad;               /* floats in tab_q */
     int64_t n_flat;
-    const double *inv_node2;      /* exp(-2 (lr0 + k drt)), k = 0..nrt */
-    const float *inv_node2f;      /* the same in float */
+    const float *inv_node2f;      /* exp(-2 (lr0 + k drt)), k = 0..nrt */
     float u_k1, u_k0, u_max, band, fr_clamp;
     double inv_drt, u_max64, band64, fr_clamp64;     /* the FP64 painter's: 1/drt, nrt - 1, the band around cell
                                                         boundaries (in cells) that takes the exact arithmetic */

@@ -49,10 +49,6 @@ __device__ static inline void pin4(uint4 v)
 {
     asm volatile("" ::"v"(v.x), "v"(v.y), "v"(v.z), "v"(v.w));
 }
-__device__ static inline void pin2(uint2 v)
-{
-    asm volatile("" ::"v"(v.x), "v"(v.y));
-}
 
 __global__ void k_fill_u32(uint32_t *p, int64_t n, uint32_t v)
 {
@@ -679,8 +675,8 @@ int p2m_sort_pairs(uint32_t *keys, uint32_t *vals, unsigned long long n, int64_t
     return e == hipSuccess ? 0 : -1;
 }
 
-/* exclusive scan of uint32 counts into uint64 offsets with a 64-bit accumulator */
-/* Exclusive scan of up to 16384 counts by one workgroup, consecutive ones a
+/* Exclusive scan of uint32 counts into uint64 offsets with a 64-bit
+ * accumulator.  Up to 16384 counts by one workgroup, consecutive ones a
  * thread: one launch instead of two (2569 counts: 5 us instead of 6 us and the
  * gap between them). */
 #define SCAN_SMALL 16384
@@ -930,7 +926,7 @@ __device__ static inline unsigned long long start_bits(unsigned long long *bits,
 }
 
 /* where wave w of nw (1 to 8) starts in n pairs: equal shares, the last ones
- * shorter; no division but by constants */
+ * shorter; divided by constants up to four waves (all that k_tile_fast takes) */
 __device__ static inline uint32_t wave_share(uint32_t n, int w, int nw)
 {
     uint32_t c;
@@ -1756,8 +1752,9 @@ struct FastWave {
     int32_t cidx[WSEG];            /* wave's pixel number of the azimuth origin: p - cidx = ip - ip_c */
     int32_t colbase[WSEG];
     uint32_t slot[WSEG];           /* halo; ASK_RUN: its deferred pixels must lie in the exact run */
-    int16_t qoff[WSEG];            /* in-tile pixel minus the wave's pixel number (-4096 .. 2047) */
+    int16_t qoff[WSEG];            /* in-tile pixel minus the wave's pixel number (-64 * 128 .. 2047) */
 };
+static_assert(WSEG * 128 <= 32768, "qoff: 64 segments of at most a row of the widest tile");
 
 /* sin^2(x) for |x| <= 2: the odd Taylor polynomial of sin to x^15 (the
  * next term is below 3e-10 there, 6e-12 at pi/2), squared; one branch-free

@@ -105,17 +105,21 @@ __device__ static inline double mt_fit(float A0, float am, float az, double mh, 
  * whose rule of 2 MT_M nodes is symmetric, so MT_M = 8 evaluations do.
  * Against sums in extended precision over b in (0.002, 4) and the profiles'
  * ranges of exponents both agree to 1e-15.  The rest of the last block, of
- * any length up to 256, has a rule of its own length (of at most MT_N points
- * every point itself).
+ * any length, has a rule of its own length (of at most MT_N points every
+ * point itself).
  *
  * Layout: rule N (1..MT_MAXN) holds MT_N pairs (t, w): t = q - 1/2 counted
  * from the block's start; then the half rules of S = 16 * 2^j, MT_M pairs
- * each. */
+ * each.  b is at most MT_RMAX, so S at most 128; the blocks are then of 16 to
+ * 128 points, and the last one starts at 256. */
 #define MT_N 11
 #define MT_M 8
-#define MT_MAXN 256
+#define MT_MAXN 145
 #define MT_S0 16
-#define MT_NSTART 5
+#define MT_NSTART 4
+#define MT_RMAX 4.0                      /* in virial radii, integrate_profiles.f90:12-95 */
+static_assert((MT_S0 << MT_NSTART) * MT_DS > 0.5 * MT_RMAX, "a larger start block than the rules hold");
+static_assert((int)(MT_RMAX / MT_DS) + 1 - 256 <= MT_MAXN && MT_MAXN >= 128, "a longer block than the rules hold");
 #define MT_RULE_DOUBLES (2 * (MT_MAXN * MT_N + MT_NSTART * MT_M))
 
 __device__ static inline double gram_b2(double k, double N)      /* squared off-diagonal of the Jacobi matrix */
@@ -226,8 +230,8 @@ __global__ void __launch_bounds__(64) k_maptable_cells(MTArgs A)
 /* One work item per node, r fastest.  Bound: FP64 VALU.  The reference's
  * two sums take up to 401 points each and five powers a point; here both
  * share their nodes (one square root, three logarithms and three exponentials
- * a node for both) and take 44 to 60 nodes for y, and 11 more for the rest
- * of rho's sum.  A wave takes the start block that its smallest b allows.
+ * a node for both) and take 30 to 71 nodes for y, by the start block, and 11
+ * more for the rest of rho's sum.  A wave takes the start block that its smallest b allows.
  * 100 x 100 x 200 nodes: 0.98 ms (15.9 ms point by point). */
 __global__ void __launch_bounds__(256) k_make_maptable(MTArgs A)
 {
@@ -238,7 +242,7 @@ __global__ void __launch_bounds__(256) k_make_maptable(MTArgs A)
     const int64_t cmi = nd / A.nrt;
     const CellCM c = A.cm[cmi];
     const double b = A.proj[(cmi / A.nmht) * A.nrt + k] / c.rvir;
-    const double rmaxp = 4.0;
+    const double rmaxp = MT_RMAX;
     const bool in = !(b > rmaxp);
     double bmin = in ? b : rmaxp;
     for (int o = 32; o > 0; o >>= 1) bmin = fmin(bmin, __shfl_xor(bmin, o));

@@ -1,7 +1,7 @@
 /* Tile pieces of a ring run: the run [lo, lo+np) of a ring of npr pixels
  * (wrapping past npr to 0) cut at the tile boundaries of width 2^log2w.
- * Host and device code share these, so the enumeration order used to
- * assign segment slots is the one used to write the segments. */
+ * No kernel cuts runs like this (the painters clip a run to the rows of their
+ * tiles, clip_run); the host checks of run geometry use it. */
 #ifndef P2M_PIECES_H
 #define P2M_PIECES_H
 
