@@ -93,10 +93,12 @@ struct p2m_ctx {
     hipEvent_t ev[10] = {};
     hipStream_t fs_stream = nullptr;            /* the flat-sky painter, beside the binning */
     hipEvent_t ev_dec = nullptr, ev_fs = nullptr;
-    unsigned long long *h_pin = nullptr;   /* pinned host words for mid-call readbacks */
-    char *h_prod = nullptr;                /* host copy of the products' scratch, pinned if that is to be had */
-    bool prod_pinned = true;
-    char *d_prod = nullptr;                /* the products' scratch */
+    /* one host block, page-locked if that is to be had, of words for readbacks
+     * and of a copy of the products' scratch */
+    unsigned long long *h_pin = nullptr;
+    char *h_prod = nullptr;
+    bool host_pinned = true;
+    char *d_prod = nullptr;                /* the products' scratch, in d_ctr's allocation */
     bool have_run = false;
     bool have_table[P2M_MAXMAPS] = {false};
     p2m_run run;
@@ -342,16 +344,14 @@ int p2m_create(p2m_ctx **out, const p2m_config *cfg)
         int e = scratch_for_device(cfg->device, &sp);
         if (e) { p2m_destroy(c); return e; }
     }
-    if (hipHostMalloc((void **)&c->h_pin, sizeof(unsigned long long) * (Ctr::ALL + 8), hipHostMallocDefault) != hipSuccess) {
+    const size_t pin_bytes = sizeof(unsigned long long) * (Ctr::ALL + 8), host_bytes = pin_bytes + P2M_PROD_BYTES + P2M_PROD_PART_BYTES;
+    if (hipHostMalloc((void **)&c->h_pin, host_bytes, hipHostMallocDefault) != hipSuccess) {
         (void)hipGetLastError();
-        c->h_pin = nullptr;
+        c->host_pinned = false;
+        c->h_pin = (unsigned long long *)malloc(host_bytes);
+        if (!c->h_pin) { p2m_destroy(c); return P2M_E_NOMEM; }
     }
-    if (hipHostMalloc((void **)&c->h_prod, P2M_PROD_BYTES + P2M_PROD_PART_BYTES, hipHostMallocDefault) != hipSuccess) {
-        (void)hipGetLastError();
-        c->prod_pinned = false;
-        c->h_prod = (char *)malloc(P2M_PROD_BYTES + P2M_PROD_PART_BYTES);
-        if (!c->h_prod) { p2m_destroy(c); return P2M_E_NOMEM; }
-    }
+    c->h_prod = (char *)c->h_pin + pin_bytes;
     c->hpnpix = cfg->nside > 0 ? 12LL * cfg->nside * cfg->nside : 0;
     c->fsnpix = (int64_t)cfg->npix_fs * cfg->npix_fs;
     int rc = 0;
@@ -372,8 +372,8 @@ int p2m_create(p2m_ctx **out, const p2m_config *cfg)
             rc |= dmalloc((void **)&c->d_fs_hash, sizeof(unsigned long long) * c->fsnpix);
         }
     }
-    if (!rc) rc |= dmalloc((void **)&c->d_ctr, sizeof(unsigned long long) * Ctr::ALL);
-    if (!rc) rc |= dmalloc((void **)&c->d_prod, P2M_PROD_BYTES);
+    if (!rc) rc |= dmalloc((void **)&c->d_ctr, sizeof(unsigned long long) * Ctr::ALL + P2M_PROD_BYTES);
+    if (!rc) c->d_prod = (char *)(c->d_ctr + Ctr::ALL);
     if (rc) { p2m_destroy(c); return P2M_E_NOMEM; }
     *out = c;
     int e = p2m_clear(c);
@@ -408,10 +408,9 @@ void p2m_destroy(p2m_ctx *c)
     dfree(c->d_cand);
     dfree(c->d_hot); dfree(c->d_pair_halo); dfree(c->d_keys); dfree(c->d_sort_tmp);
     for (int i = 0; i < 10; ++i) if (c->ev[i]) (void)hipEventDestroy(c->ev[i]);
-    if (c->h_pin) (void)hipHostFree(c->h_pin);
-    if (c->h_prod && c->prod_pinned) (void)hipHostFree(c->h_prod);
-    if (!c->prod_pinned) free(c->h_prod);
-    dfree(c->d_prod); dfree(c->d_conv);
+    if (c->h_pin && c->host_pinned) (void)hipHostFree(c->h_pin);
+    if (!c->host_pinned) free(c->h_pin);
+    dfree(c->d_conv);
     if (c->ev_dec) (void)hipEventDestroy(c->ev_dec);
     if (c->ev_fs) (void)hipEventDestroy(c->ev_fs);
     if (c->fs_stream) (void)hipStreamDestroy(c->fs_stream);
@@ -642,7 +641,7 @@ static int scan_counts(p2m_ctx *c, const uint32_t *cnt, unsigned long long *off,
 /* counter block summed over its shards (blocks until the stream is idle) */
 static int read_counters(p2m_ctx *c, unsigned long long out[Ctr::TOTAL], unsigned long long *raw = nullptr)
 {
-    unsigned long long hbuf[Ctr::ALL], *h = c->h_pin ? c->h_pin : hbuf;
+    unsigned long long *h = c->h_pin;
     HIPCHK(hipMemcpyAsync(h, c->d_ctr, sizeof(*h) * Ctr::ALL, hipMemcpyDeviceToHost, c->stream));
     HIPCHK(hipStreamSynchronize(c->stream));
     if (raw) memcpy(raw, h, sizeof(*h) * Ctr::ALL);
@@ -810,10 +809,9 @@ static int paint_halos(p2m_ctx *c, int64_t n_halo, int64_t n_flat, unsigned long
         if (recount) p2m_launch_pair_count(b, c->stream);
         if (n_halo > 0) { int rc = scan_counts(c, c->d_n_pairs, c->d_pair_off, n_halo + 1); if (rc) return rc; }
         if (recount && n_halo > 0) {
-            unsigned long long hv = 0, *hp = c->h_pin ? c->h_pin : &hv;
-            HIPCHK(hipMemcpyAsync(hp, c->d_pair_off + n_halo, sizeof(*hp), hipMemcpyDeviceToHost, c->stream));
+            HIPCHK(hipMemcpyAsync(c->h_pin, c->d_pair_off + n_halo, sizeof(*c->h_pin), hipMemcpyDeviceToHost, c->stream));
             HIPCHK(hipStreamSynchronize(c->stream));
-            c->counted_pairs = *hp;
+            c->counted_pairs = *c->h_pin;
         }
         c->counted_log2w = c->log2w;
         const unsigned long long n_pairs = c->counted_pairs;
