@@ -87,7 +87,7 @@ typedef struct {
      * of (halo, tile) pairs, sorted by tile), healpix painting, flat-sky painting (the tiled
      * modes run it on a second stream beside the binning) */
     double  ms_total, ms_decode, ms_bin, ms_paint, ms_finish;
-    int32_t tile_w, tile_wg;  /* tile shape used (autotuned or set) */
+    int32_t tile_w, tile_wg;  /* tile shape painted with: pixels (autotuned or set), lanes as launched */
     double  ms_tile;          /* the tile painter kernel alone, within ms_paint (0 for plain FP64) */
     /* catalogue handed over in host memory: bytes copied to the device, the
      * copy stream's time from the call's start to its last copy, and whether
